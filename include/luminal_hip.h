@@ -195,7 +195,7 @@ lhip_status lhip_q8_0_matvec_fused_f32_cfg(const void *const *planar_dev, float 
  * launch.  Every such call on a device shares that array: calls with m <= 128 that
  * may overlap on one device (different streams, different host threads) race on it
  * and must be ordered by the caller.  Results do not depend on timing.
- * Above 128 rows the same array holds the planes of the K-sliced plans (few 256x128 tiles and a long K; the column
+ * Above 128 rows the same array holds the planes of the K-sliced plans (few 128x256 tiles; the column
  * tiles that more than 256 tiles leave over after whole rounds of 256 workgroups: tile ids 120 + S and 200 of
  * lhip_q8_0_matmul_bf16_cfg), so the same rule applies to every shape for which
  * lhip_q8_0_matmul_bf16_workspace_nbytes is not zero; lhip_q8_0_matmul_bf16_ws takes the planes from the caller
@@ -212,19 +212,20 @@ lhip_status lhip_q8_0_matmul_bf16_f32out(const void *planar_dev, const void *x_d
  * lhip_q8_0_matmul_bf16_f32out followed by lhip_swiglu_f32_bf16out(interleaved).  N % 4 == 0. */
 lhip_status lhip_q8_0_matmul_bf16_swiglu(const void *planar_dev, const void *x_dev, void *out_dev, int64_t m, int64_t n,
                                          int64_t k, void *stream);
-/* Same with the output tile chosen by the caller: tile 0 = 256x128 (8 waves),
- * 1 = 128x128, 2 = 128x64, 3 = 64x64 (4 waves each),
+/* Same with the output tile chosen by the caller: tile 0 = the large tiles, 256x256 and 128x256 (8 waves; the library
+ * cuts N between the two heights so that the last round of workgroups ends early), 1 = 128x128, 2 = 128x64,
+ * 3 = 64x64 (4 waves each),
  * 5 = the weight-streaming kernel described above, here for any m <= 8192 in passes of 128 rows
  * (LHIP_ERR_UNSUPPORTED for shapes it does not cover),
- * 50 + S = the same with S slices of K (S clamped to K / 512), 120 + S = the 256x128
+ * 50 + S = the same with S slices of K (S clamped to K / 512), 120 + S = the 128x256
  * tile over S slices of K with the partial sums in the same scratch array (2 <= S <= 16,
- * K / 64 / S a whole multiple of 4, S * m * N <= 8 Mi; what the plain entry
- * points take for K >= 8192 when whole-K tiles would leave most of the chip idle, so
+ * K / 64 / S a whole multiple of 4, S * m * N <= 8 Mi; the plain entry points take two to eight slices, even or not,
+ * when whole-K tiles would leave most of the chip idle, so
  * the note on overlapping calls above applies to those shapes too),
- * 200 = the 256x128 tile in whole rounds of 256 workgroups and the column tiles left over in 2 to 8 slices of K
- * through the same scratch array (what the plain entry points take when more than 256 tiles would end in a
- * partly filled round: K >= 2048, the number of 256-row tiles a divisor of 256; LHIP_ERR_UNSUPPORTED where there
- * is no such remainder). */
+ * 200 = more than 256 tiles of 128x256 that would end in a partly filled round of workgroups, in whichever of two ways
+ * ends first: tile 0, or whole rounds and the column tiles left over in 2 to 8 slices of K
+ * through the same scratch array (K >= 2048, the number of 256-row tiles a divisor of 256; LHIP_ERR_UNSUPPORTED where
+ * there is no such remainder; a workspace of the recommended size holds the slices whether they are taken or not). */
 lhip_status lhip_q8_0_matmul_bf16_cfg(const void *planar_dev, const void *x_dev, void *y_dev, int64_t m, int64_t n,
                                       int64_t k, int tile, void *stream);
 

@@ -1,46 +1,40 @@
 // Q8_0 GEMM for prefill:  Y[M][N] = X[M][K] . W[N][K]^T, bf16 activations,
-// f32 accumulation on the matrix cores, bf16 output.
+// f32 accumulation on the matrix cores, bf16 (or f32, or SwiGLU) output: the choice of the kernel per shape, and the
+// tile kernel for small products.
 //
 // The reference has no such kernel on CUDA (its QuantizedMatmul re-runs the
 // matvec once per activation row, crates/luminal_cuda/src/quantized.rs:146-164);
 // the design precedent is the Metal backend's GEMM, which dequantises a weight
 // tile into threadgroup memory and feeds the matrix unit
 // (crates/luminal_metal/src/quantized.rs:54-61,63-199).  That kernel rounds
-// q * d to the activation type first; this one keeps the weights exact:
-//   * a workgroup owns a BM x BN output tile and walks K in steps of 64 (two
-//     Q8_0 blocks);
-//   * activations go global -> registers -> LDS as bf16; weight codes go global
-//     (planar int8, 16-byte loads) -> registers -> bf16 (an int8 is exact in
-//     bf16: one sign-extending byte conversion and a pack) -> LDS, and the two
-//     block scales of the K tile go to LDS as f32;
-//   * LDS is double-buffered and the global loads run D tiles ahead in
-//     rotating register sets; one barrier per tile separates LDS writers from
-//     readers;
-//   * each wavefront computes a 64 x 64 sub-tile with v_mfma_f32_32x32x16_bf16:
-//     a Q8_0 block is two chained steps into a zeroed accumulator, and the
-//     block's scale multiplies that f32 block sum, acc += d * sum, the
-//     arithmetic of the matvec kernels (quantized.rs:93-96: sumf += sumq * d);
-//     LDS rows are padded by 16 bytes so the 16-byte operand reads of 8
-//     consecutive lanes hit all banks once;
-//   * workgroups that share a weight tile (same N tile, different M tiles) get
-//     consecutive slots on the same XCD (block id modulo 8), so the weight tile
-//     is fetched from HBM once and re-read from that XCD's L2; the M tiles are
-//     walked in groups of 8, so that the activation tiles of a group stay in
-//     that L2 while the XCD's N tiles pass.  What the counters show fetched
-//     beyond the algorithmic bytes is activations (every XCD reads all of X for
-//     each round of its N tiles), not weights.
+// q * d to the activation type first; these keep the weights exact: the int8
+// codes go to the matrix cores as they are (exact in bf16) and the block's scale
+// multiplies the f32 sum of the block's products.  Three kernels share the shapes:
+//   * at most 128 rows: q8_gemm_skinny.hip, bound by streaming the weights;
+//   * more rows: q8_gemm_wide.hip, tiles of 256x256 and 128x256, over slices of K
+//     where those are few;
+//   * more rows but too few such tiles and a K too short to slice: the kernel in
+//     this file, tiles of 128x128 down to 64x64 by four waves.
+// The kernel in this file walks K in steps of 64 (two Q8_0 blocks); activations go
+// global -> registers -> LDS as bf16, codes global -> registers -> bf16 (one
+// sign-extending byte conversion and a pack) -> LDS, the two block scales of the K
+// tile to LDS as f32; LDS is double-buffered and the global loads run D tiles ahead
+// in rotating register sets; a block is two chained v_mfma_f32_32x32x16_bf16 into a
+// zeroed accumulator; LDS rows are padded by 16 bytes so the 16-byte operand reads
+// of 8 consecutive lanes hit all banks once.
 // With bf16 activations every product is exact, so the only roundings are those
 // of the f32 additions (and the one of the bf16 store).  Rounding q * d to bf16
 // instead leaves a relative error of 2^-9 per weight, proportional to the sum
 // of |w x| and therefore large on every output that cancels: measured 3.5 to
 // 5.1 under max |y - t| / max(|t|, 1e-3 rms(t)) on the Llama-3-8B shapes, where
-// this kernel scores 3.9e-3 (the bf16 store alone) and 1e-4 to 5e-4 on its f32 output.
+// these kernels score 3.9e-3 (the bf16 store alone) and 1e-4 to 5e-4 on the f32 output.
 #include <hip/hip_fp16.h>
 
 #include <type_traits>
 #include <utility>
 
 #include "common.h"
+#include "q8_gemm_wide.h"
 
 namespace lhip {
 
@@ -62,21 +56,19 @@ __device__ __forceinline__ void gm_static_for(F &&f) {
 constexpr int kBK = 64;             // K per tile: two Q8_0 blocks
 constexpr int kRowBytes = 144;      // 64 bf16 + 16 bytes of padding
 
-// Tile BM x BN by WM x WN waves of at most 64 x 64 each.  LDS per buffer: activations BM x 64 bf16, codes BN x 64 as
+// Tile BM x BN by WM x WN waves of at most 64 x 64 each (M tiles in groups of m_group per XCD, as in q8_gemm_wide.hip).  LDS per buffer: activations BM x 64 bf16, codes BN x 64 as
 // bf16 (rows of 144 bytes), and the BN x 2 block scales of the K tile as f32.  The lane that owns column n of a
 // 32 x 32 accumulator tile needs one scale per block: it reads both scales of the K tile with one 8-byte LDS read.
 // The per-block fma costs one v_fma per output element and block on the vector ALU, the same number of cycles the
 // block's two MFMAs take on the matrix pipe.
 // D = register prefetch depth in K tiles (D > 1 needs K % (64*D) == 0 and D even).
-// N = weight rows of this launch; ldy = row pitch of y in weight rows (N, or more when the launch writes the leading
-// columns of a wider output; the SwiGLU form stores pairs at half that pitch).
 // OutT = __bf16 (rounded to nearest even) or float (the accumulators as they are).
 template <int BM, int BN, int WM, int WN, int D, typename OutT>
 __global__ __launch_bounds__(WM *WN * 64) void q8_gemm_bf16_kernel(const int8_t *__restrict__ qs,
                                                                  const __half *__restrict__ ds,
-                                                                 const __bf16 *__restrict__ x, OutT *__restrict__ y_all,
+                                                                 const __bf16 *__restrict__ x, OutT *__restrict__ y,
                                                                  int M, int N, int K, int m_tiles, int n_tiles,
-                                                                 int swiglu, int kt_slice, int m_group, int ldy) {
+                                                                 int swiglu, int m_group) {
     constexpr int T = WM * WN * 64;
     constexpr int TM = BM / WM, TN = BN / WN;
     constexpr int FM = TM / 32, FN = TN / 32;  // 32x32 accumulator tiles per wave
@@ -115,9 +107,7 @@ __global__ __launch_bounds__(WM *WN * 64) void q8_gemm_bf16_kernel(const int8_t 
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / WN, wn = wave % WN;
     const int nblk = K >> 5;
-    const int kt0 = kt_slice > 0 ? static_cast<int>(blockIdx.y) * kt_slice : 0;
-    const int KT = kt_slice > 0 ? min(kt_slice, K / kBK - kt0) : K / kBK;
-    OutT *__restrict__ y = y_all + (kt_slice > 0 ? static_cast<size_t>(blockIdx.y) * M * N : 0);
+    const int KT = K / kBK;
 
     const __bf16 *a_src[A_CHUNKS];
     int a_dst[A_CHUNKS];
@@ -125,7 +115,7 @@ __global__ __launch_bounds__(WM *WN * 64) void q8_gemm_bf16_kernel(const int8_t 
     for (int i = 0; i < A_CHUNKS; ++i) {
         const int c = tid + i * T;
         const int row = c >> 3, col = (c & 7) * 8;
-        a_src[i] = x + static_cast<size_t>(min(m0 + row, M - 1)) * K + col + kt0 * kBK;
+        a_src[i] = x + static_cast<size_t>(min(m0 + row, M - 1)) * K + col;
         a_dst[i] = row * kRowBytes + col * 2;
     }
     const int8_t *b_src[B_CHUNKS];
@@ -137,8 +127,8 @@ __global__ __launch_bounds__(WM *WN * 64) void q8_gemm_bf16_kernel(const int8_t 
         const int c = tid + i * T;
         const int row = c >> 2, q16 = c & 3;
         const int grow = min(n0 + row, N - 1);
-        b_src[i] = qs + static_cast<size_t>(grow) * K + q16 * 16 + kt0 * kBK;
-        d_src[i] = reinterpret_cast<const uint32_t *>(ds + static_cast<size_t>(grow) * nblk) + kt0;
+        b_src[i] = qs + static_cast<size_t>(grow) * K + q16 * 16;
+        d_src[i] = reinterpret_cast<const uint32_t *>(ds + static_cast<size_t>(grow) * nblk);
         b_dst[i] = row * kRowBytes + q16 * 32;
         s_dst[i] = q16 == 0 ? row * 8 : -1;
     }
@@ -318,7 +308,7 @@ __global__ __launch_bounds__(WM *WN * 64) void q8_gemm_bf16_kernel(const int8_t 
                             typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
                             const bf16x2 pk = {static_cast<__bf16>(act), static_cast<__bf16>(act2)};
                             *reinterpret_cast<bf16x2 *>(reinterpret_cast<__bf16 *>(y) +
-                                                        static_cast<size_t>(row) * (ldy >> 1) + (col >> 1)) = pk;
+                                                        static_cast<size_t>(row) * (N >> 1) + (col >> 1)) = pk;
                         }
                     }
                 }
@@ -333,7 +323,7 @@ __global__ __launch_bounds__(WM *WN * 64) void q8_gemm_bf16_kernel(const int8_t 
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
                 const int row = m0 + wm * TM + i * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-                if (row < M && col < N) y[static_cast<size_t>(row) * ldy + col] = static_cast<OutT>(acc[i][j][v]);
+                if (row < M && col < N) y[static_cast<size_t>(row) * N + col] = static_cast<OutT>(acc[i][j][v]);
             }
         }
 }
@@ -362,23 +352,23 @@ struct GemmScratch {
 lhip_status q8_gemm_reduce_launch(const float *part, void *y, int m, int n, int slices, int out, hipStream_t s, int ldy = 0);
 constexpr int kTileSkinny = 5;        // K slices chosen by the library
 constexpr int kTileSkinnySplit = 50;  // + number of K slices
-constexpr int kTileSliced = 120;      // + number of K slices: the 256x128 tile over slices of K, then a reduction
-constexpr int kTileTail = 200;        // the 256x128 tile in whole rounds of 256 workgroups, the last columns over K slices
+constexpr int kTileSliced = 120;      // + number of K slices: the large tile over slices of K, then a reduction
+constexpr int kTileTail = 200;        // more than one round of large tiles, whatever ends its last round first
 
-// A product of more than 256 tiles of 256x128 runs in rounds of 256 workgroups (one per CU), and a last round that
-// is partly filled takes as long as a full one: 896 tiles (gate/up at 2048 rows) are 3.5 rounds of work in the time
-// of 4.  The plan below gives the whole rounds to the plain kernel and the remaining column tiles to the K-sliced
-// form (f32 partial planes in the scratch array, added in slice order), so that the remainder fills the chip for
-// 1 / slices of a round: `n_main` leading weight rows in whole rounds, `slices` K slices for the rest (0: no such
-// plan).  Needs the M tiles to divide 256, a remainder of at most half a round, K long enough for the saving to
-// exceed the reduction launch, and room for the planes.
+// A product of more than 256 tiles of 128x256 runs in rounds of 256 workgroups (one per CU), and a last round that
+// is partly filled takes as long as a full one.  The plan below gives whole rounds to one launch and the remaining
+// column tiles to a K-sliced one (f32 partial planes in the scratch array, added in slice order), so that the
+// remainder fills the chip for 1 / slices of a round: `n_main` leading weight rows in whole rounds, `slices` K slices
+// for the rest (0: no such plan).  Needs the M tiles to divide 256, K long enough, and room for the planes.
+// Mixing 256x256 and 128x256 tiles in one launch (q8_gemm_wide.hip) is the other way to end a last round early, and the
+// better one unless the remainder is small; gemm_tail_pays compares them.
 struct GemmTail {
     int n_main = 0, slices = 0;
 };
 static GemmTail gemm_tail_plan(int64_t m, int64_t n, int64_t k, int out, const void *y, size_t room) {
     GemmTail none;
     if (m <= 128 || k < 2048 || n % 4 != 0 || !aligned(y, out == kOutF32 ? 16 : (out == kOutBf16 ? 8 : 4))) return none;
-    const int64_t m_tiles = (m + 255) / 256, n_tiles = (n + 127) / 128;
+    const int64_t m_tiles = (m + 255) / 256, n_tiles = (n + 127) / 128;  // halves of a 256x256 tile: 256x128 or 128x256
     if (m_tiles * n_tiles <= 256 || 256 % m_tiles != 0) return none;
     const int64_t per_round = 256 / m_tiles;                 // column tiles of one round
     const int64_t main_tiles = n_tiles / per_round * per_round;
@@ -396,15 +386,23 @@ static GemmTail gemm_tail_plan(int64_t m, int64_t n, int64_t k, int out, const v
     return none;
 }
 
-// M tiles per group of the raster (see the kernel).  Measured on the FFN, QKV and lm_head shapes: groups of 8 are
-// 5 % faster than one group of all the M tiles at M = 8192 (32 M tiles), 1 % at 4096, and the same launch at or below
-// 2048 (at most 8 M tiles); groups of 4 or 6 are within 1 % of 8.
+// Whether the sliced remainder ends before one launch of mixed tiles: half units of a 128x256 tile over all of K (0.64
+// us per 64 of K), the remainder's share of a round, and 25 us for its launch, its planes and their sum.  Measured,
+// sliced remainder against mixed tiles: 2048 x 14336 x 4096 313 against 273 us.
+static bool gemm_tail_pays(const GemmTail &t, int64_t m, int64_t n, int64_t k) {
+    if (t.slices < 2) return false;
+    const double unit = 0.64 * static_cast<double>(k / kBK);
+    return static_cast<double>(q8_gemm_wide_ends(m, t.n_main)) * unit + 2.0 * unit / t.slices + 25.0 <
+           static_cast<double>(q8_gemm_wide_ends(m, n)) * unit;
+}
+
+// M tiles per group of the raster: the activation tiles of a group of rows stay in an XCD's L2 while its N tiles pass.
 constexpr int kGemmMGroup = 8;
 static int gemm_m_group(int m_tiles) { return m_tiles < kGemmMGroup ? m_tiles : kGemmMGroup; }
 
 template <int BM, int BN, int WM, int WN, int D, typename OutT>
 static lhip_status launch_gemm_t(const int8_t *qs, const __half *ds, const void *x, void *y, int m, int n, int k,
-                               int swiglu, hipStream_t s, int slices = 1, int ldy = 0) {
+                               int swiglu, hipStream_t s) {
     const int m_tiles = (m + BM - 1) / BM, n_tiles = (n + BN - 1) / BN;
     const int n_tiles_pad = (n_tiles + 7) / 8 * 8;
     if (static_cast<int64_t>(m_tiles) * n_tiles_pad > 0x7fffffff) return LHIP_ERR_INVALID_SHAPE;  // the grid's x extent
@@ -412,10 +410,9 @@ static lhip_status launch_gemm_t(const int8_t *qs, const __half *ds, const void 
     auto kern = q8_gemm_bf16_kernel<BM, BN, WM, WN, D, OutT>;
     static LdsOptIn opt;
     if (lhip_status st = lds_opt_in(opt, reinterpret_cast<const void *>(kern), lds_bytes)) return st;
-    const int kt_slice = slices > 1 ? (k / kBK + slices - 1) / slices : 0;
-    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(m_tiles * n_tiles_pad), static_cast<unsigned>(slices)),
-                       dim3(WM * WN * 64), lds_bytes, s, qs, ds, static_cast<const __bf16 *>(x), static_cast<OutT *>(y), m,
-                       n, k, m_tiles, n_tiles, swiglu, kt_slice, gemm_m_group(m_tiles), ldy > 0 ? ldy : n);
+    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(m_tiles * n_tiles_pad)), dim3(WM * WN * 64), lds_bytes, s, qs, ds,
+                       static_cast<const __bf16 *>(x), static_cast<OutT *>(y), m, n, k, m_tiles, n_tiles, swiglu,
+                       gemm_m_group(m_tiles));
     LHIP_CHECK_LAUNCH();
     return LHIP_OK;
 }
@@ -446,18 +443,17 @@ static lhip_status gemm_dispatch(const void *planar_dev, const void *x_dev, void
                                      scratch.own, scratch.ws, scratch.floats);
     }
     if (tile > kTileSliced && tile <= kTileSliced + 16) {
-        // Few output tiles and a long K (the down projection of a 512-token prompt: 64 tiles of 256x128): slices of K
-        // fill the chip, f32 partial planes go to the scratch array and are added in slice order.
+        // Few output tiles (the down projection of a 512-token prompt: 64 tiles of 128x256): slices of K fill the chip,
+        // f32 partial planes go to the scratch array and are added in slice order.
         const int slices = tile - kTileSliced;
         const int kt = ki / kBK;
         size_t cap = scratch.room();
         float *part = scratch.own ? scratch.ws : q8_gemm_scratch(&cap);
         if (!part) return scratch.own ? LHIP_ERR_UNSUPPORTED : LHIP_ERR_HIP;
-        if (slices < 2 || kt % slices != 0 || (kt / slices) % 4 != 0 || static_cast<size_t>(slices) * mi * ni > cap ||
-            ni % 4 != 0 || !aligned(y_dev, out == kOutF32 ? 16 : (out == kOutBf16 ? 8 : 4)))
+        if (slices < 2 || !q8_gemm_wide_supports(ki) || (slices - 1) * ((kt + slices - 1) / slices) >= kt ||
+            static_cast<size_t>(slices) * mi * ni > cap || ni % 4 != 0 || !aligned(y_dev, out == kOutF32 ? 16 : (out == kOutBf16 ? 8 : 4)))
             return LHIP_ERR_UNSUPPORTED;
-        if (lhip_status st = launch_gemm_t<256, 128, 4, 2, 4, float>(qs, ds, x_dev, part, mi, ni, ki, 0, s, slices))
-            return st;
+        if (lhip_status st = q8_gemm_wide_launch(qs, ds, x_dev, kWdBf16, part, mi, ni, ki, kOutF32, s, slices)) return st;
         return q8_gemm_reduce_launch(part, y_dev, mi, ni, slices, out, s);
     }
     if (tile == kTileTail) {
@@ -465,19 +461,15 @@ static lhip_status gemm_dispatch(const void *planar_dev, const void *x_dev, void
         float *part = scratch.own ? scratch.ws : q8_gemm_scratch(&cap);
         if (!part) return scratch.own ? LHIP_ERR_UNSUPPORTED : LHIP_ERR_HIP;
         const GemmTail t = gemm_tail_plan(m, n, k, out, y_dev, cap);
-        if (t.slices < 2) return LHIP_ERR_UNSUPPORTED;
+        if (t.slices < 2 || !q8_gemm_wide_supports(k)) return LHIP_ERR_UNSUPPORTED;
+        if (!gemm_tail_pays(t, m, n, k)) return q8_gemm_wide_launch(qs, ds, x_dev, kWdBf16, y_dev, mi, ni, ki, out, s);
         const int n_tail = ni - t.n_main;
         // whole rounds: the leading n_main weight rows, written into the full-width output
-        if (lhip_status st = out == kOutF32
-                                 ? launch_gemm_t<256, 128, 4, 2, 4, float>(qs, ds, x_dev, y_dev, mi, t.n_main, ki, 0, s, 1, ni)
-                                 : launch_gemm_t<256, 128, 4, 2, 4, __bf16>(qs, ds, x_dev, y_dev, mi, t.n_main, ki,
-                                                                            out == kOutSwiglu, s, 1, ni))
-            return st;
+        if (lhip_status st = q8_gemm_wide_launch(qs, ds, x_dev, kWdBf16, y_dev, mi, t.n_main, ki, out, s, 1, ni)) return st;
         // the rest: K slices of the trailing weight rows into the planes, then their sum into the trailing columns
         const int8_t *qs_tail = qs + static_cast<size_t>(t.n_main) * ki;
         const __half *ds_tail = ds + static_cast<size_t>(t.n_main) * (ki / 32);
-        if (lhip_status st = launch_gemm_t<256, 128, 4, 2, 4, float>(qs_tail, ds_tail, x_dev, part, mi, n_tail, ki, 0, s, t.slices))
-            return st;
+        if (lhip_status st = q8_gemm_wide_launch(qs_tail, ds_tail, x_dev, kWdBf16, part, mi, n_tail, ki, kOutF32, s, t.slices)) return st;
         const size_t col0 = out == kOutSwiglu ? t.n_main / 2 : t.n_main;
         void *y_tail = out == kOutF32 ? static_cast<void *>(static_cast<float *>(y_dev) + col0)
                                       : static_cast<void *>(static_cast<__bf16 *>(y_dev) + col0);
@@ -490,7 +482,9 @@ static lhip_status gemm_dispatch(const void *planar_dev, const void *x_dev, void
            : depth == 2 ? launch_gemm<BM, BN, WM, WN, 2>(out, qs, ds, x_dev, y_dev, mi, ni, ki, s)      \
                         : launch_gemm<BM, BN, WM, WN, 1>(out, qs, ds, x_dev, y_dev, mi, ni, ki, s)
     switch (tile) {
-        case 0: LHIP_TILE(256, 128, 4, 2);
+        case 0:
+            if (!q8_gemm_wide_supports(k)) return LHIP_ERR_UNSUPPORTED;
+            return q8_gemm_wide_launch(qs, ds, x_dev, kWdBf16, y_dev, mi, ni, ki, out, s);
         case 1: LHIP_TILE(128, 128, 2, 2);
         case 2: LHIP_TILE(128, 64, 2, 2);
         case 3: LHIP_TILE(64, 64, 2, 2);
@@ -505,22 +499,24 @@ static int gemm_auto_tile(int64_t m, int64_t n, int64_t k, int out, const void *
         q8_gemm_skinny_supports(static_cast<int>(m), static_cast<int>(n), static_cast<int>(k), out, y))
         return kTileSkinny;
     auto blocks = [&](int bm, int bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); };
-    // Few 256x128 tiles: slices of K until the chip is full, when the partial planes (written and read once more:
-    // 4 * slices / K bytes per flop) fit the scratch array.  A workgroup walks K at about 1.2 us per 64-wide tile
-    // whatever M is, so with fewer workgroups than CUs the K loop is the critical path and slicing it pays at every K
-    // (measured, us, whole K -> sliced: 4096 x 4096 at 256 / 512 / 1024 rows 75 -> 30 / 75 -> 38 / 78 -> 58;
-    // 1024 x 4096 at 512 rows 72 -> 23; 4096 x 14336 at 256 / 512 / 1024 rows 237 -> 56 / 240 -> 89 / 249 -> 163).
-    if (m > 128 && n % 4 == 0 && aligned(y, out == kOutF32 ? 16 : (out == kOutBf16 ? 8 : 4))) {
-        const int64_t b0 = blocks(256, 128), kt = k / kBK;
-        for (int slices = 8; slices >= 2; slices >>= 1)
-            if (b0 * slices <= 256 && kt % slices == 0 && (kt / slices) % 4 == 0 &&
-                static_cast<size_t>(slices) * m * n <= room)
-                return kTileSliced + slices;
+    // Few 128x256 tiles: slices of K until the chip is full (at most eight, of at least four 64-wide tiles), when the
+    // partial planes (written and read once more: 4 * slices / K bytes per flop) fit the scratch array.  A workgroup walks
+    // K at 1.3 us per 64-wide tile whatever M is, so with fewer workgroups than CUs the K loop is the critical path and
+    // slicing it pays at every K (measured, us, whole K -> sliced: 4096 x 4096 at 512 rows 90 -> 38, 4096 x 14336 at 512
+    // rows 300 -> 93, 2880 x 2880 at 777 rows 54 -> 38 over three uneven slices).
+    const int64_t kt = k / kBK, b0 = blocks(128, 256);
+    if (m > 32 && q8_gemm_wide_supports(k)) {  // (up to 128 rows only what the weight-streaming kernel does not cover)
+        if (n % 4 == 0 && aligned(y, out == kOutF32 ? 16 : (out == kOutBf16 ? 8 : 4)))
+            for (int64_t slices = 256 / b0 < 8 ? 256 / b0 : 8; slices >= 2; --slices) {
+                const int64_t per = (kt + slices - 1) / slices;
+                if (per >= 4 && (slices - 1) * per < kt && static_cast<size_t>(slices) * m * n <= room)
+                    return kTileSliced + static_cast<int>(slices);
+            }
+        if (gemm_tail_plan(m, n, k, out, y, room).slices >= 2) return kTileTail;
+        // the large tiles from 32 workgroups on (faster there than the smaller ones even with an eighth of the CUs
+        // busy: their K loop is the shortest per flop)
+        if (b0 >= 32) return 0;
     }
-    // Otherwise the 256x128 tile from 64 workgroups on (measured faster than the smaller tiles there even with a
-    // quarter of the CUs busy: its K loop is the shortest per flop), smaller tiles for small products.
-    if (m > 128 && k % (kBK * 4) == 0 && gemm_tail_plan(m, n, k, out, y, room).slices >= 2) return kTileTail;
-    if (m > 128 && blocks(256, 128) >= 64) return 0;
     return blocks(128, 64) >= 64 ? 2 : 3;
 }
 
@@ -532,6 +528,7 @@ extern "C" {
 
 lhip_status lhip_q8_0_matmul_bf16_cfg(const void *planar_dev, const void *x_dev, void *y_dev, int64_t m, int64_t n,
                                       int64_t k, int tile, void *stream) {
+    if (tile > kTileSliced && tile <= kTileSliced + 16 && k % (kBK * 4 * (tile - kTileSliced)) != 0) return LHIP_ERR_UNSUPPORTED;
     return gemm_dispatch(planar_dev, x_dev, y_dev, m, n, k, tile, kOutBf16, stream);
 }
 
