@@ -102,16 +102,18 @@ lhip_status lhip_q8_0_matmul_f32(const void *planar_dev, const float *x_dev, flo
                                  int64_t k, void *stream);
 
 /* The same operator for several activation rows on the matrix cores.  The reference's launch (quantized.rs:159) is
- * one matvec per activation row, i.e. the weights are streamed once per row; this form streams them once per 64
- * rows.  The int8 codes go to the matrix cores as they are (exact in bf16), x as three bf16 limbs (an f16 x as
- * two) whose sum is the value exactly; per Q8_0 block the limb products are summed in f32 and the block's scale is applied to that
- * sum, as the matvec kernels do.  Every product is exact, so the result differs from the matvec form only by the
- * order of the f32 additions (measured 5e-7 to 9e-7 of the rms for both), and products of small integers stay
- * exact.  The f16 form is the f32 form on the widened inputs, rounded once.  Any m >= 1.
+ * one matvec per activation row, i.e. the weights are streamed once per row; this form streams them once per 64 or 128
+ * rows.  The int8 codes go to the matrix cores as they are (exact in bf16 and f16), x as three bf16 limbs whose sum is
+ * the value exactly (an f16 x as two, or as it is); per Q8_0 block the products are summed in f32 and the block's scale
+ * is applied to that sum, as the matvec kernels do.  Every product is exact, so the result differs from the matvec form
+ * only by the order of the f32 additions (measured 1e-7 to 9e-7 of the rms for both), and products of small integers stay
+ * exact.  The f16 form is the f32 form's sum on the widened inputs, rounded once: bit for bit up to 64 rows and for small
+ * products, within the order of the f32 additions above.  Any m >= 1.
  * LHIP_ERR_UNSUPPORTED unless K % 512 == 0, N % 4 == 0, x 16-byte and y 16-byte (f16: 8-byte) aligned.
  * lhip_q8_0_matmul_f32 and lhip_q8_0_matmul_f16 take this form by themselves from a few rows on (two for N*K >=
  * 2^28 codes, three from 2^25, four from 2^23, six below: the measured crossovers with the matvec form) where those
- * conditions hold (the _cfg entry never does).  May keep partial sums in the library's scratch array, see the
+ * conditions hold, and from three to fifteen rows on, by size, for every other K >= 256 and every N (the _cfg entry
+ * never does).  May keep partial sums in the library's scratch array, see the
  * note on overlapping calls at lhip_q8_0_matmul_bf16. */
 lhip_status lhip_q8_0_matmul_f32_gemm(const void *planar_dev, const float *x_dev, float *y_dev, int64_t m, int64_t n,
                                       int64_t k, void *stream);

@@ -31,6 +31,8 @@
 #include <algorithm>
 
 #include "common.h"
+#include "q8_gemm_rows.h"
+#include "q8_gemm_wide.h"
 
 namespace lhip {
 
@@ -560,16 +562,14 @@ bool q8_gemm_split_supports(int n, int k, const void *x, const void *y, bool f16
     return k % kSkUnit == 0 && n % 4 == 0 && aligned(x, 16) && aligned(y, f16 ? 8 : 16);
 }
 
-// y (m, N) = x (m, K) W^T for f32 or f16 activations and results, any m: passes of 64 rows, each streaming the
-// weights once, as blockIdx.z of one launch; K is sliced only while strips x passes leave the chip unfilled.  At most
-// kSkMaxPasses passes per launch (the grid's z extent).  `splits` = 0: chosen here.  The caller has checked
-// q8_gemm_split_supports.
+// Passes of 64 rows of the kernel above, each streaming the weights once, as blockIdx.z of one launch; K is sliced only
+// while strips x passes leave the chip unfilled.  At most kSkMaxPasses passes per launch (the grid's z extent).
 constexpr int64_t kSkMaxPasses = 1024;
 
 // K slices of one chunk of mc rows: as many as fill the chip, within `room` floats of partial planes.
-static int split_slices(int mc, int n, int k, int splits_arg, size_t room) {
+static int split_slices(int mc, int n, int k, size_t room) {
     const int units = k / kSkUnit, strips = (n + kSkRows - 1) / kSkRows, passes = (mc + 63) / 64;
-    int splits = splits_arg > 0 ? splits_arg : 256 / (strips * passes);
+    int splits = 256 / (strips * passes);
     if (splits < 1) splits = 1;
     if (splits > units) splits = units;
     while (splits > 1 && static_cast<size_t>(splits) * mc * n > room) --splits;
@@ -577,28 +577,112 @@ static int split_slices(int mc, int n, int k, int splits_arg, size_t room) {
     return (units + per - 1) / per;  // no empty slice
 }
 
-// Floats of partial planes the plan of q8_gemm_split_launch uses for (m, n, k) when it has the library's own
-// scratch array to itself: what a caller's workspace must hold for the same plan (and the same bits).
+// ---- the choice of the kernel for the f32 / f16 operators
+
+// How a product is run: by passes of 64 rows of the kernel above (kStream), by q8_gemm_rows.hip (kRows: `n_main` leading
+// weight rows in whole rounds of workgroups, the others over `slices` K slices; n_main = 0: all of them), or by the
+// tiles of q8_gemm_wide.hip (kWide).
+struct RowsPlan {
+    enum Kind { kStream, kRows, kWide } kind = kStream;
+    int n_main = 0, slices = 1;
+    size_t floats = 0;  // of partial planes
+};
+
+// The plan that ends first, by what each kernel takes (us, measured): a workgroup of the streaming kernel 0.49 (f32) or
+// 0.38 (f16) per block of K, one of q8_gemm_rows.hip 1.2 or 0.66, a 128x256 tile of q8_gemm_wide.hip 0.64 (f16); 256
+// workgroups at a time, some microseconds per launch, and 3 plus 8 TB/s for the sum of the slices.  The lines this draws
+// (streaming -> chosen, us): 14336 x 4096 f32 at 64 rows 38 -> (54), at 128 61 -> 54, at 256 120 -> 97, at 512 239 ->
+// 162; f16 at 64 rows 34 -> (36), at 128 50 -> 36, at 512 188 -> 90; 4096 x 4096 f32 at 256 rows 39 -> (41), at 300 63 ->
+// 44.  Up to 64 rows, and for fewer than sixteen 128x256 tiles, the streaming kernel's narrower strips stay ahead.
+static RowsPlan rows_plan(int64_t m, int n, int k, bool f16, size_t room, bool stream) {
+    RowsPlan best;
+    const int64_t m_tiles = (m + 127) / 128, n_tiles = (n + 255) / 256;
+    if (stream && (m <= 64 || m_tiles * n_tiles < 16)) return best;
+    const double nblk = k / 32, block = f16 ? 0.66 : 1.2;
+    auto rounds = [](int64_t workgroups) { return static_cast<double>((workgroups + 255) / 256); };
+    auto sum_us = [&](int64_t slices, int64_t cols) { return 3.0 + static_cast<double>(slices * m * cols) * 4.0 / 8e6; };
+    double best_us = 1e30;
+    if (stream) {
+        const int mc = static_cast<int>(m < 64 * kSkMaxPasses ? m : 64 * kSkMaxPasses);
+        const int splits = split_slices(mc, n, k, room);
+        best_us = 6.0 + rounds(((n + kSkRows - 1) / kSkRows) * ((m + 63) / 64) * splits) * (nblk / splits) * (f16 ? 0.38 : 0.49) +
+                  (splits > 1 ? sum_us(splits, n) : 0.0);
+    }
+    if (f16 && q8_gemm_wide_supports(k)) {
+        const double us = 8.0 + static_cast<double>(q8_gemm_wide_ends(m, n)) * 0.32 * nblk;
+        if (us < best_us) best_us = us, best.kind = RowsPlan::kWide;
+    }
+    // all columns, or those that whole rounds leave over, in 1 to 16 slices
+    const int64_t per_round = m_tiles < 256 ? 256 / m_tiles : 1;
+    const int64_t main_tiles = n_tiles / per_round * per_round;
+    for (int64_t lead : {int64_t{0}, main_tiles}) {
+        if (lead == n_tiles || (lead > 0 && m_tiles > 256)) continue;
+        const int64_t cols = n - lead * 256, tiles = m_tiles * (n_tiles - lead);
+        const double main_us = lead > 0 ? rounds(m_tiles * lead) * nblk * block + 8.0 : 0.0;
+        for (int slices = 1; slices <= 16; ++slices) {
+            if (lead > 0 && slices == 1) continue;
+            const int per = q8_gemm_rows_slice_blocks(k, slices);
+            if (static_cast<int64_t>(slices - 1) * per >= k / 32) break;
+            const size_t floats = slices > 1 ? static_cast<size_t>(slices) * m * cols : 0;
+            if (floats > room || (slices > 1 && tiles * slices > 0x7ffffff0)) break;  // (the grid's x extent)
+            const double us = main_us + 8.0 + rounds(tiles * slices) * per * block + (slices > 1 ? sum_us(slices, cols) : 0.0);
+            if (us < best_us) {
+                best_us = us;
+                best.kind = RowsPlan::kRows;
+                best.n_main = static_cast<int>(lead * 256);
+                best.slices = slices;
+                best.floats = floats;
+            }
+        }
+    }
+    return best;
+}
+
+// Floats of partial planes the plan for (m, n, k) uses when it has the library's own scratch array to itself: what a
+// caller's workspace must hold for the same plan (and the same bits) with either activation type.
 size_t q8_gemm_split_workspace_floats(int64_t m, int n, int k) {
+    const bool stream = k % kSkUnit == 0 && n % 4 == 0;
     size_t most = 0;
-    for (int64_t m0 = 0; m0 < m; m0 += 64 * kSkMaxPasses) {
-        const int mc = static_cast<int>(m - m0 < 64 * kSkMaxPasses ? m - m0 : 64 * kSkMaxPasses);
-        const int splits = split_slices(mc, n, k, 0, kSkScratchFloats);
-        if (splits > 1) most = std::max(most, static_cast<size_t>(splits) * mc * n);
+    for (bool f16 : {false, true}) {
+        const RowsPlan plan = rows_plan(m, n, k, f16, kSkScratchFloats, stream);
+        if (plan.kind != RowsPlan::kStream) {
+            most = std::max(most, plan.floats);
+            continue;
+        }
+        for (int64_t m0 = 0; m0 < m; m0 += 64 * kSkMaxPasses) {
+            const int mc = static_cast<int>(m - m0 < 64 * kSkMaxPasses ? m - m0 : 64 * kSkMaxPasses);
+            const int splits = split_slices(mc, n, k, kSkScratchFloats);
+            if (splits > 1) most = std::max(most, static_cast<size_t>(splits) * mc * n);
+        }
     }
     return most;
 }
 
+// y (m, N) = x (m, K) W^T for f32 or f16 activations and results, any m; x 16-byte aligned.
 // `own_workspace`: partial planes go to `ws` (ws_floats floats; none: no K slices) and the library's scratch array
 // is not touched, so calls may overlap in time.
 lhip_status q8_gemm_split_launch(const int8_t *qs, const __half *ds, const void *x, void *y, int64_t m, int n, int k,
-                                 bool f16, int splits_arg, hipStream_t s, bool own_workspace, float *ws, size_t ws_floats) {
+                                 bool f16, hipStream_t s, bool own_workspace, float *ws, size_t ws_floats) {
     const size_t esz = f16 ? 2 : 4;
+    const size_t room = own_workspace ? (ws ? std::min(ws_floats, kSkScratchFloats) : 0) : kSkScratchFloats;
+    const bool stream = q8_gemm_split_supports(n, k, x, y, f16);
+    RowsPlan plan = rows_plan(m, n, k, f16, kSkScratchFloats, stream);
+    if (plan.floats > room) plan = rows_plan(m, n, k, f16, room, stream);
+    float *scratch = own_workspace ? ws : (plan.kind == RowsPlan::kRows && plan.slices > 1 ? sk_scratch_ptr() : nullptr);
+    if (plan.kind == RowsPlan::kWide) return q8_gemm_wide_launch(qs, ds, x, kWdF16, y, static_cast<int>(m), n, k, kWdOutF16, s);
+    if (plan.kind == RowsPlan::kRows) {
+        if (plan.slices > 1 && !scratch) return LHIP_ERR_HIP;
+        const int mi = static_cast<int>(m), tail = n - plan.n_main;
+        if (plan.n_main > 0)
+            if (lhip_status st = q8_gemm_rows_launch(qs, ds, x, y, mi, plan.n_main, k, f16, 1, nullptr, n, s)) return st;
+        return q8_gemm_rows_launch(qs + static_cast<size_t>(plan.n_main) * k, ds + static_cast<size_t>(plan.n_main) * (k / 32), x,
+                                   static_cast<unsigned char *>(y) + static_cast<size_t>(plan.n_main) * esz, mi, tail, k, f16,
+                                   plan.slices, scratch, n, s);
+    }
     for (int64_t m0 = 0; m0 < m; m0 += 64 * kSkMaxPasses) {
         const int mc = static_cast<int>(m - m0 < 64 * kSkMaxPasses ? m - m0 : 64 * kSkMaxPasses);
         const int passes = (mc + 63) / 64;
-        const size_t room = own_workspace ? (ws ? std::min(ws_floats, kSkScratchFloats) : 0) : kSkScratchFloats;
-        const int splits = split_slices(mc, n, k, splits_arg, room);
+        const int splits = split_slices(mc, n, k, room);
         float *part = nullptr;
         if (splits > 1) {
             part = own_workspace ? ws : sk_scratch_ptr();

@@ -9,9 +9,7 @@
 
 namespace lhip {
 
-// Activations as the kernel reads them: (m, k) bf16, (m, k) f16, or three bf16 planes of (m, k) whose sum is the f32
-// value (q8_gemm_wide_split).
-enum WdType { kWdBf16, kWdF16, kWdF32Planes };
+enum WdType { kWdBf16, kWdF16 };  // activations
 // Results; the numbers are those of the output forms in q8_gemm.hip and q8_gemm_skinny.hip.
 enum { kWdOutBf16 = 0, kWdOutF32 = 1, kWdOutSwiglu = 2, kWdOutF16 = 4 };
 
@@ -22,8 +20,6 @@ bool q8_gemm_wide_supports(int64_t k);
 // rows, for a product that fills the leading columns of a wider one.
 lhip_status q8_gemm_wide_launch(const int8_t *qs, const __half *ds, const void *x, WdType type, void *y, int m, int n, int k,
                                 int out, hipStream_t s, int slices = 1, int ldy = 0);
-// f32 (m, k) -> the three planes.
-lhip_status q8_gemm_wide_split(const float *x, void *planes, int64_t m, int64_t k, hipStream_t s);
 // When a launch of that product ends, in half units of a 128x256 tile's time over all of K (1.3 us per 64 of K).
 int64_t q8_gemm_wide_ends(int64_t m, int64_t n);
 

@@ -1,16 +1,15 @@
 // Q8_0 weights x many activation rows on the matrix cores:  Y[M][N] = X[M][K] . W[N][K]^T.
 //
-// The tile kernel behind the prompt products (bf16 activations: lhip_q8_0_matmul_bf16 and its forms; f16 and f32
-// activations: lhip_q8_0_matmul_f16 / _f32 from a hundred rows or so on).  Weights stay exact: the int8 codes go to the
+// The tile kernel behind the prompt products (bf16 activations: lhip_q8_0_matmul_bf16 and its forms; f16 activations of
+// many rows: lhip_q8_0_matmul_f16).  Weights stay exact: the int8 codes go to the
 // matrix cores as they are (exact in bf16 and in f16), the sum of a Q8_0 block's products is formed there in f32, and
 // the block's scale multiplies that sum on the vector ALU, acc += d * sum - the arithmetic of the reference's matvec
-// kernel (crates/luminal_cuda/src/quantized.rs:93-96).  Activations are bf16 or f16 as given, or f32 as three bf16
-// planes whose sum is the value exactly (q8_gemm_wide_split_kernel; one matrix step per plane).
+// kernel (crates/luminal_cuda/src/quantized.rs:93-96).  Activations are bf16 or f16 as given, so every product is exact.
 //
 // What bounds it: the scale costs one vector fma per output element and block, 64 cycles per 32 x 32 outputs and
-// block against 64 cycles of matrix steps, and a matrix step holds the vector pipe for about ten cycles of its own, so
-// one activation plane is bound by the vector pipe (a register-only loop of that mix: 1330 TFLOP/s of useful work on
-// random data), three planes by the matrix pipe.  Hence:
+// block against 64 cycles of matrix steps, and a matrix step holds the vector pipe for about ten cycles of its own: the
+// kernel is bound by the vector pipe (a register-only loop of that mix: 1330 TFLOP/s of useful work on random data).
+// Hence:
 //   * v_mfma_f32_16x16x32: a block is ONE step (nothing is read back as an accumulator), and on random data the part
 //     holds 2.2 GHz with it where the 32x32x16 form drops to 1.6-1.9;
 //   * a wave owns 32 weight rows of the tile and all of its BM activation rows, so a code is converted to bf16 / f16
@@ -54,13 +53,11 @@ __device__ __forceinline__ void wd_static_for(F &&f) {
 
 constexpr int kWdBN = 256;  // weight rows per workgroup: eight waves of 32
 
-// BM activation rows, LIMBS planes of them, KB Q8_0 blocks of K per tile.
-template <int BM, int LIMBS, int KB>
+// BM activation rows; a tile is 64 of K, two Q8_0 blocks.
+template <int BM>
 struct WdShape {
-    static constexpr int A_ROW = KB * 64;                    // bytes of a plane's row
-    static constexpr int A_PLANE = BM * A_ROW;
-    static constexpr int A_BYTES = LIMBS * A_PLANE;
-    static constexpr int B_ROW = KB * 32;
+    static constexpr int A_ROW = 128, B_ROW = 64;            // bytes of an activation row and of a row of codes
+    static constexpr int A_BYTES = BM * A_ROW;
     static constexpr int B_WAVE = 32 * B_ROW;                // the codes of a wave's weight rows
     static constexpr int B_BYTES = 8 * B_WAVE;
     static constexpr int S_BYTES = 8 * 256;                  // one dword (two blocks' scales) per lane
@@ -104,7 +101,8 @@ __device__ __forceinline__ uint32_t wd_codes2(uint32_t w, int h) {
 }
 
 template <typename XT>
-__device__ __forceinline__ wd_f32x4 wd_mfma(const wd_u32x4 &a, const wd_u32x4 &b, const wd_f32x4 &c) {
+__device__ __forceinline__ wd_f32x4 wd_mfma(const wd_u32x4 &a, const wd_u32x4 &b) {
+    const wd_f32x4 c = {0.f, 0.f, 0.f, 0.f};
     if constexpr (std::is_same<XT, __bf16>::value)
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(wd_bf16x8, a), __builtin_bit_cast(wd_bf16x8, b), c, 0, 0, 0);
     else
@@ -132,15 +130,15 @@ __device__ __forceinline__ bool wd_tile(int id, int m_tiles, int n_tiles, int sl
     return true;
 }
 
-// One tile: rows m0 .. of x, weight rows n0 .. below n_end, K tiles kt0 .. kt0 + KT - 1 of KB blocks each.
+// One tile: rows m0 .. of x, weight rows n0 .. below n_end, K tiles kt0 .. kt0 + KT - 1.
 // `y` already points at this K slice's plane; ldy = row pitch of y in weight rows.
-template <int BM, int LIMBS, int KB, typename XT, int OUT>
+template <int BM, typename XT, int OUT>
 __device__ __forceinline__ void wd_tile_body(unsigned char *lds, const int8_t *__restrict__ qs, const __half *__restrict__ ds,
-                                             const XT *__restrict__ x, size_t x_plane, void *__restrict__ y, int M, int K, int m0,
-                                             int n0, int n_end, int kt0, int KT, int ldy) {
-    using S = WdShape<BM, LIMBS, KB>;
+                                             const XT *__restrict__ x, void *__restrict__ y, int M, int K, int m0, int n0,
+                                             int n_end, int kt0, int KT, int ldy) {
+    using S = WdShape<BM>;
     constexpr int NI = BM / 16;    // 16-row fragments
-    constexpr int NF = KB * NI;    // (block, fragment) pairs of a tile
+    constexpr int NF = 2 * NI;     // (block, fragment) pairs of a tile
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, g = lane >> 4;
@@ -149,43 +147,39 @@ __device__ __forceinline__ void wd_tile_body(unsigned char *lds, const int8_t *_
 
     // ---- requests.  A wave brings in 1/8 of the activation rows, and the codes and scales of its own 32 weight rows.
     // Rows past the end repeat the last one.
-    auto a_swizzle = [](int row) { return KB == 2 ? (row >> 1) & 7 : (4 - (row >> 2)) & 3; };
+    auto a_swizzle = [](int row) { return (row >> 1) & 7; };
     auto b_swizzle = [](int row) { return (4 - (row >> 2)) & 3; };
     const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char *)lds));
-    constexpr int A_PPR = S::A_ROW / 16, A_RPR = 64 / A_PPR;        // pieces per row, rows per request
-    constexpr int A_PER = S::A_REQ / LIMBS;                         // requests per plane
-    constexpr int B_PPR = S::B_ROW / 16, B_RPR = 64 / B_PPR;
-    uint32_t a_off[A_PER], b_off[S::B_REQ], s_off;
+    uint32_t a_off[S::A_REQ], b_off[S::B_REQ], s_off;
 #pragma unroll
-    for (int q = 0; q < A_PER; ++q) {
-        const int row = (wave * A_PER + q) * A_RPR + lane / A_PPR;
-        const int piece = (lane % A_PPR) ^ a_swizzle(row);
+    for (int q = 0; q < S::A_REQ; ++q) {  // eight rows per request
+        const int row = (wave * S::A_REQ + q) * 8 + (lane >> 3);
+        const int piece = (lane & 7) ^ a_swizzle(row);
         a_off[q] = static_cast<uint32_t>(min(m0 + row, M - 1) - m0) * static_cast<uint32_t>(K) * 2u + piece * 16u;
     }
     const int wn0 = n0 + wave * 32, wbase = min(wn0, last_n);
 #pragma unroll
-    for (int q = 0; q < S::B_REQ; ++q) {
-        const int row = q * B_RPR + lane / B_PPR;
-        const int piece = KB == 2 ? (lane & 3) ^ b_swizzle(row) : lane & 1;
+    for (int q = 0; q < S::B_REQ; ++q) {  // sixteen rows per request
+        const int row = q * 16 + (lane >> 2);
+        const int piece = (lane & 3) ^ b_swizzle(row);
         b_off[q] = static_cast<uint32_t>(min(wn0 + row, last_n) - wbase) * static_cast<uint32_t>(K) + piece * 16u;
     }
     s_off = static_cast<uint32_t>(min(wn0 + (lane & 31), last_n) - wbase) * static_cast<uint32_t>(nblk) * 2u;
-    const unsigned char *xb = reinterpret_cast<const unsigned char *>(x) + (static_cast<size_t>(m0) * K + static_cast<size_t>(kt0) * (KB * 32)) * 2;
-    const int8_t *qb = qs + static_cast<size_t>(wbase) * K + static_cast<size_t>(kt0) * (KB * 32);
-    const __half *db = ds + static_cast<size_t>(wbase) * nblk;
+    const unsigned char *xb = reinterpret_cast<const unsigned char *>(x) + (static_cast<size_t>(m0) * K + static_cast<size_t>(kt0) * 64) * 2;
+    const int8_t *qb = qs + static_cast<size_t>(wbase) * K + static_cast<size_t>(kt0) * 64;
+    const __half *db = ds + static_cast<size_t>(wbase) * nblk + static_cast<size_t>(kt0) * 2;
     auto request_piece = [&](int t, int stage, auto pc) __attribute__((always_inline)) {
         constexpr int p = decltype(pc)::value;
         static_assert(p >= 0 && p < S::REQ, "no such request");
         const int tt = min(t, KT - 1);  // past the end: the last tile again, never used
         const uint32_t st = lds0 + stage * S::STAGE;
         if constexpr (p < S::A_REQ) {
-            constexpr int l = p / A_PER, q = p % A_PER;
-            wd_request<16>(xb + l * x_plane + static_cast<size_t>(tt) * (KB * 64), a_off[q], st + l * S::A_PLANE + (wave * A_PER + q) * 1024);
+            wd_request<16>(xb + static_cast<size_t>(tt) * 128, a_off[p], st + (wave * S::A_REQ + p) * 1024);
         } else if constexpr (p < S::A_REQ + S::B_REQ) {
             constexpr int q = p - S::A_REQ;
-            wd_request<16>(qb + static_cast<size_t>(tt) * (KB * 32), b_off[q], st + S::A_BYTES + wave * S::B_WAVE + q * 1024);
-        } else {  // the dword that holds the tile's scales (KB = 1: the pair of blocks it belongs to)
-            wd_request<4>(db + ((static_cast<size_t>(kt0 + tt) * KB) & ~size_t{1}), s_off, st + S::A_BYTES + S::B_BYTES + wave * 256);
+            wd_request<16>(qb + static_cast<size_t>(tt) * 64, b_off[q], st + S::A_BYTES + wave * S::B_WAVE + q * 1024);
+        } else {  // a row's two scales are one aligned dword (K / 32 is even)
+            wd_request<4>(db + static_cast<size_t>(tt) * 2, s_off, st + S::A_BYTES + S::B_BYTES + wave * 256);
         }
     };
     auto request = [&](int t, int stage) __attribute__((always_inline)) {
@@ -194,9 +188,8 @@ __device__ __forceinline__ void wd_tile_body(unsigned char *lds, const int8_t *_
 
     // ---- operands
     const int a_lane = r * S::A_ROW + (g ^ a_swizzle(r)) * 16;  // fragment i: + i * 16 rows; block 1: ^ 64
-    const int b_lane = S::A_BYTES + wave * S::B_WAVE + r * S::B_ROW +
-                       (KB == 2 ? ((g >> 1) ^ b_swizzle(r)) * 16 : (g >> 1) * 16) + (g & 1) * 8;  // n tile 1: + 16 rows; block 1: ^ 32
-    const int s_lane = S::A_BYTES + S::B_BYTES + wave * 256 + r * 4;                              // n tile 1: + 64
+    const int b_lane = S::A_BYTES + wave * S::B_WAVE + r * S::B_ROW + ((g >> 1) ^ b_swizzle(r)) * 16 + (g & 1) * 8;  // n tile 1: + 16 rows; block 1: ^ 32
+    const int s_lane = S::A_BYTES + S::B_BYTES + wave * 256 + r * 4;  // n tile 1: + 64
     wd_f32x4 acc[NI][2];
 #pragma unroll
     for (int i = 0; i < NI; ++i)
@@ -204,16 +197,12 @@ __device__ __forceinline__ void wd_tile_body(unsigned char *lds, const int8_t *_
         for (int j = 0; j < 2; ++j) acc[i][j] = wd_f32x4{0.f, 0.f, 0.f, 0.f};
     constexpr int AHEAD = 3, RING = AHEAD + 1;  // activation fragments requested from LDS ahead of their use
     static_assert(NF % RING == 0, "the ring has the same phase in every tile");
-    wd_u32x4 ar[RING][LIMBS];
+    wd_u32x4 ar[RING];
     wd_u32x4 bf[2][2];   // weight operands of two successive blocks, [block parity][n tile]
     wd_u32x2 raw[2];     // codes of the block after this one
     float sc[2][2];      // scales [block parity][n tile]
     uint32_t sraw[2];    // the next tile's
     wd_f32x4 sum[2];     // block sums whose scaling is still to be issued
-    auto a_read = [&](wd_u32x4 (&dst)[LIMBS], const unsigned char *p) __attribute__((always_inline)) {
-#pragma unroll
-        for (int l = 0; l < LIMBS; ++l) dst[l] = *reinterpret_cast<const wd_u32x4 *>(p + l * S::A_PLANE);
-    };
     auto read_raw = [&](const unsigned char *p) __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < 2; ++j) raw[j] = *reinterpret_cast<const wd_u32x2 *>(p + j * 16 * S::B_ROW);
@@ -223,15 +212,11 @@ __device__ __forceinline__ void wd_tile_body(unsigned char *lds, const int8_t *_
         for (int j = 0; j < 2; ++j) sraw[j] = *reinterpret_cast<const uint32_t *>(st + s_lane + j * 64);
     };
     auto half_of = [](uint32_t w, int h) { return __half2float(__ushort_as_half(static_cast<unsigned short>(w >> (16 * h)))); };
-    auto set_scales = [&](int t) __attribute__((always_inline)) {  // those of K tile t, from sraw
+    auto set_scales = [&]() __attribute__((always_inline)) {  // from sraw
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            if constexpr (KB == 2) {
-                sc[0][j] = half_of(sraw[j], 0);
-                sc[1][j] = half_of(sraw[j], 1);
-            } else {
-                sc[0][j] = ((kt0 + t) & 1) ? half_of(sraw[j], 1) : half_of(sraw[j], 0);
-            }
+            sc[0][j] = half_of(sraw[j], 0);
+            sc[1][j] = half_of(sraw[j], 1);
         }
     };
     auto convert = [&](int b, int p) __attribute__((always_inline)) {  // piece p of 8
@@ -243,16 +228,15 @@ __device__ __forceinline__ void wd_tile_body(unsigned char *lds, const int8_t *_
     wd_wait_requests<(S::STAGES - 2) * S::REQ>();
     wd_barrier();
 #pragma unroll
-    for (int f = 0; f < AHEAD; ++f) a_read(ar[f], lds + a_lane + f * 16 * S::A_ROW);
+    for (int f = 0; f < AHEAD; ++f) ar[f] = *reinterpret_cast<const wd_u32x4 *>(lds + a_lane + f * 16 * S::A_ROW);
     read_raw(lds + b_lane);
     read_scales(lds);
-    set_scales(0);
+    set_scales();
 #pragma unroll
     for (int p = 0; p < 8; ++p) convert(0, p);
 
-    constexpr int MID = NF / 2;                                     // where the barrier stands
-    constexpr int STEP = (NF - MID) / S::REQ >= 2 ? 2 : 1;          // fragments between two requests
-    static_assert(1 + (S::REQ - 1) * STEP < NF - MID || KB == 1, "the requests fit the second half");
+    constexpr int STEP = NI / S::REQ >= 2 ? 2 : 1;  // fragments between two requests
+    static_assert(1 + (S::REQ - 1) * STEP < NI, "the requests fit the second half");
     int stage = 0;
     for (int t = 0; t < KT; ++t) {
         const int next = stage == S::STAGES - 1 ? 0 : stage + 1, last = stage == 0 ? S::STAGES - 1 : stage - 1;
@@ -260,10 +244,9 @@ __device__ __forceinline__ void wd_tile_body(unsigned char *lds, const int8_t *_
         const unsigned char *a0 = st + a_lane, *a1 = st + (a_lane ^ 64), *a2 = st_next + a_lane;
         wd_static_for<NF>([&](auto fc) __attribute__((always_inline)) {
             constexpr int f = decltype(fc)::value, b = f / NI, i = f % NI;
-            constexpr int pb = KB == 2 ? b : 0;                     // this block's operands and scales
-            constexpr int fp = (f + NF - 1) % NF, bp = fp / NI, ip = fp % NI;  // the fragment before this one
-            if constexpr (KB == 2 && f == 0) read_raw(st + (b_lane ^ 32));  // block 1
-            if constexpr (f == MID) {
+            constexpr int bp = (f - 1) / NI, ip = (f + NI - 1) % NI;  // the fragment before this one (f > 0)
+            if constexpr (f == 0) read_raw(st + (b_lane ^ 32));  // block 1
+            if constexpr (f == NI) {
                 // This wave's requests for the next tile have landed, and behind the barrier everybody's; the buffer of
                 // the tile before this one is free.
                 wd_wait_requests<(S::STAGES - 3) * S::REQ>();
@@ -271,59 +254,40 @@ __device__ __forceinline__ void wd_tile_body(unsigned char *lds, const int8_t *_
                 read_raw(st_next + b_lane);
                 read_scales(st_next);
             }
-            if constexpr (KB == 2) {
-                if constexpr (f > MID && (f - MID - 1) % STEP == 0 && (f - MID - 1) / STEP < S::REQ)
-                    request_piece(t + S::STAGES - 1, last, std::integral_constant<int, (f - MID - 1) / STEP>{});
-            } else if constexpr (f >= MID) {  // few fragments: two requests behind each
-                constexpr int p = (f - MID) * 2;
-                if constexpr (p < S::REQ) request_piece(t + S::STAGES - 1, last, std::integral_constant<int, p>{});
-                if constexpr (p + 1 < S::REQ) request_piece(t + S::STAGES - 1, last, std::integral_constant<int, p + 1>{});
-            }
+            if constexpr (f > NI && (f - NI - 1) % STEP == 0 && (f - NI - 1) / STEP < S::REQ)
+                request_piece(t + S::STAGES - 1, last, std::integral_constant<int, (f - NI - 1) / STEP>{});
             constexpr int fa = f + AHEAD;
-            a_read(ar[fa % RING], (fa < NF ? (KB == 2 && fa >= NI ? a1 : a0) : a2) + (fa % NI) * 16 * S::A_ROW);
+            ar[fa % RING] = *reinterpret_cast<const wd_u32x4 *>((fa < NI ? a0 : (fa < NF ? a1 : a2)) + (fa % NI) * 16 * S::A_ROW);
             wd_f32x4 s[2];
-            wd_static_for<LIMBS>([&](auto lc) __attribute__((always_inline)) {
-                constexpr int l = LIMBS - 1 - decltype(lc)::value;  // small limbs first
-                wd_static_for<2>([&](auto jc) __attribute__((always_inline)) {
-                    constexpr int j = decltype(jc)::value;
-                    const wd_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-                    // The fences hold the order: left alone, the scheduler issues the matrix steps first and keeps their
-                    // sums alive.  The sums of the fragment before are scaled under this one's matrix steps.
-                    __builtin_amdgcn_sched_barrier(0);
-                    s[j] = wd_mfma<XT>(ar[f % RING][l], bf[KB == 2 ? pb : 0][j], l == LIMBS - 1 ? zero : s[j]);
-                    asm volatile("" : "+v"(s[j]));
-                    __builtin_amdgcn_sched_barrier(0);
-                    if constexpr (l == LIMBS - 1 && f > 0) {
+            wd_static_for<2>([&](auto jc) __attribute__((always_inline)) {
+                constexpr int j = decltype(jc)::value;
+                // The fences hold the order: left alone, the scheduler issues the matrix steps first and keeps their sums
+                // alive.  The sums of the fragment before are scaled under this one's matrix steps.
+                __builtin_amdgcn_sched_barrier(0);
+                s[j] = wd_mfma<XT>(ar[f % RING], bf[b][j]);
+                asm volatile("" : "+v"(s[j]));
+                __builtin_amdgcn_sched_barrier(0);
+                if constexpr (f > 0) {
 #pragma unroll
-                        for (int v = 0; v < 4; ++v) acc[ip][j][v] = fmaf(sc[KB == 2 ? bp : 0][j], sum[j][v], acc[ip][j][v]);
-                        asm volatile("" : "+v"(acc[ip][j]));
-                    }
-                });
+                    for (int v = 0; v < 4; ++v) acc[ip][j][v] = fmaf(sc[bp][j], sum[j][v], acc[ip][j][v]);
+                    asm volatile("" : "+v"(acc[ip][j]));
+                }
             });
             sum[0] = s[0];
             sum[1] = s[1];
-            if constexpr (KB == 2) {  // the codes of the block after this one
-                constexpr int C0 = NI >= 16 ? 4 : 3, PER = NI >= 16 ? 1 : 2;
-                if constexpr (i >= C0 && (i - C0) * PER < 8) {
+            // the codes of the block after this one
+            constexpr int C0 = NI >= 16 ? 4 : 3, PER = NI >= 16 ? 1 : 2;
+            if constexpr (i >= C0 && (i - C0) * PER < 8) {
 #pragma unroll
-                    for (int p = (i - C0) * PER; p < (i - C0) * PER + PER; ++p) convert(b ^ 1, p);
-                }
-            } else if constexpr (f >= MID + 2) {
-                constexpr int PER = 8 / (NF - MID - 2);
-#pragma unroll
-                for (int p = (f - MID - 2) * PER; p < (f - MID - 2) * PER + PER; ++p) convert(1, p);
+                for (int p = (i - C0) * PER; p < (i - C0) * PER + PER; ++p) convert(b ^ 1, p);
             }
         });
         // the last fragment's sums, with this tile's scales
 #pragma unroll
         for (int j = 0; j < 2; ++j)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) acc[NI - 1][j][v] = fmaf(sc[KB - 1][j], sum[j][v], acc[NI - 1][j][v]);
-        set_scales(t + 1);
-        if constexpr (KB == 1) {
-#pragma unroll
-            for (int j = 0; j < 2; ++j) bf[0][j] = bf[1][j];
-        }
+            for (int v = 0; v < 4; ++v) acc[NI - 1][j][v] = fmaf(sc[1][j], sum[j][v], acc[NI - 1][j][v]);
+        set_scales();
         stage = next;
     }
     wd_wait_requests<0>();  // no request outlives its buffer, which the epilogue now takes over
@@ -408,51 +372,25 @@ __device__ __forceinline__ void wd_tile_body(unsigned char *lds, const int8_t *_
 // Weight rows below n_big in tiles of 256x256 (the first big_blocks workgroups), the others in tiles of 128x256
 // (wd_big_rows chooses the cut).  With `slices` > 1 every slice of kt_slice K tiles goes into an f32 plane of (M, N) of its
 // own.
-template <int LIMBS, int KB, typename XT, int OUT>
+template <typename XT, int OUT>
 __global__ __launch_bounds__(512) void q8_gemm_wide_kernel(const int8_t *__restrict__ qs, const __half *__restrict__ ds,
                                                            const XT *__restrict__ x, void *__restrict__ y, int M, int N, int K,
                                                            int n_big, int big_blocks, int slices, int kt_slice, int ldy) {
     extern __shared__ __attribute__((aligned(16))) unsigned char wd_lds[];
-    const int kt_all = K / (KB * 32);
-    const size_t x_plane = static_cast<size_t>(M) * K * 2;
+    const int kt_all = K / 64;
     int mt, nt, slice;
-    if constexpr (LIMBS == 1) {
-        if (static_cast<int>(blockIdx.x) < big_blocks) {
-            const int m_tiles = (M + 255) / 256;
-            if (!wd_tile(blockIdx.x, m_tiles, n_big / kWdBN, 1, min(m_tiles, 8), mt, nt, slice)) return;
-            wd_tile_body<256, LIMBS, KB, XT, OUT>(wd_lds, qs, ds, x, x_plane, y, M, K, mt * 256, nt * kWdBN, n_big, 0, kt_all, ldy);
-            return;
-        }
+    if (static_cast<int>(blockIdx.x) < big_blocks) {
+        const int m_tiles = (M + 255) / 256;
+        if (!wd_tile(blockIdx.x, m_tiles, n_big / kWdBN, 1, min(m_tiles, 8), mt, nt, slice)) return;
+        wd_tile_body<256, XT, OUT>(wd_lds, qs, ds, x, y, M, K, mt * 256, nt * kWdBN, n_big, 0, kt_all, ldy);
+        return;
     }
     const int m_tiles = (M + 127) / 128;
     if (!wd_tile(static_cast<int>(blockIdx.x) - big_blocks, m_tiles, (N - n_big + kWdBN - 1) / kWdBN, slices, min(m_tiles, 16), mt, nt, slice))
         return;
     const int kt0 = slice * kt_slice;
     if (slices > 1) y = static_cast<float *>(y) + static_cast<size_t>(slice) * M * N;
-    wd_tile_body<128, LIMBS, KB, XT, OUT>(wd_lds, qs, ds, x, x_plane, y, M, K, mt * 128, n_big + nt * kWdBN, N, kt0,
-                                          min(kt_slice, kt_all - kt0), ldy);
-}
-
-// f32 activations -> three bf16 planes whose sum is the value exactly (three successive roundings to nearest: 8 + 8 + 8
-// significant bits), the layout the tile kernel's requests read.  One pass over x, bound by memory.
-__global__ __launch_bounds__(256) void q8_gemm_wide_split_kernel(const wd_f32x4 *__restrict__ x, wd_u32x2 *__restrict__ planes,
-                                                                 size_t quads) {
-    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-    for (size_t i = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x; i < quads; i += static_cast<size_t>(gridDim.x) * 256) {
-        wd_f32x4 v = x[i];
-#pragma unroll
-        for (int l = 0; l < 3; ++l) {
-            wd_u32x2 w;
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const bf16x2 p = {static_cast<__bf16>(v[2 * h]), static_cast<__bf16>(v[2 * h + 1])};
-                w[h] = __builtin_bit_cast(uint32_t, p);
-                v[2 * h] -= __uint_as_float(w[h] << 16);
-                v[2 * h + 1] -= __uint_as_float(w[h] & 0xffff0000u);
-            }
-            planes[l * quads + i] = w;
-        }
-    }
+    wd_tile_body<128, XT, OUT>(wd_lds, qs, ds, x, y, M, K, mt * 128, n_big + nt * kWdBN, N, kt0, min(kt_slice, kt_all - kt0), ldy);
 }
 
 // How many weight rows go to 256x256 tiles.  A tile of either height takes the same time whatever its neighbours do, a
@@ -485,20 +423,20 @@ int64_t q8_gemm_wide_ends(int64_t m, int64_t n) {
     return end;
 }
 
-template <int LIMBS, int KB, typename XT, int OUT>
+template <typename XT, int OUT>
 static lhip_status wd_launch_t(const int8_t *qs, const __half *ds, const void *x, void *y, int m, int n, int k, int slices,
                                int ldy, hipStream_t s) {
-    const int n_big = LIMBS == 1 && slices == 1 ? wd_big_rows(m, n) : 0;
+    const int n_big = slices == 1 ? wd_big_rows(m, n) : 0;
     auto blocks = [](int64_t m_tiles, int64_t n_tiles) { return (m_tiles * n_tiles + 7) / 8 * 8; };  // whole eights, see wd_tile
     const int64_t big = blocks((m + 255) / 256, n_big / kWdBN);
     const int64_t small = blocks((m + 127) / 128, static_cast<int64_t>((n - n_big + kWdBN - 1) / kWdBN) * slices);
     if (big + small > 0x7fffffff) return LHIP_ERR_INVALID_SHAPE;  // the grid's x extent
-    auto kern = q8_gemm_wide_kernel<LIMBS, KB, XT, OUT>;
-    constexpr int lds_small = WdShape<128, LIMBS, KB>::LDS;
-    constexpr int lds_most = LIMBS == 1 && WdShape<256, 1, 2>::LDS > lds_small ? WdShape<256, 1, 2>::LDS : lds_small;
+    auto kern = q8_gemm_wide_kernel<XT, OUT>;
+    constexpr int lds_small = WdShape<128>::LDS, lds_most = WdShape<256>::LDS;
+    static_assert(lds_most >= lds_small, "the opt-in covers both heights");
     static LdsOptIn opt;
     if (lhip_status st = lds_opt_in(opt, reinterpret_cast<const void *>(kern), lds_most)) return st;
-    const int kt = k / (KB * 32), kt_slice = (kt + slices - 1) / slices;
+    const int kt = k / 64, kt_slice = (kt + slices - 1) / slices;
     if (slices < 1 || (slices - 1) * kt_slice >= kt) return LHIP_ERR_UNSUPPORTED;  // an empty slice
     hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(big + small)), dim3(512),
                        static_cast<unsigned>(n_big > 0 ? lds_most : lds_small), s, qs, ds, static_cast<const XT *>(x), y, m, n, k,
@@ -511,32 +449,16 @@ bool q8_gemm_wide_supports(int64_t k) { return k % 64 == 0 && k <= kWdMaxK; }
 
 lhip_status q8_gemm_wide_launch(const int8_t *qs, const __half *ds, const void *x, WdType type, void *y, int m, int n, int k,
                                 int out, hipStream_t s, int slices, int ldy) {
-#define LHIP_WD(LIMBS, KB, XT, OUT) return wd_launch_t<LIMBS, KB, XT, OUT>(qs, ds, x, y, m, n, k, slices, ldy, s)
-    switch (type) {
-        case kWdBf16:
-            if (out == kWdOutF32) LHIP_WD(1, 2, __bf16, kWdOutF32);
-            if (out == kWdOutBf16) LHIP_WD(1, 2, __bf16, kWdOutBf16);
-            if (out == kWdOutSwiglu) LHIP_WD(1, 2, __bf16, kWdOutSwiglu);
-            break;
-        case kWdF16:
-            if (out == kWdOutF32) LHIP_WD(1, 2, _Float16, kWdOutF32);
-            if (out == kWdOutF16) LHIP_WD(1, 2, _Float16, kWdOutF16);
-            break;
-        case kWdF32Planes:
-            if (out == kWdOutF32) LHIP_WD(3, 1, __bf16, kWdOutF32);
-            break;
+#define LHIP_WD(XT, OUT) return wd_launch_t<XT, OUT>(qs, ds, x, y, m, n, k, slices, ldy, s)
+    if (type == kWdBf16) {
+        if (out == kWdOutF32) LHIP_WD(__bf16, kWdOutF32);
+        if (out == kWdOutBf16) LHIP_WD(__bf16, kWdOutBf16);
+        if (out == kWdOutSwiglu) LHIP_WD(__bf16, kWdOutSwiglu);
+    } else if (out == kWdOutF16) {
+        LHIP_WD(_Float16, kWdOutF16);
     }
 #undef LHIP_WD
     return LHIP_ERR_UNSUPPORTED;
-}
-
-lhip_status q8_gemm_wide_split(const float *x, void *planes, int64_t m, int64_t k, hipStream_t s) {
-    const size_t quads = static_cast<size_t>(m) * k / 4;
-    const size_t blocks = (quads + 255) / 256;
-    hipLaunchKernelGGL(q8_gemm_wide_split_kernel, dim3(static_cast<unsigned>(blocks < 2048 ? blocks : 2048)), dim3(256), 0, s,
-                       reinterpret_cast<const wd_f32x4 *>(x), static_cast<wd_u32x2 *>(planes), quads);
-    LHIP_CHECK_LAUNCH();
-    return LHIP_OK;
 }
 
 }  // namespace lhip

@@ -28,7 +28,7 @@ namespace lhip {
 // q8_gemm_skinny.hip: the matrix-core form with f32-accurate (head + tail bf16) operands for several activation rows.
 bool q8_gemm_split_supports(int n, int k, const void *x, const void *y, bool f16);
 lhip_status q8_gemm_split_launch(const int8_t *qs, const __half *ds, const void *x, void *y, int64_t m, int n, int k,
-                                 bool f16, int splits, hipStream_t s, bool own_workspace = false, float *ws = nullptr,
+                                 bool f16, hipStream_t s, bool own_workspace = false, float *ws = nullptr,
                                  size_t ws_floats = 0);
 size_t q8_gemm_split_workspace_floats(int64_t m, int n, int k);
 // From this many activation rows on the plain operators take that form where the shape allows it: the weights are
@@ -41,6 +41,17 @@ static int split_min_rows(int64_t n, int64_t k) {
     return codes >= (int64_t{256} << 20) ? 2 : codes >= (int64_t{32} << 20) ? 3 : codes >= (int64_t{8} << 20) ? 4 : 6;
 }
 
+// Whether a product of m rows is one for the matrix cores.  The streaming kernel's shapes (K in steps of 512, N of 4)
+// from split_min_rows on.  Every other K from 256 on by q8_gemm_rows.hip, whose workgroups take 256 weight rows and whose
+// result is a sum of K slices, 10 to 14 us at least, against one matvec per row.  Measured, matvecs -> matrix cores, us:
+// 2880 x 2880 f32 at 8 / 45 / 200 rows 19.5 -> 16.3 / 97 -> 18 / 423 -> 28, f16 at 8 / 45 rows 12.9 -> 15.8 / 48 -> 17;
+// 1000 x 4480 f32 at 12 rows 18.8 -> 18.9.  A K below 256 is a matvec of one or two microseconds per row.
+static bool on_matrix_cores(int64_t m, int64_t n, int64_t k, const void *x, const void *y, bool f16) {
+    if (q8_gemm_split_supports(static_cast<int>(n), static_cast<int>(k), x, y, f16)) return m >= split_min_rows(n, k);
+    const int64_t codes = n * k;
+    const int64_t min_rows = codes >= (int64_t{32} << 20) ? 3 : codes >= (int64_t{16} << 20) ? 6 : codes >= (int64_t{8} << 20) ? 8 : 12;
+    return k >= 256 && aligned(x, 16) && m >= (f16 ? min_rows * 5 / 4 : min_rows);
+}
 
 }  // namespace lhip
 
@@ -544,12 +555,15 @@ static lhip_status check_args(const void *planar, const float *x, float *y, int6
 
 using namespace lhip;
 
-extern "C" {
+static lhip_status matrix_cores(const void *planar, const void *x, void *y, int64_t m, int64_t n, int64_t k, bool f16, void *stream,
+                                bool own_workspace = false, void *ws = nullptr, size_t ws_nbytes = 0) {
+    auto *base = static_cast<const uint8_t *>(planar);
+    return q8_gemm_split_launch(reinterpret_cast<const int8_t *>(base), reinterpret_cast<const __half *>(base + q8_scale_offset(n, k)),
+                                x, y, m, static_cast<int>(n), static_cast<int>(k), f16, as_stream(stream), own_workspace,
+                                static_cast<float *>(ws), ws ? ws_nbytes / sizeof(float) : 0);
+}
 
-lhip_status lhip_q8_0_matmul_f32_gemm(const void *planar_dev, const float *x_dev, float *y_dev, int64_t m, int64_t n,
-                                      int64_t k, void *stream);
-lhip_status lhip_q8_0_matmul_f16_gemm(const void *planar_dev, const void *x_f16_dev, void *y_f16_dev, int64_t m,
-                                      int64_t n, int64_t k, void *stream);
+extern "C" {
 
 lhip_status lhip_q8_0_matmul_f32_cfg(const void *planar_dev, const float *x_dev, float *y_dev, int64_t m, int64_t n,
                                      int64_t k, int rows_per_wave, int k_unroll, int blocks_per_cu,
@@ -571,8 +585,8 @@ lhip_status lhip_q8_0_matmul_f32_cfg(const void *planar_dev, const float *x_dev,
 lhip_status lhip_q8_0_matmul_f32(const void *planar_dev, const float *x_dev, float *y_dev, int64_t m, int64_t n,
                                  int64_t k, void *stream) {
     if (lhip_status s = check_args(planar_dev, x_dev, y_dev, m, n, k)) return s;
-    if (m >= split_min_rows(n, k) && q8_gemm_split_supports(static_cast<int>(n), static_cast<int>(k), x_dev, y_dev, false))
-        return lhip_q8_0_matmul_f32_gemm(planar_dev, x_dev, y_dev, m, n, k, stream);
+    if (on_matrix_cores(m, n, k, x_dev, y_dev, false))
+        return matrix_cores(planar_dev, x_dev, y_dev, m, n, k, false, stream);
     int r, u, b, w;
     choose(static_cast<int>(n), static_cast<int>(k), &r, &u, &b, &w);
     return lhip_q8_0_matmul_f32_cfg(planar_dev, x_dev, y_dev, m, n, k, r, u, b, w, stream);
@@ -608,8 +622,8 @@ lhip_status lhip_q8_0_matmul_f16(const void *planar_dev, const void *x_f16_dev, 
     if (m <= 0 || m > kMaxDim) return LHIP_ERR_INVALID_SHAPE;
     // Rows of x start at multiples of K halves; K % 32 == 0 keeps them 8-byte aligned.
     if (!aligned(planar_dev, 256) || !aligned(x_f16_dev, 8) || !aligned(y_f16_dev, 2)) return LHIP_ERR_MISALIGNED;
-    if (m >= split_min_rows(n, k) && q8_gemm_split_supports(static_cast<int>(n), static_cast<int>(k), x_f16_dev, y_f16_dev, true))
-        return lhip_q8_0_matmul_f16_gemm(planar_dev, x_f16_dev, y_f16_dev, m, n, k, stream);
+    if (on_matrix_cores(m, n, k, x_f16_dev, y_f16_dev, true))
+        return matrix_cores(planar_dev, x_f16_dev, y_f16_dev, m, n, k, true, stream);
     auto *base = static_cast<const uint8_t *>(planar_dev);
     int r, u, b, w;
     choose(static_cast<int>(n), static_cast<int>(k), &r, &u, &b, &w);
@@ -629,10 +643,7 @@ lhip_status lhip_q8_0_matmul_f32_gemm(const void *planar_dev, const float *x_dev
                                       int64_t k, void *stream) {
     if (lhip_status s = check_args(planar_dev, x_dev, y_dev, m, n, k)) return s;
     if (!q8_gemm_split_supports(static_cast<int>(n), static_cast<int>(k), x_dev, y_dev, false)) return LHIP_ERR_UNSUPPORTED;
-    auto *base = static_cast<const uint8_t *>(planar_dev);
-    return q8_gemm_split_launch(reinterpret_cast<const int8_t *>(base),
-                                reinterpret_cast<const __half *>(base + q8_scale_offset(n, k)), x_dev, y_dev, m,
-                                static_cast<int>(n), static_cast<int>(k), false, 0, as_stream(stream));
+    return matrix_cores(planar_dev, x_dev, y_dev, m, n, k, false, stream);
 }
 
 lhip_status lhip_q8_0_matmul_f16_gemm(const void *planar_dev, const void *x_f16_dev, void *y_f16_dev, int64_t m,
@@ -643,15 +654,12 @@ lhip_status lhip_q8_0_matmul_f16_gemm(const void *planar_dev, const void *x_f16_
     if (!aligned(planar_dev, 256) || !aligned(x_f16_dev, 8) || !aligned(y_f16_dev, 2)) return LHIP_ERR_MISALIGNED;
     if (!q8_gemm_split_supports(static_cast<int>(n), static_cast<int>(k), x_f16_dev, y_f16_dev, true))
         return LHIP_ERR_UNSUPPORTED;
-    auto *base = static_cast<const uint8_t *>(planar_dev);
-    return q8_gemm_split_launch(reinterpret_cast<const int8_t *>(base),
-                                reinterpret_cast<const __half *>(base + q8_scale_offset(n, k)), x_f16_dev, y_f16_dev, m,
-                                static_cast<int>(n), static_cast<int>(k), true, 0, as_stream(stream));
+    return matrix_cores(planar_dev, x_f16_dev, y_f16_dev, m, n, k, true, stream);
 }
 
 size_t lhip_q8_0_matmul_workspace_nbytes(int64_t m, int64_t n, int64_t k) {
     if (check_q8_shape(n, k) != LHIP_OK || m <= 0 || m > kMaxDim) return 0;
-    if (m < split_min_rows(n, k) || k % 512 != 0 || n % 4 != 0) return 0;  // the matvec kernels keep nothing outside their outputs
+    if (!on_matrix_cores(m, n, k, nullptr, nullptr, false)) return 0;  // the matvec kernels keep nothing outside their outputs
     return q8_gemm_split_workspace_floats(m, static_cast<int>(n), static_cast<int>(k)) * sizeof(float);
 }
 
@@ -659,13 +667,8 @@ lhip_status lhip_q8_0_matmul_f32_ws(const void *planar_dev, const float *x_dev, 
                                     int64_t k, void *workspace_dev, size_t workspace_nbytes, void *stream) {
     if (lhip_status s = check_args(planar_dev, x_dev, y_dev, m, n, k)) return s;
     if (workspace_dev && !aligned(workspace_dev, 256)) return LHIP_ERR_MISALIGNED;
-    if (m >= split_min_rows(n, k) && q8_gemm_split_supports(static_cast<int>(n), static_cast<int>(k), x_dev, y_dev, false)) {
-        auto *base = static_cast<const uint8_t *>(planar_dev);
-        return q8_gemm_split_launch(reinterpret_cast<const int8_t *>(base),
-                                    reinterpret_cast<const __half *>(base + q8_scale_offset(n, k)), x_dev, y_dev, m,
-                                    static_cast<int>(n), static_cast<int>(k), false, 0, as_stream(stream), true,
-                                    static_cast<float *>(workspace_dev), workspace_dev ? workspace_nbytes / sizeof(float) : 0);
-    }
+    if (on_matrix_cores(m, n, k, x_dev, y_dev, false))
+        return matrix_cores(planar_dev, x_dev, y_dev, m, n, k, false, stream, true, workspace_dev, workspace_nbytes);
     return lhip_q8_0_matmul_f32(planar_dev, x_dev, y_dev, m, n, k, stream);  // matvec kernels: no shared state
 }
 
@@ -676,13 +679,8 @@ lhip_status lhip_q8_0_matmul_f16_ws(const void *planar_dev, const void *x_f16_de
     if (m <= 0 || m > kMaxDim) return LHIP_ERR_INVALID_SHAPE;
     if (!aligned(planar_dev, 256) || !aligned(x_f16_dev, 8) || !aligned(y_f16_dev, 2)) return LHIP_ERR_MISALIGNED;
     if (workspace_dev && !aligned(workspace_dev, 256)) return LHIP_ERR_MISALIGNED;
-    if (m >= split_min_rows(n, k) && q8_gemm_split_supports(static_cast<int>(n), static_cast<int>(k), x_f16_dev, y_f16_dev, true)) {
-        auto *base = static_cast<const uint8_t *>(planar_dev);
-        return q8_gemm_split_launch(reinterpret_cast<const int8_t *>(base),
-                                    reinterpret_cast<const __half *>(base + q8_scale_offset(n, k)), x_f16_dev, y_f16_dev, m,
-                                    static_cast<int>(n), static_cast<int>(k), true, 0, as_stream(stream), true,
-                                    static_cast<float *>(workspace_dev), workspace_dev ? workspace_nbytes / sizeof(float) : 0);
-    }
+    if (on_matrix_cores(m, n, k, x_f16_dev, y_f16_dev, true))
+        return matrix_cores(planar_dev, x_f16_dev, y_f16_dev, m, n, k, true, stream, true, workspace_dev, workspace_nbytes);
     return lhip_q8_0_matmul_f16(planar_dev, x_f16_dev, y_f16_dev, m, n, k, stream);
 }
 

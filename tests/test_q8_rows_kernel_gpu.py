@@ -1,0 +1,72 @@
+"""The f32 / f16 operators at the sizes where the kernel for many rows and for any K (q8_gemm_rows.hip) has an edge, through
+lhip_q8_0_matmul_f32 / _f16, against the f64 product.
+
+A result adds, per Q8_0 block, at most 96 exact products in f32 and then one scaled sum per block and one per K slice (at
+most 16): its error is below (96 + K / 32 + 16) * 2^-24 of the sum of the terms' magnitudes, and an f16 result is that
+rounded once (2^-11 of its size, 2^-25 where it is subnormal).
+"""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+from luminal_amd import capi, synth  # noqa: E402
+from luminal_amd.quantized import Q8Weight, QuantizedMatmul  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+# K of 8, 9, 10, 11 and 33 blocks: whole groups of four and every remainder; m of one wave's rows and around a tile; N of
+# one row, around a tile, odd (the slices' sum and the stores element by element); last: leading columns in whole rounds
+# of workgroups and the rest over K slices
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16], ids=["f32", "f16"])
+@pytest.mark.parametrize("m,n,k", [(16, 1, 256), (17, 255, 288), (127, 257, 320), (128, 258, 352), (129, 1001, 1056),
+                                   (300, 516, 4128), (200, 4096, 1024), (300, 28671, 1280)])
+def test_rows_kernel_edges(oracle, dtype, m, n, k):
+    qs, d = synth.q8_0_random(n, k, seed=m + n + k)
+    raw = synth.q8_0_raw_blocks(qs, d)
+    x = torch.from_numpy(synth.activations(m, k, seed=m * n)).to(DEV).to(dtype)
+    y = QuantizedMatmul().process(x, Q8Weight.from_raw(raw, n, k, DEV)).cpu().numpy().astype(np.float64)
+    xf = x.cpu().numpy().astype(np.float64)
+    wf = oracle.q8_0_dequant(raw, qs.size).reshape(qs.shape).astype(np.float64).T
+    truth, bound = xf @ wf, (np.abs(xf) @ np.abs(wf)) * (96 + k // 32 + 16) * 2.0 ** -24
+    if dtype == torch.float16:
+        bound += np.abs(truth) * 2.0 ** -11 + 2.0 ** -25
+    assert y.shape == (m, n) and np.all(np.abs(y - truth) <= bound)
+
+
+def test_f16_subnormal_activations_are_not_flushed():
+    """Every f16 subnormal times codes of one and power-of-two scales: exact in f32, exact again as f16."""
+    m, n, k = 128, 4096, 1024
+    x = np.zeros((m, k), np.float16)
+    x[np.arange(1023) % m, np.arange(1023)] = (np.arange(1, 1024, dtype=np.uint16)).view(np.float16)
+    w = Q8Weight.from_raw(synth.q8_0_raw_blocks(np.ones((n, k), np.int8), np.ones((n, k // 32), np.float16)), n, k, DEV)
+    y = QuantizedMatmul().process(torch.from_numpy(x).to(DEV), w).cpu().numpy()
+    want = x.astype(np.float64).sum(axis=1)
+    assert np.array_equal(y.astype(np.float64), np.repeat(want.astype(np.float16).astype(np.float64)[:, None], n, axis=1))
+
+
+@pytest.mark.parametrize("m,n,k", [(45, 2880, 2880), (128, 14336, 4096)])
+def test_workspace_form_of_any_k(m, n, k):
+    """The K slices of these products in the caller's workspace: the plain call's bits with the recommended size, the
+    product within the f32 bound of the order of its sums without one."""
+    lib = capi.load_library()
+    s = torch.cuda.current_stream().cuda_stream
+    w = Q8Weight.from_raw(synth.q8_0_raw_blocks(*synth.q8_0_random(n, k, seed=1)), n, k, DEV)
+    for dtype, plain, ws in ((torch.float32, lib.lhip_q8_0_matmul_f32, lib.lhip_q8_0_matmul_f32_ws),
+                             (torch.float16, lib.lhip_q8_0_matmul_f16, lib.lhip_q8_0_matmul_f16_ws)):
+        x = torch.from_numpy(synth.activations(m, k, seed=2)).to(DEV).to(dtype)
+        nbytes = lib.lhip_q8_0_matmul_workspace_nbytes(m, n, k)
+        assert nbytes > 0
+        space = torch.empty(nbytes, dtype=torch.uint8, device=DEV)
+        y, y_ws, y_none = (torch.full((m, n), float("nan"), device=DEV, dtype=dtype) for _ in range(3))
+        capi.check(plain(w.planar.data_ptr(), x.data_ptr(), y.data_ptr(), m, n, k, s), "plain")
+        capi.check(ws(w.planar.data_ptr(), x.data_ptr(), y_ws.data_ptr(), m, n, k, space.data_ptr(), nbytes, s), "ws")
+        capi.check(ws(w.planar.data_ptr(), x.data_ptr(), y_none.data_ptr(), m, n, k, None, 0, s), "none")
+        torch.cuda.synchronize()
+        assert torch.equal(y.view(torch.uint8), y_ws.view(torch.uint8))
+        eps = 2.0 ** -24 if dtype == torch.float32 else 2.0 ** -10
+        size = x.float().abs() @ w.dequantize().abs().t()
+        assert bool(((y.float() - y_none.float()).abs() <= size * 2 * (96 + k // 32 + 16) * 2.0 ** -24 + y.float().abs() * eps).all())
