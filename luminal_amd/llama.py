@@ -18,7 +18,7 @@ import numpy as np
 import torch
 
 from . import capi
-from .quantized import DecodeProgram, FusedMatvec, Q8Weight
+from .quantized import DecodeProgram, FusedMatvec, Q8Weight, _stream as _s
 
 
 @dataclass(frozen=True)
@@ -43,10 +43,6 @@ class LlamaConfig:
 
 
 LLAMA3_8B = LlamaConfig()
-
-
-def _s() -> int:
-    return torch.cuda.current_stream().cuda_stream
 
 
 class LlamaQ8:

@@ -7,10 +7,7 @@ import numpy as np
 import torch
 
 from . import capi
-
-
-def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+from .quantized import _stream, launch
 
 
 class Mxfp4Weight:
@@ -70,9 +67,8 @@ def route_topk(logits: torch.Tensor, topk: int):
     t, e = logits.shape
     sel = torch.empty((t, topk), dtype=torch.int32, device=logits.device)
     wts = torch.empty((t, topk), dtype=torch.float32, device=logits.device)
-    with torch.cuda.device(logits.device):
-        capi.check(lib.lhip_moe_route_topk(logits.data_ptr(), sel.data_ptr(), wts.data_ptr(), t, e, topk, _stream()),
-                   "lhip_moe_route_topk")
+    capi.check(launch(logits.device, lib.lhip_moe_route_topk, logits.data_ptr(), sel.data_ptr(), wts.data_ptr(), t, e, topk),
+               "lhip_moe_route_topk")
     return sel, wts
 
 
@@ -100,10 +96,9 @@ class MoEExperts:
         if self._ws is None or self._ws.numel() < need:
             self._ws = torch.empty(need, dtype=torch.uint8, device=x.device)
         y = torch.empty((t, self.h), dtype=torch.bfloat16, device=x.device)
-        with torch.cuda.device(x.device):
-            st = lib.lhip_mxfp4_moe_bf16_mode(self.gu.planar.data_ptr(), self.dn.planar.data_ptr(), x.data_ptr(),
-                                              sel.contiguous().data_ptr(), wts.contiguous().data_ptr(), y.data_ptr(), t,
-                                              self.h, self.i, self.e, topk, mode, self._ws.data_ptr(), _stream())
+        sel, wts = sel.contiguous(), wts.contiguous()  # (held until the launch)
+        st = launch(x.device, lib.lhip_mxfp4_moe_bf16_mode, self.gu.planar.data_ptr(), self.dn.planar.data_ptr(), x.data_ptr(),
+                    sel.data_ptr(), wts.data_ptr(), y.data_ptr(), t, self.h, self.i, self.e, topk, mode, self._ws.data_ptr())
         capi.check(st, "lhip_mxfp4_moe_bf16_mode")
         self._last = (t, topk, mode)
         return y
