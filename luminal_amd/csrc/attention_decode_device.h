@@ -25,6 +25,7 @@ namespace lhip {
 
 constexpr int kDecThreads = 256;
 constexpr int kDecTile = 64;
+constexpr int kDecCachedKeys = 32;
 
 __device__ __forceinline__ float wave_max64(float v) {
     for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
@@ -58,6 +59,11 @@ __device__ __forceinline__ void stg4(float4 *p, const float4 &v) {
     lhip_f32x4 t;
     t.x = v.x; t.y = v.y; t.z = v.z; t.w = v.w;
     *as_global(reinterpret_cast<lhip_f32x4 *>(p)) = t;
+}
+
+__device__ __forceinline__ float4 ldg4_nt(const float4 *p) {
+    const lhip_f32x4 v = __builtin_nontemporal_load(as_global(reinterpret_cast<const lhip_f32x4 *>(p)));
+    return make_float4(v[0], v[1], v[2], v[3]);
 }
 
 // ---- agent-coherent accessors (relaxed atomics at agent scope: single instructions with the coherence bit set)
@@ -209,11 +215,16 @@ struct AttnShared {
 // the caches when the range holds the new position, attention over the range, partial state to the workspace.
 //
 // Inside a workgroup (256 working threads), per tile of 64 keys:
-//   scores: 4 lanes per key, each reading float4 columns sub, sub+4, ... of the row, so a
-//           quad covers 64 contiguous bytes per load; q for the G heads comes from LDS;
+//   scores: 8 lanes per key, each reading float4 columns sub, sub+8, ... of the row, so that
+//           a load covers whole 128-byte lines, two keys per lane; q for the G heads comes from LDS;
 //   online softmax: wave w owns heads w, w+4: lane = key;
 //   P.V:    HD/4 lanes cover a V row as float4, 256/(HD/4) key groups split the tile.
-// The K and V loads of a tile are all issued before the first use.
+// The K and V loads of a tile are all issued before the first use.  Behind a long context they are what bounds the
+// kernel (8000 keys: 65 MB), and how they are asked for decides the rate: whole lines a load, and past the caches where
+// a range has more than kDecCachedKeys keys.  With the merge, 32 query heads on 8 of 128, cached half lines -> this:
+// 1000 / 2040 / 2100 / 4000 / 8000 / 12000 keys 11.3 / 13.6 / 17.5 / 20.6 / 28.3 / 35.2 -> 11.4 / 12.4 / 15.4 / 16.6 /
+// 23.8 / 30.4 us; at 300 keys loads past the caches cost 0.3 us more (11.1 against 10.8).  Two or three tiles in flight
+// (as many sets of registers) change nothing.
 template <int G, int HD, int THREADS, typename IO>
 __device__ __forceinline__ void attention_decode_body(IO io, AttnShared<G, HD> &sh, int kvh, int split,
                                                       const float *__restrict__ qkv, float *__restrict__ k_cache,
@@ -242,19 +253,32 @@ __device__ __forceinline__ void attention_decode_body(IO io, AttnShared<G, HD> &
     // ---- cache rows of a tile of keys: all loads issued before the first use.  The first tile is requested at
     // once, ahead of the wait for q: the caches do not depend on it (the row of the new position, which may not
     // have been written yet, is replaced from LDS below).
-    const int sub = tid & 3, kslot = (tid >> 2) & (kDecTile - 1);  // scores: 4 lanes per key
-    const int c4 = tid % C4, kgp = (tid / C4) % KG;                // P.V: column and key group
-    float4 kreg[J];
+    const int sub = tid & 7, kslot = (tid >> 3) & (kDecTile / 2 - 1);  // scores: 8 lanes per key, keys kslot and kslot + 32
+    const int c4 = tid % C4, kgp = (tid / C4) % KG;                    // P.V: column and key group
+    float4 kreg[2][J / 2];
     float4 vreg[KPG];
-    auto load_tile = [&](int t0) {
-        const int key = t0 + kslot;
-        const float4 *krow = kc4 + static_cast<size_t>(key < k1 ? key : k0) * C4;
+    const bool past_caches = k1 - k0 > kDecCachedKeys;  // uniform
+    auto load_rows = [&](int t0, auto load) __attribute__((always_inline)) {
 #pragma unroll
-        for (int j = 0; j < J; ++j) kreg[j] = ldg4(krow + j * 4 + sub);
+        for (int i = 0; i < 2; ++i) {
+            const int key = t0 + kslot + i * (kDecTile / 2);
+            const float4 *krow = kc4 + static_cast<size_t>(key < k1 ? key : k0) * C4;
+#pragma unroll
+            for (int j = 0; j < J / 2; ++j) kreg[i][j] = load(krow + j * 8 + sub);
+        }
 #pragma unroll
         for (int u = 0; u < KPG; ++u) {
             const int vkey = t0 + kgp + KG * u;
-            vreg[u] = ldg4(vc4 + static_cast<size_t>(vkey < k1 ? vkey : k0) * C4 + c4);
+            vreg[u] = load(vc4 + static_cast<size_t>(vkey < k1 ? vkey : k0) * C4 + c4);
+        }
+    };
+    auto load_tile = [&](int t0) __attribute__((always_inline)) {
+        if (past_caches) {
+            asm volatile("" ::: "memory");  // (or the two branches' loads become one, and cached)
+            load_rows(t0, [](const float4 *p) { return ldg4_nt(p); });
+            asm volatile("" ::: "memory");
+        } else {
+            load_rows(t0, [](const float4 *p) { return ldg4(p); });
         }
     };
     if (on && k0 < k1) load_tile(k0);
@@ -306,37 +330,42 @@ __device__ __forceinline__ void attention_decode_body(IO io, AttnShared<G, HD> &
     for (int g = 0; g < G; ++g) acc[g] = make_float4(0, 0, 0, 0);
     for (int t0 = k0; t0 < k1; t0 += kDecTile) {
         // ---- the tile's cache rows; the new position is served from LDS (its cache row may not have landed)
-        const int key = t0 + kslot;
-        const bool live = key < k1;
         if (on) {
             if (t0 != k0) load_tile(t0);
-            if (key == pos) {
 #pragma unroll
-                for (int j = 0; j < J; ++j) kreg[j] = sh.knew[j * 4 + sub];
-            }
+            for (int i = 0; i < 2; ++i)
+                if (t0 + kslot + i * (kDecTile / 2) == pos) {
+#pragma unroll
+                    for (int j = 0; j < J / 2; ++j) kreg[i][j] = sh.knew[j * 8 + sub];
+                }
 #pragma unroll
             for (int u = 0; u < KPG; ++u)
                 if (t0 + kgp + KG * u == pos) vreg[u] = sh.vnew[c4];
             // ---- scores
-            float s[G];
 #pragma unroll
-            for (int g = 0; g < G; ++g) {
-                float d = 0.f;
+            for (int i = 0; i < 2; ++i) {
+                const int slot = kslot + i * (kDecTile / 2);
+                float s[G];
 #pragma unroll
-                for (int j = 0; j < J; ++j) {
-                    const float4 qv = sh.q_s[g][j * 4 + sub];
-                    d = fmaf(qv.x, kreg[j].x, d);
-                    d = fmaf(qv.y, kreg[j].y, d);
-                    d = fmaf(qv.z, kreg[j].z, d);
-                    d = fmaf(qv.w, kreg[j].w, d);
+                for (int g = 0; g < G; ++g) {
+                    float d = 0.f;
+#pragma unroll
+                    for (int j = 0; j < J / 2; ++j) {
+                        const float4 qv = sh.q_s[g][j * 8 + sub], kv = kreg[i][j];
+                        d = fmaf(qv.x, kv.x, d);
+                        d = fmaf(qv.y, kv.y, d);
+                        d = fmaf(qv.z, kv.z, d);
+                        d = fmaf(qv.w, kv.w, d);
+                    }
+                    d += __shfl_xor(d, 1);
+                    d += __shfl_xor(d, 2);
+                    d += __shfl_xor(d, 4);
+                    s[g] = d * inv_sqrt;
                 }
-                d += __shfl_xor(d, 1);
-                d += __shfl_xor(d, 2);
-                s[g] = d * inv_sqrt;
-            }
-            if (sub == 0) {
+                if (sub == 0) {
 #pragma unroll
-                for (int g = 0; g < G; ++g) sh.p_s[g][kslot] = live ? s[g] : -INFINITY;
+                    for (int g = 0; g < G; ++g) sh.p_s[g][slot] = t0 + slot < k1 ? s[g] : -INFINITY;
+                }
             }
         }
         __syncthreads();
