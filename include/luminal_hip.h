@@ -112,9 +112,10 @@ lhip_status lhip_q8_0_matmul_f32(const void *planar_dev, const float *x_dev, flo
  * LHIP_ERR_UNSUPPORTED unless K % 512 == 0, N % 4 == 0, x 16-byte and y 16-byte (f16: 8-byte) aligned.
  * lhip_q8_0_matmul_f32 and lhip_q8_0_matmul_f16 take this form by themselves from a few rows on (two for N*K >=
  * 2^28 codes, three from 2^25, four from 2^23, six below: the measured crossovers with the matvec form) where those
- * conditions hold, and from three to fifteen rows on, by size, for every other K >= 256 and every N (the _cfg entry
- * never does).  May keep partial sums in the library's scratch array, see the
- * note on overlapping calls at lhip_q8_0_matmul_bf16. */
+ * conditions hold, and may then keep partial sums in the library's scratch array, see the note on overlapping calls at
+ * lhip_q8_0_matmul_bf16.  For every other K >= 256 and every N they keep nothing outside their outputs: the matrix cores
+ * without K slices where the rows are many enough for that, else one matvec per row; the _ws forms below with a workspace
+ * slice K there and take the matrix cores from three to fifteen rows on, by size.  The _cfg entry never does. */
 lhip_status lhip_q8_0_matmul_f32_gemm(const void *planar_dev, const float *x_dev, float *y_dev, int64_t m, int64_t n,
                                       int64_t k, void *stream);
 lhip_status lhip_q8_0_matmul_f16_gemm(const void *planar_dev, const void *x_f16_dev, void *y_f16_dev, int64_t m,
@@ -252,7 +253,8 @@ lhip_status lhip_q8_0_gather_f16(const void *planar_dev, const float *idx_dev, v
  * in time on one device (different streams) race; the reference's operators (quantized.rs:116-149) have no such
  * constraint.  These forms keep the partial sums in the caller's workspace instead and touch no shared state:
  *   workspace_dev of lhip_q8_0_matmul_workspace_nbytes(m, n, k) bytes (256-byte aligned; 0 bytes: none is needed,
- *   NULL is fine) gives the plan, and the bits, of the plain call;
+ *   NULL is fine) gives the plan, and the bits, of the plain call where K % 512 == 0 and N % 4 == 0, and the plan with K
+ *   slices elsewhere, where the plain call has none;
  *   a smaller one, or NULL, means fewer or no K slices: same accuracy, last bits may differ, and a short-and-small
  *   product (few rows, few weight rows) leaves compute units idle.
  * Calls sharing a workspace must be ordered on one stream.  Other arguments and errors as the plain forms. */

@@ -46,11 +46,21 @@ static int split_min_rows(int64_t n, int64_t k) {
 // result is a sum of K slices, 10 to 14 us at least, against one matvec per row.  Measured, matvecs -> matrix cores, us:
 // 2880 x 2880 f32 at 8 / 45 / 200 rows 19.5 -> 16.3 / 97 -> 18 / 423 -> 28, f16 at 8 / 45 rows 12.9 -> 15.8 / 48 -> 17;
 // 1000 x 4480 f32 at 12 rows 18.8 -> 18.9.  A K below 256 is a matvec of one or two microseconds per row.
-static bool on_matrix_cores(int64_t m, int64_t n, int64_t k, const void *x, const void *y, bool f16) {
+// Without room for the slices' planes - the plain operators, which for these K keep nothing outside their outputs, so that
+// calls on several streams may overlap - it is one slice, 1.2 (f32) or 0.66 us (f16) per block of K and round of 256
+// workgroups, against matvecs of 0.17 or 0.085 us per 2^20 codes and row (where they are cheapest, so that nothing gets
+// slower).  Measured, matvecs -> one slice -> sliced, us: 2880 x 2880 f32 at 96 rows 203 -> 86 -> 26, f16 at 128 rows 109 ->
+// 52 -> 21; 14336 x 4128 f32 at 32 rows 367 -> 80 -> 32; 512 x 14304 f32 at 512 rows 1073 -> 424 -> 47.
+static bool on_matrix_cores(int64_t m, int64_t n, int64_t k, const void *x, const void *y, bool f16, size_t room_floats) {
     if (q8_gemm_split_supports(static_cast<int>(n), static_cast<int>(k), x, y, f16)) return m >= split_min_rows(n, k);
+    if (k < 256 || !aligned(x, 16)) return false;
     const int64_t codes = n * k;
     const int64_t min_rows = codes >= (int64_t{32} << 20) ? 3 : codes >= (int64_t{16} << 20) ? 6 : codes >= (int64_t{8} << 20) ? 8 : 12;
-    return k >= 256 && aligned(x, 16) && m >= (f16 ? min_rows * 5 / 4 : min_rows);
+    if (m < (f16 ? min_rows * 5 / 4 : min_rows)) return false;
+    if (room_floats >= q8_gemm_split_workspace_floats(m, static_cast<int>(n), static_cast<int>(k))) return true;
+    const int64_t rounds = ((m + 127) / 128 * ((n + 255) / 256) + 255) / 256;
+    return static_cast<double>(m) * static_cast<double>(codes) * (f16 ? 0.085 : 0.17) / (1 << 20) >
+           8.0 + static_cast<double>(rounds * (k / 32)) * (f16 ? 0.66 : 1.2);
 }
 
 }  // namespace lhip
@@ -585,8 +595,9 @@ lhip_status lhip_q8_0_matmul_f32_cfg(const void *planar_dev, const float *x_dev,
 lhip_status lhip_q8_0_matmul_f32(const void *planar_dev, const float *x_dev, float *y_dev, int64_t m, int64_t n,
                                  int64_t k, void *stream) {
     if (lhip_status s = check_args(planar_dev, x_dev, y_dev, m, n, k)) return s;
-    if (on_matrix_cores(m, n, k, x_dev, y_dev, false))
-        return matrix_cores(planar_dev, x_dev, y_dev, m, n, k, false, stream);
+    if (on_matrix_cores(m, n, k, x_dev, y_dev, false, 0))
+        return matrix_cores(planar_dev, x_dev, y_dev, m, n, k, false, stream,
+                            !q8_gemm_split_supports(static_cast<int>(n), static_cast<int>(k), x_dev, y_dev, false));
     int r, u, b, w;
     choose(static_cast<int>(n), static_cast<int>(k), &r, &u, &b, &w);
     return lhip_q8_0_matmul_f32_cfg(planar_dev, x_dev, y_dev, m, n, k, r, u, b, w, stream);
@@ -622,8 +633,9 @@ lhip_status lhip_q8_0_matmul_f16(const void *planar_dev, const void *x_f16_dev, 
     if (m <= 0 || m > kMaxDim) return LHIP_ERR_INVALID_SHAPE;
     // Rows of x start at multiples of K halves; K % 32 == 0 keeps them 8-byte aligned.
     if (!aligned(planar_dev, 256) || !aligned(x_f16_dev, 8) || !aligned(y_f16_dev, 2)) return LHIP_ERR_MISALIGNED;
-    if (on_matrix_cores(m, n, k, x_f16_dev, y_f16_dev, true))
-        return matrix_cores(planar_dev, x_f16_dev, y_f16_dev, m, n, k, true, stream);
+    if (on_matrix_cores(m, n, k, x_f16_dev, y_f16_dev, true, 0))
+        return matrix_cores(planar_dev, x_f16_dev, y_f16_dev, m, n, k, true, stream,
+                            !q8_gemm_split_supports(static_cast<int>(n), static_cast<int>(k), x_f16_dev, y_f16_dev, true));
     auto *base = static_cast<const uint8_t *>(planar_dev);
     int r, u, b, w;
     choose(static_cast<int>(n), static_cast<int>(k), &r, &u, &b, &w);
@@ -659,7 +671,7 @@ lhip_status lhip_q8_0_matmul_f16_gemm(const void *planar_dev, const void *x_f16_
 
 size_t lhip_q8_0_matmul_workspace_nbytes(int64_t m, int64_t n, int64_t k) {
     if (check_q8_shape(n, k) != LHIP_OK || m <= 0 || m > kMaxDim) return 0;
-    if (!on_matrix_cores(m, n, k, nullptr, nullptr, false)) return 0;  // the matvec kernels keep nothing outside their outputs
+    if (!on_matrix_cores(m, n, k, nullptr, nullptr, false, SIZE_MAX)) return 0;  // the matvec kernels keep nothing outside their outputs
     return q8_gemm_split_workspace_floats(m, static_cast<int>(n), static_cast<int>(k)) * sizeof(float);
 }
 
@@ -667,7 +679,7 @@ lhip_status lhip_q8_0_matmul_f32_ws(const void *planar_dev, const float *x_dev, 
                                     int64_t k, void *workspace_dev, size_t workspace_nbytes, void *stream) {
     if (lhip_status s = check_args(planar_dev, x_dev, y_dev, m, n, k)) return s;
     if (workspace_dev && !aligned(workspace_dev, 256)) return LHIP_ERR_MISALIGNED;
-    if (on_matrix_cores(m, n, k, x_dev, y_dev, false))
+    if (on_matrix_cores(m, n, k, x_dev, y_dev, false, workspace_dev ? workspace_nbytes / sizeof(float) : 0))
         return matrix_cores(planar_dev, x_dev, y_dev, m, n, k, false, stream, true, workspace_dev, workspace_nbytes);
     return lhip_q8_0_matmul_f32(planar_dev, x_dev, y_dev, m, n, k, stream);  // matvec kernels: no shared state
 }
@@ -679,7 +691,7 @@ lhip_status lhip_q8_0_matmul_f16_ws(const void *planar_dev, const void *x_f16_de
     if (m <= 0 || m > kMaxDim) return LHIP_ERR_INVALID_SHAPE;
     if (!aligned(planar_dev, 256) || !aligned(x_f16_dev, 8) || !aligned(y_f16_dev, 2)) return LHIP_ERR_MISALIGNED;
     if (workspace_dev && !aligned(workspace_dev, 256)) return LHIP_ERR_MISALIGNED;
-    if (on_matrix_cores(m, n, k, x_f16_dev, y_f16_dev, true))
+    if (on_matrix_cores(m, n, k, x_f16_dev, y_f16_dev, true, workspace_dev ? workspace_nbytes / sizeof(float) : 0))
         return matrix_cores(planar_dev, x_f16_dev, y_f16_dev, m, n, k, true, stream, true, workspace_dev, workspace_nbytes);
     return lhip_q8_0_matmul_f16(planar_dev, x_f16_dev, y_f16_dev, m, n, k, stream);
 }

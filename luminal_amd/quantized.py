@@ -33,6 +33,13 @@ def launch(device: torch.device, entry_point, *args) -> int:
         return entry_point(*args, _raw_stream(index))
 
 
+def _workspace(nbytes: int, device: torch.device):
+    """The (address, size) arguments of a `_ws` operator and what owns them: a call's partial sums in memory of its own
+    stream, so that calls on several streams never share any."""
+    space = torch.empty(nbytes, dtype=torch.uint8, device=device)
+    return (space.data_ptr(), nbytes), space
+
+
 def _ptr(t: torch.Tensor) -> int:
     return t.data_ptr()
 
@@ -127,13 +134,20 @@ class QuantizedMatmul:
         if dtype == torch.float16:
             if self.cfg:
                 raise TypeError("QuantizedMatmul: a launch shape can be chosen for f32 activations only")
-            capi.check(launch(device, lib.lhip_q8_0_matmul_f16, *args), "lhip_q8_0_matmul_f16")
-            return out
+            plain, with_workspace = lib.lhip_q8_0_matmul_f16, lib.lhip_q8_0_matmul_f16_ws
+        else:
+            plain, with_workspace = lib.lhip_q8_0_matmul_f32, lib.lhip_q8_0_matmul_f32_ws
         if self.cfg:
             st = launch(device, lib.lhip_q8_0_matmul_f32_cfg, *args, *self.cfg)
         else:
-            st = launch(device, lib.lhip_q8_0_matmul_f32, *args)
-        capi.check(st, "lhip_q8_0_matmul_f32")
+            # up to 64 rows of a K in steps of 512 the library's own scratch array serves, without the allocation
+            need = lib.lhip_q8_0_matmul_workspace_nbytes(m, n, k) if m > 64 or (m > 1 and (k % 512 or n % 4)) else 0
+            if need:
+                room, _space = _workspace(need, device)
+                st = launch(device, with_workspace, *args, *room)
+            else:
+                st = launch(device, plain, *args)
+        capi.check(st, "lhip_q8_0_matmul_f16" if dtype == torch.float16 else "lhip_q8_0_matmul_f32")
         return out
 
 
@@ -156,9 +170,16 @@ class QuantizedMatmulBf16:
         x = x.contiguous()
         n, k, device = w.n, w.k, x.device
         out = torch.empty((*x.shape[:-1], n), dtype=torch.bfloat16, device=device)
-        args = (w.planar.data_ptr(), x.data_ptr(), out.data_ptr(), x.numel() // k, n, k)
+        m = x.numel() // k
+        args = (w.planar.data_ptr(), x.data_ptr(), out.data_ptr(), m, n, k)
         if self.tile is None:
-            st = launch(device, lib.lhip_q8_0_matmul_bf16, *args)
+            # up to 128 rows the library's own scratch array serves, without the allocation
+            need = lib.lhip_q8_0_matmul_bf16_workspace_nbytes(m, n, k, 0) if m > 128 else 0
+            if need:
+                room, _space = _workspace(need, device)
+                st = launch(device, lib.lhip_q8_0_matmul_bf16_ws, *args, 0, *room)
+            else:
+                st = launch(device, lib.lhip_q8_0_matmul_bf16, *args)
         else:
             st = launch(device, lib.lhip_q8_0_matmul_bf16_cfg, *args, self.tile)
         capi.check(st, "lhip_q8_0_matmul_bf16")
