@@ -155,9 +155,10 @@ __global__ __launch_bounds__(768) void q8_gemm_rows_kernel(const int8_t *__restr
 #pragma unroll
         for (int w = 0; w < XW; ++w) xraw[set][w] = reinterpret_cast<const rw_u32x4 *>(x_src + static_cast<size_t>(bb) * 32)[w];
     };
-    // an f32 as three bf16 limbs whose sum it is: three successive roundings to nearest (8 + 8 + 8 significant bits)
+    // An f32 as three bf16 limbs whose sum it is: its upper half, that of what is left, and the rest (8 + 8 + 8 significant
+    // bits).  What is left lies between 0 and the value; taken as the median of the three it is 0 behind +inf and -inf behind
+    // -inf, where the difference is NaN, and the limbs still sum to the value.
     auto split_x = [&](int set) __attribute__((always_inline)) {
-        typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 #pragma unroll
         for (int w = 0; w < XW; ++w) asm volatile("" : "+v"(xraw[set][w]));  // the arithmetic stays here, behind the loads' wait
         if constexpr (L == 1) {
@@ -168,10 +169,10 @@ __global__ __launch_bounds__(768) void q8_gemm_rows_kernel(const int8_t *__restr
                 float a = __uint_as_float(xraw[set][e >> 1][(e & 1) * 2]), b = __uint_as_float(xraw[set][e >> 1][(e & 1) * 2 + 1]);
 #pragma unroll
                 for (int l = 0; l < L; ++l) {
-                    const bf16x2 h = {static_cast<__bf16>(a), static_cast<__bf16>(b)};
-                    xop[l][e] = __builtin_bit_cast(uint32_t, h);
-                    a -= __uint_as_float(xop[l][e] << 16);
-                    b -= __uint_as_float(xop[l][e] & 0xffff0000u);
+                    xop[l][e] = __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
+                    if (l + 1 == L) break;
+                    a = __builtin_amdgcn_fmed3f(a - __uint_as_float(__float_as_uint(a) & 0xffff0000u), 0.f, a);
+                    b = __builtin_amdgcn_fmed3f(b - __uint_as_float(__float_as_uint(b) & 0xffff0000u), 0.f, b);
                 }
             }
         }

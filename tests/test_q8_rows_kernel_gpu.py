@@ -102,3 +102,29 @@ def test_calls_of_any_k_overlap_on_two_streams(m, k):
     torch.cuda.synchronize()
     for i in range(2):
         assert all(torch.equal(y, want[i]) for y in outs[i]) and all(torch.equal(y, plain[i]) for y in raw[i])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16], ids=["f32", "f16"])
+def test_infinities_nan_and_the_largest_values_as_in_one_row_calls(dtype):
+    """Activations that are not finite, and the type's largest, against the matvec form row by row: the same infinities,
+    NaN in the same places (an infinity times a code of zero among them), finite sums within the order of the additions."""
+    m, n, k = 17, 257, 2848
+    lib = capi.load_library()
+    qs, d = synth.q8_0_random(n, k, seed=7)
+    qs[:, 11] = np.arange(n) % 3 - 1
+    w = Q8Weight.from_raw(synth.q8_0_raw_blocks(qs, d), n, k, DEV)
+    x = torch.from_numpy(synth.activations(m, k, seed=8)).to(DEV).to(dtype)
+    x[3, 5], x[4, 7], x[5, 9], x[6, 11] = float("inf"), float("-inf"), float("nan"), torch.finfo(dtype).max
+    x[7, 11], x[8, 11], x[9, 11] = -torch.finfo(dtype).max, float("inf"), float("-inf")
+    assert lib.lhip_q8_0_matmul_workspace_nbytes(m, n, k) > 0  # not one matvec per row
+    op = QuantizedMatmul()
+    got = op.process(x, w).cpu().numpy().astype(np.float64)
+    one = np.concatenate([op.process(x[i:i + 1], w).cpu().numpy() for i in range(m)]).astype(np.float64)
+    finite = np.isfinite(one)
+    assert np.array_equal(np.isnan(got), np.isnan(one)) and np.array_equal(got[np.isinf(one)], one[np.isinf(one)])
+    assert np.isinf(one).any() and np.isnan(one).any() and np.array_equal(np.isfinite(got), finite)
+    # both forms' errors are below (96 + K / 32 + 16) 2^-24 of the sum of the magnitudes, a half rounds each once
+    size = np.abs(np.where(np.isfinite(x.cpu().numpy()), x.cpu().numpy(), 0)).astype(np.float64) @ \
+        np.abs(w.dequantize().cpu().numpy().astype(np.float64)).T
+    bound = size * 2 * (96 + k // 32 + 16) * 2.0 ** -24 + (np.abs(one) * 2.0 ** -10 + 2.0 ** -24 if dtype == torch.float16 else 0)
+    assert np.all(np.abs(got[finite] - one[finite]) <= bound[finite])
