@@ -18,7 +18,7 @@ import numpy as np
 import torch
 
 from . import capi
-from .quantized import DecodeProgram, FusedMatvec, Q8Weight, _stream as _s
+from .quantized import DecodeProgram, FusedMatvec, Q8Weight, _stream as _s, _workspace, rows_workspace_nbytes
 
 
 @dataclass(frozen=True)
@@ -113,8 +113,12 @@ class LlamaQ8:
     def _matmul(self, w: Q8Weight, x, y, m, bf16):
         lib = self.lib
         if not bf16:
-            capi.check(lib.lhip_q8_0_matmul_f32(w.planar.data_ptr(), x.data_ptr(), y.data_ptr(), m, w.n, w.k, _s()),
-                       "lhip_q8_0_matmul_f32")
+            room, _space = _workspace(rows_workspace_nbytes(lib, m, w.n, w.k), x.device) if m > 1 else ((None, 0), None)
+            if room[1]:
+                st = lib.lhip_q8_0_matmul_f32_ws(w.planar.data_ptr(), x.data_ptr(), y.data_ptr(), m, w.n, w.k, *room, _s())
+            else:
+                st = lib.lhip_q8_0_matmul_f32(w.planar.data_ptr(), x.data_ptr(), y.data_ptr(), m, w.n, w.k, _s())
+            capi.check(st, "lhip_q8_0_matmul_f32")
             return
         xb = self._buf("xb", (m, w.k), torch.bfloat16)
         yb = self._buf("yb", (m, w.n), torch.bfloat16)

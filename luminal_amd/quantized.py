@@ -40,6 +40,12 @@ def _workspace(nbytes: int, device: torch.device):
     return (space.data_ptr(), nbytes), space
 
 
+def rows_workspace_nbytes(lib, m: int, n: int, k: int) -> int:
+    """Workspace that an f32 or f16 product is given: up to 64 rows of a K in steps of 512 the library's own scratch array
+    serves, without the allocation."""
+    return lib.lhip_q8_0_matmul_workspace_nbytes(m, n, k) if m > 64 or (m > 1 and (k % 512 or n % 4)) else 0
+
+
 def _ptr(t: torch.Tensor) -> int:
     return t.data_ptr()
 
@@ -140,8 +146,7 @@ class QuantizedMatmul:
         if self.cfg:
             st = launch(device, lib.lhip_q8_0_matmul_f32_cfg, *args, *self.cfg)
         else:
-            # up to 64 rows of a K in steps of 512 the library's own scratch array serves, without the allocation
-            need = lib.lhip_q8_0_matmul_workspace_nbytes(m, n, k) if m > 64 or (m > 1 and (k % 512 or n % 4)) else 0
+            need = rows_workspace_nbytes(lib, m, n, k)
             if need:
                 room, _space = _workspace(need, device)
                 st = launch(device, with_workspace, *args, *room)
