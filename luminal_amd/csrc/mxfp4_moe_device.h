@@ -41,17 +41,18 @@ struct MoePlan {
     // GEMMs walk a run column block by column block, so that the workgroups that read the same weights run together.
     int *tile_run0, *tile_runlen;
     int *n_tiles;      // [1]
-    int max_tiles;     // entries of the three tile arrays
+    int max_tiles;     // entries of the tile arrays
+    int fragment;      // rows of a matrix step: a tile is some number of these, but for the end of an expert
     // 0: tiles are listed in expert order from entry 0.  Otherwise the list is cut into eight ranges of this many
     // entries, one per XCD (range x is read by the workgroups whose dispatch number is x modulo 8), and the
-    // tiles, still in expert order, are dealt to the ranges in eight contiguous, equal shares: the tiles of an
+    // tiles, an expert's behind each other, are dealt to the ranges in eight contiguous, equal shares: the tiles of an
     // expert, and all column blocks of a tile, then run on one XCD and find each other's weights and
     // activation rows in its L2.
     int tiles_per_xcd;
 };
 
 __device__ __forceinline__ void moe_plan_block(const int *__restrict__ sel, int R, int E, int BM, const MoePlan &p) {
-    __shared__ int cnt[1024], off[1025], cur[1024];
+    __shared__ int cnt[1024], off[1025], cur[1024], pos[1024];
     for (int e = threadIdx.x; e < E; e += 1024) {
         cnt[e] = 0;
         cur[e] = 0;
@@ -69,26 +70,37 @@ __device__ __forceinline__ void moe_plan_block(const int *__restrict__ sel, int 
         if (e >= 0 && e < E) atomicAdd(&cnt[e], 1);
     }
     __syncthreads();
+    // The list's order of experts: by rows, the most first, dealt to eight shares back and forth, share behind share.  Cut
+    // into eight ranges of as many tiles, the ranges then have about as many rows each, and tall tiles start first.
+    for (int e = threadIdx.x; e < E; e += 1024) {
+        int rank = 0;
+        for (int q = 0; q < E; ++q) rank += cnt[q] > cnt[e] || (cnt[q] == cnt[e] && q < e);
+        const int turn = rank >> 3, whole = E >> 3, more = E & 7;
+        const bool back = turn & 1, last_back = whole & 1;
+        const int share = back ? 7 - (rank & 7) : rank & 7;
+        const int extra = last_back ? max(share - (8 - more), 0) : min(share, more);  // experts of the last turn in the shares before
+        pos[e] = share * whole + extra + turn;
+    }
+    __syncthreads();
     // Thread e lays out expert e: its first slot and first tile are prefix sums over the experts before it
     // (E <= 1024 broadcast reads from LDS), then it writes its own tiles.
-    // ceil(cnt / BM) tiles of equal height (a multiple of 16 rows): 140 rows with BM = 128 become 80 + 60 rather
+    // ceil(cnt / BM) tiles that differ by at most a fragment: 140 rows with BM = 128 become 80 + 60 rather
     // than 128 + 12, and the GEMM skips the row fragments a tile does not have.
     for (int e = threadIdx.x; e < E; e += 1024) {
         int o = 0, nt = 0, total = 0;
         for (int q = 0; q < E; ++q) {
             const int tq = (cnt[q] + BM - 1) / BM;  // equals the number of tiles written for q below
-            if (q < e) {
-                o += cnt[q];
-                nt += tq;
-            }
+            if (q < e) o += cnt[q];
+            if (pos[q] < pos[e]) nt += tq;
             total += tq;
         }
         off[e] = o;
         p.offsets[e] = o;
         const int tiles_e = (cnt[e] + BM - 1) / BM;
-        const int per = tiles_e ? ((cnt[e] + tiles_e - 1) / tiles_e + 15) / 16 * 16 : 0;
+        const int frags_e = (cnt[e] + p.fragment - 1) / p.fragment;
         const int nt_first = nt, nt_end = nt + tiles_e;
-        for (int m0 = 0; m0 < cnt[e]; m0 += per) {
+        for (int m0 = 0, i = 0; m0 < cnt[e]; ++i) {
+            const int per = (frags_e / tiles_e + (i < frags_e % tiles_e ? 1 : 0)) * p.fragment;
             int at = nt, run_first = nt_first, run_end = nt_end;
             if (p.tiles_per_xcd) {  // tile nt of `total` goes to range x = floor(8 nt / total), behind that range's earlier tiles
                 const int x = nt * 8 / total;
@@ -102,12 +114,13 @@ __device__ __forceinline__ void moe_plan_block(const int *__restrict__ sel, int 
             p.tile_rows[at] = min(per, cnt[e] - m0);
             p.tile_run0[at] = at - (nt - run_first);
             p.tile_runlen[at] = run_end - run_first;
+            m0 += per;
             ++nt;
         }
         if (e == E - 1) {
             off[E] = o + cnt[e];
             p.offsets[E] = o + cnt[e];
-            *p.n_tiles = nt;
+            *p.n_tiles = total;
         }
     }
     __syncthreads();
@@ -176,6 +189,7 @@ struct MoeWorkspace {
 
 static inline MoeWorkspace carve(void *base, int64_t T, int64_t H, int64_t I, int64_t E, int64_t topk) {
     MoeWorkspace w{};
+    w.plan.fragment = 16;
     const int64_t R = T * topk;
     const int64_t max_tiles = R / 16 + E + 8;  // tiles of at least 16 rows, one partial tile per expert, rounded up to eight
     size_t off = 0;

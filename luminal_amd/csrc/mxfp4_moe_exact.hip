@@ -20,12 +20,9 @@
 // In LDS an activation row of a chunk lies in two planes of 128 bytes (steps 0-1, steps 2-3), piece (g, d) at
 // byte 16 (g + 4 (d & 1)) of plane d >> 1, which gives the fragment reads the addresses r * pitch + 16 g + 64 (d & 1)
 // that were measured free of bank conflicts at a pitch of 160 bytes.
-#include "mxfp4_moe_device.h"
+#include "mxfp4_moe_exact_device.h"
 
 namespace lhip {
-
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
 
 // The 32 codes of one block (four dwords, even k in the low nibble) times 2^(code - 127), as the four weight
 // operands of the block's matrix steps.
@@ -45,11 +42,6 @@ __device__ __forceinline__ void mx_expand_block(const mu32x4 &q, uint32_t scale_
 __device__ __forceinline__ int exact_piece_offset(int j, int plane_bytes) {
     const int g = j >> 2, d = j & 3;
     return (d >> 1) * plane_bytes + (g + 4 * (d & 1)) * 16;
-}
-
-// up * swish(gate) with the hardware exp2 and reciprocal (1 ulp each), as the block-scaled form computes it.
-__device__ __forceinline__ float exact_swiglu(float gate, float up) {
-    return up * (gate * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504f * gate)));
 }
 
 // ---------------------------------------------------------------------------
@@ -83,20 +75,6 @@ __global__ __launch_bounds__(256) void mx_dequant_bf16_kernel(const uint8_t *__r
 // is expanded once per row tile whatever the tile's height, and an activation fragment is read from LDS once per
 // chunk.  GATED: fragments come in pairs, gate rows and the matching up rows; output bf16 up * swish(gate), else f32.
 // ---------------------------------------------------------------------------
-struct MoeExactArgs {
-    const __bf16 *a;      // activation rows, K elements each
-    const int *a_index;   // slot -> routed entry (GEMM 1) or nullptr (rows are slots)
-    int a_div;            // routed entry / a_div = activation row
-    const uint8_t *w_nib, *w_sc;
-    int rows_per_expert;
-    int K, Kp;
-    int N;
-    const int *tile_expert, *tile_row0, *tile_rows, *n_tiles;
-    const int *tile_run0, *tile_runlen;
-    int tiles_per_xcd;
-    void *out;            // bf16 [R][N] (gated) or f32 [R][N]
-};
-
 template <int MT, int NT, bool GATED, int WR, int D>
 __global__ __launch_bounds__(256 * WR) void mx_moe_gemm_exact_kernel(MoeExactArgs g) {
     static_assert(!GATED || NT % 2 == 0, "gated tiles pair each gate fragment with its up fragment");
@@ -110,38 +88,9 @@ __global__ __launch_bounds__(256 * WR) void mx_moe_gemm_exact_kernel(MoeExactArg
 
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];  // 3 x A_BUF
 
-    // Tile and column block of this workgroup (see MoePlan::tiles_per_xcd for the per-XCD list).
-    // Within a run of tiles of one expert the workgroups are ordered column block by column block: the tiles that
-    // read the same weights are dispatched next to each other and share one fetch of them out of the XCD's L2.
-    int tile = blockIdx.y, cb = blockIdx.x;
-    int expert, row0, rows;
-    if (g.tiles_per_xcd) {
-        const int linear = blockIdx.y * gridDim.x + blockIdx.x;
-        const int turn = linear >> 3, cols = static_cast<int>(gridDim.x);
-        const int base = (linear & 7) * g.tiles_per_xcd;
-        const int entry = turn / cols;
-        cb = turn - entry * cols;
-        tile = base + entry;
-        // (the entry's own tile is read in the same trip to memory; only a workgroup inside a run pays a second one,
-        // and not for the expert, which the run shares)
-        expert = g.tile_expert[tile];
-        row0 = g.tile_row0[tile];
-        rows = g.tile_rows[tile];
-        const int run0 = g.tile_run0[tile], runlen = g.tile_runlen[tile];
-        if (runlen > 1) {
-            const int local = turn - (run0 - base) * cols;  // position among the run's runlen * cols workgroups
-            cb = local / runlen;
-            tile = run0 + (local - cb * runlen);
-            row0 = g.tile_row0[tile];
-            rows = g.tile_rows[tile];
-        }
-    } else {
-        expert = g.tile_expert[tile];
-        row0 = g.tile_row0[tile];
-        rows = g.tile_rows[tile];
-    }
+    int tile, cb, expert, row0, rows;
+    exact_tile(g, tile, cb, expert, row0, rows);
     if (rows == 0) return;
-
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -604,17 +553,16 @@ static lhip_status launch_exact_gemm(const MoeExactArgs &a, int col_blocks, int 
     return LHIP_OK;
 }
 
-// Tile height of the exact form for R routed rows over E experts: the smallest of 16, 32, 64 rows that holds an
+// Tile height of the exact form for R routed rows over E experts, in 16-row fragments: 16 or 32 rows where such a tile holds an
 // expert with two standard deviations more rows than the average (so that nearly every expert is one tile and its
-// weights are read and expanded once); experts with more than 64 rows are cut into equal tiles of at most 64, whose
-// later reads of the weights come out of the XCD's L2.  Measured on the benchmark layer (us per layer, 64-row tiles as
-// four-wave workgroups two to a CU / 128-row tiles as eight-wave workgroups): T = 256 134 / 194, T = 512 187 / 207,
-// T = 1024 274 / 342, T = 2048 458 / 530; and 16- / 32- / 64-row tiles: T = 32 87 / 94 / 110, T = 64 90 / 95 / 110,
-// T = 128 132 / 99 / 114.
-static inline int exact_tile_fragments(int R, int E) {
+// weights are read and expanded once), else 96 (`tall`, mxfp4_moe_tall.hip), cut into equal parts for experts with more.  Measured
+// on the benchmark layer (us per layer, 16 / 32 / 96 rows): T = 32 87 / 94 / -, T = 64 90 / 95 / -, T = 128 132 / 99 / 103; 64-row
+// tiles of the kernel below, which stood in the place of the 96-row ones, against those: T = 192 121 / 112, T = 256 126 / 117, T = 512
+// 183 / 147, T = 768 214 / 202, T = 1024 274 / 246, T = 2048 455 / 399.
+static inline int exact_tile_fragments(int R, int E, bool tall) {
     const int avg = (R + E - 1) / E;
     const int need = avg + 2 * static_cast<int>(sqrtf(static_cast<float>(avg)) + 0.5f);
-    return need <= 16 ? 1 : need <= 32 ? 2 : 4;
+    return need <= 16 ? 1 : need <= 32 || !tall ? 2 : kTallRows / 16;
 }
 
 lhip_status moe_exact_forward(const uint8_t *gu, const uint8_t *dn, const __bf16 *x, const int32_t *sel_dev,
@@ -656,11 +604,12 @@ lhip_status moe_exact_forward(const uint8_t *gu, const uint8_t *dn, const __bf16
         return LHIP_OK;
     }
 
-    const int mt = exact_tile_fragments(R, E);
+    const int mt = exact_tile_fragments(R, E, moe_tall_supports(T, H, I));
     const int BM = 16 * mt;
     const int max_tiles = (R / BM + E + 7) / 8 * 8;
     w.plan.max_tiles = max_tiles;
     w.plan.tiles_per_xcd = max_tiles / 8;
+    w.plan.fragment = BM == kTallRows ? 32 : 16;
     hipLaunchKernelGGL(moe_plan_kernel, dim3(1), dim3(1024), 0, s, sel_dev, R, E, BM, w.plan);
     LHIP_CHECK_LAUNCH();
 
@@ -676,7 +625,7 @@ lhip_status moe_exact_forward(const uint8_t *gu, const uint8_t *dn, const __bf16
     switch (mt) {
         case 1: st = launch_exact_gemm<1, 4, true, 1, 4>(a1, cb1, max_tiles, s); break;
         case 2: st = launch_exact_gemm<2, 4, true, 1, 4>(a1, cb1, max_tiles, s); break;
-        default: st = launch_exact_gemm<4, 4, true, 1, 2>(a1, cb1, max_tiles, s); break;
+        default: st = moe_tall_gemm(a1, true, max_tiles, s); break;
     }
     if (st) return st;
     MoeExactArgs a2{};
@@ -686,11 +635,11 @@ lhip_status moe_exact_forward(const uint8_t *gu, const uint8_t *dn, const __bf16
     a2.tile_expert = w.plan.tile_expert; a2.tile_row0 = w.plan.tile_row0; a2.tile_rows = w.plan.tile_rows;
     a2.n_tiles = w.plan.n_tiles; a2.tiles_per_xcd = w.plan.tiles_per_xcd; a2.out = w.out;
     a2.tile_run0 = w.plan.tile_run0; a2.tile_runlen = w.plan.tile_runlen;
-    const int cb2 = (H + 127) / 128, cb2w = (H + 255) / 256;
+    const int cb2 = (H + 127) / 128;
     switch (mt) {
         case 1: st = launch_exact_gemm<1, 2, false, 1, 4>(a2, cb2, max_tiles, s); break;
         case 2: st = launch_exact_gemm<2, 2, false, 1, 4>(a2, cb2, max_tiles, s); break;
-        default: st = launch_exact_gemm<4, 4, false, 1, 2>(a2, cb2w, max_tiles, s); break;
+        default: st = moe_tall_gemm(a2, false, max_tiles, s); break;
     }
     if (st) return st;
     return moe_launch_combine(w.out, w.plan.slot_of, wts_dev, y, T, H, topk, s);

@@ -1,0 +1,68 @@
+// What the two grouped GEMMs of the exact expert layer share (mxfp4_moe_exact.hip: row tiles of 16 and 32, mxfp4_moe_tall.hip: of
+// 96): arguments, the tile a workgroup takes, SwiGLU.
+#pragma once
+
+#include "mxfp4_moe_device.h"
+
+namespace lhip {
+
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+
+// up * swish(gate) with the hardware exp2 and reciprocal (1 ulp each), as the block-scaled form computes it.
+__device__ __forceinline__ float exact_swiglu(float gate, float up) {
+    return up * (gate * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504f * gate)));
+}
+
+struct MoeExactArgs {
+    const __bf16 *a;      // activation rows, K elements each
+    const int *a_index;   // slot -> routed entry (GEMM 1) or nullptr (rows are slots)
+    int a_div;            // routed entry / a_div = activation row
+    const uint8_t *w_nib, *w_sc;
+    int rows_per_expert;
+    int K, Kp;
+    int N;
+    const int *tile_expert, *tile_row0, *tile_rows, *n_tiles;
+    const int *tile_run0, *tile_runlen;
+    int tiles_per_xcd;
+    void *out;            // bf16 [R][N] (gated) or f32 [R][N]
+};
+
+// Tile and column block of this workgroup (see MoePlan::tiles_per_xcd for the per-XCD list).
+// Within a run of tiles of one expert the workgroups are ordered column block by column block: the tiles that
+// read the same weights are dispatched next to each other and share one fetch of them out of the XCD's L2.
+__device__ __forceinline__ void exact_tile(const MoeExactArgs &g, int &tile, int &cb, int &expert, int &row0, int &rows) {
+    tile = blockIdx.y, cb = blockIdx.x;
+    if (g.tiles_per_xcd) {
+        const int linear = blockIdx.y * gridDim.x + blockIdx.x;
+        const int turn = linear >> 3, cols = static_cast<int>(gridDim.x);
+        const int base = (linear & 7) * g.tiles_per_xcd;
+        const int entry = turn / cols;
+        cb = turn - entry * cols;
+        tile = base + entry;
+        // (the entry's own tile is read in the same trip to memory; only a workgroup inside a run pays a second one,
+        // and not for the expert, which the run shares)
+        expert = g.tile_expert[tile];
+        row0 = g.tile_row0[tile];
+        rows = g.tile_rows[tile];
+        const int run0 = g.tile_run0[tile], runlen = g.tile_runlen[tile];
+        if (runlen > 1) {
+            const int local = turn - (run0 - base) * cols;  // position among the run's runlen * cols workgroups
+            cb = local / runlen;
+            tile = run0 + (local - cb * runlen);
+            row0 = g.tile_row0[tile];
+            rows = g.tile_rows[tile];
+        }
+    } else {
+        expert = g.tile_expert[tile];
+        row0 = g.tile_row0[tile];
+        rows = g.tile_rows[tile];
+    }
+}
+
+// mxfp4_moe_tall.hip.  Whether its 32-bit offsets reach everywhere for t tokens of width h and experts of width i.
+constexpr int kTallRows = 96;
+bool moe_tall_supports(int64_t t, int64_t h, int64_t i);
+lhip_status moe_tall_gemm(const MoeExactArgs &a, bool gated, int max_tiles, hipStream_t s);
+
+}  // namespace lhip

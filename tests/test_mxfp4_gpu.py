@@ -320,6 +320,49 @@ def test_moe_lopsided_routing(oracle, t, e, h, i, topk, hot, mode):
         check_stages(oracle, layer, xf, w_gu, w_dn, sel_h, wts_h, y, tokens=live, mode=mode)
 
 
+@pytest.mark.parametrize("h,i", [(96, 160), (416, 320), (128, 96)])
+def test_moe_rows_per_expert_at_the_edges_of_the_96_row_tiles(oracle, h, i):
+    """Experts of 0, 1, 33, 64, 96, 97, 129 and 193 rows in one call (fragments of 32, tiles of 96, their remainders), K that
+    ends inside a stage of 64, column blocks with waves that have no columns.  The row of x behind another one's end starts
+    with infinities, which must not reach it through the padding of K."""
+    counts, e = (97, 33, 0, 96, 1, 193, 64, 129), 8
+    layer, w_gu, w_dn = make_layer(oracle, e, h, i, seed=h + i)
+    rng = np.random.default_rng(h)
+    sel = rng.permutation(np.repeat(np.arange(e, dtype=np.int32), counts))[:, None]
+    t = len(sel)
+    x = (rng.standard_normal((t, h)) * 0.05).astype(np.float32)
+    x[5, :32] = np.inf
+    bits = oracle.f32_to_bf16_bits(x)
+    xf = oracle.bf16_bits_to_f32(bits)
+    wts = rng.uniform(0.5, 1.0, (t, 1)).astype(np.float32)
+    xd = torch.from_numpy(bits.view(np.int16)).to(DEV).view(torch.bfloat16)
+    y = layer.process(xd, torch.from_numpy(np.ascontiguousarray(sel)).to(DEV), torch.from_numpy(wts).to(DEV), EXACT).float().cpu().numpy()
+    others = np.flatnonzero(np.arange(t) != 5)
+    assert np.isfinite(y[others]).all()
+    check_stages_exact(layer, xf, w_gu, w_dn, sel, wts, y, tokens=others)
+
+
+def test_moe_rows_beyond_32_bit_offsets(oracle):
+    """More than 4 GiB of x: tiles whose kernel does not count in 32 bits."""
+    e, h, i = 2, 32768, 32
+    t = (1 << 32) // (2 * h) + 40
+    layer, w_gu, w_dn = make_layer(oracle, e, h, i, seed=3)
+    rng = np.random.default_rng(4)
+    bits = oracle.f32_to_bf16_bits((rng.standard_normal((8, h)) * 0.05).astype(np.float32))
+    xd = torch.from_numpy(bits.view(np.int16)).to(DEV).view(torch.bfloat16).repeat((t + 7) // 8, 1)[:t]
+    sel = torch.arange(t, dtype=torch.int32, device=DEV).remainder_(3).clamp_(max=e - 1)[:, None].contiguous()
+    wts = torch.ones((t, 1), device=DEV)
+    y = layer.process(xd, sel, wts, EXACT)
+    # rows of equal activations and expert are equal wherever they lie; the first are held to the oracle
+    period = y[:24]
+    last = t - 24 - (t - 24) % 24
+    assert torch.equal(y[last:last + 24], period)
+    first = period.float().cpu().numpy()
+    xf = np.tile(oracle.bf16_bits_to_f32(bits), (3, 1))
+    truth = oracle.moe_forward(xf, w_gu, w_dn, sel[:24].cpu().numpy(), wts[:24].cpu().numpy(), act_bf16=True)
+    assert norm_err(first, truth) < NORM_TOL[EXACT]
+
+
 @MODES
 def test_moe_activation_split_is_exact_on_wide_dynamic_range(oracle, mode):
     # activations spanning many binades inside one 32-block: the hi/lo fp8 split must not lose the small ones
