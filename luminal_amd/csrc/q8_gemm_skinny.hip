@@ -567,6 +567,8 @@ static int split_slices(int mc, int n, int k, size_t room) {
 
 // ---- the choice of the kernel for the f32 / f16 operators
 
+constexpr int kMaxRowsSlices = 40;
+
 // How a product is run: by passes of 64 rows of the kernel above (kStream), by q8_gemm_rows.hip (kRows: `n_main` leading
 // weight rows in whole rounds of workgroups, the others over `slices` K slices; n_main = 0: all of them), or by the
 // tiles of q8_gemm_wide.hip (kWide).
@@ -576,12 +578,23 @@ struct RowsPlan {
     size_t floats = 0;  // of partial planes
 };
 
+// What q8_gemm_rows.hip takes for up to 64 rows, us: per block of K that the slowest compute unit walks, for the sum of the slices
+// and its planes.  Fitted to 420 sizes (6 % of standard deviation).
+static double few_rows_us(int64_t m, int64_t n, bool f16, int64_t blocks, int slices) {
+    const double sum = slices > 1 ? (f16 ? 4.1 : 3.8) + static_cast<double>(slices * m * n) * 4e-6 * 0.56 : 0.0;
+    return static_cast<double>(blocks) * (f16 ? 0.63 : 0.78) + sum;
+}
+
 // The plan that ends first, by what each kernel takes (us, measured): a workgroup of the streaming kernel 0.49 (f32) or
 // 0.38 (f16) per block of K, one of q8_gemm_rows.hip 1.2 or 0.66, a 128x256 tile of q8_gemm_wide.hip 0.64 (f16); 256
-// workgroups at a time, some microseconds per launch, and 3 plus 8 TB/s for the sum of the slices.  The lines this draws
-// (streaming -> chosen, us): 14336 x 4096 f32 at 64 rows 38 -> (54), at 128 61 -> 54, at 256 120 -> 97, at 512 239 ->
-// 162; f16 at 64 rows 34 -> (36), at 128 50 -> 36, at 512 188 -> 90; 4096 x 4096 f32 at 256 rows 39 -> (41), at 300 63 ->
-// 44.  Up to 64 rows, and for fewer than sixteen 128x256 tiles, the streaming kernel's narrower strips stay ahead.
+// workgroups at a time, some microseconds per launch, and 3 plus 8 TB/s for the sum of the slices; up to 64 rows what
+// few_rows_us says.  The lines this draws (streaming -> chosen, us): 14336 x 4096 f32 at 64 rows 38 -> (54), at 128 61 -> 54,
+// at 256 120 -> 97, at 512 239 -> 162; f16 at 64 rows 34 -> (36), at 128 50 -> 36, at 512 188 -> 90; 4096 x 4096 f32 at 256
+// rows 39 -> (41), at 300 63 -> 44.  Up to 64 rows, and for fewer than sixteen 128x256 tiles, the streaming kernel's narrower
+// strips stay ahead.  A number of slices that leaves one empty is passed over; with 16 slices at most, and none behind the
+// first number that leaves one empty, few weight rows or a K of 90 blocks left most compute units idle: 45 x 2880 x 2880 f32
+// 6 -> 12 slices 18.1 -> 15.3 us, 45 x 1000 x 4480 18.9 -> 13.6, 300 x 1000 x 8000 37.4 -> 27.2, f16 400 x 1000 x 8992 30.4 ->
+// 25.7.
 static RowsPlan rows_plan(int64_t m, int n, int k, bool f16, size_t room, bool stream) {
     RowsPlan best;
     const int64_t m_tiles = (m + 127) / 128, n_tiles = (n + 255) / 256;
@@ -600,20 +613,21 @@ static RowsPlan rows_plan(int64_t m, int n, int k, bool f16, size_t room, bool s
         const double us = 8.0 + static_cast<double>(q8_gemm_wide_ends(m, n)) * 0.32 * nblk;
         if (us < best_us) best_us = us, best.kind = RowsPlan::kWide;
     }
-    // all columns, or those that whole rounds leave over, in 1 to 16 slices
+    // all columns, or those that whole rounds leave over, in K slices
     const int64_t per_round = m_tiles < 256 ? 256 / m_tiles : 1;
     const int64_t main_tiles = n_tiles / per_round * per_round;
     for (int64_t lead : {int64_t{0}, main_tiles}) {
         if (lead == n_tiles || (lead > 0 && m_tiles > 256)) continue;
         const int64_t cols = n - lead * 256, tiles = m_tiles * (n_tiles - lead);
-        const double main_us = lead > 0 ? rounds(m_tiles * lead) * nblk * block + 8.0 : 0.0;
-        for (int slices = 1; slices <= 16; ++slices) {
+        const double main_us = lead > 0 ? rounds(m_tiles * lead) * nblk * (m <= 64 ? (f16 ? 0.63 : 0.78) : block) + 8.0 : 0.0;
+        for (int slices = 1; slices <= kMaxRowsSlices; ++slices) {
             if (lead > 0 && slices == 1) continue;
             const int per = q8_gemm_rows_slice_blocks(k, slices);
-            if (static_cast<int64_t>(slices - 1) * per >= k / 32) break;
+            if (static_cast<int64_t>(slices - 1) * per >= k / 32) continue;  // an empty slice (the next number may have none)
             const size_t floats = slices > 1 ? static_cast<size_t>(slices) * m * cols : 0;
             if (floats > room || (slices > 1 && tiles * slices > 0x7ffffff0)) break;  // (the grid's x extent)
-            const double us = main_us + 8.0 + rounds(tiles * slices) * per * block + (slices > 1 ? sum_us(slices, cols) : 0.0);
+            const double us = main_us + (m <= 64 ? few_rows_us(m, cols, f16, static_cast<int64_t>(rounds(tiles * slices)) * per, slices)
+                                                 : 8.0 + rounds(tiles * slices) * per * block + (slices > 1 ? sum_us(slices, cols) : 0.0));
             if (us < best_us) {
                 best_us = us;
                 best.kind = RowsPlan::kRows;
