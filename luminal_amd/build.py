@@ -98,6 +98,31 @@ def build_module(verbose: bool = True) -> str:
     return MODULE
 
 
+TORCH_OPS_SRC = os.path.join(HERE, "host", "torch_ops.cpp")
+TORCH_OPS = os.path.join(HERE, "_torch_ops.so")
+
+
+def build_torch_ops(verbose: bool = True) -> str:
+    """Compile the operators' native host path (a Python extension against the installed torch) with the host compiler; it links
+    against libluminal_hip.so, which has to be there."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    cxx = os.environ.get("CXX") or shutil.which("g++") or shutil.which("c++")
+    if not cxx:
+        raise RuntimeError("no host C++ compiler found (g++)")
+    if verbose:
+        print(f"[luminal_amd.build] {cxx} -> {TORCH_OPS}", file=sys.stderr)
+    _run([cxx, "-std=c++17", "-O2", "-Wall", "-fPIC", "-shared", "-fvisibility=hidden",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+          *[f"-isystem{p}" for p in (*cpp_extension.include_paths(), sysconfig.get_paths()["include"])], "-o", TORCH_OPS, TORCH_OPS_SRC,
+          "-L" + HERE, "-lluminal_hip", *["-L" + p for p in cpp_extension.library_paths()],
+          "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-Wl,-rpath,$ORIGIN"])
+    return TORCH_OPS
+
+
 HOST_TEST_SRC = os.path.join(os.path.dirname(HERE), "tests", "cpp", "host_mirror_test.cpp")
 HOST_TEST_BIN = os.path.join(os.path.dirname(HERE), "tests", "cpp", "_build", "host_mirror_test")
 
@@ -118,4 +143,5 @@ def build_host_test(verbose: bool = True) -> str:
 
 if __name__ == "__main__":
     build(incremental="--incremental" in sys.argv)
+    build_torch_ops()
     build_host_test()

@@ -52,6 +52,15 @@ def bf16_workspace_nbytes(lib, m: int, n: int, k: int, out_form: int) -> int:
     return lib.lhip_q8_0_matmul_bf16_workspace_nbytes(m, n, k, out_form) if m > 128 or k % 512 else 0
 
 
+# The whole call of an operator in native code (host/torch_ops.cpp): the plain case, or None.  It is linked against the torch it
+# was built with; where that is not the one that runs, the operators below do the same through ctypes.
+try:
+    from ._torch_ops import quantized_matmul as _native_matmul
+except ImportError:
+    def _native_matmul(*_):
+        return None
+
+
 def _ptr(t: torch.Tensor) -> int:
     return t.data_ptr()
 
@@ -131,6 +140,11 @@ class QuantizedMatmul:
         self.cfg = (rows_per_wave, k_unroll, blocks_per_cu, waves_per_block) if rows_per_wave else None
 
     def process(self, x: torch.Tensor, w: Q8Weight) -> torch.Tensor:
+        if self.cfg is None:
+            device = _current_device()
+            out = _native_matmul(x, w.planar, w.n, w.k, False, device, _raw_stream(device))
+            if out is not None:
+                return out
         lib = capi.load_library()
         dtype, n, k = x.dtype, w.n, w.k
         if dtype not in (torch.float32, torch.float16) or not x.is_cuda:
@@ -172,6 +186,11 @@ class QuantizedMatmulBf16:
         self.tile = tile
 
     def process(self, x: torch.Tensor, w: Q8Weight) -> torch.Tensor:
+        if self.tile is None:
+            device = _current_device()
+            out = _native_matmul(x, w.planar, w.n, w.k, True, device, _raw_stream(device))
+            if out is not None:
+                return out
         lib = capi.load_library()
         if x.dtype != torch.bfloat16 or not x.is_cuda:
             raise TypeError("QuantizedMatmulBf16 expects bf16 activations on the GPU")
