@@ -246,7 +246,7 @@ def test_decode_attention_equals_rope_append_attention(hq, hkv, hd, pos0):
 
 
 @pytest.mark.parametrize("hq,hkv,hd", [(8, 2, 128), (32, 8, 128), (4, 4, 64), (16, 2, 64), (4, 2, 128), (8, 8, 128)])
-@pytest.mark.parametrize("S,pos0", [(8, 0), (33, 0), (70, 5), (64, 64), (129, 31)])
+@pytest.mark.parametrize("S,pos0", [(8, 0), (33, 0), (70, 5), (64, 64), (129, 31), (15, 1), (16, 16), (17, 47)])
 def test_prompt_attention_on_matrix_cores(hq, hkv, hd, S, pos0):
     """Calls of 8 or more tokens take the matrix-core kernel: against the f64 softmax(QK)V over the cache, for
     query blocks and key tiles that are ragged, start mid-cache and span several tiles."""
