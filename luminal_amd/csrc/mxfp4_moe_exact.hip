@@ -555,14 +555,14 @@ static lhip_status launch_exact_gemm(const MoeExactArgs &a, int col_blocks, int 
 
 // Tile height of the exact form for R routed rows over E experts, in 16-row fragments: 16 or 32 rows where such a tile holds an
 // expert with two standard deviations more rows than the average (so that nearly every expert is one tile and its
-// weights are read and expanded once), else 96 (`tall`, mxfp4_moe_tall.hip), cut into equal parts for experts with more.  Measured
-// on the benchmark layer (us per layer, 16 / 32 / 96 rows): T = 32 87 / 94 / -, T = 64 90 / 95 / -, T = 128 132 / 99 / 103; 64-row
-// tiles of the kernel below, which stood in the place of the 96-row ones, against those: T = 192 121 / 112, T = 256 126 / 117, T = 512
-// 183 / 147, T = 768 214 / 202, T = 1024 274 / 246, T = 2048 455 / 399.
+// weights are read and expanded once), else 96 (`tall`, mxfp4_moe_tall.hip), cut into equal parts for experts with more; but 64
+// around 40 rows, which fragments of 16 fit better than that kernel's of 32.  Measured on the benchmark layer (us per layer, 16 / 32 /
+// 64 / 96 rows): T = 32 87 / 94 / 110 / -, T = 64 90 / 95 / 110 / -, T = 128 132 / 99 / 114 / 103, T = 192 - / - / 126 / 114, T = 256 128 /
+// 127, T = 288 133 / 136, T = 320 135 / 139, T = 352 137 / 138, T = 384 140 / 138, T = 512 191 / 155, T = 768 221 / 210, T = 1024 284 / 237.
 static inline int exact_tile_fragments(int R, int E, bool tall) {
     const int avg = (R + E - 1) / E;
     const int need = avg + 2 * static_cast<int>(sqrtf(static_cast<float>(avg)) + 0.5f);
-    return need <= 16 ? 1 : need <= 32 || !tall ? 2 : kTallRows / 16;
+    return need <= 16 ? 1 : need <= 32 ? 2 : (avg >= 34 && avg <= 44) || !tall ? 4 : kTallRows / 16;
 }
 
 lhip_status moe_exact_forward(const uint8_t *gu, const uint8_t *dn, const __bf16 *x, const int32_t *sel_dev,
@@ -609,6 +609,9 @@ lhip_status moe_exact_forward(const uint8_t *gu, const uint8_t *dn, const __bf16
     const int max_tiles = (R / BM + E + 7) / 8 * 8;
     w.plan.max_tiles = max_tiles;
     w.plan.tiles_per_xcd = max_tiles / 8;
+    // Experts listed by their rows where many are more than one tile, us, own order / by rows: T = 320 136 / 139, T = 416 141 / 145,
+    // T = 448 153 / 149, T = 512 158 / 155, T = 640 173 / 175, T = 768 217 / 210, T = 1024 243 / 237.
+    w.plan.by_rows = BM == kTallRows && R >= 56 * E;
     w.plan.fragment = BM == kTallRows ? 32 : 16;
     hipLaunchKernelGGL(moe_plan_kernel, dim3(1), dim3(1024), 0, s, sel_dev, R, E, BM, w.plan);
     LHIP_CHECK_LAUNCH();
@@ -625,6 +628,7 @@ lhip_status moe_exact_forward(const uint8_t *gu, const uint8_t *dn, const __bf16
     switch (mt) {
         case 1: st = launch_exact_gemm<1, 4, true, 1, 4>(a1, cb1, max_tiles, s); break;
         case 2: st = launch_exact_gemm<2, 4, true, 1, 4>(a1, cb1, max_tiles, s); break;
+        case 4: st = launch_exact_gemm<4, 4, true, 1, 2>(a1, cb1, max_tiles, s); break;
         default: st = moe_tall_gemm(a1, true, max_tiles, s); break;
     }
     if (st) return st;
@@ -635,10 +639,11 @@ lhip_status moe_exact_forward(const uint8_t *gu, const uint8_t *dn, const __bf16
     a2.tile_expert = w.plan.tile_expert; a2.tile_row0 = w.plan.tile_row0; a2.tile_rows = w.plan.tile_rows;
     a2.n_tiles = w.plan.n_tiles; a2.tiles_per_xcd = w.plan.tiles_per_xcd; a2.out = w.out;
     a2.tile_run0 = w.plan.tile_run0; a2.tile_runlen = w.plan.tile_runlen;
-    const int cb2 = (H + 127) / 128;
+    const int cb2 = (H + 127) / 128, cb2w = (H + 255) / 256;
     switch (mt) {
         case 1: st = launch_exact_gemm<1, 2, false, 1, 4>(a2, cb2, max_tiles, s); break;
         case 2: st = launch_exact_gemm<2, 2, false, 1, 4>(a2, cb2, max_tiles, s); break;
+        case 4: st = launch_exact_gemm<4, 4, false, 1, 2>(a2, cb2w, max_tiles, s); break;
         default: st = moe_tall_gemm(a2, false, max_tiles, s); break;
     }
     if (st) return st;

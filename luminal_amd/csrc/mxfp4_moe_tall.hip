@@ -14,8 +14,8 @@
 //     compiler's waits for them count the direct loads too, and stop at those;
 //   * activation fragments that the tile does not have are not requested (all 96 rows always: 5 % slower at T = 1024).
 // Measured on the benchmark layer (32 experts of 2880 x 2880, top 4), us per layer, before (64-row tiles of mx_moe_gemm_exact_kernel,
-// activations through registers, experts in their own order in the tile list) -> now: T = 192 121 -> 112, T = 512 183 -> 147,
-// T = 1024 274 -> 246 (830 TFLOP/s of useful work), T = 2048 455 -> 399.  Tiles of 128 rows and 64 are level or slower there (T = 1024 289
+// activations through registers, experts in their own order in the tile list) -> now: T = 192 126 -> 114, T = 512 191 -> 155,
+// T = 1024 284 -> 237 (860 TFLOP/s of useful work), T = 2048 455 -> 393.  Tiles of 128 rows and 64 are level or slower there (T = 1024 289
 // and 259, T = 512 173 and 172), of 160 rows at two workgroups a CU 241 at T = 1024 and 174 at T = 512.
 #include <algorithm>
 
