@@ -1,12 +1,12 @@
 // Q8_0 weights x activations for few activation rows (short prompts, small batches; up to 128 rows per pass).
 //
 // With so few activation rows the product is bound by streaming the weights, not by the matrix cores, and the
-// 128/256-row tiles of q8_gemm.hip leave most of the chip idle.  Here a workgroup owns a strip of 128 weight rows
+// 128/256-row tiles of q8_gemm.hip leave most of the chip idle.  Here a workgroup owns a strip of up to 128 weight rows
 // (and, when the strips alone would not fill the chip, a slice of K) and streams it from HBM straight into
 // registers in matrix-core operand order:
 //
-//   * eight compute waves of 16 weight rows each (seven, i.e. strips of 112 rows, where that cuts N into a number
-//     of workgroups that fills the 256 CUs better: sk_plan).  The int8 codes go to the matrix cores as they are (an int8 is
+//   * eight compute waves of 16 weight rows each, or seven, four, three or two (strips of 112, 64, 48 or 32 rows) where
+//     those end first: sk_plan.  The int8 codes go to the matrix cores as they are (an int8 is
 //     exact in bf16); an MFMA step (v_mfma_f32_16x16x32_bf16) is one Q8_0 block, a lane supplies eight of its
 //     codes, and the block's scale multiplies the f32 block sum: acc += d * sum, the arithmetic of the matvec
 //     kernels (crates/luminal_cuda/src/quantized.rs:93-96).  Eight groups of 64 k per row block are in flight per
@@ -29,6 +29,7 @@
 #include <utility>
 
 #include <algorithm>
+#include <cmath>
 
 #include "common.h"
 #include "q8_gemm_rows.h"
@@ -43,7 +44,7 @@ typedef uint32_t sk_u32x4 __attribute__((ext_vector_type(4)));
 
 enum { kSkOutBf16 = 0, kSkOutF32 = 1, kSkOutSwiglu = 2, kSkOutPartial = 3, kSkOutF16 = 4 };  // first three as in q8_gemm.hip
 
-constexpr int kSkRows = 128;    // weight rows per workgroup of eight compute waves (seven: 112)
+constexpr int kSkRows = 128;    // weight rows per workgroup of eight compute waves (CW: 16 * CW)
 constexpr int kSkPitch = 160;   // bytes per activation row of a panel in LDS
 constexpr int kSkStages = 3;    // LDS buffers
 constexpr int kSkUnit = 512;     // K slices are whole multiples of this (eight groups of 64 k)
@@ -95,8 +96,9 @@ __device__ __forceinline__ void sk_store4(void *y, float *part, int split, int M
 // RING = groups in flight per wave; a slice is a multiple of RING groups.
 // XT = __bf16, __half or float: the loaders write x as NL = 1, 2 or 3 bf16 planes per tile whose sum is the value
 // exactly (an f16 has 11 significant bits, which two limbs hold; an f32's 24 take three).
-// CW = compute waves: 8, or 7 where strips of 112 weight rows cut N into a number of workgroups that fills the chip
-// (14336 rows are 112 strips of 128 but 128 of 112: with two K slices 224 or 256 workgroups for the 256 CUs).
+// CW = compute waves: 8, or as few as sk_plan finds to end first (a strip is one workgroup per K slice and CU, so narrower
+// strips fill the chip with fewer slices, whose planes cost 16-30 % of a product of few rows; a workgroup's time per k
+// falls by less than its rows do, see the table there).
 template <int MT, int OUT, int RING, typename XT, int CW = 8>
 __global__ __launch_bounds__((CW + 4) * 64) void q8_gemm_skinny_kernel(const int8_t *__restrict__ qs, const __half *__restrict__ ds,
                                                              const XT *__restrict__ x, void *__restrict__ y,
@@ -105,7 +107,7 @@ __global__ __launch_bounds__((CW + 4) * 64) void q8_gemm_skinny_kernel(const int
     constexpr int NL = sizeof(XT) == 4 ? 3 : (std::is_same<XT, __bf16>::value ? 1 : 2);  // bf16 limbs of an activation
     using S = SkShape<MT, NL>;
     constexpr int G = S::G;
-    static_assert(CW == 8 || CW == 7, "compute waves");
+    static_assert(CW >= 2 && CW <= 8, "compute waves");
     extern __shared__ __attribute__((aligned(16))) unsigned char sk_lds[];
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -264,6 +266,7 @@ __global__ __launch_bounds__((CW + 4) * 64) void q8_gemm_skinny_kernel(const int
         for (int cb = 0; cb < MT; ++cb) acc[cb] = sk_f32x4{0.f, 0.f, 0.f, 0.f};
 
         constexpr int UNITS = 2 * MT;  // (block, column block) pairs of a group
+        constexpr int kPending = NL == 1 ? 2 : 0;
         auto b_read = [&](const unsigned char *xb, int i, int limb) __attribute__((always_inline)) {
             return *reinterpret_cast<const sk_bf16x8 *>(xb + limb * S::PLANE + (i % MT) * 16 * kSkPitch + (i / MT) * 64);
         };
@@ -278,6 +281,23 @@ __global__ __launch_bounds__((CW + 4) * 64) void q8_gemm_skinny_kernel(const int
             bq[0][l] = b_read(xb_cur, 0, l);
             bq[1][l] = UNITS > 1 ? b_read(xb_cur, 1 % UNITS, l) : b_read(xb_cur, 0, l);
         }
+        // A unit's block sums are added kPending units after their MFMA, when they are there: with bf16 activations (one MFMA
+        // per unit) a wave alone on its SIMD otherwise waits out every MFMA (64 x 512 x 1024 8.1 -> 7.0 us, 128 x 4096 x 1024
+        // 12.4 -> 10.3, 16 x 14336 x 4096 16.4 -> 16.2; two units, one gives half of it).  The limbs of f32 / f16 activations fill
+        // the pipe by themselves: 64 x 14336 x 4096 f32 37.9 -> 38.6 us with it.
+        sk_f32x4 sum[4];
+        float dv[2][2][4];  // scales of this group and of the one before it
+        static_for<kPending>([&](auto ic) __attribute__((always_inline)) {
+            sum[(4 - kPending + decltype(ic)::value) % 4] = sk_f32x4{0.f, 0.f, 0.f, 0.f};
+        });
+#pragma unroll
+        for (int v = 0; v < 4; ++v) dv[1][0][v] = dv[1][1][v] = 0.f;
+        auto add_unit = [&](auto uc, auto ic) __attribute__((always_inline)) {  // unit i of group u, i < 0: of the group before
+            constexpr int i = decltype(ic)::value, u = decltype(uc)::value + (i < 0 ? 7 : 8), j = i < 0 ? i + UNITS : i;
+            constexpr int slot = (u * UNITS + j) % 4;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) acc[j % MT][v] = fmaf(dv[u & 1][j / MT][v], sum[slot][v], acc[j % MT][v]);
+        };
         int stage = 0;
         int R = 0;
         do {  // a slice is never empty: no guard, so the requests above stay where the fences put them
@@ -309,12 +329,11 @@ __global__ __launch_bounds__((CW + 4) * 64) void q8_gemm_skinny_kernel(const int
                         const float hi = static_cast<float>(static_cast<signed char>(w >> (16 * (e & 1) + 8)));
                         a_bf[b][e] = (__float_as_uint(lo) >> 16) | (__float_as_uint(hi) & 0xffff0000u);
                     }
-                float dv[2][4];
 #pragma unroll
                 for (int b = 0; b < 2; ++b)
 #pragma unroll
                     for (int v = 0; v < 4; ++v)
-                        dv[b][v] = __half2float(__ushort_as_half(static_cast<unsigned short>(d_reg[u >> 2][v][u & 3] >> (16 * b))));
+                        dv[u & 1][b][v] = __half2float(__ushort_as_half(static_cast<unsigned short>(d_reg[u >> 2][v][u & 3] >> (16 * b))));
                 load_a(u, gl + RING);
                 static_for<UNITS>([&](auto ic) __attribute__((always_inline)) {
                     constexpr int i = decltype(ic)::value;
@@ -329,8 +348,8 @@ __global__ __launch_bounds__((CW + 4) * 64) void q8_gemm_skinny_kernel(const int
 #pragma unroll
                     for (int l = NL - 1; l >= 0; --l)
                         t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bq[U % 4][l], t, 0, 0, 0);
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) acc[i % MT][v] = fmaf(dv[i / MT][v], t[v], acc[i % MT][v]);
+                    sum[U % 4] = t;
+                    add_unit(uc, std::integral_constant<int, i - kPending>{});
                 });
                 // a set of scales is requested again once its last group has read it (requested earlier, the load
                 // gets other registers and a copy at the end of the trip that waits for every load in flight)
@@ -342,6 +361,9 @@ __global__ __launch_bounds__((CW + 4) * 64) void q8_gemm_skinny_kernel(const int
                 }
             });
         } while ((R += RING / 4) < n_rounds);
+        static_for<kPending>([&](auto ic) __attribute__((always_inline)) {
+            add_unit(std::integral_constant<int, RING - 1>{}, std::integral_constant<int, UNITS - kPending + decltype(ic)::value>{});
+        });
         const int n = n0 + 4 * g;
         if (n < N) {
 #pragma unroll
@@ -429,16 +451,49 @@ static int sk_splits_for(int strips, int m, int n, int k, size_t room) {
 }
 
 // Compute waves per workgroup (strips of 16 rows each) for `splits` K slices (0: the slices are chosen with them).
-// A workgroup's time goes with the weights it streams (rows x its share of K) and the launch takes as many rounds of
-// 256 workgroups as it has workgroups: eight waves unless seven make that product smaller.
 struct SkPlan {
     int cw, splits;
 };
+constexpr int kSkWaves[] = {8, 7, 4, 3, 2};
+
+// What the kernel takes for one pass of bf16 rows, us.  A workgroup walks 512 of K in the time of its table (the vector
+// instructions of its waves: conversions, and four fmas per MFMA) or in the time that the weights and activations of all of
+// them take from memory and L2, whichever is longer (joined by a fourth power); a CU runs them one after the other; the sum
+// of the slices is a launch and its planes.  Fitted to 2800 measurements, the numbers of slices around those that fill the
+// chip for 240 sizes (m of 16 to 128, N of 512 to 28672, K of 1024 to 14336).
+// `groups` workgroups of kSkWaves[cw_index] compute waves walk `per` units of K; a plan that cannot come below `limit` is not
+// worked out.
+static double sk_us(int cw_index, int slices, unsigned groups, int per, int m, int n, double limit) {
+    static const double walk[4][5] = {{3.11, 2.60, 1.33, 1.10, 0.98},   // up to 16 activation rows
+                                      {3.34, 2.96, 1.68, 1.42, 1.23},   // 32
+                                      {5.24, 4.61, 2.69, 2.18, 1.99},   // 64
+                                      {5.96, 5.44, 3.62, 3.29, 3.10}};  // 128
+    static const double weights[4] = {6.2e6, 7.0e6, 5.8e6, 7.0e6}, activations = 20e6;  // bytes per us
+    static const double fixed[4] = {3.2, 3.35, 3.65, 4.45};
+    const int rows = m <= 16 ? 0 : (m <= 32 ? 1 : (m <= 64 ? 2 : 3)), strip = 16 * kSkWaves[cw_index];
+    const double walks = static_cast<double>((groups + 255) / 256 * static_cast<unsigned>(per));
+    const double rest = fixed[rows] + (slices > 1 ? 2.0 + 0.52 * static_cast<double>(slices) * m * n * 4e-6 : 0.0);
+    if (rest + walks * walk[rows][cw_index] >= limit) return limit;
+    const double stream = static_cast<double>(groups < 256 ? groups : 256) *
+                          (strip * (kSkUnit + kSkUnit / 16) / weights[rows] + (16 << rows) * 2 * kSkUnit / activations);
+    const double w2 = walk[rows][cw_index] * walk[rows][cw_index], s2 = stream * stream;
+    return rest + walks * sqrt(sqrt(w2 * w2 + s2 * s2));
+}
+
+// A workgroup's time goes with the weights it streams (rows x its share of K) and the launch takes as many rounds of
+// 256 workgroups as it has workgroups: eight waves, or seven if they make that product smaller, with the K slices that
+// fill the chip.  That is right for many rows; one pass of up to 128 takes any other strip and number of slices that
+// sk_us puts 6 % below (its own spread).  m x N x K, us: 16 x 14336 x 4096 7 waves, 2 slices 18.7 -> 4 waves, none 16.4;
+// 16 x 4096 x 4096 8 waves, 8 slices 10.5 -> 4 waves, 4 slices 9.1; 64 x 4096 x 4096 18.1 -> 13.5; 128 x 4096 x 4096 21.4 -> 18.2;
+// 16 x 4096 x 1024 8.4 -> 5.0; as it was: 32 x 10240 x 8192 29.3, 64 x 8192 x 14336 47.7.  Over the 240 sizes it is within
+// 1.4 % of the best of all plans (the first rule alone: 17 %), and at none more than 1 % behind the first rule.
 static SkPlan sk_plan(int m, int n, int k, size_t room, int splits = 0) {
     const int units = k / kSkUnit, passes = (m + 127) / 128;
     SkPlan best{8, 1};
     long best_cost = -1;
-    for (int cw = 8; cw >= 7; --cw) {
+    int best_index = 0;
+    for (int i = 0; i < 2; ++i) {
+        const int cw = kSkWaves[i];
         const int strips = (n + cw * 16 - 1) / (cw * 16);
         int s = splits > 0 ? (splits > units ? units : splits) : sk_splits_for(strips, m, n, k, room);
         const int per = (units + s - 1) / s;
@@ -447,7 +502,24 @@ static SkPlan sk_plan(int m, int n, int k, size_t room, int splits = 0) {
         const long cost = rounds * cw * per;
         if (best_cost < 0 || cost < best_cost) {
             best_cost = cost;
+            best_index = i;
             best = SkPlan{cw, s};
+        }
+    }
+    if (passes > 1) return best;
+    auto strips_of = [n](int i) { return static_cast<unsigned>((n + 16 * kSkWaves[i] - 1) / (16 * kSkWaves[i])); };
+    auto per_of = [units](int s) { return static_cast<int>(static_cast<unsigned>(units + s - 1) / static_cast<unsigned>(s)); };
+    const int fixed_s = splits > 0 ? best.splits : 0;
+    double best_us = 0.94 * sk_us(best_index, best.splits, strips_of(best_index) * best.splits, per_of(best.splits), m, n, 1e30);
+    for (int i = 0; i < static_cast<int>(sizeof(kSkWaves) / sizeof(kSkWaves[0])); ++i) {
+        const unsigned strips = strips_of(i);
+        for (int s = fixed_s ? fixed_s : 1; s <= (fixed_s ? fixed_s : units); ++s) {
+            // (two rounds of workgroups are enough for any strip)
+            if (s > 1 && !fixed_s && (strips * s > 512 || static_cast<size_t>(s) * m * n > room)) break;
+            const int per = per_of(s);
+            if ((s - 1) * per >= units) continue;  // an empty slice
+            const double us = sk_us(i, s, strips * s, per, m, n, best_us);
+            if (us < best_us) best_us = us, best = SkPlan{kSkWaves[i], s};
         }
     }
     return best;
@@ -524,8 +596,14 @@ lhip_status q8_gemm_skinny_launch(const int8_t *qs, const __half *ds, const void
         if (!part) return LHIP_ERR_HIP;
     }
     const __bf16 *x = static_cast<const __bf16 *>(x_bf16);
-    const lhip_status st = plan.cw == 7 ? sk_launch_rows<7>(out, qs, ds, x, y, part, m, n, k, splits, s)
-                                        : sk_launch_rows<8>(out, qs, ds, x, y, part, m, n, k, splits, s);
+    lhip_status st;
+    switch (plan.cw) {
+        case 2: st = sk_launch_rows<2>(out, qs, ds, x, y, part, m, n, k, splits, s); break;
+        case 3: st = sk_launch_rows<3>(out, qs, ds, x, y, part, m, n, k, splits, s); break;
+        case 4: st = sk_launch_rows<4>(out, qs, ds, x, y, part, m, n, k, splits, s); break;
+        case 7: st = sk_launch_rows<7>(out, qs, ds, x, y, part, m, n, k, splits, s); break;
+        default: st = sk_launch_rows<8>(out, qs, ds, x, y, part, m, n, k, splits, s); break;
+    }
     if (st != LHIP_OK || splits == 1) return st;
     return q8_gemm_reduce_launch(part, y, m, n, splits, out, s);
 }

@@ -168,6 +168,32 @@ def test_weight_streaming_gemm_vs_oracle(oracle, m, n, k):
         assert np.all(np.abs(y - auto) <= step) and np.mean(y == auto) > 0.98, slices
 
 
+@pytest.mark.parametrize("m,n,k", [
+    (1, 36, 512), (16, 100, 1024), (17, 8188, 1024), (32, 28, 2048),            # strips of 32 rows: ragged, none full
+    (16, 8212, 1024), (33, 12276, 1024),                                        # 48: one row more than 256 strips of 32 hold
+    (65, 8212, 1024), (128, 12300, 1024), (16, 16388, 1024), (64, 14332, 512),  # 64, and one round of them exceeded
+    (16, 4100, 4096), (64, 4092, 4096), (31, 500, 8192), (128, 2044, 8192),     # narrow strips over K slices
+])
+def test_weight_streaming_gemm_by_every_strip_width(oracle, m, n, k):
+    """Sizes on the edges of the strips of 32, 48, 64 and 112 / 128 weight rows, with and without K slices.  The block
+    sums are f32 (32 exact products) and so are their K / 32 additions, so an element is off by less than
+    (32 + K / 32) 2^-24 times the sum of the magnitudes of its terms; the bf16 form is the f32 output rounded once."""
+    qs, d = synth.q8_0_random(n, k, seed=m + n + k)
+    xf, bits = bf16_activations(oracle, m, k, seed=m + 1)
+    w = upload(qs, d)
+    x = torch.from_numpy(bits.view(np.int16)).to(DEV).view(torch.bfloat16)
+    lib, st = capi.load_library(), torch.cuda.current_stream().cuda_stream
+    y32 = torch.full((m, n), float("nan"), device=DEV)
+    capi.check(lib.lhip_q8_0_matmul_bf16_f32out(w.planar.data_ptr(), x.data_ptr(), y32.data_ptr(), m, n, k, st), "f32out")
+    y16 = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=DEV)
+    capi.check(lib.lhip_q8_0_matmul_bf16(w.planar.data_ptr(), x.data_ptr(), y16.data_ptr(), m, n, k, st), "bf16")
+    weight = torch.from_numpy((qs.reshape(n, k // 32, 32).astype(np.float64) * d.astype(np.float64)[:, :, None]).reshape(n, k))
+    x64 = torch.from_numpy(xf.astype(np.float64).reshape(m, k))
+    err = (y32.cpu().double() - x64 @ weight.T).abs()
+    assert bool((err <= (32 + k // 32) * 2.0 ** -24 * (x64.abs() @ weight.abs().T)).all())
+    assert torch.equal(y16, y32.to(torch.bfloat16))
+
+
 @pytest.mark.parametrize("m,n,k", [(129, 260, 1024), (300, 128, 512), (512, 1024, 4096)])
 def test_weight_streaming_gemm_in_passes(oracle, m, n, k):
     """More than 128 rows through the weight-streaming kernel (tile id 5): passes of 128 rows in one launch."""
