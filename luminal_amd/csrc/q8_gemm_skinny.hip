@@ -266,7 +266,7 @@ __global__ __launch_bounds__((CW + 4) * 64) void q8_gemm_skinny_kernel(const int
         for (int cb = 0; cb < MT; ++cb) acc[cb] = sk_f32x4{0.f, 0.f, 0.f, 0.f};
 
         constexpr int UNITS = 2 * MT;  // (block, column block) pairs of a group
-        constexpr int kPending = NL == 1 ? 2 : 0;
+        constexpr int kPending = NL == 1 || (NL == 3 && MT <= 2 && CW <= 4) ? 2 : 0;
         auto b_read = [&](const unsigned char *xb, int i, int limb) __attribute__((always_inline)) {
             return *reinterpret_cast<const sk_bf16x8 *>(xb + limb * S::PLANE + (i % MT) * 16 * kSkPitch + (i / MT) * 64);
         };
@@ -283,8 +283,9 @@ __global__ __launch_bounds__((CW + 4) * 64) void q8_gemm_skinny_kernel(const int
         }
         // A unit's block sums are added kPending units after their MFMA, when they are there: with bf16 activations (one MFMA
         // per unit) a wave alone on its SIMD otherwise waits out every MFMA (64 x 512 x 1024 8.1 -> 7.0 us, 128 x 4096 x 1024
-        // 12.4 -> 10.3, 16 x 14336 x 4096 16.4 -> 16.2; two units, one gives half of it).  The limbs of f32 / f16 activations fill
-        // the pipe by themselves: 64 x 14336 x 4096 f32 37.9 -> 38.6 us with it.
+        // 12.4 -> 10.3, 16 x 14336 x 4096 16.4 -> 16.2; two units, one gives half of it).  So does the chain of three of an f32
+        // for up to 32 rows in narrow strips (2-7 % of the product); elsewhere the limbs fill the pipe by themselves and
+        // it costs 1-4 % (64 x 14336 x 4096 f32 37.9 -> 38.6 us).
         sk_f32x4 sum[4];
         float dv[2][2][4];  // scales of this group and of the one before it
         static_for<kPending>([&](auto ic) __attribute__((always_inline)) {
@@ -453,31 +454,64 @@ static int sk_splits_for(int strips, int m, int n, int k, size_t room) {
 // Compute waves per workgroup (strips of 16 rows each) for `splits` K slices (0: the slices are chosen with them).
 struct SkPlan {
     int cw, splits;
+    double of_base = 1.0;  // its time over that of strips of 128 (112) rows in the slices that fill the chip, by sk_us
 };
 constexpr int kSkWaves[] = {8, 7, 4, 3, 2};
 
-// What the kernel takes for one pass of bf16 rows, us.  A workgroup walks 512 of K in the time of its table (the vector
-// instructions of its waves: conversions, and four fmas per MFMA) or in the time that the weights and activations of all of
-// them take from memory and L2, whichever is longer (joined by a fourth power); a CU runs them one after the other; the sum
-// of the slices is a launch and its planes.  Fitted to 2800 measurements, the numbers of slices around those that fill the
-// chip for 240 sizes (m of 16 to 128, N of 512 to 28672, K of 1024 to 14336).
+// What the kernel takes for one pass of activation rows, us.  A workgroup walks 512 of K in the time of its table (the
+// vector instructions of its waves: conversions, and four fmas per block and 16 rows) or in the time that the weights and
+// activations of all of them take from memory and L2, whichever is longer (joined by a fourth power); a CU runs them one
+// after the other; the sum of the slices is a launch and its planes.
+struct SkTimes {
+    double walk[4][5];                // by activation rows (16, 32, 64, 128) and kSkWaves (0: not built)
+    double weights[4], activations;   // bytes per us
+    double fixed[4], sum, planes;     // us, us, us per MB
+    int x_bytes;
+};
+// bf16: fitted to 2800 measurements, the numbers of slices around those that fill the chip for 240 sizes (m of 16 to 128, N
+// of 512 to 28672, K of 1024 to 14336).
+static constexpr SkTimes kSkBf16 = {{{3.11, 2.60, 1.33, 1.10, 0.98}, {3.34, 2.96, 1.68, 1.42, 1.23},
+                                     {5.24, 4.61, 2.69, 2.18, 1.99}, {5.96, 5.44, 3.62, 3.29, 3.10}},
+                                    {6.2e6, 7.0e6, 5.8e6, 7.0e6}, 20e6, {3.2, 3.35, 3.65, 4.45}, 2.0, 0.52, 2};
+// f32, and f16 too (so that both take the same plan, and an f16 result is the f32 form's rounded once; its own fit would
+// gain 0.5 %): 1400 measurements for 120 sizes (m of 16 to 64).
+static constexpr SkTimes kSkF32 = {{{3.15, 0.0, 1.64, 1.46, 1.34}, {4.12, 0.0, 2.67, 2.52, 2.37}, {6.58, 0.0, 4.57, 4.41, 4.15}, {}},
+                                   {5.44e6, 5.59e6, 7.0e6, 7.0e6}, 20e6, {3.5, 3.6, 4.2, 0.0}, 1.7, 0.97, 4};
+
 // `groups` workgroups of kSkWaves[cw_index] compute waves walk `per` units of K; a plan that cannot come below `limit` is not
 // worked out.
-static double sk_us(int cw_index, int slices, unsigned groups, int per, int m, int n, double limit) {
-    static const double walk[4][5] = {{3.11, 2.60, 1.33, 1.10, 0.98},   // up to 16 activation rows
-                                      {3.34, 2.96, 1.68, 1.42, 1.23},   // 32
-                                      {5.24, 4.61, 2.69, 2.18, 1.99},   // 64
-                                      {5.96, 5.44, 3.62, 3.29, 3.10}};  // 128
-    static const double weights[4] = {6.2e6, 7.0e6, 5.8e6, 7.0e6}, activations = 20e6;  // bytes per us
-    static const double fixed[4] = {3.2, 3.35, 3.65, 4.45};
-    const int rows = m <= 16 ? 0 : (m <= 32 ? 1 : (m <= 64 ? 2 : 3)), strip = 16 * kSkWaves[cw_index];
-    const double walks = static_cast<double>((groups + 255) / 256 * static_cast<unsigned>(per));
-    const double rest = fixed[rows] + (slices > 1 ? 2.0 + 0.52 * static_cast<double>(slices) * m * n * 4e-6 : 0.0);
-    if (rest + walks * walk[rows][cw_index] >= limit) return limit;
+static double sk_us(const SkTimes &t, int cw_index, int slices, unsigned groups, int per, int m, int n, double limit) {
+    const int rows = m <= 16 ? 0 : (m <= 32 ? 1 : (m <= 64 || t.x_bytes == 4 ? 2 : 3)), strip = 16 * kSkWaves[cw_index];
+    const double walk = t.walk[rows][cw_index], walks = static_cast<double>((groups + 255) / 256 * static_cast<unsigned>(per));
+    const double rest = t.fixed[rows] + (slices > 1 ? t.sum + t.planes * static_cast<double>(slices) * m * n * 4e-6 : 0.0);
+    if (walk == 0.0 || rest + walks * walk >= limit) return limit;
     const double stream = static_cast<double>(groups < 256 ? groups : 256) *
-                          (strip * (kSkUnit + kSkUnit / 16) / weights[rows] + (16 << rows) * 2 * kSkUnit / activations);
-    const double w2 = walk[rows][cw_index] * walk[rows][cw_index], s2 = stream * stream;
+                          (strip * (kSkUnit + kSkUnit / 16) / t.weights[rows] + (16 << rows) * t.x_bytes * kSkUnit / t.activations);
+    const double w2 = walk * walk, s2 = stream * stream;
     return rest + walks * sqrt(sqrt(w2 * w2 + s2 * s2));
+}
+
+// `base`, or the strip and number of slices (fixed_s: that one) that sk_us puts below `margin` of it.
+static SkPlan sk_faster_plan(const SkTimes &t, SkPlan base, double margin, int m, int n, int k, size_t room, int fixed_s, int passes = 1) {
+    const int units = k / kSkUnit;
+    auto strips_of = [n, passes](int cw) { return static_cast<unsigned>((n + 16 * cw - 1) / (16 * cw) * passes); };
+    auto per_of = [units](int s) { return static_cast<int>(static_cast<unsigned>(units + s - 1) / static_cast<unsigned>(s)); };
+    SkPlan best = base;
+    const int base_index = base.cw == 8 ? 0 : 1;
+    const double base_us = sk_us(t, base_index, base.splits, strips_of(base.cw) * base.splits, per_of(base.splits), m, n, 1e30);
+    double best_us = margin * base_us;
+    for (int i = 0; i < static_cast<int>(sizeof(kSkWaves) / sizeof(kSkWaves[0])); ++i) {
+        const unsigned strips = strips_of(kSkWaves[i]);
+        for (int s = fixed_s ? fixed_s : 1; s <= (fixed_s ? fixed_s : units); ++s) {
+            // (two rounds of workgroups are enough for any strip)
+            if (s > 1 && !fixed_s && (strips * s > 512 || static_cast<size_t>(s) * m * n > room)) break;
+            const int per = per_of(s);
+            if ((s - 1) * per >= units) continue;  // an empty slice
+            const double us = sk_us(t, i, s, strips * s, per, m, n, best_us);
+            if (us < best_us) best_us = us, best = SkPlan{kSkWaves[i], s, us / base_us};
+        }
+    }
+    return best;
 }
 
 // A workgroup's time goes with the weights it streams (rows x its share of K) and the launch takes as many rounds of
@@ -491,9 +525,7 @@ static SkPlan sk_plan(int m, int n, int k, size_t room, int splits = 0) {
     const int units = k / kSkUnit, passes = (m + 127) / 128;
     SkPlan best{8, 1};
     long best_cost = -1;
-    int best_index = 0;
-    for (int i = 0; i < 2; ++i) {
-        const int cw = kSkWaves[i];
+    for (int cw = 8; cw >= 7; --cw) {
         const int strips = (n + cw * 16 - 1) / (cw * 16);
         int s = splits > 0 ? (splits > units ? units : splits) : sk_splits_for(strips, m, n, k, room);
         const int per = (units + s - 1) / s;
@@ -502,27 +534,10 @@ static SkPlan sk_plan(int m, int n, int k, size_t room, int splits = 0) {
         const long cost = rounds * cw * per;
         if (best_cost < 0 || cost < best_cost) {
             best_cost = cost;
-            best_index = i;
             best = SkPlan{cw, s};
         }
     }
-    if (passes > 1) return best;
-    auto strips_of = [n](int i) { return static_cast<unsigned>((n + 16 * kSkWaves[i] - 1) / (16 * kSkWaves[i])); };
-    auto per_of = [units](int s) { return static_cast<int>(static_cast<unsigned>(units + s - 1) / static_cast<unsigned>(s)); };
-    const int fixed_s = splits > 0 ? best.splits : 0;
-    double best_us = 0.94 * sk_us(best_index, best.splits, strips_of(best_index) * best.splits, per_of(best.splits), m, n, 1e30);
-    for (int i = 0; i < static_cast<int>(sizeof(kSkWaves) / sizeof(kSkWaves[0])); ++i) {
-        const unsigned strips = strips_of(i);
-        for (int s = fixed_s ? fixed_s : 1; s <= (fixed_s ? fixed_s : units); ++s) {
-            // (two rounds of workgroups are enough for any strip)
-            if (s > 1 && !fixed_s && (strips * s > 512 || static_cast<size_t>(s) * m * n > room)) break;
-            const int per = per_of(s);
-            if ((s - 1) * per >= units) continue;  // an empty slice
-            const double us = sk_us(i, s, strips * s, per, m, n, best_us);
-            if (us < best_us) best_us = us, best = SkPlan{kSkWaves[i], s};
-        }
-    }
-    return best;
+    return passes > 1 ? best : sk_faster_plan(kSkBf16, best, 0.94, m, n, k, room, splits > 0 ? best.splits : 0);
 }
 
 // The plan for `room` floats of partial planes: the one the library's own array allows wherever it fits (so that a
@@ -611,17 +626,27 @@ lhip_status q8_gemm_skinny_launch(const int8_t *qs, const __half *ds, const void
 // ---- the f32-accurate ("split") form behind the f32 / f16 operators
 
 // m rows in all; passes of 64 rows (one: the tile height follows m).
-template <typename XT, int OUT>
-static lhip_status sk_launch_split_rows(const int8_t *qs, const __half *ds, const XT *x, void *y, float *part, int m, int n,
-                                        int k, int splits, int passes, hipStream_t s) {
+template <typename XT, int OUT, int CW>
+static lhip_status sk_launch_split_strips(const int8_t *qs, const __half *ds, const XT *x, void *y, float *part, int m, int n,
+                                          int k, int splits, int passes, hipStream_t s) {
     if (splits > 1) {
-        if (passes == 1 && m <= 16) return sk_launch_t<1, kSkOutPartial, XT>(qs, ds, x, y, part, m, n, k, splits, 1, s);
-        if (passes == 1 && m <= 32) return sk_launch_t<2, kSkOutPartial, XT>(qs, ds, x, y, part, m, n, k, splits, 1, s);
-        return sk_launch_t<4, kSkOutPartial, XT>(qs, ds, x, y, part, m, n, k, splits, passes, s);
+        if (passes == 1 && m <= 16) return sk_launch_t<1, kSkOutPartial, XT, CW>(qs, ds, x, y, part, m, n, k, splits, 1, s);
+        if (passes == 1 && m <= 32) return sk_launch_t<2, kSkOutPartial, XT, CW>(qs, ds, x, y, part, m, n, k, splits, 1, s);
+        return sk_launch_t<4, kSkOutPartial, XT, CW>(qs, ds, x, y, part, m, n, k, splits, passes, s);
     }
-    if (passes == 1 && m <= 16) return sk_launch_t<1, OUT, XT>(qs, ds, x, y, part, m, n, k, 1, 1, s);
-    if (passes == 1 && m <= 32) return sk_launch_t<2, OUT, XT>(qs, ds, x, y, part, m, n, k, 1, 1, s);
-    return sk_launch_t<4, OUT, XT>(qs, ds, x, y, part, m, n, k, 1, passes, s);
+    if (passes == 1 && m <= 16) return sk_launch_t<1, OUT, XT, CW>(qs, ds, x, y, part, m, n, k, 1, 1, s);
+    if (passes == 1 && m <= 32) return sk_launch_t<2, OUT, XT, CW>(qs, ds, x, y, part, m, n, k, 1, 1, s);
+    return sk_launch_t<4, OUT, XT, CW>(qs, ds, x, y, part, m, n, k, 1, passes, s);
+}
+template <typename XT, int OUT>
+static lhip_status sk_launch_split_rows(int cw, const int8_t *qs, const __half *ds, const XT *x, void *y, float *part, int m,
+                                        int n, int k, int splits, int passes, hipStream_t s) {
+    switch (cw) {
+        case 2: return sk_launch_split_strips<XT, OUT, 2>(qs, ds, x, y, part, m, n, k, splits, passes, s);
+        case 3: return sk_launch_split_strips<XT, OUT, 3>(qs, ds, x, y, part, m, n, k, splits, passes, s);
+        case 4: return sk_launch_split_strips<XT, OUT, 4>(qs, ds, x, y, part, m, n, k, splits, passes, s);
+        default: return sk_launch_split_strips<XT, OUT, 8>(qs, ds, x, y, part, m, n, k, splits, passes, s);
+    }
 }
 
 bool q8_gemm_split_supports(int n, int k, const void *x, const void *y, bool f16) {
@@ -632,8 +657,9 @@ bool q8_gemm_split_supports(int n, int k, const void *x, const void *y, bool f16
 // while strips x passes leave the chip unfilled.  At most kSkMaxPasses passes per launch (the grid's z extent).
 constexpr int64_t kSkMaxPasses = 1024;
 
-// K slices of one chunk of mc rows: as many as fill the chip, within `room` floats of partial planes.
-static int split_slices(int mc, int n, int k, size_t room) {
+// K slices of one chunk of mc rows in strips of 128 weight rows: as many as fill the chip, within `room` floats of partial
+// planes.
+static int split_base_slices(int mc, int n, int k, size_t room) {
     const int units = k / kSkUnit, strips = (n + kSkRows - 1) / kSkRows, passes = (mc + 63) / 64;
     int splits = 256 / (strips * passes);
     if (splits < 1) splits = 1;
@@ -641,6 +667,22 @@ static int split_slices(int mc, int n, int k, size_t room) {
     while (splits > 1 && static_cast<size_t>(splits) * mc * n > room) --splits;
     const int per = (units + splits - 1) / splits;
     return (units + per - 1) / per;  // no empty slice
+}
+// The plan of a chunk: those, or up to 1024 rows any other strip and number of slices that sk_us puts 3 % below.  m x N x K, f32
+// and f16, us: 16 x 4096 x 1024 9.2 -> 5.9 and 8.9 -> 5.8, 32 x 4096 x 4096 13.9 -> 12.7 and 12.8 -> 11.6, 64 x 2048 x 4096 17.4 -> 13.8
+// and 16.2 -> 12.6, 16 x 14336 x 4096 21.2 -> 19.4 and 19.7 -> 17.6, 256 x 512 x 4096 17.3 -> 13.6 and 15.8 -> 12.4, 1000 x 256 x 1024
+// 16.2 -> 11.4 and 14.7 -> 9.5; as it was: 16 x 8192 x 8192 23.2 and 21.4.  Mean of 500 sizes of up to 64 rows 0.87, of 900 above
+// that 0.85 (0.82 - 0.88 by type and rows), at none more than 2 % behind.
+static SkPlan split_plan_for(int mc, int n, int k, size_t room) {
+    const int passes = (mc + 63) / 64;
+    const SkPlan base{8, split_base_slices(mc, n, k, room)};
+    return passes > 16 ? base : sk_faster_plan(kSkF32, base, 0.97, mc, n, k, room, 0, passes);
+}
+// The library array's plan wherever it fits, as sk_plan_within.
+static SkPlan split_plan(int mc, int n, int k, size_t room) {
+    const SkPlan plan = split_plan_for(mc, n, k, kSkScratchFloats);
+    if (plan.splits == 1 || static_cast<size_t>(plan.splits) * mc * n <= room) return plan;
+    return split_plan_for(mc, n, k, room);
 }
 
 // ---- the choice of the kernel for the f32 / f16 operators
@@ -681,11 +723,12 @@ static RowsPlan rows_plan(int64_t m, int n, int k, bool f16, size_t room, bool s
     auto rounds = [](int64_t workgroups) { return static_cast<double>((workgroups + 255) / 256); };
     auto sum_us = [&](int64_t slices, int64_t cols) { return 3.0 + static_cast<double>(slices * m * cols) * 4.0 / 8e6; };
     double best_us = 1e30;
-    if (stream) {
+    if (stream) {  // (0.49 and 0.38 us are those of strips of 128 rows)
         const int mc = static_cast<int>(m < 64 * kSkMaxPasses ? m : 64 * kSkMaxPasses);
-        const int splits = split_slices(mc, n, k, room);
+        const int splits = split_base_slices(mc, n, k, room);
         best_us = 6.0 + rounds(((n + kSkRows - 1) / kSkRows) * ((m + 63) / 64) * splits) * (nblk / splits) * (f16 ? 0.38 : 0.49) +
                   (splits > 1 ? sum_us(splits, n) : 0.0);
+        if (mc == m) best_us *= split_plan(mc, n, k, room).of_base;
     }
     if (f16 && q8_gemm_wide_supports(k)) {
         const double us = 8.0 + static_cast<double>(q8_gemm_wide_ends(m, n)) * 0.32 * nblk;
@@ -731,7 +774,7 @@ size_t q8_gemm_split_workspace_floats(int64_t m, int n, int k) {
         }
         for (int64_t m0 = 0; m0 < m; m0 += 64 * kSkMaxPasses) {
             const int mc = static_cast<int>(m - m0 < 64 * kSkMaxPasses ? m - m0 : 64 * kSkMaxPasses);
-            const int splits = split_slices(mc, n, k, kSkScratchFloats);
+            const int splits = split_plan(mc, n, k, kSkScratchFloats).splits;
             if (splits > 1) most = std::max(most, static_cast<size_t>(splits) * mc * n);
         }
     }
@@ -762,7 +805,8 @@ lhip_status q8_gemm_split_launch(const int8_t *qs, const __half *ds, const void 
     for (int64_t m0 = 0; m0 < m; m0 += 64 * kSkMaxPasses) {
         const int mc = static_cast<int>(m - m0 < 64 * kSkMaxPasses ? m - m0 : 64 * kSkMaxPasses);
         const int passes = (mc + 63) / 64;
-        const int splits = split_slices(mc, n, k, room);
+        const SkPlan strips = split_plan(mc, n, k, room);
+        const int splits = strips.splits;
         float *part = nullptr;
         if (splits > 1) {
             part = own_workspace ? ws : sk_scratch_ptr();
@@ -770,9 +814,9 @@ lhip_status q8_gemm_split_launch(const int8_t *qs, const __half *ds, const void 
         }
         const auto *xc = static_cast<const unsigned char *>(x) + static_cast<size_t>(m0) * k * esz;
         auto *yc = static_cast<unsigned char *>(y) + static_cast<size_t>(m0) * n * esz;
-        lhip_status st = f16 ? sk_launch_split_rows<__half, kSkOutF16>(qs, ds, reinterpret_cast<const __half *>(xc), yc, part,
+        lhip_status st = f16 ? sk_launch_split_rows<__half, kSkOutF16>(strips.cw, qs, ds, reinterpret_cast<const __half *>(xc), yc, part,
                                                                        mc, n, k, splits, passes, s)
-                             : sk_launch_split_rows<float, kSkOutF32>(qs, ds, reinterpret_cast<const float *>(xc), yc, part,
+                             : sk_launch_split_rows<float, kSkOutF32>(strips.cw, qs, ds, reinterpret_cast<const float *>(xc), yc, part,
                                                                       mc, n, k, splits, passes, s);
         if (st != LHIP_OK) return st;
         if (splits > 1)
