@@ -325,6 +325,7 @@ enum { kOutBf16 = 0, kOutF32 = 1, kOutSwiglu = 2 };
 // q8_gemm_skinny.hip: the weight-streaming kernel for at most 128 activation rows.
 bool q8_gemm_skinny_supports(int m, int n, int k, int out, const void *y);
 int q8_gemm_skinny_splits(int m, int n, int k, size_t room);
+double q8_gemm_skinny_us(int m, int n, int k, size_t room);
 lhip_status q8_gemm_skinny_launch(const int8_t *qs, const __half *ds, const void *x_bf16, void *y, int m, int n, int k,
                                   int out, int splits, hipStream_t s, bool own_workspace = false, float *ws = nullptr,
                                   size_t ws_floats = 0);
@@ -431,8 +432,9 @@ static lhip_status gemm_dispatch(const void *planar_dev, const void *x_dev, void
     const bool wide = q8_gemm_wide_supports(k);  // where not, asked for by name: the same product by tiles of 128x128
     if (tile == kTileSkinny || (tile > kTileSkinnySplit && tile <= kTileSkinnySplit + 64)) {
         if (!q8_gemm_skinny_supports(mi, ni, ki, out, y_dev)) return LHIP_ERR_UNSUPPORTED;
+        // (a plain call of a K that is no multiple of 512 has no room: gemm_plain_room)
         return q8_gemm_skinny_launch(qs, ds, x_dev, y_dev, mi, ni, ki, out, tile == kTileSkinny ? 0 : tile - kTileSkinnySplit, s,
-                                     scratch.own, scratch.ws, scratch.floats);
+                                     scratch.own || k % 512 != 0, scratch.ws, scratch.floats);
     }
     if (tile > kTileSliced && tile <= kTileSliced + 16) {
         // Few output tiles (the down projection of a 512-token prompt: 64 tiles of 128x256): slices of K fill the chip,
@@ -521,15 +523,17 @@ static double gemm_sliced_us(int64_t m, int64_t n, int64_t slices, int64_t per, 
            0.33e-6 * 4.0 * static_cast<double>(slices * m) * static_cast<double>(n);
 }
 
-static int gemm_auto_tile(int64_t m, int64_t n, int64_t k, int out, const void *y, size_t room) {
-    // Few activation rows: the product is bound by the weight stream
-    if (m <= 128 && n <= kMaxDim && k <= kMaxDim &&
-        q8_gemm_skinny_supports(static_cast<int>(m), static_cast<int>(n), static_cast<int>(k), out, y))
-        return kTileSkinny;
+// The tiles (kTile...) for a product that the weight-streaming kernel does not take, and their time, us.
+static int gemm_tiles(int64_t m, int64_t n, int64_t k, int out, const void *y, size_t room, double *us) {
     const int64_t kt = k / kBK, b0 = (m + 127) / 128 * ((n + 255) / 256);
-    if (m <= 32) return (m + 127) / 128 * ((n + 63) / 64) >= 64 ? 2 : 3;
+    if (m <= 32) {
+        const int tile = (m + 127) / 128 * ((n + 63) / 64) >= 64 ? 2 : 3;
+        *us = tile == 2 ? 4.3 + static_cast<double>(kt) : 3.0 + 0.6 * (k % (kBK * 2) != 0 ? 1.12 : 1.0) * static_cast<double>(kt);
+        return tile;
+    }
     int tile;
-    const double unsliced = gemm_unsliced_us(m, n, k, &tile) + (tile == 2 ? 2.2 : tile == 3 ? 1.3 : 0.0);
+    *us = gemm_unsliced_us(m, n, k, &tile);
+    const double unsliced = *us + (tile == 2 ? 2.2 : tile == 3 ? 1.3 : 0.0);
     // Few 128x256 tiles: slices of K until the chip is full (at most eight, of at least four 64-wide tiles), when the
     // partial planes fit the scratch array and cost less than the shorter walk saves (measured, us, whole K -> sliced: 4096 x
     // 4096 at 512 rows 73 -> 36, 4096 x 14336 at 512 rows 244 -> 85, 2880 x 2880 at 777 rows 54 -> 33 over three uneven
@@ -539,11 +543,31 @@ static int gemm_auto_tile(int64_t m, int64_t n, int64_t k, int out, const void *
             for (int64_t slices = 256 / b0 < 8 ? 256 / b0 : 8; slices >= 2; --slices) {
                 const int64_t per = (kt + slices - 1) / slices;
                 if (per < 4 || (slices - 1) * per >= kt || static_cast<size_t>(slices) * m * n > room) continue;
-                if (gemm_sliced_us(m, n, slices, per, b0 * slices) < unsliced) return kTileSliced + static_cast<int>(slices);
+                const double sliced = gemm_sliced_us(m, n, slices, per, b0 * slices);
+                if (sliced < unsliced) {
+                    *us = sliced;
+                    return kTileSliced + static_cast<int>(slices);
+                }
             }
         if (gemm_tail_plan(m, n, k, out, y, room).slices >= 2) return kTileTail;
     }
     return tile;
+}
+
+static int gemm_auto_tile(int64_t m, int64_t n, int64_t k, int out, const void *y, size_t room) {
+    double us;
+    // Few activation rows: the product is bound by the weight stream.  A K that is no multiple of 512 is one for that kernel
+    // unless the tiles end within a tenth of it, which they do for a K of one step and for many weight rows.  Measured, us,
+    // tiles -> streamed, without and with a workspace: 16 x 2880 x 2880 33 -> 9.9 and 33 -> 8.6, 45 x 2880 x 2880 33 -> 17 and 15.9 ->
+    // 13.4, 128 x 4096 x 4160 79 -> 36 and 22.5 -> 20, 16 x 28672 x 960 24 -> 10.7; the other way 128 x 28672 x 320 11.5 <- 13.7,
+    // 80 x 28672 x 4160 with one 54 <- 60.
+    if (m <= 128 && n <= kMaxDim && k <= kMaxDim &&
+        q8_gemm_skinny_supports(static_cast<int>(m), static_cast<int>(n), static_cast<int>(k), out, y)) {
+        if (k % 512 == 0) return kTileSkinny;
+        const int tile = gemm_tiles(m, n, k, out, y, room, &us);
+        return 1.1 * q8_gemm_skinny_us(static_cast<int>(m), static_cast<int>(n), static_cast<int>(k), room) < us ? kTileSkinny : tile;
+    }
+    return gemm_tiles(m, n, k, out, y, room, &us);
 }
 
 }  // namespace lhip
@@ -555,6 +579,7 @@ extern "C" {
 lhip_status lhip_q8_0_matmul_bf16_cfg(const void *planar_dev, const void *x_dev, void *y_dev, int64_t m, int64_t n,
                                       int64_t k, int tile, void *stream) {
     if (tile > kTileSliced && tile <= kTileSliced + 16 && k % (kBK * 4 * (tile - kTileSliced)) != 0) return LHIP_ERR_UNSUPPORTED;
+    if ((tile == kTileSkinny || (tile > kTileSkinnySplit && tile <= kTileSkinnySplit + 64)) && k % 512 != 0) return LHIP_ERR_UNSUPPORTED;
     return gemm_dispatch(planar_dev, x_dev, y_dev, m, n, k, tile, kOutBf16, stream);
 }
 

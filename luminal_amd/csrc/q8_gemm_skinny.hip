@@ -1,4 +1,5 @@
-// Q8_0 weights x activations for few activation rows (short prompts, small batches; up to 128 rows per pass).
+// Q8_0 weights x activations for few activation rows (short prompts, small batches; up to 128 rows per pass); bf16
+// activations for any K in steps of 64, f32 and f16 ones for K in steps of 512.
 //
 // With so few activation rows the product is bound by streaming the weights, not by the matrix cores, and the
 // 128/256-row tiles of q8_gemm.hip leave most of the chip idle.  Here a workgroup owns a strip of up to 128 weight rows
@@ -47,7 +48,7 @@ enum { kSkOutBf16 = 0, kSkOutF32 = 1, kSkOutSwiglu = 2, kSkOutPartial = 3, kSkOu
 constexpr int kSkRows = 128;    // weight rows per workgroup of eight compute waves (CW: 16 * CW)
 constexpr int kSkPitch = 160;   // bytes per activation row of a panel in LDS
 constexpr int kSkStages = 3;    // LDS buffers
-constexpr int kSkUnit = 512;     // K slices are whole multiples of this (eight groups of 64 k)
+constexpr int kSkUnit = 512;     // K slices are whole multiples of this (eight groups of 64 k); the last may end sooner
 constexpr size_t kSkScratchFloats = size_t{8} << 20;  // 32 MiB of partial sums
 
 static __device__ __align__(256) float sk_scratch[kSkScratchFloats];
@@ -99,7 +100,10 @@ __device__ __forceinline__ void sk_store4(void *y, float *part, int split, int M
 // CW = compute waves: 8, or as few as sk_plan finds to end first (a strip is one workgroup per K slice and CU, so narrower
 // strips fill the chip with fewer slices, whose planes cost 16-30 % of a product of few rows; a workgroup's time per k
 // falls by less than its rows do, see the table there).
-template <int MT, int OUT, int RING, typename XT, int CW = 8>
+// RAG: any K in steps of 64 that is no multiple of 512, at least 256.  The last slice then ends inside a ring: groups are
+// counted up to a whole one, x is zero behind K, codes behind it are the last group's again and the scales of the last
+// ring are shifted into place with zeros behind them.  (16 x 2880 x 2880 9.9 us against 9.6 for a K of 3072.)
+template <int MT, int OUT, int RING, typename XT, int CW = 8, bool RAG = false>
 __global__ __launch_bounds__((CW + 4) * 64) void q8_gemm_skinny_kernel(const int8_t *__restrict__ qs, const __half *__restrict__ ds,
                                                              const XT *__restrict__ x, void *__restrict__ y,
                                                              float *__restrict__ part, int M, int N, int K,
@@ -114,7 +118,7 @@ __global__ __launch_bounds__((CW + 4) * 64) void q8_gemm_skinny_kernel(const int
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int strip = blockIdx.x, split = blockIdx.y;
     const int g_begin = split * slice_groups;
-    const int n_groups = min(slice_groups, (K >> 6) - g_begin);
+    const int n_groups = min(slice_groups, RAG ? (((K + 63) >> 6) + 7) / 8 * 8 - g_begin : (K >> 6) - g_begin);
     const int n_tiles = n_groups / G;
     // blockIdx.z takes 16 * MT activation rows of the M in all (one launch streams the weights once per pass)
     const int m_base = static_cast<int>(blockIdx.z) * (16 * MT);
@@ -122,19 +126,20 @@ __global__ __launch_bounds__((CW + 4) * 64) void q8_gemm_skinny_kernel(const int
     // the strips advance at the same pace and would otherwise all ask the same memory channels for the same k at
     // the same time (measured: 39 -> 36 us for 28672 x 4096 at 16 rows).  With many rows the strips reading the
     // same activation tile at the same time is worth more (57 against 64 us at 128 rows).
-    const int rot = MT <= 2 ? (strip % (n_groups / RING)) * RING : 0;
+    const int rot = MT <= 2 && !RAG ? (strip % (n_groups / RING)) * RING : 0;
 
     if (wave >= CW) {
         // ---------------- loaders: x tiles -> LDS, two tiles ahead of the compute waves
         const int lt = tid - CW * 64;
         const XT *src[S::CH];
-        int dst[S::CH];
+        int dst[S::CH], k_left[S::CH];  // (k_left: RAG only)
 #pragma unroll
         for (int i = 0; i < S::CH; ++i) {
             const int c = lt + i * 256;
             const int m = c / (G * 8), j = c % (G * 8);
             const int panel = j >> 3, jj = j & 7;
             src[i] = x + static_cast<size_t>(min(m_base + m, M - 1)) * K + (static_cast<size_t>(g_begin) + panel) * 64 + jj * 8;
+            k_left[i] = K - (g_begin + panel) * 64 - jj * 8;
             dst[i] = panel * S::PANEL + m * kSkPitch + jj * 16;  // pieces in natural order: an MFMA step is one Q8_0 block
         }
         constexpr int XL = sizeof(XT) == 4 ? 2 : 1;  // 16-byte loads per piece of 8 k
@@ -144,15 +149,24 @@ __global__ __launch_bounds__((CW + 4) * 64) void q8_gemm_skinny_kernel(const int
             if (tt >= n_tiles) tt -= n_tiles;
             const size_t off = static_cast<size_t>(tt) * (G * 64);
 #pragma unroll
-            for (int i = 0; i < S::CH; ++i)
+            for (int i = 0; i < S::CH; ++i) {
+                const XT *from = src[i] + off;
+                if constexpr (RAG) {  // a piece behind K: read from the row's first k, stored as zero
+                    if (static_cast<int>(off) >= k_left[i]) from = src[i] + (k_left[i] - K);
+                }
 #pragma unroll
-                for (int l = 0; l < XL; ++l)
-                    xr[slot][i][l] = reinterpret_cast<const sk_u32x4 *>(src[i] + off)[l];
+                for (int l = 0; l < XL; ++l) xr[slot][i][l] = reinterpret_cast<const sk_u32x4 *>(from)[l];
+            }
         };
-        auto store_x = [&](int slot, int stage) __attribute__((always_inline)) {
+        auto store_x = [&](int slot, int stage, int t) __attribute__((always_inline)) {
             unsigned char *base = sk_lds + stage * S::STAGE;
 #pragma unroll
             for (int i = 0; i < S::CH; ++i) {
+                if constexpr (RAG) {
+                    if (t * (G * 64) >= k_left[i])
+#pragma unroll
+                        for (int l = 0; l < XL; ++l) xr[slot][i][l] = sk_u32x4{0, 0, 0, 0};
+                }
                 if constexpr (NL == 1) {
                     *reinterpret_cast<sk_u32x4 *>(base + dst[i]) = xr[slot][i][0];
                 } else {
@@ -181,9 +195,9 @@ __global__ __launch_bounds__((CW + 4) * 64) void q8_gemm_skinny_kernel(const int
         };
         load_x(0, 0);
         load_x(1, 1);
-        store_x(0, 0);
+        store_x(0, 0, 0);
         load_x(0, 2);
-        store_x(1, 1);
+        store_x(1, 1, 1);
         load_x(1, 3);
         __syncthreads();
         int stage = 2;  // buffer of tile t + 2
@@ -191,12 +205,12 @@ __global__ __launch_bounds__((CW + 4) * 64) void q8_gemm_skinny_kernel(const int
                                                 // are exact (the loads of a slot are two tiles old when it is stored)
             // The fences keep the arithmetic on one slot's values (the limb split) behind the barrier before it:
             // moved up, it waits for loads that are only one tile old instead of two.
-            store_x(0, stage);  // tile t + 2 (a buffer last read for tile t - 1)
+            store_x(0, stage, t + 2);  // tile t + 2 (a buffer last read for tile t - 1)
             load_x(0, t + 4);
             stage = stage == 2 ? 0 : stage + 1;
             __syncthreads();
             __builtin_amdgcn_sched_barrier(0);
-            store_x(1, stage);  // tile t + 3
+            store_x(1, stage, t + 3);  // tile t + 3
             load_x(1, t + 5);
             stage = stage == 2 ? 0 : stage + 1;
             __syncthreads();
@@ -235,7 +249,7 @@ __global__ __launch_bounds__((CW + 4) * 64) void q8_gemm_skinny_kernel(const int
         sk_u32x4 a_reg[RING];
         sk_u32x4 d_reg[RING / 4][4];
         auto load_a = [&](int u, int group) __attribute__((always_inline)) {
-            int gg = min(group, n_groups - 1) + rot;
+            int gg = min(group, (RAG ? min(n_groups, ((K + 63) >> 6) - g_begin) : n_groups) - 1) + rot;
             if (gg >= n_groups) gg -= n_groups;
             if constexpr (WIDE) {
                 a_reg[u] = *reinterpret_cast<const sk_u32x4 *>(a_ptr + static_cast<size_t>(gg) * 64);
@@ -251,8 +265,24 @@ __global__ __launch_bounds__((CW + 4) * 64) void q8_gemm_skinny_kernel(const int
         auto load_d = [&](int set, int round) __attribute__((always_inline)) {
             int rr = min(round, n_rounds - 1) + rot / 4;
             if (rr >= n_rounds) rr -= n_rounds;
+            if constexpr (RAG) {  // at any multiple of two bytes; eight scales of the row, its last ones where it ends sooner
+                typedef sk_u32x4 sk_u32x4_2 __attribute__((aligned(2)));
+                const int first = min(rr * 8, (K >> 5) - 2 * g_begin - 8);
 #pragma unroll
-            for (int v = 0; v < 4; ++v) d_reg[set][v] = *reinterpret_cast<const sk_u32x4 *>(d_ptr[v] + static_cast<size_t>(rr) * 8);
+                for (int v = 0; v < 4; ++v) d_reg[set][v] = *reinterpret_cast<const sk_u32x4_2 *>(d_ptr[v] + first);
+            } else {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) d_reg[set][v] = *reinterpret_cast<const sk_u32x4 *>(d_ptr[v] + static_cast<size_t>(rr) * 8);
+            }
+        };
+        // The scales of round rr, which load_d may have read from `shift` scales before its first: zeros behind the row.
+        auto settle_d = [&](int set, int rr) __attribute__((always_inline)) {
+            const int shift = 8 * rr - min(8 * rr, (K >> 5) - 2 * g_begin - 8);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const unsigned __int128 all = __builtin_bit_cast(unsigned __int128, d_reg[set][v]);
+                d_reg[set][v] = __builtin_bit_cast(sk_u32x4, shift < 8 ? all >> (16 * (shift & 7)) : static_cast<unsigned __int128>(0));
+            }
         };
         // same order of requests in the prologue as in the loop: a0 .. a3, d0, a4 .. a7, d1
 #pragma unroll
@@ -302,6 +332,11 @@ __global__ __launch_bounds__((CW + 4) * 64) void q8_gemm_skinny_kernel(const int
         int stage = 0;
         int R = 0;
         do {  // a slice is never empty: no guard, so the requests above stay where the fences put them
+            if constexpr (RAG) {  // (one body for every ring: a second for the last spills)
+                if (R + RING / 4 >= n_rounds)
+#pragma unroll
+                    for (int set = 0; set < RING / 4; ++set) settle_d(set, R + set);
+            }
             static_for<RING>([&](auto uc) __attribute__((always_inline)) {
                 constexpr int u = decltype(uc)::value;
                 constexpr bool tile_ends = (u + 1) % G == 0;
@@ -441,8 +476,9 @@ lhip_status q8_gemm_reduce_launch(const float *part, void *y, int m, int n, int 
 
 // K slices for a product: enough workgroups for the 256 CUs, slices of whole 512-k units, partial sums within the
 // scratch array.
+static int sk_units(int k) { return k / kSkUnit + (k % kSkUnit != 0); }
 static int sk_splits_for(int strips, int m, int n, int k, size_t room) {
-    const int units = k / kSkUnit, passes = (m + 127) / 128;
+    const int units = sk_units(k), passes = (m + 127) / 128;
     int s = 256 / (strips * passes);
     if (s < 1) s = 1;
     if (s > units) s = units;
@@ -457,6 +493,7 @@ struct SkPlan {
     double of_base = 1.0;  // its time over that of strips of 128 (112) rows in the slices that fill the chip, by sk_us
 };
 constexpr int kSkWaves[] = {8, 7, 4, 3, 2};
+constexpr bool sk_ragged_waves(int cw) { return cw % 2 == 0; }  // those built for a K that is no multiple of 512
 
 // What the kernel takes for one pass of activation rows, us.  A workgroup walks 512 of K in the time of its table (the
 // vector instructions of its waves: conversions, and four fmas per block and 16 rows) or in the time that the weights and
@@ -493,7 +530,7 @@ static double sk_us(const SkTimes &t, int cw_index, int slices, unsigned groups,
 
 // `base`, or the strip and number of slices (fixed_s: that one) that sk_us puts below `margin` of it.
 static SkPlan sk_faster_plan(const SkTimes &t, SkPlan base, double margin, int m, int n, int k, size_t room, int fixed_s, int passes = 1) {
-    const int units = k / kSkUnit;
+    const int units = sk_units(k);
     auto strips_of = [n, passes](int cw) { return static_cast<unsigned>((n + 16 * cw - 1) / (16 * cw) * passes); };
     auto per_of = [units](int s) { return static_cast<int>(static_cast<unsigned>(units + s - 1) / static_cast<unsigned>(s)); };
     SkPlan best = base;
@@ -501,6 +538,7 @@ static SkPlan sk_faster_plan(const SkTimes &t, SkPlan base, double margin, int m
     const double base_us = sk_us(t, base_index, base.splits, strips_of(base.cw) * base.splits, per_of(base.splits), m, n, 1e30);
     double best_us = margin * base_us;
     for (int i = 0; i < static_cast<int>(sizeof(kSkWaves) / sizeof(kSkWaves[0])); ++i) {
+        if (k % kSkUnit != 0 && !sk_ragged_waves(kSkWaves[i])) continue;
         const unsigned strips = strips_of(kSkWaves[i]);
         for (int s = fixed_s ? fixed_s : 1; s <= (fixed_s ? fixed_s : units); ++s) {
             // (two rounds of workgroups are enough for any strip)
@@ -522,10 +560,10 @@ static SkPlan sk_faster_plan(const SkTimes &t, SkPlan base, double margin, int m
 // 16 x 4096 x 1024 8.4 -> 5.0; as it was: 32 x 10240 x 8192 29.3, 64 x 8192 x 14336 47.7.  Over the 240 sizes it is within
 // 1.4 % of the best of all plans (the first rule alone: 17 %), and at none more than 1 % behind the first rule.
 static SkPlan sk_plan(int m, int n, int k, size_t room, int splits = 0) {
-    const int units = k / kSkUnit, passes = (m + 127) / 128;
+    const int units = sk_units(k), passes = (m + 127) / 128;
     SkPlan best{8, 1};
     long best_cost = -1;
-    for (int cw = 8; cw >= 7; --cw) {
+    for (int cw = 8; cw >= (k % kSkUnit == 0 ? 7 : 8); --cw) {
         const int strips = (n + cw * 16 - 1) / (cw * 16);
         int s = splits > 0 ? (splits > units ? units : splits) : sk_splits_for(strips, m, n, k, room);
         const int per = (units + s - 1) / s;
@@ -550,23 +588,34 @@ static SkPlan sk_plan_within(int m, int n, int k, size_t room, int splits = 0) {
 
 int q8_gemm_skinny_splits(int m, int n, int k, size_t room) { return sk_plan_within(m, n, k, room).splits; }
 
+// What the plan takes, us (one pass: up to 128 rows).
+double q8_gemm_skinny_us(int m, int n, int k, size_t room) {
+    const SkPlan plan = sk_plan_within(m, n, k, room);
+    int index = 0;
+    while (kSkWaves[index] != plan.cw) ++index;
+    const unsigned strips = static_cast<unsigned>((n + 16 * plan.cw - 1) / (16 * plan.cw));
+    return sk_us(kSkBf16, index, plan.splits, strips * plan.splits, (sk_units(k) + plan.splits - 1) / plan.splits, m, n, 1e30);
+}
+
 constexpr int kSkMaxRows = 128 * 64;  // passes are the grid's z extent
 
 bool q8_gemm_skinny_supports(int m, int n, int k, int out, const void *y) {
-    return m >= 1 && m <= kSkMaxRows && k % kSkUnit == 0 && n % 4 == 0 && aligned(y, out == kSkOutF32 ? 16 : (out == kSkOutBf16 ? 8 : 4));
+    return m >= 1 && m <= kSkMaxRows && k % 64 == 0 && k >= 256 && n % 4 == 0 && aligned(y, out == kSkOutF32 ? 16 : (out == kSkOutBf16 ? 8 : 4));
 }
 
 template <typename XT>
 constexpr int sk_limbs() { return sizeof(XT) == 4 ? 3 : (std::is_same<XT, __bf16>::value ? 1 : 2); }
 
-template <int MT, int OUT, typename XT, int CW = 8>
+template <int MT, int OUT, typename XT, int CW = 8, bool RAG = false>
 static lhip_status sk_launch_t(const int8_t *qs, const __half *ds, const XT *x, void *y, float *part, int m, int n,
                                int k, int splits, int passes, hipStream_t s) {
-    auto kern = q8_gemm_skinny_kernel<MT, OUT, 8, XT, CW>;
+    if constexpr (!RAG && sk_ragged_waves(CW) && std::is_same<XT, __bf16>::value)
+        if (k % kSkUnit != 0) return sk_launch_t<MT, OUT, XT, CW, true>(qs, ds, x, y, part, m, n, k, splits, passes, s);
+    auto kern = q8_gemm_skinny_kernel<MT, OUT, 8, XT, CW, RAG>;
     constexpr size_t lds_bytes = SkShape<MT, sk_limbs<XT>()>::LDS;
     static LdsOptIn opt;  // opting in to more than 64 KiB of dynamic LDS is a per-function attribute
     if (lhip_status st = lds_opt_in(opt, reinterpret_cast<const void *>(kern), lds_bytes)) return st;
-    const int units = k / kSkUnit, per = (units + splits - 1) / splits;
+    const int units = sk_units(k), per = (units + splits - 1) / splits;
     hipLaunchKernelGGL(kern,
                        dim3(static_cast<unsigned>((n + CW * 16 - 1) / (CW * 16)), static_cast<unsigned>(splits),
                             static_cast<unsigned>(passes)),

@@ -194,6 +194,41 @@ def test_weight_streaming_gemm_by_every_strip_width(oracle, m, n, k):
     assert torch.equal(y16, y32.to(torch.bfloat16))
 
 
+@pytest.mark.parametrize("m,n,k", [
+    (1, 36, 256), (16, 100, 320), (17, 260, 448), (33, 64, 576), (128, 132, 704),  # one to eleven groups of 64
+    (16, 8196, 960), (64, 16388, 1088), (65, 28, 1472), (128, 8252, 1984),         # strips of 32, 64, 128
+    (5, 2880, 2880), (45, 2880, 2880), (100, 2880, 2880), (31, 516, 14272), (128, 1028, 4160),
+])
+def test_weight_streaming_gemm_of_any_k(oracle, m, n, k):
+    """A K that ends inside a step of 512: without K slices (the plain call) and with them (a workspace), to the bound of
+    test_weight_streaming_gemm_by_every_strip_width with one more addition per slice; an infinite activation at the end
+    of K reaches its row only, and nothing behind K reaches any (the next row of x is infinite there)."""
+    qs, d = synth.q8_0_random(n, k, seed=m + n + k)
+    d = np.maximum(d, np.float16(2.0 ** -14))
+    qs[:, -1] = 3
+    xf, bits = bf16_activations(oracle, m, k, seed=m + 1)
+    w = upload(qs, d)
+    x = torch.from_numpy(bits.view(np.int16)).to(DEV).view(torch.bfloat16)
+    lib, st = capi.load_library(), torch.cuda.current_stream().cuda_stream
+    weight = torch.from_numpy((qs.reshape(n, k // 32, 32).astype(np.float64) * d.astype(np.float64)[:, :, None]).reshape(n, k))
+    x64 = torch.from_numpy(xf.astype(np.float64).reshape(m, k))
+    truth, bound = x64 @ weight.T, (32 + k // 32 + 32) * 2.0 ** -24 * (x64.abs() @ weight.abs().T)
+    nbytes = lib.lhip_q8_0_matmul_bf16_workspace_nbytes(m, n, k, 1)
+    space = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=DEV)
+    y, y_ws = (torch.full((m, n), float("nan"), device=DEV) for _ in range(2))
+    for infinite in (False, True):
+        if infinite:
+            x[m // 2, k - 1] = float("inf")
+        capi.check(lib.lhip_q8_0_matmul_bf16_f32out(w.planar.data_ptr(), x.data_ptr(), y.data_ptr(), m, n, k, st), "plain")
+        capi.check(lib.lhip_q8_0_matmul_bf16_ws(w.planar.data_ptr(), x.data_ptr(), y_ws.data_ptr(), m, n, k, 1,
+                                                space.data_ptr() if nbytes else None, nbytes, st), "ws")
+        for got in (y.cpu().double(), y_ws.cpu().double()):
+            if infinite:
+                assert bool((got[m // 2] == float("inf")).all())
+                got[m // 2] = truth[m // 2]
+            assert bool(((got - truth).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("m,n,k", [(129, 260, 1024), (300, 128, 512), (512, 1024, 4096)])
 def test_weight_streaming_gemm_in_passes(oracle, m, n, k):
     """More than 128 rows through the weight-streaming kernel (tile id 5): passes of 128 rows in one launch."""
