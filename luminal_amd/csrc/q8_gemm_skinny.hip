@@ -823,7 +823,8 @@ size_t q8_gemm_split_workspace_floats(int64_t m, int n, int k) {
         }
         for (int64_t m0 = 0; m0 < m; m0 += 64 * kSkMaxPasses) {
             const int mc = static_cast<int>(m - m0 < 64 * kSkMaxPasses ? m - m0 : 64 * kSkMaxPasses);
-            const int splits = split_plan(mc, n, k, kSkScratchFloats).splits;
+            // (at least what strips of 128 rows want, so that narrower ones without slices do not turn the answer into 0, "a matvec")
+            const int splits = std::max(split_plan(mc, n, k, kSkScratchFloats).splits, split_base_slices(mc, n, k, kSkScratchFloats));
             if (splits > 1) most = std::max(most, static_cast<size_t>(splits) * mc * n);
         }
     }
