@@ -99,6 +99,16 @@ def test_a_ragged_k_takes_the_matrix_cores_where_its_matvecs_are_dearer(m, n, k,
     assert (capi.load_library().lhip_q8_0_matmul_workspace_nbytes(m, n, k) > 0) == rows
 
 
+@pytest.mark.parametrize("m,n,k,bf16", [(48, 20564, 8192, False), (64, 17956, 8192, False), (4000, 2180, 512, False),
+                                        (17, 16780, 8192, True), (48, 17956, 14336, True), (65, 20564, 11264, True)])
+def test_products_whose_plain_calls_may_overlap_keep_no_partial_sums(m, n, k, bf16):
+    """Strips of 128 weight rows (112) fill the chip without K slices here, so nothing goes through the library's array;
+    no narrower strip or further number of slices may change that."""
+    lib = capi.load_library()
+    need = lib.lhip_q8_0_matmul_bf16_workspace_nbytes(m, n, k, 0) if bf16 else lib.lhip_q8_0_matmul_workspace_nbytes(m, n, k)
+    assert need == 0
+
+
 def test_operators_can_be_imported_with_a_torch_that_has_no_gpu_backend():
     code = ("import torch\n"
             "for name in ('_cuda_getDevice', '_cuda_getCurrentRawStream'):\n"
