@@ -193,9 +193,9 @@ lhip_status lhip_q8_0_matvec_fused_f32_cfg(const void *const *planar_dev, float 
  * more rounding.  K must be a multiple of 64 (LHIP_ERR_UNSUPPORTED otherwise).
  *
  * With m <= 128 (and K % 512 == 0, N % 4 == 0, y aligned to 8 bytes; 16 for the f32
- * form below) the three entry points take a kernel that is bound by streaming the
- * weights rather than by the matrix cores.  When the 128-row strips of the weight
- * alone would not fill the chip it also splits K, keeps the f32 partial sums in a
+ * form below; any other K >= 256 where it ends first) the three entry points take a kernel that is bound by streaming the
+ * weights rather than by the matrix cores.  When K % 512 == 0 and strips of 112 or 128 weight rows
+ * alone would not fill the chip it may also split K, keeps the f32 partial sums in a
  * 32 MiB scratch array that the library owns (a __device__ array: nothing is
  * allocated, one copy per device) and adds them in a fixed order in a second
  * launch.  Every such call on a device shares that array: calls with m <= 128 that
