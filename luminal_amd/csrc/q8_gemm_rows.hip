@@ -29,22 +29,25 @@
 
 namespace lhip {
 
-constexpr int kRwBN = 256;                      // weight rows per workgroup
+constexpr int kRwBN = 256;                      // weight rows per workgroup, at most
 constexpr int kRwPlane = kRwBN * 64 + 64;       // bytes of one block's codes as bf16 / f16, and a shift of the banks
 constexpr int kRwBuf = 4 * kRwPlane + 4 * kRwBN * 4;  // a group of four blocks and its scales as f32
 constexpr int kRwLds = 2 * kRwBuf;
 enum { kRwOutF32 = 1, kRwOutF16 = 4 };  // as in q8_gemm_skinny.hip
 
-// Workgroup tile: 128 activation rows (a compute wave: 16) x 256 weight rows, over slice_blocks blocks of K; with more than one
+// Workgroup tile: 128 activation rows (a compute wave: 16) x 16 FR weight rows (256, or fewer where these end sooner: a tile's time
+// goes nearly with its weight rows, and the launch's with its rounds of 256 tiles; the LDS is laid out for 256), over slice_blocks blocks of K; with more than one
 // slice each goes into an f32 plane of (M, N) of its own.  ldy = row pitch of y (N, or more when the launch fills some columns
 // of a wider output).
-template <typename XT, int OUT>
+template <typename XT, int OUT, int FR>
 __global__ __launch_bounds__(768) void q8_gemm_rows_kernel(const int8_t *__restrict__ qs, const unsigned short *__restrict__ ds,
                                                            const XT *__restrict__ x, void *__restrict__ y, int M, int N, int K,
                                                            int m_tiles, int n_tiles, int slices, int slice_blocks, int ldy) {
     constexpr bool kF16 = !std::is_same<XT, float>::value;
     constexpr int L = kF16 ? 1 : 3;                            // operands per value
     constexpr int XW = sizeof(XT) == 4 ? 2 : 1;                // 16-byte loads per 8 values
+    constexpr int BN = 16 * FR, PP = FR / 2;                   // weight rows; pairs of fragments
+    static_assert(FR % 2 == 0 && BN <= kRwBN, "pairs of fragments");
     extern __shared__ __attribute__((aligned(16))) unsigned char rw_lds[];
     int mt, nt, slice;
     {
@@ -61,7 +64,7 @@ __global__ __launch_bounds__(768) void q8_gemm_rows_kernel(const int8_t *__restr
     const int nblk = K >> 5;
     const int blk0 = slice * slice_blocks, nb = min(slice_blocks, nblk - blk0);  // this slice's blocks
     const int groups = (nb + 3) >> 2;
-    const int m0 = mt * 128 + wave * 16, n0 = nt * kRwBN;
+    const int m0 = mt * 128 + wave * 16, n0 = nt * BN;
     const bool idle = m0 >= M;  // a wave without rows only stages
 
     auto swz = [](int row) { return (4 - (row >> 2)) & 3; };
@@ -69,26 +72,26 @@ __global__ __launch_bounds__(768) void q8_gemm_rows_kernel(const int8_t *__restr
         // ---- loaders: a group's codes -> registers -> bf16 / f16 in LDS, two groups ahead of their use.  Thread
         // (row lt / 8 + 32 q, piece lt % 8) holds 16 codes of a group's 128.
         const int lt = tid - 512, wp = lt & 7, wrow = lt >> 3;
-        const int8_t *w_src[8];
+        const int8_t *w_src[PP];
 #pragma unroll
-        for (int q = 0; q < 8; ++q)
+        for (int q = 0; q < PP; ++q)
             w_src[q] = qs + static_cast<size_t>(min(n0 + q * 32 + wrow, N - 1)) * K + static_cast<size_t>(blk0) * 32;
         const int w_dst = (wp >> 1) * kRwPlane + wrow * 64 + (((wp & 1) * 2) ^ swz(wrow)) * 16;  // second half: ^ 16; pass q: + 32 rows
         const unsigned short *s_src = ds + static_cast<size_t>(min(n0 + lt, N - 1)) * nblk + blk0;
         const int s_dst = 4 * kRwPlane + ((lt >> 5) * 16 + (lt & 15)) * 8 + ((lt >> 4) & 1) * 4;
-        mma_u32x4 wreg[2][8];
+        mma_u32x4 wreg[2][PP];
         unsigned short sreg[2][4];
         auto load_w = [&](int set, int grp) __attribute__((always_inline)) {
             // pieces of blocks past the slice's end repeat its last block's (never multiplied)
             const int b = min(grp * 4 + (wp >> 1), nb - 1);
 #pragma unroll
-            for (int q = 0; q < 8; ++q) wreg[set][q] = *reinterpret_cast<const mma_u32x4 *>(w_src[q] + b * 32 + (wp & 1) * 16);
+            for (int q = 0; q < PP; ++q) wreg[set][q] = *reinterpret_cast<const mma_u32x4 *>(w_src[q] + b * 32 + (wp & 1) * 16);
 #pragma unroll
             for (int h = 0; h < 4; ++h) sreg[set][h] = s_src[min(grp * 4 + h, nb - 1)];
         };
         auto store_w = [&](int set, unsigned char *buf) __attribute__((always_inline)) {
 #pragma unroll
-            for (int q = 0; q < 8; ++q) {
+            for (int q = 0; q < PP; ++q) {
                 asm volatile("" : "+v"(wreg[set][q]));
                 const mma_u32x4 &w = wreg[set][q];
                 const mma_u32x4 lo = {codes2<kF16>(w[0], 0), codes2<kF16>(w[0], 1), codes2<kF16>(w[1], 0), codes2<kF16>(w[1], 1)};
@@ -141,23 +144,23 @@ __global__ __launch_bounds__(768) void q8_gemm_rows_kernel(const int8_t *__restr
         }
     };
 
-    mma_f32x4 acc[16];
+    mma_f32x4 acc[FR];
 #pragma unroll
-    for (int j = 0; j < 16; ++j) acc[j] = mma_f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < FR; ++j) acc[j] = mma_f32x4{0.f, 0.f, 0.f, 0.f};
 
     const int b_lane = r * 64 + ((g ^ swz(r)) * 16);
     const int s_lane = 4 * kRwPlane + r * 8;
-    // NB blocks of a group, from block B0 on: eight pairs of weight fragments each against the wave's rows.
+    // NB blocks of a group, from block B0 on: PP pairs of weight fragments each against the wave's rows.
     auto blocks = [&](const unsigned char *buf, int blk, auto nbc, auto first) __attribute__((always_inline)) {
         constexpr int NB = decltype(nbc)::value, B0 = decltype(first)::value, RING = 4, AHEAD = 2;
         mma_u32x4 br[RING][2];
         float sc[RING][2];
         auto read_b = [&](int p) __attribute__((always_inline)) {
-            const int b = B0 + p / 8;
+            const int b = B0 + p / PP;
 #pragma unroll
             for (int j = 0; j < 2; ++j)
-                br[p % RING][j] = *reinterpret_cast<const mma_u32x4 *>(buf + b * kRwPlane + b_lane + (2 * (p % 8) + j) * 16 * 64);
-            const float2 s2 = *reinterpret_cast<const float2 *>(buf + s_lane + b * kRwBN * 4 + (p % 8) * 128);
+                br[p % RING][j] = *reinterpret_cast<const mma_u32x4 *>(buf + b * kRwPlane + b_lane + (2 * (p % PP) + j) * 16 * 64);
+            const float2 s2 = *reinterpret_cast<const float2 *>(buf + s_lane + b * kRwBN * 4 + (p % PP) * 128);
             sc[p % RING][0] = s2.x;
             sc[p % RING][1] = s2.y;
         };
@@ -165,18 +168,18 @@ __global__ __launch_bounds__(768) void q8_gemm_rows_kernel(const int8_t *__restr
         for (int p = 0; p < AHEAD; ++p) read_b(p);
         mma_f32x4 last[2];
         auto scale = [&](int p, int j) __attribute__((always_inline)) {  // the sums of pair p
-            mma_f32x4 &a = acc[2 * (p % 8) + j];
+            mma_f32x4 &a = acc[2 * (p % PP) + j];
 #pragma unroll
             for (int v = 0; v < 4; ++v) a[v] = fmaf(sc[p % RING][j], last[j][v], a[v]);
             asm volatile("" : "+v"(a));
         };
-        static_for<8 * NB>([&](auto pc) __attribute__((always_inline)) {
-            constexpr int p = decltype(pc)::value, b = B0 + p / 8;
-            if constexpr (p % 8 == 0) {
+        static_for<PP * NB>([&](auto pc) __attribute__((always_inline)) {
+            constexpr int p = decltype(pc)::value, b = B0 + p / PP;
+            if constexpr (p % PP == 0) {
                 split_x(b & 1);
                 load_x(b & 1, blk + b + 2);
             }
-            if constexpr (p + AHEAD < 8 * NB) read_b(p + AHEAD);
+            if constexpr (p + AHEAD < PP * NB) read_b(p + AHEAD);
             mma_f32x4 s[2];
             // The fences hold this order: the two fragments' chains alternate, small limbs first, and the scaling of the
             // pair before stands in the middle of them.
@@ -195,8 +198,8 @@ __global__ __launch_bounds__(768) void q8_gemm_rows_kernel(const int8_t *__restr
             last[0] = s[0];
             last[1] = s[1];
         });
-        scale(8 * NB - 1, 0);
-        scale(8 * NB - 1, 1);
+        scale(PP * NB - 1, 0);
+        scale(PP * NB - 1, 1);
     };
     if (idle) {
         for (int grp = 0; grp <= groups; ++grp) __syncthreads();
@@ -218,7 +221,7 @@ __global__ __launch_bounds__(768) void q8_gemm_rows_kernel(const int8_t *__restr
     if ((nb & 3) >= 3) blocks(buf, whole_groups * 4, one, std::integral_constant<int, 2>{});
     if (nb & 3) __syncthreads();
 
-    // ---- epilogue: element v of lane (r, g) is row 4 g + v, column r of its 16 x 16 tile; rows of 256 through LDS
+    // ---- epilogue: element v of lane (r, g) is row 4 g + v, column r of its 16 x 16 tile; rows of 16 FR through LDS
     constexpr int EP = 260;
     float *ep = reinterpret_cast<float *>(rw_lds) + wave * (16 * EP);
     static_assert(8 * 16 * EP * 4 <= kRwLds, "epilogue buffer");
@@ -227,9 +230,10 @@ __global__ __launch_bounds__(768) void q8_gemm_rows_kernel(const int8_t *__restr
     const int col = n0 + lane * 4;
     const bool whole = ldy % 4 == 0 && (reinterpret_cast<uintptr_t>(yo) & (4 * sizeof(OT) - 1)) == 0;
 #pragma unroll
-    for (int j = 0; j < 16; ++j)
+    for (int j = 0; j < FR; ++j)
 #pragma unroll
         for (int v = 0; v < 4; ++v) ep[(4 * g + v) * EP + j * 16 + r] = acc[j][v];
+    if (lane * 4 >= BN) return;  // the next tile's columns
 #pragma unroll 4
     for (int q = 0; q < 16; ++q) {
         const int row = m0 + q;
@@ -271,15 +275,15 @@ __global__ __launch_bounds__(256) void q8_gemm_rows_reduce_kernel(const float *_
     y[m * ldy + (i - m * N)] = static_cast<OT>(v);
 }
 
-template <typename XT, int OUT>
-static lhip_status rw_launch_t(const int8_t *qs, const __half *ds, const void *x, void *y, int m, int n, int k, int slices, int ldy,
+template <typename XT, int OUT, int FR>
+static lhip_status rw_launch_w(const int8_t *qs, const __half *ds, const void *x, void *y, int m, int n, int k, int slices, int ldy,
                                hipStream_t s) {
-    const int m_tiles = (m + 127) / 128, n_tiles = (n + kRwBN - 1) / kRwBN;
+    const int m_tiles = (m + 127) / 128, n_tiles = (n + 16 * FR - 1) / (16 * FR);
     const int64_t total = static_cast<int64_t>(m_tiles) * n_tiles * slices;
     if (total > 0x7ffffff0) return LHIP_ERR_INVALID_SHAPE;  // the grid's x extent
     const int per = q8_gemm_rows_slice_blocks(k, slices);
     if (static_cast<int64_t>(slices - 1) * per >= k / 32) return LHIP_ERR_UNSUPPORTED;  // an empty slice
-    auto kern = q8_gemm_rows_kernel<XT, OUT>;
+    auto kern = q8_gemm_rows_kernel<XT, OUT, FR>;
     static LdsOptIn opt;
     if (lhip_status st = lds_opt_in(opt, reinterpret_cast<const void *>(kern), kRwLds)) return st;
     hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>((total + 7) / 8 * 8)), dim3(768), kRwLds, s, qs,
@@ -289,19 +293,30 @@ static lhip_status rw_launch_t(const int8_t *qs, const __half *ds, const void *x
     return LHIP_OK;
 }
 
+template <typename XT, int OUT>
+static lhip_status rw_launch_t(int width, const int8_t *qs, const __half *ds, const void *x, void *y, int m, int n, int k, int slices,
+                               int ldy, hipStream_t s) {
+    switch (width) {
+        case 128: return rw_launch_w<XT, OUT, 8>(qs, ds, x, y, m, n, k, slices, ldy, s);
+        case 192: return rw_launch_w<XT, OUT, 12>(qs, ds, x, y, m, n, k, slices, ldy, s);
+        case 224: return rw_launch_w<XT, OUT, 14>(qs, ds, x, y, m, n, k, slices, ldy, s);
+        default: return rw_launch_w<XT, OUT, 16>(qs, ds, x, y, m, n, k, slices, ldy, s);
+    }
+}
+
 int q8_gemm_rows_slice_blocks(int64_t k, int slices) {
     return static_cast<int>(((k / 32 + slices - 1) / slices + 3) / 4 * 4);
 }
 
 lhip_status q8_gemm_reduce_launch(const float *part, void *y, int m, int n, int slices, int out, hipStream_t s, int ldy = 0);
 
-lhip_status q8_gemm_rows_launch(const int8_t *qs, const __half *ds, const void *x, void *y, int m, int n, int k, bool f16, int slices,
-                                float *part, int ldy, hipStream_t s) {
+lhip_status q8_gemm_rows_launch(const int8_t *qs, const __half *ds, const void *x, void *y, int m, int n, int k, bool f16, int width,
+                                int slices, float *part, int ldy, hipStream_t s) {
     if (slices == 1)
-        return f16 ? rw_launch_t<__half, kRwOutF16>(qs, ds, x, y, m, n, k, 1, ldy, s)
-                   : rw_launch_t<float, kRwOutF32>(qs, ds, x, y, m, n, k, 1, ldy, s);
-    if (lhip_status st = f16 ? rw_launch_t<__half, kRwOutF32>(qs, ds, x, part, m, n, k, slices, n, s)
-                             : rw_launch_t<float, kRwOutF32>(qs, ds, x, part, m, n, k, slices, n, s))
+        return f16 ? rw_launch_t<__half, kRwOutF16>(width, qs, ds, x, y, m, n, k, 1, ldy, s)
+                   : rw_launch_t<float, kRwOutF32>(width, qs, ds, x, y, m, n, k, 1, ldy, s);
+    if (lhip_status st = f16 ? rw_launch_t<__half, kRwOutF32>(width, qs, ds, x, part, m, n, k, slices, n, s)
+                             : rw_launch_t<float, kRwOutF32>(width, qs, ds, x, part, m, n, k, slices, n, s))
         return st;
     if (n % 4 == 0 && ldy % 4 == 0 && aligned(y, f16 ? 8 : 16))
         return q8_gemm_reduce_launch(part, y, m, n, slices, f16 ? kRwOutF16 : kRwOutF32, s, ldy);

@@ -745,15 +745,15 @@ constexpr int kMaxRowsSlices = 40;
 // tiles of q8_gemm_wide.hip (kWide).
 struct RowsPlan {
     enum Kind { kStream, kRows, kWide } kind = kStream;
-    int n_main = 0, slices = 1;
+    int n_main = 0, slices = 1, width = 256;  // width = weight rows of a tile (of the n_main: 256)
     size_t floats = 0;  // of partial planes
 };
 
 // What q8_gemm_rows.hip takes for up to 64 rows, us: per block of K that the slowest compute unit walks, for the sum of the slices
 // and its planes.  Fitted to 420 sizes (6 % of standard deviation).
-static double few_rows_us(int64_t m, int64_t n, bool f16, int64_t blocks, int slices) {
+static double few_rows_us(int64_t m, int64_t n, bool f16, double blocks, int slices) {
     const double sum = slices > 1 ? (f16 ? 4.1 : 3.8) + static_cast<double>(slices * m * n) * 4e-6 * 0.56 : 0.0;
-    return static_cast<double>(blocks) * (f16 ? 0.63 : 0.78) + sum;
+    return blocks * (f16 ? 0.63 : 0.78) + sum;
 }
 
 // The plan that ends first, by what each kernel takes (us, measured): a workgroup of the streaming kernel 0.49 (f32) or
@@ -773,8 +773,9 @@ static RowsPlan rows_plan(int64_t m, int n, int k, bool f16, size_t room, bool s
     const double nblk = k / 32, block = f16 ? 0.66 : 1.2;
     auto rounds = [](int64_t workgroups) { return static_cast<double>((workgroups + 255) / 256); };
     auto sum_us = [&](int64_t slices, int64_t cols) { return 3.0 + static_cast<double>(slices * m * cols) * 4.0 / 8e6; };
-    double best_us = 1e30, early_us = 1e30;
-    RowsPlan early;  // the best of up to 16 slices that come before a number leaving one empty
+    double best_us = 1e30, early_us = 1e30, bare_us = 1e30;
+    RowsPlan early;  // the best of tiles of 256 in up to 16 slices that come before a number leaving one empty
+    RowsPlan bare;   // the best that has no planes
     bool planes = false;
     if (stream) {  // (0.49 and 0.38 us are those of strips of 128 rows)
         const int mc = static_cast<int>(m < 64 * kSkMaxPasses ? m : 64 * kSkMaxPasses);
@@ -788,7 +789,7 @@ static RowsPlan rows_plan(int64_t m, int n, int k, bool f16, size_t room, bool s
         const double us = 8.0 + static_cast<double>(q8_gemm_wide_ends(m, n)) * 0.32 * nblk;
         if (us < best_us) best_us = us, best.kind = RowsPlan::kWide;
     }
-    early = best, early_us = best_us;
+    early = bare = best, early_us = bare_us = best_us;
     // all columns, or those that whole rounds leave over, in K slices
     const int64_t per_round = m_tiles < 256 ? 256 / m_tiles : 1;
     const int64_t main_tiles = n_tiles / per_round * per_round;
@@ -796,6 +797,9 @@ static RowsPlan rows_plan(int64_t m, int n, int k, bool f16, size_t room, bool s
         if (lead == n_tiles || (lead > 0 && m_tiles > 256)) continue;
         const int64_t cols = n - lead * 256, tiles = m_tiles * (n_tiles - lead);
         const double main_us = lead > 0 ? rounds(m_tiles * lead) * nblk * (m <= 64 ? (f16 ? 0.63 : 0.78) : block) + 8.0 : 0.0;
+        constexpr int widths[] = {256, 224, 192, 128};
+        int64_t tiles_of[4];
+        for (int i = 0; i < 4; ++i) tiles_of[i] = m_tiles * ((cols + widths[i] - 1) / widths[i]);
         bool gap = false;
         for (int slices = 1; slices <= kMaxRowsSlices; ++slices) {
             if (lead > 0 && slices == 1) continue;
@@ -807,20 +811,29 @@ static RowsPlan rows_plan(int64_t m, int n, int k, bool f16, size_t room, bool s
             }
             const size_t floats = slices > 1 ? static_cast<size_t>(slices) * m * cols : 0;
             if (floats > room || (slices > 1 && tiles * slices > 0x7ffffff0)) break;  // (the grid's x extent)
-            const double us = main_us + (m <= 64 ? few_rows_us(m, cols, f16, static_cast<int64_t>(rounds(tiles * slices)) * per, slices)
-                                                 : 8.0 + rounds(tiles * slices) * per * block + (slices > 1 ? sum_us(slices, cols) : 0.0));
-            RowsPlan plan;
-            plan.kind = RowsPlan::kRows;
-            plan.n_main = static_cast<int>(lead * 256);
-            plan.slices = slices;
-            plan.floats = floats;
-            if (us < best_us) best_us = us, best = plan;
-            if (!gap && us < early_us) early_us = us, early = plan;
+            for (int i = 0; i < 4; ++i) {
+                const int width = widths[i];
+                const int64_t all = tiles_of[i] * slices;
+                if (i > 0 && (lead > 0 || (slices > 1 && all > 256))) break;  // (a second round of slices pays a start and an end of its own)
+                const double walk = (width + 20.0) / 276.0, blocks = rounds(all) * per;
+                double us = main_us + (m <= 64 ? few_rows_us(m, cols, f16, blocks * walk, slices)
+                                               : 8.0 + blocks * walk * block + (slices > 1 ? sum_us(slices, cols) : 0.0));
+                RowsPlan plan;
+                plan.kind = RowsPlan::kRows;
+                plan.n_main = static_cast<int>(lead * 256);
+                plan.slices = slices;
+                plan.width = width;
+                plan.floats = floats;
+                if (i == 0 && !gap && us < early_us) early_us = us, early = plan;
+                if (i > 0) us *= 1.06;  // only where clearly ahead
+                if (us < best_us) best_us = us, best = plan;
+                if (floats == 0 && us < bare_us) bare_us = us, bare = plan;
+            }
         }
     }
     // A product of which the plain call keeps nothing in the library's array, so that its calls may overlap, keeps nothing there by
-    // the further numbers of slices either.
-    return stream && early.floats == 0 && !(early.kind == RowsPlan::kStream && planes) ? early : best;
+    // the further numbers of slices and widths either.
+    return stream && early.floats == 0 && !(early.kind == RowsPlan::kStream && planes) ? bare : best;
 }
 
 // Floats of partial planes the plan for (m, n, k) uses when it has the library's own scratch array to itself: what a
@@ -860,10 +873,10 @@ lhip_status q8_gemm_split_launch(const int8_t *qs, const __half *ds, const void 
         if (plan.slices > 1 && !scratch) return LHIP_ERR_HIP;
         const int mi = static_cast<int>(m), tail = n - plan.n_main;
         if (plan.n_main > 0)
-            if (lhip_status st = q8_gemm_rows_launch(qs, ds, x, y, mi, plan.n_main, k, f16, 1, nullptr, n, s)) return st;
+            if (lhip_status st = q8_gemm_rows_launch(qs, ds, x, y, mi, plan.n_main, k, f16, 256, 1, nullptr, n, s)) return st;
         return q8_gemm_rows_launch(qs + static_cast<size_t>(plan.n_main) * k, ds + static_cast<size_t>(plan.n_main) * (k / 32), x,
                                    static_cast<unsigned char *>(y) + static_cast<size_t>(plan.n_main) * esz, mi, tail, k, f16,
-                                   plan.slices, scratch, n, s);
+                                   plan.width, plan.slices, scratch, n, s);
     }
     for (int64_t m0 = 0; m0 < m; m0 += 64 * kSkMaxPasses) {
         const int mc = static_cast<int>(m - m0 < 64 * kSkMaxPasses ? m - m0 : 64 * kSkMaxPasses);
