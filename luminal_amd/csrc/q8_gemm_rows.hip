@@ -16,8 +16,9 @@
 //     waves instead, that work stands in front of their matrix steps (512 x 14336 x 4096 f32: 176 -> 161 us);
 //   * the operand reads run two pairs of fragments ahead, the scaling of a pair runs under the next pair's steps.
 // Measured, whole operator, passes of 64 rows of q8_gemm_skinny.hip -> this kernel: f32 14336 x 4096 at 256 / 512 rows
-// 120 -> 86 / 239 -> 162 us; 2880 x 2880 at 45 rows (K is no multiple of 512: one matvec per row before) 97 -> 18, of which
-// the sum of the slices takes 3.
+// 120 -> 83 / 239 -> 145 us; 2880 x 2880 at 45 rows (K is no multiple of 512: one matvec per row before) 97 -> 13, of which
+// the sum of the slices takes 3.  Tiles of 224 weight rows fill the chip at 256 x 14336 (128 tiles x 2 slices, 85 -> 83), of 128 at 45
+// x 2880 (23 tiles x 8 slices for 12 x 12, 14.6 -> 12.2).
 #include <hip/hip_fp16.h>
 
 #include <type_traits>

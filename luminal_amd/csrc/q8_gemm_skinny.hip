@@ -762,7 +762,9 @@ static double few_rows_us(int64_t m, int64_t n, bool f16, double blocks, int sli
 // few_rows_us says.  The lines this draws (streaming -> chosen, us): 14336 x 4096 f32 at 64 rows 38 -> (54), at 128 61 -> 54,
 // at 256 120 -> 97, at 512 239 -> 162; f16 at 64 rows 34 -> (36), at 128 50 -> 36, at 512 188 -> 90; 4096 x 4096 f32 at 256
 // rows 39 -> (41), at 300 63 -> 44.  Up to 64 rows, and for fewer than sixteen 128x256 tiles, the streaming kernel's narrower
-// strips stay ahead.  A number of slices that leaves one empty is passed over; with 16 slices at most, and none behind the
+// strips stay ahead.  Tiles of 224, 192 or 128 weight rows are taken where the plan puts them 6 % ahead: in one round, or without
+// slices (45 x 2880 x 2880 f32 12 slices of 256 14.6 -> 8 of 128 12.2, 300 x 6144 x 4096 54.8 -> 52.6 at 224, 485 x 9721 x 3488 117 -> 100
+// unsliced at 192, f16 387 x 1138 x 2432 25.8 -> 20.1; in two rounds of slices 138 x 9702 x 5056 72 <- 78).  A number of slices that leaves one empty is passed over; with 16 slices at most, and none behind the
 // first number that leaves one empty, few weight rows or a K of 90 blocks left most compute units idle: 45 x 2880 x 2880 f32
 // 6 -> 12 slices 18.1 -> 15.3 us, 45 x 1000 x 4480 18.9 -> 13.6, 300 x 1000 x 8000 37.4 -> 27.2, f16 400 x 1000 x 8992 30.4 ->
 // 25.7.
@@ -806,6 +808,7 @@ static RowsPlan rows_plan(int64_t m, int n, int k, bool f16, size_t room, bool s
             const int per = q8_gemm_rows_slice_blocks(k, slices);
             gap = gap || slices > 16;
             if (static_cast<int64_t>(slices - 1) * per >= k / 32) {  // an empty slice (the next number may have none)
+                if (per == 4) break;  // (the smallest: every further number leaves one empty)
                 gap = true;
                 continue;
             }
