@@ -140,15 +140,16 @@ class QuantizedMatmul:
         self.cfg = (rows_per_wave, k_unroll, blocks_per_cu, waves_per_block) if rows_per_wave else None
 
     def process(self, x: torch.Tensor, w: Q8Weight) -> torch.Tensor:
-        if self.cfg is None:
-            device = _current_device()
-            out = _native_matmul(x, w.planar, w.n, w.k, False, device, _raw_stream(device))
-            if out is not None:
-                return out
         lib = capi.load_library()
         dtype, n, k = x.dtype, w.n, w.k
+        # (before anything asks for the current device: without a GPU that raises an error of its own)
         if dtype not in (torch.float32, torch.float16) or not x.is_cuda:
             raise TypeError("QuantizedMatmul expects f32 or f16 activations on the GPU")
+        if self.cfg is None:
+            device = _current_device()
+            out = _native_matmul(x, w.planar, n, k, False, device, _raw_stream(device))
+            if out is not None:
+                return out
         if x.shape[-1] != k:
             raise capi.LhipError(capi.LHIP_ERR_INVALID_SHAPE, "QuantizedMatmul",
                                  f"activation K {x.shape[-1]} != weight K {k}")
@@ -186,14 +187,14 @@ class QuantizedMatmulBf16:
         self.tile = tile
 
     def process(self, x: torch.Tensor, w: Q8Weight) -> torch.Tensor:
+        lib = capi.load_library()
+        if x.dtype != torch.bfloat16 or not x.is_cuda:
+            raise TypeError("QuantizedMatmulBf16 expects bf16 activations on the GPU")
         if self.tile is None:
             device = _current_device()
             out = _native_matmul(x, w.planar, w.n, w.k, True, device, _raw_stream(device))
             if out is not None:
                 return out
-        lib = capi.load_library()
-        if x.dtype != torch.bfloat16 or not x.is_cuda:
-            raise TypeError("QuantizedMatmulBf16 expects bf16 activations on the GPU")
         if x.shape[-1] != w.k:
             raise capi.LhipError(capi.LHIP_ERR_INVALID_SHAPE, "QuantizedMatmulBf16",
                                  f"activation K {x.shape[-1]} != weight K {w.k}")

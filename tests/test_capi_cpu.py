@@ -117,6 +117,18 @@ def test_operators_can_be_imported_with_a_torch_that_has_no_gpu_backend():
     subprocess.run([sys.executable, "-c", code], check=True, cwd=ROOT, timeout=300)
 
 
+@pytest.mark.parametrize("op,dtype", [("QuantizedMatmul", "float32"), ("QuantizedMatmul", "float16"), ("QuantizedMatmulBf16", "bfloat16"),
+                                      ("QuantizedMatmul", "int8"), ("QuantizedMatmulBf16", "float32")])
+def test_operators_refuse_host_activations_before_they_ask_for_a_gpu(op, dtype):
+    """TypeError, also where there is no GPU whose number or stream could be asked for."""
+    torch = pytest.importorskip("torch")
+    from luminal_amd import quantized
+
+    w = quantized.Q8Weight(torch.zeros(quantized.Q8Weight.planar_nbytes(64, 128), dtype=torch.uint8), 64, 128)
+    with pytest.raises(TypeError):
+        getattr(quantized, op)().process(torch.zeros((2, 128), dtype=getattr(torch, dtype)), w)
+
+
 def test_argument_validation_before_any_device_work():
     lib = capi.load_library()
     ok_ptr = 0x1000  # never dereferenced: validation fails first
