@@ -12,6 +12,9 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
+
+from .capi import header_digest
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -99,14 +102,12 @@ def build_module(verbose: bool = True) -> str:
 
 
 TORCH_OPS_SRC = os.path.join(HERE, "host", "torch_ops.cpp")
-TORCH_OPS = os.path.join(HERE, "_torch_ops.so")
+TORCH_OPS = os.path.join(HERE, "_torch_ops" + sysconfig.get_config_var("EXT_SUFFIX"))  # importable by this Python only
 
 
 def build_torch_ops(verbose: bool = True) -> str:
     """Compile the operators' native host path (a Python extension against the installed torch) with the host compiler; it links
     against libluminal_hip.so, which has to be there."""
-    import sysconfig
-
     import torch
     from torch.utils import cpp_extension
 
@@ -117,6 +118,7 @@ def build_torch_ops(verbose: bool = True) -> str:
         print(f"[luminal_amd.build] {cxx} -> {TORCH_OPS}", file=sys.stderr)
     _run([cxx, "-std=c++17", "-O2", "-Wall", "-fPIC", "-shared", "-fvisibility=hidden",
           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+          f'-DLHIP_TORCH_VERSION="{torch.__version__}"', f'-DLHIP_C_HEADER="{header_digest()}"',
           *[f"-isystem{p}" for p in (*cpp_extension.include_paths(), sysconfig.get_paths()["include"])], "-o", TORCH_OPS, TORCH_OPS_SRC,
           "-L" + HERE, "-lluminal_hip", *["-L" + p for p in cpp_extension.library_paths()],
           "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-Wl,-rpath,$ORIGIN"])

@@ -2,10 +2,12 @@
 from __future__ import annotations
 
 import ctypes as C
+import hashlib
 import os
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libluminal_hip.so")
+HEADER = os.path.join(os.path.dirname(HERE), "include", "luminal_hip.h")
 
 LHIP_OK = 0
 LHIP_ERR_NULL_PTR = 1
@@ -137,6 +139,15 @@ def load_library(path: str | None = None) -> C.CDLL:
     if path is None:
         _lib = lib
     return lib
+
+
+def header_digest() -> str | None:
+    """Of the C header, which a native caller of the library is built with; None where only the package is installed."""
+    try:
+        with open(HEADER, "rb") as f:
+            return hashlib.sha256(f.read()).hexdigest()
+    except OSError:
+        return None
 
 
 def status_string(s: int) -> str:

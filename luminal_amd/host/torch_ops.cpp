@@ -68,4 +68,13 @@ PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_torch_ops", nullptr, -1, meth
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__torch_ops() { return PyModule_Create(&module_def); }
+// What it was built for, which quantized.py compares with what runs: at::Tensor's layout goes with the one, the C ABI's signatures with
+// the other.  (The file's name goes with the Python.)
+PyMODINIT_FUNC PyInit__torch_ops() {
+    PyObject *module = PyModule_Create(&module_def);
+    if (module && (PyModule_AddStringConstant(module, "torch_version", LHIP_TORCH_VERSION) || PyModule_AddStringConstant(module, "c_header", LHIP_C_HEADER))) {
+        Py_DECREF(module);
+        return nullptr;
+    }
+    return module;
+}

@@ -52,13 +52,24 @@ def bf16_workspace_nbytes(lib, m: int, n: int, k: int, out_form: int) -> int:
     return lib.lhip_q8_0_matmul_bf16_workspace_nbytes(m, n, k, out_form) if m > 128 or k % 512 else 0
 
 
-# The whole call of an operator in native code (host/torch_ops.cpp): the plain case, or None.  It is linked against the torch it
-# was built with; where that is not the one that runs, the operators below do the same through ctypes.
-try:
-    from ._torch_ops import quantized_matmul as _native_matmul
-except ImportError:
-    def _native_matmul(*_):
+def _native_operator():
+    """The whole call of an operator in native code (host/torch_ops.cpp): its result, or None for all but the plain case.  Where it
+    is not built, or not for this torch and this C header (for this Python, says its file's name), every call is left to the
+    operators below, which do the same through ctypes."""
+    def none(*_):
         return None
+
+    try:
+        from . import _torch_ops
+    except ImportError:
+        return none
+    built_for = getattr(_torch_ops, "torch_version", None), getattr(_torch_ops, "c_header", None)
+    if built_for != (str(torch.__version__), capi.header_digest() or built_for[1]):
+        return none
+    return _torch_ops.quantized_matmul
+
+
+_native_matmul = _native_operator()
 
 
 def _ptr(t: torch.Tensor) -> int:
