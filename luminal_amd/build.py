@@ -105,12 +105,23 @@ TORCH_OPS_SRC = os.path.join(HERE, "host", "torch_ops.cpp")
 TORCH_OPS = os.path.join(HERE, "_torch_ops" + sysconfig.get_config_var("EXT_SUFFIX"))  # importable by this Python only
 
 
-def build_torch_ops(verbose: bool = True) -> str:
+def build_torch_ops(verbose: bool = True) -> str | None:
     """Compile the operators' native host path (a Python extension against the installed torch) with the host compiler; it links
-    against libluminal_hip.so, which has to be there."""
-    import torch
-    from torch.utils import cpp_extension
-
+    against libluminal_hip.so, which has to be there.  The operators do without it where torch's or Python's headers are not
+    installed: None then, and no file of an earlier build is left."""
+    if os.path.exists(TORCH_OPS):
+        os.remove(TORCH_OPS)
+    try:
+        import torch
+        from torch.utils import cpp_extension
+    except ImportError as e:
+        print(f"[luminal_amd.build] no native host path: {e}", file=sys.stderr)
+        return None
+    includes = [*cpp_extension.include_paths(), sysconfig.get_paths()["include"]]
+    for header in ("Python.h", os.path.join("torch", "csrc", "autograd", "python_variable.h")):
+        if not any(os.path.exists(os.path.join(p, header)) for p in includes):
+            print(f"[luminal_amd.build] no native host path: {header} is not installed", file=sys.stderr)
+            return None
     cxx = os.environ.get("CXX") or shutil.which("g++") or shutil.which("c++")
     if not cxx:
         raise RuntimeError("no host C++ compiler found (g++)")
@@ -119,7 +130,7 @@ def build_torch_ops(verbose: bool = True) -> str:
     _run([cxx, "-std=c++17", "-O2", "-Wall", "-fPIC", "-shared", "-fvisibility=hidden",
           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
           f'-DLHIP_TORCH_VERSION="{torch.__version__}"', f'-DLHIP_C_HEADER="{header_digest()}"',
-          *[f"-isystem{p}" for p in (*cpp_extension.include_paths(), sysconfig.get_paths()["include"])], "-o", TORCH_OPS, TORCH_OPS_SRC,
+          *[f"-isystem{p}" for p in includes], "-o", TORCH_OPS, TORCH_OPS_SRC,
           "-L" + HERE, "-lluminal_hip", *["-L" + p for p in cpp_extension.library_paths()],
           "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-Wl,-rpath,$ORIGIN"])
     return TORCH_OPS

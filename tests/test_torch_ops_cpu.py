@@ -47,3 +47,21 @@ def test_the_extension_is_named_for_the_python_it_is_built_for():
 def test_the_built_extension_names_what_it_was_built_for():
     ops = pytest.importorskip("luminal_amd._torch_ops")
     assert (ops.torch_version, ops.c_header) == (str(torch.__version__), capi.header_digest())
+
+
+@pytest.mark.parametrize("missing", ["torch", "Python's headers", "torch's headers"])
+def test_the_build_goes_on_without_it_where_headers_are_missing(monkeypatch, tmp_path, missing):
+    from torch.utils import cpp_extension
+
+    stale = tmp_path / "_torch_ops.so"
+    stale.write_bytes(b"an earlier build's")
+    monkeypatch.setattr(build, "TORCH_OPS", str(stale))
+    monkeypatch.setattr(build, "_run", lambda cmd: pytest.fail("compiled"))
+    if missing == "torch":
+        monkeypatch.setitem(sys.modules, "torch.utils", None)
+    elif missing == "Python's headers":
+        monkeypatch.setattr(build.sysconfig, "get_paths", lambda: {"include": str(tmp_path)})
+    else:
+        monkeypatch.setattr(cpp_extension, "include_paths", lambda: [str(tmp_path)])
+    assert build.build_torch_ops(verbose=False) is None
+    assert not stale.exists()  # (it would go with another library)
