@@ -23,7 +23,7 @@
 // What bounds it: the matrix pipe (128 steps of 32 cycles a tile and wave at HD = 128) and, for a prompt of a few hundred tokens, the
 // serial chain of the last block's tiles, with most of the chip idle.  Hence blocks of 16 queries (with v_mfma_f32_32x32x2 and blocks of 32,
 // as before, twice the chain on half the workgroups), operands requested from LDS ahead of their use (the compiler waited
-// for each where it was read: 49 us and not 34 at 300 tokens), two buffers and one barrier a tile.  32 heads on 8 of 128, us, before ->
+// for each where it was read: 49 us and not 34 at 300 tokens), two buffers and one barrier a tile (but see BUFS).  32 heads on 8 of 128, us, before ->
 // now: 16 tokens 11.9 -> 6.7, 100 31 -> 14.8, 300 69 -> 34, 512 109 -> 53, 1000 207 -> 129, 2000 575 -> 350 (94 TFLOP/s of 157).
 #include "common.h"
 
@@ -45,10 +45,15 @@ __global__ __launch_bounds__(64 * G) __attribute__((amdgpu_waves_per_eu(1, 2))) 
     constexpr int LD = TILE_F4 / THREADS;  // float4 per thread and tile and matrix
     static_assert(TILE_F4 % THREADS == 0 && THREADS % (HD / 4) == 0, "whole rounds of whole rows");
     constexpr bool PREFETCH = LD <= 4;     // keep the next tile in registers during the sweep of this one
-    // Two buffers of a tile; 16-byte piece p of a K row lies at p ^ (key % 16), of a V row at p ^ (key / 4 % 2), which gives the
-    // operand reads below 16 lanes on 16 different slots.
-    __shared__ __attribute__((aligned(16))) float k_s[2][kPfTileK * HD];
-    __shared__ __attribute__((aligned(16))) float v_s[2][kPfTileK * HD];
+    // Two buffers of a tile, and one for a single wave: it waits for nobody, so the second gives it nothing, and with twice the LDS half
+    // the waves fit a CU (32 heads on 32 of 128, two buffers -> one, us: 300 tokens 39 -> 37, 1000 232 -> 150, 2000 876 -> 517; two waves,
+    // 32 on 16: 1000 tokens 112 <- 141).
+    constexpr int BUFS = G == 1 ? 1 : 2;
+    static_assert(BUFS == 2 || !PREFETCH, "a tile requested ahead is stored in the other buffer");
+    // 16-byte piece p of a K row lies at p ^ (key % 16), of a V row at p ^ (key / 4 % 2), which gives the operand reads below
+    // 16 lanes on 16 different slots.
+    __shared__ __attribute__((aligned(16))) float k_s[BUFS][kPfTileK * HD];
+    __shared__ __attribute__((aligned(16))) float v_s[BUFS][kPfTileK * HD];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -119,7 +124,7 @@ __global__ __launch_bounds__(64 * G) __attribute__((amdgpu_waves_per_eu(1, 2))) 
     }
     __syncthreads();
     for (int t = 0; t < n_tiles; ++t) {
-        const float *kb = k_s[t & 1], *vb = v_s[t & 1];
+        const float *kb = k_s[t % BUFS], *vb = v_s[t % BUFS];
         if (PREFETCH && t + 1 < n_tiles) load_tile(t + 1);
         v4f s_acc[2] = {v4f{0.f, 0.f, 0.f, 0.f}, v4f{0.f, 0.f, 0.f, 0.f}};
         // Operands are requested from LDS ahead of their use; the fences hold that order.
@@ -190,9 +195,10 @@ __global__ __launch_bounds__(64 * G) __attribute__((amdgpu_waves_per_eu(1, 2))) 
                 o_acc[j0 + e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vr[u % RING][e], s_acc[step >> 2][step & 3], o_acc[j0 + e], 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
         }
-        if (t + 1 < n_tiles) {  // the other buffer was last read a tile ago, behind a barrier
-            if (PREFETCH) store_tile((t + 1) & 1);
-            else copy_tile(t + 1, (t + 1) & 1);
+        if (BUFS == 1) __syncthreads();  // the only buffer has been read
+        if (t + 1 < n_tiles) {           // (of two, the other was last read a tile ago, behind a barrier)
+            if (PREFETCH) store_tile((t + 1) % BUFS);
+            else copy_tile(t + 1, (t + 1) % BUFS);
         }
         __syncthreads();
     }
