@@ -553,16 +553,24 @@ static lhip_status launch_exact_gemm(const MoeExactArgs &a, int col_blocks, int 
     return LHIP_OK;
 }
 
-// Tile height of the exact form for R routed rows over E experts, in 16-row fragments: 16 or 32 rows where such a tile holds an
-// expert with two standard deviations more rows than the average (so that nearly every expert is one tile and its
-// weights are read and expanded once), else 96 (`tall`, mxfp4_moe_tall.hip), cut into equal parts for experts with more; but 64
-// around 40 rows, which fragments of 16 fit better than that kernel's of 32.  Measured on the benchmark layer (us per layer, 16 / 32 /
-// 64 / 96 rows): T = 32 87 / 94 / 110 / -, T = 64 90 / 95 / 110 / -, T = 128 132 / 99 / 114 / 103, T = 192 - / - / 126 / 114, T = 256 128 /
-// 127, T = 288 133 / 136, T = 320 135 / 139, T = 352 137 / 138, T = 384 140 / 138, T = 512 191 / 155, T = 768 221 / 210, T = 1024 284 / 237.
-static inline int exact_tile_fragments(int R, int E, bool tall) {
+// Tile height of the exact form for R routed rows over E experts of H x I, in 16-row fragments: 16 or 32 rows where such a tile holds
+// an expert with two standard deviations more rows than the average (so that nearly every expert is one tile and its weights are
+// read and expanded once), else 64, or 96 (`tall`, mxfp4_moe_tall.hip), cut into equal parts for experts with more.
+// A stage of the 96-row kernel takes longer when its workgroup is alone on a compute unit, and two of its workgroups end no
+// sooner than two of 64 rows; it wins with the third.  So it is taken with two workgroups a compute unit in the first product and one
+// and a half in the second, and there where its tiles are fewer (more than 50 rows an expert: many are two tiles of 64) or
+// hold one fragment of 32 (less than 28).  Measured on 16 layers (4 to 128 experts, H of 1024 to 4096, I of 512 to 14336) at 24 to
+// 384 rows an expert: over 64 rows everywhere 0.98, the better of both 0.97, 96 rows everywhere 1.05.  us, 64 / 96 rows: 32 experts of
+// 2880 x 2880, top 4, T = 192 115 / 108, T = 256 121 / 127, T = 384 142 / 146, T = 512 180 / 153, T = 1024 261 / 233; 8 experts of 4096 x
+// 14336, top 2, T = 128 218 / 314, T = 384 331 / 440; 64 of 2048 x 1408, top 6, T = 512 98 / 106, T = 683 140 / 115; 12 of 2880 x 2880, top 3,
+// T = 192 80 / 85.  16- / 32- / 64-row tiles of the first: T = 32 87 / 94 / 110, T = 64 90 / 95 / 110, T = 128 132 / 99 / 114.
+static inline int exact_tile_fragments(int R, int E, int H, int I, bool tall) {
     const int avg = (R + E - 1) / E;
     const int need = avg + 2 * static_cast<int>(sqrtf(static_cast<float>(avg)) + 0.5f);
-    return need <= 16 ? 1 : need <= 32 ? 2 : (avg >= 34 && avg <= 44) || !tall ? 4 : kTallRows / 16;
+    if (need <= 32) return need <= 16 ? 1 : 2;
+    const int64_t tiles = R / kTallRows + E / 2 > E ? R / kTallRows + E / 2 : E;  // about as many as there will be
+    const bool filled = tiles * ((I + 127) / 128) >= 2 * 256 && tiles * ((H + 255) / 256) * 2 >= 3 * 256;
+    return tall && filled && (avg < 28 || avg > 50) ? kTallRows / 16 : 4;
 }
 
 lhip_status moe_exact_forward(const uint8_t *gu, const uint8_t *dn, const __bf16 *x, const int32_t *sel_dev,
@@ -604,7 +612,7 @@ lhip_status moe_exact_forward(const uint8_t *gu, const uint8_t *dn, const __bf16
         return LHIP_OK;
     }
 
-    const int mt = exact_tile_fragments(R, E, moe_tall_supports(T, H, I));
+    const int mt = exact_tile_fragments(R, E, H, I, moe_tall_supports(T, H, I));
     const int BM = 16 * mt;
     const int max_tiles = (R / BM + E + 7) / 8 * 8;
     w.plan.max_tiles = max_tiles;

@@ -320,12 +320,13 @@ def test_moe_lopsided_routing(oracle, t, e, h, i, topk, hot, mode):
         check_stages(oracle, layer, xf, w_gu, w_dn, sel_h, wts_h, y, tokens=live, mode=mode)
 
 
-@pytest.mark.parametrize("h,i", [(96, 160), (416, 320), (128, 96)])
-def test_moe_rows_per_expert_at_the_edges_of_the_96_row_tiles(oracle, h, i):
+@pytest.mark.parametrize("e,h,i", [(384, 96, 160), (192, 416, 320), (512, 128, 96)])
+def test_moe_rows_per_expert_at_the_edges_of_the_96_row_tiles(oracle, e, h, i):
     """Experts of 0, 1, 33, 64, 96, 97, 129 and 193 rows in one call (fragments of 32, tiles of 96, their remainders), K that
-    ends inside a stage of 64, column blocks with waves that have no columns.  The row of x behind another one's end starts
-    with infinities, which must not reach it through the padding of K."""
-    counts, e = (97, 33, 0, 96, 1, 193, 64, 129), 8
+    ends inside a stage of 64, column blocks with waves that have no columns; so many experts that these narrow layers fill the
+    chip, without which such tiles are not taken.  The row of x behind another one's end starts with infinities, which must not
+    reach it through the padding of K."""
+    counts = np.tile((97, 33, 0, 96, 1, 193, 64, 129), e // 8)
     layer, w_gu, w_dn = make_layer(oracle, e, h, i, seed=h + i)
     rng = np.random.default_rng(h)
     sel = rng.permutation(np.repeat(np.arange(e, dtype=np.int32), counts))[:, None]
@@ -339,7 +340,21 @@ def test_moe_rows_per_expert_at_the_edges_of_the_96_row_tiles(oracle, h, i):
     y = layer.process(xd, torch.from_numpy(np.ascontiguousarray(sel)).to(DEV), torch.from_numpy(wts).to(DEV), EXACT).float().cpu().numpy()
     others = np.flatnonzero(np.arange(t) != 5)
     assert np.isfinite(y[others]).all()
+    # the tokens of the first, some middle and the last experts
+    of = sel[others, 0]
+    others = others[(of < 8) | (of >= e - 8) | ((of >= e // 2) & (of < e // 2 + 8))]
     check_stages_exact(layer, xf, w_gu, w_dn, sel, wts, y, tokens=others)
+
+
+@pytest.mark.parametrize("e,h,i,rows", [(512, 96, 128, 26), (511, 128, 96, 51), (397, 160, 192, 52)])
+def test_moe_random_rows_per_expert_in_96_row_tiles(oracle, e, h, i, rows):
+    """Routed at random, on both sides of the rows per expert between which tiles of 64 rows are taken instead, and numbers of
+    experts that are no multiple of the eight shares of the tile list (or of the four counts a thread reads at once)."""
+    layer, w_gu, w_dn = make_layer(oracle, e, h, i, seed=e)
+    t = e * rows // 2
+    xf, sel, wts, y = run_layer(oracle, layer, t, h, e, 2, seed=rows, scale=0.05)
+    assert np.isfinite(y).all()
+    check_stages_exact(layer, xf, w_gu, w_dn, sel, wts, y, tokens=np.concatenate([np.arange(300), np.arange(t - 300, t)]))
 
 
 def test_moe_rows_beyond_32_bit_offsets(oracle):
