@@ -617,9 +617,6 @@ lhip_status moe_exact_forward(const uint8_t *gu, const uint8_t *dn, const __bf16
     const int max_tiles = (R / BM + E + 7) / 8 * 8;
     w.plan.max_tiles = max_tiles;
     w.plan.tiles_per_xcd = max_tiles / 8;
-    // Experts listed by their rows where many are more than one tile, us, own order / by rows: T = 320 136 / 139, T = 416 141 / 145,
-    // T = 448 153 / 149, T = 512 158 / 155, T = 640 173 / 175, T = 768 217 / 210, T = 1024 243 / 237.
-    w.plan.by_rows = BM == kTallRows && R >= 56 * E;
     w.plan.fragment = BM == kTallRows ? 32 : 16;
     hipLaunchKernelGGL(moe_plan_kernel, dim3(1), dim3(1024), 0, s, sel_dev, R, E, BM, w.plan);
     LHIP_CHECK_LAUNCH();
