@@ -85,7 +85,8 @@ def build(verbose: bool = True, incremental: bool = False, jobs: int | None = No
         print(f"[luminal_amd.build] {cc}: {len(todo)} of {len(srcs)} sources -> {LIB}", file=sys.stderr)
     jobs = jobs or min(8, os.cpu_count() or 1, int(os.environ.get("MAX_JOBS", "8")))
     with ThreadPoolExecutor(max_workers=max(1, jobs)) as pool:
-        list(pool.map(lambda s: _run([cc, *COMMON, *DEVICE_FLAGS, "-c", "-o", _object_path(s), s]), todo))
+        # (last name first: q8_*, the ones that take longest)
+        list(pool.map(lambda s: _run([cc, *COMMON, *DEVICE_FLAGS, "-c", "-o", _object_path(s), s]), reversed(todo)))
     _run([cc, *COMMON, "-shared", "-o", LIB, *[_object_path(s) for s in srcs]])
     if todo or not os.path.exists(MODULE):
         build_module(verbose)
