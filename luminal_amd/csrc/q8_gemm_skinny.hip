@@ -142,8 +142,9 @@ static SkPlan sk_faster_plan(const SkTimes &t, SkPlan base, double margin, int m
         if (k % kSkUnit != 0 && !sk_ragged_waves(kSkWaves[i])) continue;
         const unsigned strips = strips_of(kSkWaves[i]);
         for (int s = fixed_s ? fixed_s : 1; s <= (fixed_s ? fixed_s : base.splits > 1 ? units : 1); ++s) {
-            // (two rounds of workgroups are enough for any strip)
-            if (s > 1 && !fixed_s && (strips * s > 512 || static_cast<size_t>(s) * m * n > room)) break;
+            // K is sliced within one round of 256 workgroups: another pays a start and an end of its own, which the tables do not hold (us,
+            // in one round / two: 3 x 5460 x 5632 bf16 15.2 / 18.0, 33 x 2728 x 11776 f32 29.0 / 31.7, 5 x 9320 x 7168 25.7 / 27.8).
+            if (s > 1 && !fixed_s && (strips * s > 256 || static_cast<size_t>(s) * m * n > room)) break;
             const int per = per_of(s);
             if ((s - 1) * per >= units) continue;  // an empty slice
             const double us = sk_us(t, i, s, strips * s, per, m, n, best_us);
@@ -159,7 +160,7 @@ static SkPlan sk_faster_plan(const SkTimes &t, SkPlan base, double margin, int m
 // sk_us puts 6 % below (its own spread).  m x N x K, us: 16 x 14336 x 4096 7 waves, 2 slices 18.7 -> 4 waves, none 16.4;
 // 16 x 4096 x 4096 8 waves, 8 slices 10.5 -> 4 waves, 4 slices 9.1; 64 x 4096 x 4096 18.1 -> 13.5; 128 x 4096 x 4096 21.4 -> 18.2;
 // 16 x 4096 x 1024 8.4 -> 5.0; as it was: 32 x 10240 x 8192 29.3, 64 x 8192 x 14336 47.7.  Over the 240 sizes it is within
-// 1.4 % of the best of all plans (the first rule alone: 17 %), and at none more than 1 % behind the first rule.
+// 1.4 % of the best of all plans (the first rule alone: 17 %); mean of 1158 others 0.78 of the first rule's time.
 static SkPlan sk_plan(int m, int n, int k, size_t room, int splits = 0) {
     const int units = sk_units(k), passes = (m + 127) / 128;
     SkPlan best{8, 1};
@@ -249,8 +250,8 @@ static int split_base_slices(int mc, int n, int k, size_t room) {
 // The plan of a chunk: those, or up to 1024 rows any other strip and number of slices that sk_us puts 3 % below.  m x N x K, f32
 // and f16, us: 16 x 4096 x 1024 9.2 -> 5.9 and 8.9 -> 5.8, 32 x 4096 x 4096 13.9 -> 12.7 and 12.8 -> 11.6, 64 x 2048 x 4096 17.4 -> 13.8
 // and 16.2 -> 12.6, 16 x 14336 x 4096 21.2 -> 19.4 and 19.7 -> 17.6, 256 x 512 x 4096 17.3 -> 13.6 and 15.8 -> 12.4, 1000 x 256 x 1024
-// 16.2 -> 11.4 and 14.7 -> 9.5; as it was: 16 x 8192 x 8192 23.2 and 21.4.  Mean of 500 sizes of up to 64 rows 0.87, of 900 above
-// that 0.85 (0.82 - 0.88 by type and rows), at none more than 2 % behind.
+// 16.2 -> 11.4 and 14.7 -> 9.5; as it was: 16 x 8192 x 8192 23.2 and 21.4.  Mean of 2242 sizes of up to 64 rows 0.85, of 826
+// above that 0.83, at none more than 3 % behind.
 static SkPlan split_plan_for(int mc, int n, int k, size_t room) {
     const int passes = (mc + 63) / 64;
     const SkPlan base{8, split_base_slices(mc, n, k, room)};

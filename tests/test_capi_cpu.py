@@ -3,6 +3,7 @@ every declared symbol, and its size arithmetic and argument validation (which
 run before any HIP call) behave as documented."""
 import ctypes as C
 import os
+import random
 import re
 import subprocess
 import sys
@@ -107,6 +108,22 @@ def test_products_whose_plain_calls_may_overlap_keep_no_partial_sums(m, n, k, bf
     lib = capi.load_library()
     need = lib.lhip_q8_0_matmul_bf16_workspace_nbytes(m, n, k, 0) if bf16 else lib.lhip_q8_0_matmul_workspace_nbytes(m, n, k)
     assert need == 0
+
+
+def test_k_is_sliced_within_one_round_of_workgroups():
+    """Slices of K of the weight-streaming kernel, as its partial planes in the workspace show them: times the fewest strips that N
+    can be cut into (128 weight rows) they fit on the 256 compute units at once."""
+    lib = capi.load_library()
+    rng = random.Random(7)
+    sizes = [(3, 5460, 5632), (4, 8240, 7168), (3, 7024, 12800), (5, 9320, 7168), (33, 2728, 11776), (35, 7124, 8704)]
+    sizes += [(rng.randint(2, 64), rng.randint(64, 4000) * 4, rng.randint(1, 28) * 512) for _ in range(400)]
+    sliced = 0
+    for m, n, k in sizes:
+        for nbytes in (lib.lhip_q8_0_matmul_bf16_workspace_nbytes(m, n, k, 0), lib.lhip_q8_0_matmul_workspace_nbytes(m, n, k)):
+            slices = nbytes // (m * n * 4)
+            assert slices * m * n * 4 == nbytes and (slices <= 1 or slices * ((n + 127) // 128) <= 256), (m, n, k, slices)
+            sliced += slices > 1
+    assert sliced > 200
 
 
 def test_operators_can_be_imported_with_a_torch_that_has_no_gpu_backend():
