@@ -277,34 +277,45 @@ struct RowsPlan {
     size_t floats = 0;  // of partial planes
 };
 
-// What q8_gemm_rows.hip takes for up to 64 rows, us: per block of K that the slowest compute unit walks, for the sum of the slices
-// and its planes.  Fitted to 420 sizes (6 % of standard deviation).
-static double few_rows_us(int64_t m, int64_t n, bool f16, double blocks, int slices) {
-    const double sum = slices > 1 ? (f16 ? 4.1 : 3.8) + static_cast<double>(slices * m * n) * 4e-6 * 0.56 : 0.0;
-    return blocks * (f16 ? 0.63 : 0.78) + sum;
+// What q8_gemm_rows.hip takes, us: a launch, a start and an end for every further round of 256 workgroups, a price per block of K that a
+// workgroup walks (some of it for its 128 activation rows, some by its weight rows, some as the launch fills the chip), and for K
+// slices the launch of their sum and its planes (N in steps of four: 16 bytes a load; else four).  Fitted to 10200 launches of 4300
+// sizes; standard deviation 5 and 6 % (f32 and f16) up to 64 activation rows, of which most compute waves have none, 7 and 8 %
+// above.
+struct RowsTimes {
+    double launch, round, sum, planes, planes_odd;  // us, us, us, us per MB
+    double block, block_rows, block_fill;           // us per block; per block and 256 weight rows; per block at a full chip
+};
+static constexpr RowsTimes kRowsTimes[2][2] = {{{3.6, 2.75, 2.85, 0.51, 0.79, 0.12, 0.535, 0.105}, {5.7, 5.4, 2.0, 0.38, 0.725, 0.23, 0.71, 0.03}},
+                                               {{3.5, 2.25, 2.75, 0.455, 0.75, 0.035, 0.455, 0.14}, {5.0, 4.1, 2.9, 0.36, 0.73, 0.08, 0.45, 0.075}}};
+static double rows_us(const RowsTimes &t, int64_t workgroups, int width, int per, int slices, int64_t m, int64_t cols) {
+    const double rounds = static_cast<double>((workgroups + 255) / 256), fill = workgroups < 256 ? static_cast<double>(workgroups) / 256.0 : 1.0;
+    const double sum = slices > 1 ? t.sum + static_cast<double>(slices * m * cols) * 4e-6 * (cols % 4 == 0 ? t.planes : t.planes_odd) : 0.0;
+    return t.launch + (rounds - 1.0) * t.round + rounds * per * (t.block + t.block_rows * width / 256.0 + t.block_fill * fill) + sum;
 }
 
 // The plan that ends first, by what each kernel takes (us, measured): a workgroup of the streaming kernel 0.49 (f32) or
-// 0.38 (f16) per block of K, one of q8_gemm_rows.hip 1.2 or 0.66, a 128x256 tile of q8_gemm_wide.hip 0.64 (f16); 256
-// workgroups at a time, some microseconds per launch, and 3 plus 8 TB/s for the sum of the slices; up to 64 rows what
-// few_rows_us says.  The lines this draws (streaming -> chosen, us): 14336 x 4096 f32 at 64 rows 38 -> (54), at 128 61 -> 54,
-// at 256 120 -> 97, at 512 239 -> 162; f16 at 64 rows 34 -> (36), at 128 50 -> 36, at 512 188 -> 90; 4096 x 4096 f32 at 256
-// rows 39 -> (41), at 300 63 -> 44.  Up to 64 rows, and for fewer than sixteen 128x256 tiles, the streaming kernel's narrower
-// strips stay ahead.  Tiles of 224, 192 or 128 weight rows are taken where the plan puts them 6 % ahead: in one round, or without
-// slices (45 x 2880 x 2880 f32 12 slices of 256 14.6 -> 8 of 128 12.2, 300 x 6144 x 4096 54.8 -> 52.6 at 224, 485 x 9721 x 3488 117 -> 100
-// unsliced at 192, f16 387 x 1138 x 2432 25.8 -> 20.1; in two rounds of slices 138 x 9702 x 5056 72 <- 78).  A number of slices that leaves one empty is passed over; with 16 slices at most, and none behind the
-// first number that leaves one empty, few weight rows or a K of 90 blocks left most compute units idle: 45 x 2880 x 2880 f32
-// 6 -> 12 slices 18.1 -> 15.3 us, 45 x 1000 x 4480 18.9 -> 13.6, 300 x 1000 x 8000 37.4 -> 27.2, f16 400 x 1000 x 8992 30.4 ->
-// 25.7.
+// 0.38 (f16) per block of K, 256 workgroups at a time, a 128x256 tile of q8_gemm_wide.hip 0.64 (f16), some microseconds per
+// launch, 3 plus 8 TB/s for the sum of the slices, and q8_gemm_rows.hip what rows_us says.  The lines this draws (streaming ->
+// chosen, us): 14336 x 4096 f32 at 64 rows (40), at 128 61 -> 53, at 256 117 -> 85, at 512 235 -> 147; f16 at 128 rows 50 -> 39, at 256 95 ->
+// 57, at 512 186 -> 82; 4096 x 4096 f32 at 128 rows 25.4 -> 24.7, at 256 39 -> 36, at 300 57 -> 42, f16 at 256 32 -> 26.  Up to 64 rows, and
+// for fewer than sixteen 128x256 tiles, the streaming kernel's narrower strips stay ahead.
+// Tiles of 256 weight rows, or of 224, 192 or 128 in one round or without slices (us, 45 x 2880 x 2880 f32 12 slices of 256 14.6 -> 8 of 128
+// 12.2, 300 x 6144 x 4096 55.6 -> 54.1 at 224, 485 x 9721 x 3488 118 -> 103 unsliced at 192, f16 387 x 1138 x 2432 26.1 -> 20.0; in two rounds of
+// slices 138 x 9702 x 5056 72 <- 78).  Up to 40 slices, none of them empty (45 x 2880 x 2880 f32 6 -> 12 slices 18.1 -> 15.3 us, 45 x 1000 x
+// 4480 7 -> 18 19.3 -> 12.0, 300 x 1000 x 8000 37 -> 29, f16 400 x 1000 x 8992 30.6 -> 25.0).  Without the price of a
+// further round few rows of a wide matrix went to many: 3 x 12081 x 4736 f32 in 37 slices and seven rounds 49 us, in 5 and one 30; f16 3 x
+// 22140 x 2400 in 19 and seven 43, in 2 of 192 26.
 static RowsPlan rows_plan(int64_t m, int n, int k, bool f16, size_t room, bool stream) {
     RowsPlan best;
     const int64_t m_tiles = (m + 127) / 128, n_tiles = (n + 255) / 256;
     if (stream && (m <= 64 || m_tiles * n_tiles < 16)) return best;
-    const double nblk = k / 32, block = f16 ? 0.66 : 1.2;
+    const RowsTimes &times = kRowsTimes[f16][m > 64];
+    const double nblk = k / 32;
     auto rounds = [](int64_t workgroups) { return static_cast<double>((workgroups + 255) / 256); };
     auto sum_us = [&](int64_t slices, int64_t cols) { return 3.0 + static_cast<double>(slices * m * cols) * 4.0 / 8e6; };
     double best_us = 1e30, early_us = 1e30, bare_us = 1e30;
-    RowsPlan early;  // the best of tiles of 256 in up to 16 slices that come before a number leaving one empty
+    RowsPlan early;  // the plan by which a plain call keeps planes or none (see the end)
     RowsPlan bare;   // the best that has no planes
     bool planes = false;
     if (stream) {  // (0.49 and 0.38 us are those of strips of 128 rows)
@@ -326,7 +337,8 @@ static RowsPlan rows_plan(int64_t m, int n, int k, bool f16, size_t room, bool s
     for (int64_t lead : {int64_t{0}, main_tiles}) {
         if (lead == n_tiles || (lead > 0 && m_tiles > 256)) continue;
         const int64_t cols = n - lead * 256, tiles = m_tiles * (n_tiles - lead);
-        const double main_us = lead > 0 ? rounds(m_tiles * lead) * nblk * (m <= 64 ? (f16 ? 0.63 : 0.78) : block) + 8.0 : 0.0;
+        const double main_us = lead > 0 ? rows_us(times, m_tiles * lead, 256, k / 32, 1, m, cols) : 0.0;
+        const double first_main_us = lead > 0 ? rounds(m_tiles * lead) * nblk * (f16 ? 0.66 : 1.2) + 8.0 : 0.0;
         constexpr int widths[] = {256, 224, 192, 128};
         int64_t tiles_of[4];
         for (int i = 0; i < 4; ++i) tiles_of[i] = m_tiles * ((cols + widths[i] - 1) / widths[i]);
@@ -345,25 +357,28 @@ static RowsPlan rows_plan(int64_t m, int n, int k, bool f16, size_t room, bool s
             for (int i = 0; i < 4; ++i) {
                 const int width = widths[i];
                 const int64_t all = tiles_of[i] * slices;
-                if (i > 0 && (lead > 0 || (slices > 1 && all > 256))) break;  // (a second round of slices pays a start and an end of its own)
-                const double walk = (width + 20.0) / 276.0, blocks = rounds(all) * per;
-                double us = main_us + (m <= 64 ? few_rows_us(m, cols, f16, blocks * walk, slices)
-                                               : 8.0 + blocks * walk * block + (slices > 1 ? sum_us(slices, cols) : 0.0));
+                if (i > 0 && (lead > 0 || (slices > 1 && all > 256))) break;
+                double us = main_us + rows_us(times, all, width, per, slices, m, cols);
+                // (what the estimate is short of on average: the gap between two launches; narrow tiles that walk all of K in step)
+                if (lead > 0 || (width < 256 && slices == 1)) us *= 1.05;
                 RowsPlan plan;
                 plan.kind = RowsPlan::kRows;
                 plan.n_main = static_cast<int>(lead * 256);
                 plan.slices = slices;
                 plan.width = width;
                 plan.floats = floats;
-                if (i == 0 && !gap && us < early_us) early_us = us, early = plan;
-                if (i > 0) us *= 1.06;  // only where clearly ahead
+                if (i == 0 && !gap && stream) {
+                    const double first_us = first_main_us + 8.0 + rounds(all) * per * (f16 ? 0.66 : 1.2) + (slices > 1 ? sum_us(slices, cols) : 0.0);
+                    if (first_us < early_us) early_us = first_us, early = plan;
+                }
                 if (us < best_us) best_us = us, best = plan;
                 if (floats == 0 && us < bare_us) bare_us = us, bare = plan;
             }
         }
     }
-    // A product of which the plain call keeps nothing in the library's array, so that its calls may overlap, keeps nothing there by
-    // the further numbers of slices and widths either.
+    // A product of which the plain call kept nothing in the library's array, so that its calls may overlap, when these plans had tiles
+    // of 256 in up to 16 slices, none of them behind a number that leaves one empty, at 1.2 (f32) or 0.66 us per block (`early`), keeps
+    // nothing there now.
     return stream && early.floats == 0 && !(early.kind == RowsPlan::kStream && planes) ? bare : best;
 }
 

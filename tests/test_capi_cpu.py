@@ -126,6 +126,15 @@ def test_k_is_sliced_within_one_round_of_workgroups():
     assert sliced > 200
 
 
+@pytest.mark.parametrize("m,n,k", [(3, 12081, 4736), (6, 38616, 3296), (3, 20336, 4640), (3, 13192, 2688), (3, 22140, 2400),
+                                   (6, 34643, 2144), (3, 23136, 1600)])
+def test_few_rows_of_a_wide_matrix_take_few_slices(m, n, k):
+    """The rows kernel (a K that is no multiple of 512): slices of K for at most two rounds of 256 workgroups of 256 weight rows."""
+    nbytes = capi.load_library().lhip_q8_0_matmul_workspace_nbytes(m, n, k)
+    slices = nbytes // (m * n * 4)
+    assert slices * m * n * 4 == nbytes and slices * ((n + 255) // 256) <= 512, slices
+
+
 def test_operators_can_be_imported_with_a_torch_that_has_no_gpu_backend():
     code = ("import torch\n"
             "for name in ('_cuda_getDevice', '_cuda_getCurrentRawStream'):\n"
