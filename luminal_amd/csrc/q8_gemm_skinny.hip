@@ -114,16 +114,24 @@ static constexpr SkTimes kSkBf16 = {{{3.11, 2.60, 1.33, 1.10, 0.98}, {3.34, 2.96
 static constexpr SkTimes kSkF32 = {{{3.15, 0.0, 1.64, 1.46, 1.34}, {4.12, 0.0, 2.67, 2.52, 2.37}, {6.58, 0.0, 4.57, 4.41, 4.15}, {}},
                                    {5.44e6, 5.59e6, 7.0e6, 7.0e6}, 20e6, {3.5, 3.6, 4.2, 0.0}, 1.7, 0.97, 4};
 
-// `groups` workgroups of kSkWaves[cw_index] compute waves walk `per` units of K; a plan that cannot come below `limit` is not
-// worked out.
-static double sk_us(const SkTimes &t, int cw_index, int slices, unsigned groups, int per, int m, int n, double limit) {
-    const int rows = m <= 16 ? 0 : (m <= 32 ? 1 : (m <= 64 || t.x_bytes == 4 ? 2 : 3)), strip = 16 * kSkWaves[cw_index];
-    const double walk = t.walk[rows][cw_index], walks = static_cast<double>((groups + 255) / 256 * static_cast<unsigned>(per));
-    const double rest = t.fixed[rows] + (slices > 1 ? t.sum + t.planes * static_cast<double>(slices) * m * n * 4e-6 : 0.0);
-    if (walk == 0.0 || rest + walks * walk >= limit) return limit;
-    const double stream = static_cast<double>(groups < 256 ? groups : 256) *
-                          (strip * (kSkUnit + kSkUnit / 16) / t.weights[rows] + (16 << rows) * t.x_bytes * kSkUnit / t.activations);
-    const double w2 = walk * walk, s2 = stream * stream;
+// One strip's part of that: what a workgroup's 512 of K take by its table and, per workgroup, from memory, and what does not depend
+// on K.
+struct SkStrip {
+    double walk, stream, fixed;
+    SkStrip(const SkTimes &t, int cw_index, int m) {
+        const int rows = m <= 16 ? 0 : (m <= 32 ? 1 : (m <= 64 || t.x_bytes == 4 ? 2 : 3));
+        walk = t.walk[rows][cw_index];
+        stream = 16 * kSkWaves[cw_index] * (kSkUnit + kSkUnit / 16) / t.weights[rows] + (16 << rows) * t.x_bytes * kSkUnit / t.activations;
+        fixed = t.fixed[rows];
+    }
+};
+// `groups` workgroups of the strip walk `per` units of K; a plan that cannot come below `limit` is not worked out.
+static double sk_us(const SkTimes &t, const SkStrip &strip, int slices, unsigned groups, int per, int m, int n, double limit) {
+    const double walks = static_cast<double>((groups + 255) / 256 * static_cast<unsigned>(per));
+    const double rest = strip.fixed + (slices > 1 ? t.sum + t.planes * static_cast<double>(slices) * m * n * 4e-6 : 0.0);
+    if (strip.walk == 0.0 || rest + walks * strip.walk >= limit) return limit;
+    const double stream = static_cast<double>(groups < 256 ? groups : 256) * strip.stream;
+    const double w2 = strip.walk * strip.walk, s2 = stream * stream;
     return rest + walks * sqrt(sqrt(w2 * w2 + s2 * s2));
 }
 
@@ -136,18 +144,32 @@ static SkPlan sk_faster_plan(const SkTimes &t, SkPlan base, double margin, int m
     auto per_of = [units](int s) { return static_cast<int>(static_cast<unsigned>(units + s - 1) / static_cast<unsigned>(s)); };
     SkPlan best = base;
     const int base_index = base.cw == 8 ? 0 : 1;
-    const double base_us = sk_us(t, base_index, base.splits, strips_of(base.cw) * base.splits, per_of(base.splits), m, n, 1e30);
+    const double base_us = sk_us(t, SkStrip(t, base_index, m), base.splits, strips_of(base.cw) * base.splits, per_of(base.splits), m, n, 1e30);
     double best_us = margin * base_us;
+    // The numbers of slices, none of which leaves one empty: each is the smallest for its length of slice.  K is sliced within one round
+    // of 256 workgroups: another pays a start and an end of its own, which the tables do not hold (us, in one round / two: 3 x 5460 x 5632
+    // bf16 15.2 / 18.0, 33 x 2728 x 11776 f32 29.0 / 31.7, 5 x 9320 x 7168 25.7 / 27.8).
+    struct {
+        int slices, per;
+    } cuts[256];
+    int n_cuts = 0;
+    if (fixed_s) {
+        if ((fixed_s - 1) * per_of(fixed_s) < units) cuts[n_cuts++] = {fixed_s, per_of(fixed_s)};
+    } else {
+        const unsigned most = base.splits == 1 ? 1 : 256 / strips_of(kSkWaves[0]);  // (the widest strips are the fewest)
+        for (int s = 1, per = units;; s = per_of(per - 1), per = per_of(s)) {
+            cuts[n_cuts++] = {s, per};
+            if (per == 1 || static_cast<unsigned>(per_of(per - 1)) > most) break;
+        }
+    }
     for (int i = 0; i < static_cast<int>(sizeof(kSkWaves) / sizeof(kSkWaves[0])); ++i) {
         if (k % kSkUnit != 0 && !sk_ragged_waves(kSkWaves[i])) continue;
+        const SkStrip strip(t, i, m);
         const unsigned strips = strips_of(kSkWaves[i]);
-        for (int s = fixed_s ? fixed_s : 1; s <= (fixed_s ? fixed_s : base.splits > 1 ? units : 1); ++s) {
-            // K is sliced within one round of 256 workgroups: another pays a start and an end of its own, which the tables do not hold (us,
-            // in one round / two: 3 x 5460 x 5632 bf16 15.2 / 18.0, 33 x 2728 x 11776 f32 29.0 / 31.7, 5 x 9320 x 7168 25.7 / 27.8).
+        for (int c = 0; c < n_cuts; ++c) {
+            const int s = cuts[c].slices, per = cuts[c].per;
             if (s > 1 && !fixed_s && (strips * s > 256 || static_cast<size_t>(s) * m * n > room)) break;
-            const int per = per_of(s);
-            if ((s - 1) * per >= units) continue;  // an empty slice
-            const double us = sk_us(t, i, s, strips * s, per, m, n, best_us);
+            const double us = sk_us(t, strip, s, strips * s, per, m, n, best_us);
             if (us < best_us) best_us = us, best = SkPlan{kSkWaves[i], s, us / base_us};
         }
     }
@@ -196,7 +218,7 @@ double q8_gemm_skinny_us(int m, int n, int k, size_t room) {
     int index = 0;
     while (kSkWaves[index] != plan.cw) ++index;
     const unsigned strips = static_cast<unsigned>((n + 16 * plan.cw - 1) / (16 * plan.cw));
-    return sk_us(kSkBf16, index, plan.splits, strips * plan.splits, (sk_units(k) + plan.splits - 1) / plan.splits, m, n, 1e30);
+    return sk_us(kSkBf16, SkStrip(kSkBf16, index, m), plan.splits, strips * plan.splits, (sk_units(k) + plan.splits - 1) / plan.splits, m, n, 1e30);
 }
 
 constexpr int kSkMaxRows = 128 * 64;  // passes are the grid's z extent
@@ -268,15 +290,6 @@ static SkPlan split_plan(int mc, int n, int k, size_t room) {
 
 constexpr int kMaxRowsSlices = 40;
 
-// How a product is run: by passes of 64 rows of the kernel above (kStream), by q8_gemm_rows.hip (kRows: `n_main` leading
-// weight rows in whole rounds of workgroups, the others over `slices` K slices; n_main = 0: all of them), or by the
-// tiles of q8_gemm_wide.hip (kWide).
-struct RowsPlan {
-    enum Kind { kStream, kRows, kWide } kind = kStream;
-    int n_main = 0, slices = 1, width = 256;  // width = weight rows of a tile (of the n_main: 256)
-    size_t floats = 0;  // of partial planes
-};
-
 // What q8_gemm_rows.hip takes, us: a launch, a start and an end for every further round of 256 workgroups, a price per block of K that a
 // workgroup walks (some of it for its 128 activation rows, some by its weight rows, some as the launch fills the chip), and for K
 // slices the launch of their sum and its planes (N in steps of four: 16 bytes a load; else four).  Fitted to 10200 launches of 4300
@@ -288,10 +301,12 @@ struct RowsTimes {
 };
 static constexpr RowsTimes kRowsTimes[2][2] = {{{3.6, 2.75, 2.85, 0.51, 0.79, 0.12, 0.535, 0.105}, {5.7, 5.4, 2.0, 0.38, 0.725, 0.23, 0.71, 0.03}},
                                                {{3.5, 2.25, 2.75, 0.455, 0.75, 0.035, 0.455, 0.14}, {5.0, 4.1, 2.9, 0.36, 0.73, 0.08, 0.45, 0.075}}};
-static double rows_us(const RowsTimes &t, int64_t workgroups, int width, int per, int slices, int64_t m, int64_t cols) {
-    const double rounds = static_cast<double>((workgroups + 255) / 256), fill = workgroups < 256 ? static_cast<double>(workgroups) / 256.0 : 1.0;
-    const double sum = slices > 1 ? t.sum + static_cast<double>(slices * m * cols) * 4e-6 * (cols % 4 == 0 ? t.planes : t.planes_odd) : 0.0;
-    return t.launch + (rounds - 1.0) * t.round + rounds * per * (t.block + t.block_rows * width / 256.0 + t.block_fill * fill) + sum;
+static double rows_us(const RowsTimes &t, int64_t workgroups, int width, int per) {  // (without the sum)
+    const double rounds = static_cast<double>((workgroups + 255) >> 8), fill = workgroups < 256 ? static_cast<double>(workgroups) * (1.0 / 256.0) : 1.0;
+    return t.launch + (rounds - 1.0) * t.round + rounds * per * (t.block + t.block_rows * (width * (1.0 / 256.0)) + t.block_fill * fill);
+}
+static double rows_sum_us(const RowsTimes &t, int slices, int64_t m, int64_t cols) {
+    return slices > 1 ? t.sum + static_cast<double>(slices * m * cols) * 4e-6 * (cols % 4 == 0 ? t.planes : t.planes_odd) : 0.0;
 }
 
 // The plan that ends first, by what each kernel takes (us, measured): a workgroup of the streaming kernel 0.49 (f32) or
@@ -334,46 +349,44 @@ static RowsPlan rows_plan(int64_t m, int n, int k, bool f16, size_t room, bool s
     // all columns, or those that whole rounds leave over, in K slices
     const int64_t per_round = m_tiles < 256 ? 256 / m_tiles : 1;
     const int64_t main_tiles = n_tiles / per_round * per_round;
-    for (int64_t lead : {int64_t{0}, main_tiles}) {
-        if (lead == n_tiles || (lead > 0 && m_tiles > 256)) continue;
+    for (int part = 0; part < 2; ++part) {
+        const int64_t lead = part == 0 ? 0 : main_tiles;
+        if (part == 1 && (lead == 0 || lead == n_tiles || m_tiles > 256)) break;
         const int64_t cols = n - lead * 256, tiles = m_tiles * (n_tiles - lead);
-        const double main_us = lead > 0 ? rows_us(times, m_tiles * lead, 256, k / 32, 1, m, cols) : 0.0;
+        const double main_us = lead > 0 ? rows_us(times, m_tiles * lead, 256, k / 32) : 0.0;
         const double first_main_us = lead > 0 ? rounds(m_tiles * lead) * nblk * (f16 ? 0.66 : 1.2) + 8.0 : 0.0;
         constexpr int widths[] = {256, 224, 192, 128};
         int64_t tiles_of[4];
+#pragma unroll
         for (int i = 0; i < 4; ++i) tiles_of[i] = m_tiles * ((cols + widths[i] - 1) / widths[i]);
         bool gap = false;
-        for (int slices = 1; slices <= kMaxRowsSlices; ++slices) {
-            if (lead > 0 && slices == 1) continue;
-            const int per = q8_gemm_rows_slice_blocks(k, slices);
-            gap = gap || slices > 16;
-            if (static_cast<int64_t>(slices - 1) * per >= k / 32) {  // an empty slice (the next number may have none)
-                if (per == 4) break;  // (the smallest: every further number leaves one empty)
-                gap = true;
-                continue;
-            }
-            const size_t floats = slices > 1 ? static_cast<size_t>(slices) * m * cols : 0;
-            if (floats > room || (slices > 1 && tiles * slices > 0x7ffffff0)) break;  // (the grid's x extent)
-            for (int i = 0; i < 4; ++i) {
-                const int width = widths[i];
-                const int64_t all = tiles_of[i] * slices;
-                if (i > 0 && (lead > 0 || (slices > 1 && all > 256))) break;
-                double us = main_us + rows_us(times, all, width, per, slices, m, cols);
-                // (what the estimate is short of on average: the gap between two launches; narrow tiles that walk all of K in step)
-                if (lead > 0 || (width < 256 && slices == 1)) us *= 1.05;
-                RowsPlan plan;
-                plan.kind = RowsPlan::kRows;
-                plan.n_main = static_cast<int>(lead * 256);
-                plan.slices = slices;
-                plan.width = width;
-                plan.floats = floats;
-                if (i == 0 && !gap && stream) {
-                    const double first_us = first_main_us + 8.0 + rounds(all) * per * (f16 ? 0.66 : 1.2) + (slices > 1 ? sum_us(slices, cols) : 0.0);
+        for (int slices = 1, per = q8_gemm_rows_slice_blocks(k, 1);;) {
+            if (lead == 0 || slices > 1) {
+                const size_t floats = slices > 1 ? static_cast<size_t>(slices) * m * cols : 0;
+                if (floats > room || (slices > 1 && tiles * slices > 0x7ffffff0)) break;  // (the grid's x extent)
+                const RowsPlan plan{RowsPlan::kRows, static_cast<int>(lead * 256), slices, 256, floats};
+                const double others_us = main_us + rows_sum_us(times, slices, m, cols);
+                for (int i = 0; i < 4; ++i) {
+                    const int width = widths[i];
+                    const int64_t all = tiles_of[i] * slices;
+                    if (i > 0 && (lead > 0 || (slices > 1 && all > 256))) break;
+                    double us = others_us + rows_us(times, all, width, per);
+                    // (what the estimate is short of on average: the gap between two launches; narrow tiles that walk all of K in step)
+                    if (lead > 0 || (width < 256 && slices == 1)) us *= 1.05;
+                    if (us < best_us) best_us = us, best = plan, best.width = width;
+                    if (floats == 0 && us < bare_us) bare_us = us, bare = plan, bare.width = width;
+                }
+                if (!gap && stream) {
+                    const double first_us = first_main_us + 8.0 + rounds(tiles * slices) * per * (f16 ? 0.66 : 1.2) + (slices > 1 ? sum_us(slices, cols) : 0.0);
                     if (first_us < early_us) early_us = first_us, early = plan;
                 }
-                if (us < best_us) best_us = us, best = plan;
-                if (floats == 0 && us < bare_us) bare_us = us, bare = plan;
             }
+            if (per == 4) break;
+            const int next = (k / 32 + per - 5) / (per - 4);  // the next number whose slices are shorter: those between leave one empty
+            if (next > kMaxRowsSlices) break;
+            gap = gap || next > slices + 1 || next > 16;
+            slices = next;
+            per = q8_gemm_rows_slice_blocks(k, slices);
         }
     }
     // A product of which the plain call kept nothing in the library's array, so that its calls may overlap, when these plans had tiles
@@ -382,23 +395,23 @@ static RowsPlan rows_plan(int64_t m, int n, int k, bool f16, size_t room, bool s
     return stream && early.floats == 0 && !(early.kind == RowsPlan::kStream && planes) ? bare : best;
 }
 
-// Floats of partial planes the plan for (m, n, k) uses when it has the library's own scratch array to itself: what a
-// caller's workspace must hold for the same plan (and the same bits) with either activation type.
-size_t q8_gemm_split_workspace_floats(int64_t m, int n, int k) {
+size_t q8_gemm_split_workspace_floats(int64_t m, int n, int k, RowsPlan *plans) {
     const bool stream = k % kSkUnit == 0 && n % 4 == 0;
     size_t most = 0;
+    bool streams = false;
     for (bool f16 : {false, true}) {
         const RowsPlan plan = rows_plan(m, n, k, f16, kSkScratchFloats, stream);
-        if (plan.kind != RowsPlan::kStream) {
+        if (plan.kind == RowsPlan::kStream)
+            streams = true;
+        else
             most = std::max(most, plan.floats);
-            continue;
-        }
-        for (int64_t m0 = 0; m0 < m; m0 += 64 * kSkMaxPasses) {
-            const int mc = static_cast<int>(m - m0 < 64 * kSkMaxPasses ? m - m0 : 64 * kSkMaxPasses);
-            // (at least what strips of 128 rows want, so that narrower ones without slices do not turn the answer into 0, "a matvec")
-            const int splits = std::max(split_plan(mc, n, k, kSkScratchFloats).splits, split_base_slices(mc, n, k, kSkScratchFloats));
-            if (splits > 1) most = std::max(most, static_cast<size_t>(splits) * mc * n);
-        }
+        if (plans) plans[f16] = plan;
+    }
+    for (int64_t m0 = 0; streams && m0 < m; m0 += 64 * kSkMaxPasses) {
+        const int mc = static_cast<int>(m - m0 < 64 * kSkMaxPasses ? m - m0 : 64 * kSkMaxPasses);
+        // (at least what strips of 128 rows want, so that narrower ones without slices do not turn the answer into 0, "a matvec")
+        const int splits = std::max(split_plan(mc, n, k, kSkScratchFloats).splits, split_base_slices(mc, n, k, kSkScratchFloats));
+        if (splits > 1) most = std::max(most, static_cast<size_t>(splits) * mc * n);
     }
     return most;
 }
@@ -407,11 +420,11 @@ size_t q8_gemm_split_workspace_floats(int64_t m, int n, int k) {
 // `own_workspace`: partial planes go to `ws` (ws_floats floats; none: no K slices) and the library's scratch array
 // is not touched, so calls may overlap in time.
 lhip_status q8_gemm_split_launch(const int8_t *qs, const __half *ds, const void *x, void *y, int64_t m, int n, int k,
-                                 bool f16, hipStream_t s, bool own_workspace, float *ws, size_t ws_floats) {
+                                 bool f16, hipStream_t s, bool own_workspace, float *ws, size_t ws_floats, const RowsPlan *known) {
     const size_t esz = f16 ? 2 : 4;
     const size_t room = own_workspace ? (ws ? std::min(ws_floats, kSkScratchFloats) : 0) : kSkScratchFloats;
     const bool stream = q8_gemm_split_supports(n, k, x, y, f16);
-    RowsPlan plan = rows_plan(m, n, k, f16, kSkScratchFloats, stream);
+    RowsPlan plan = known ? *known : rows_plan(m, n, k, f16, kSkScratchFloats, stream);
     if (plan.floats > room) plan = rows_plan(m, n, k, f16, room, stream);
     float *scratch = own_workspace ? ws : (plan.kind == RowsPlan::kRows && plan.slices > 1 ? sk_scratch_ptr() : nullptr);
     if (plan.kind == RowsPlan::kWide) return q8_gemm_wide_launch(qs, ds, x, kWdF16, y, static_cast<int>(m), n, k, kWdOutF16, s);

@@ -23,14 +23,11 @@
 #include <stdio.h>
 
 #include "common.h"
+#include "q8_gemm_rows.h"
 
 namespace lhip {
-// q8_gemm_skinny.hip: the matrix-core form with f32-accurate (head + tail bf16) operands for several activation rows.
-bool q8_gemm_split_supports(int n, int k, const void *x, const void *y, bool f16);
-lhip_status q8_gemm_split_launch(const int8_t *qs, const __half *ds, const void *x, void *y, int64_t m, int n, int k,
-                                 bool f16, hipStream_t s, bool own_workspace = false, float *ws = nullptr,
-                                 size_t ws_floats = 0);
-size_t q8_gemm_split_workspace_floats(int64_t m, int n, int k);
+// The matrix-core form with f32-accurate (head + tail bf16) operands for several activation rows: q8_gemm_split_launch
+// (q8_gemm_skinny.hip).
 // From this many activation rows on the plain operators take that form where the shape allows it: the weights are
 // then streamed once per 64 rows instead of once per row.  The matrix-core form has a fixed cost (its launch, a
 // reduce launch where K is sliced, staging) that a matvec pass over a small matrix stays under.  Measured, matvec
@@ -77,14 +74,21 @@ static double rows_sliced_us(int64_t m, int64_t n, int64_t k, bool f16) {
 // workgroups, against matvecs of 0.17 or 0.085 us per 2^20 codes and row (where they are cheapest, so that nothing gets
 // slower).  Measured, matvecs -> one slice -> sliced, us: 2880 x 2880 f32 at 96 rows 203 -> 86 -> 26, f16 at 128 rows 109 ->
 // 52 -> 21; 14336 x 4128 f32 at 32 rows 367 -> 80 -> 32; 512 x 14304 f32 at 512 rows 1073 -> 424 -> 47.
-static bool on_matrix_cores(int64_t m, int64_t n, int64_t k, const void *x, const void *y, bool f16, size_t room_floats) {
+// `plan` (not for SIZE_MAX): what the answer was worked out with, for the launch; kind kNone where it was not.
+static bool on_matrix_cores(int64_t m, int64_t n, int64_t k, const void *x, const void *y, bool f16, size_t room_floats,
+                            RowsPlan *plan = nullptr) {
     if (q8_gemm_split_supports(static_cast<int>(n), static_cast<int>(k), x, y, f16)) return m >= split_min_rows(n, k);
     if (k < 256 || !aligned(x, 16)) return false;
     const int64_t codes = n * k;
     const int64_t min_rows = codes >= (int64_t{32} << 20) ? 3 : codes >= (int64_t{16} << 20) ? 6 : codes >= (int64_t{8} << 20) ? 8 : 12;
     if (m < (f16 ? min_rows * 5 / 4 : min_rows)) return false;
-    if (room_floats == SIZE_MAX || room_floats >= q8_gemm_split_workspace_floats(m, static_cast<int>(n), static_cast<int>(k)))
-        return rows_sliced_us(m, n, k, f16) < matvecs_us(m, n, k, f16);
+    bool room = room_floats == SIZE_MAX;
+    if (!room) {
+        RowsPlan plans[2];
+        room = room_floats >= q8_gemm_split_workspace_floats(m, static_cast<int>(n), static_cast<int>(k), plans);
+        if (plan && (k % 512 != 0 || n % 4 != 0)) *plan = plans[f16];
+    }
+    if (room) return rows_sliced_us(m, n, k, f16) < matvecs_us(m, n, k, f16);
     const int64_t rounds = ((m + 127) / 128 * ((n + 255) / 256) + 255) / 256;
     return static_cast<double>(m) * static_cast<double>(codes) * (f16 ? 0.085 : 0.17) / (1 << 20) >
            8.0 + static_cast<double>(rounds * (k / 32)) * (f16 ? 0.66 : 1.2);
@@ -593,11 +597,12 @@ static lhip_status check_args(const void *planar, const float *x, float *y, int6
 using namespace lhip;
 
 static lhip_status matrix_cores(const void *planar, const void *x, void *y, int64_t m, int64_t n, int64_t k, bool f16, void *stream,
-                                bool own_workspace = false, void *ws = nullptr, size_t ws_nbytes = 0) {
+                                bool own_workspace = false, void *ws = nullptr, size_t ws_nbytes = 0, const RowsPlan *plan = nullptr) {
     auto *base = static_cast<const uint8_t *>(planar);
     return q8_gemm_split_launch(reinterpret_cast<const int8_t *>(base), reinterpret_cast<const __half *>(base + q8_scale_offset(n, k)),
                                 x, y, m, static_cast<int>(n), static_cast<int>(k), f16, as_stream(stream), own_workspace,
-                                static_cast<float *>(ws), ws ? ws_nbytes / sizeof(float) : 0);
+                                static_cast<float *>(ws), ws ? ws_nbytes / sizeof(float) : 0,
+                                plan && plan->kind != RowsPlan::kNone ? plan : nullptr);
 }
 
 extern "C" {
@@ -622,9 +627,10 @@ lhip_status lhip_q8_0_matmul_f32_cfg(const void *planar_dev, const float *x_dev,
 lhip_status lhip_q8_0_matmul_f32(const void *planar_dev, const float *x_dev, float *y_dev, int64_t m, int64_t n,
                                  int64_t k, void *stream) {
     if (lhip_status s = check_args(planar_dev, x_dev, y_dev, m, n, k)) return s;
-    if (on_matrix_cores(m, n, k, x_dev, y_dev, false, 0))
+    RowsPlan plan{RowsPlan::kNone};
+    if (on_matrix_cores(m, n, k, x_dev, y_dev, false, 0, &plan))
         return matrix_cores(planar_dev, x_dev, y_dev, m, n, k, false, stream,
-                            !q8_gemm_split_supports(static_cast<int>(n), static_cast<int>(k), x_dev, y_dev, false));
+                            !q8_gemm_split_supports(static_cast<int>(n), static_cast<int>(k), x_dev, y_dev, false), nullptr, 0, &plan);
     int r, u, b, w;
     choose(static_cast<int>(n), static_cast<int>(k), &r, &u, &b, &w);
     return lhip_q8_0_matmul_f32_cfg(planar_dev, x_dev, y_dev, m, n, k, r, u, b, w, stream);
@@ -660,9 +666,10 @@ lhip_status lhip_q8_0_matmul_f16(const void *planar_dev, const void *x_f16_dev, 
     if (m <= 0 || m > kMaxDim) return LHIP_ERR_INVALID_SHAPE;
     // Rows of x start at multiples of K halves; K % 32 == 0 keeps them 8-byte aligned.
     if (!aligned(planar_dev, 256) || !aligned(x_f16_dev, 8) || !aligned(y_f16_dev, 2)) return LHIP_ERR_MISALIGNED;
-    if (on_matrix_cores(m, n, k, x_f16_dev, y_f16_dev, true, 0))
+    RowsPlan plan{RowsPlan::kNone};
+    if (on_matrix_cores(m, n, k, x_f16_dev, y_f16_dev, true, 0, &plan))
         return matrix_cores(planar_dev, x_f16_dev, y_f16_dev, m, n, k, true, stream,
-                            !q8_gemm_split_supports(static_cast<int>(n), static_cast<int>(k), x_f16_dev, y_f16_dev, true));
+                            !q8_gemm_split_supports(static_cast<int>(n), static_cast<int>(k), x_f16_dev, y_f16_dev, true), nullptr, 0, &plan);
     auto *base = static_cast<const uint8_t *>(planar_dev);
     int r, u, b, w;
     choose(static_cast<int>(n), static_cast<int>(k), &r, &u, &b, &w);
@@ -707,8 +714,9 @@ lhip_status lhip_q8_0_matmul_f32_ws(const void *planar_dev, const float *x_dev, 
                                     int64_t k, void *workspace_dev, size_t workspace_nbytes, void *stream) {
     if (lhip_status s = check_args(planar_dev, x_dev, y_dev, m, n, k)) return s;
     if (workspace_dev && !aligned(workspace_dev, 256)) return LHIP_ERR_MISALIGNED;
-    if (on_matrix_cores(m, n, k, x_dev, y_dev, false, workspace_dev ? workspace_nbytes / sizeof(float) : 0))
-        return matrix_cores(planar_dev, x_dev, y_dev, m, n, k, false, stream, true, workspace_dev, workspace_nbytes);
+    RowsPlan plan{RowsPlan::kNone};
+    if (on_matrix_cores(m, n, k, x_dev, y_dev, false, workspace_dev ? workspace_nbytes / sizeof(float) : 0, &plan))
+        return matrix_cores(planar_dev, x_dev, y_dev, m, n, k, false, stream, true, workspace_dev, workspace_nbytes, &plan);
     return lhip_q8_0_matmul_f32(planar_dev, x_dev, y_dev, m, n, k, stream);  // matvec kernels: no shared state
 }
 
@@ -719,8 +727,9 @@ lhip_status lhip_q8_0_matmul_f16_ws(const void *planar_dev, const void *x_f16_de
     if (m <= 0 || m > kMaxDim) return LHIP_ERR_INVALID_SHAPE;
     if (!aligned(planar_dev, 256) || !aligned(x_f16_dev, 8) || !aligned(y_f16_dev, 2)) return LHIP_ERR_MISALIGNED;
     if (workspace_dev && !aligned(workspace_dev, 256)) return LHIP_ERR_MISALIGNED;
-    if (on_matrix_cores(m, n, k, x_f16_dev, y_f16_dev, true, workspace_dev ? workspace_nbytes / sizeof(float) : 0))
-        return matrix_cores(planar_dev, x_f16_dev, y_f16_dev, m, n, k, true, stream, true, workspace_dev, workspace_nbytes);
+    RowsPlan plan{RowsPlan::kNone};
+    if (on_matrix_cores(m, n, k, x_f16_dev, y_f16_dev, true, workspace_dev ? workspace_nbytes / sizeof(float) : 0, &plan))
+        return matrix_cores(planar_dev, x_f16_dev, y_f16_dev, m, n, k, true, stream, true, workspace_dev, workspace_nbytes, &plan);
     return lhip_q8_0_matmul_f16(planar_dev, x_f16_dev, y_f16_dev, m, n, k, stream);
 }
 
