@@ -236,6 +236,14 @@ lhip_status lhip_q8_0_matmul_bf16_swiglu(const void *planar_dev, const void *x_d
 lhip_status lhip_q8_0_matmul_bf16_cfg(const void *planar_dev, const void *x_dev, void *y_dev, int64_t m, int64_t n,
                                       int64_t k, int tile, void *stream);
 
+/* Which kernel a call of lhip_q8_0_matmul_f32 (activations 0), _f16 (1) or _bf16 (2) takes and how it cuts the weight: for tests and
+ * profiles, which ask whether a shape reaches what it is meant to (no counterpart in the reference).  It touches no device, assumes
+ * aligned arguments and may answer differently from version to version.  workspace_nbytes: the room a `_ws` form is given,
+ * (size_t)-1 for the plain call.  plan[0] = 0: matvecs, 1: the weight-streaming kernel, 2: the f32 / f16 kernel for several
+ * rows, 3: the bf16 / f16 tiles; plan[1] = weight rows of a workgroup of kernels 1 and 2 (else 0); plan[2] = slices of K (0: of the
+ * columns that whole rounds of tiles leave over only). */
+lhip_status lhip_q8_0_matmul_plan(int64_t m, int64_t n, int64_t k, int32_t activations, size_t workspace_nbytes, int32_t plan[3]);
+
 /* Row gather: out[t][j] = dequant(W[(int)idx[t]][j]), idx carried as f32 like
  * the reference's (crates/luminal_cuda/src/quantized.rs:191-198,202-233), but
  * read from device memory.  An index outside [0, n) yields a row of zeros. */

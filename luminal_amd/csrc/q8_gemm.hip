@@ -34,6 +34,7 @@
 #include <utility>
 
 #include "common.h"
+#include "q8_gemm_rows.h"
 #include "q8_gemm_wide.h"
 #include "q8_mma_device.h"
 
@@ -568,6 +569,14 @@ static int gemm_auto_tile(int64_t m, int64_t n, int64_t k, int out, const void *
         return 1.1 * q8_gemm_skinny_us(static_cast<int>(m), static_cast<int>(n), static_cast<int>(k), room) < us ? kTileSkinny : tile;
     }
     return gemm_tiles(m, n, k, out, y, room, &us);
+}
+
+void q8_gemm_describe(int64_t m, int64_t n, int64_t k, size_t room, int32_t plan[3]) {
+    room = room == SIZE_MAX ? gemm_plain_room(k) : room < kGemmScratchFloats ? room : kGemmScratchFloats;
+    const int tile = gemm_auto_tile(m, n, k, kOutBf16, nullptr, room);
+    if (tile == kTileSkinny) return q8_gemm_skinny_describe(static_cast<int>(m), static_cast<int>(n), static_cast<int>(k), room, plan);
+    plan[0] = 3, plan[1] = 0;
+    plan[2] = tile == kTileTail ? 0 : tile > kTileSliced ? tile - kTileSliced : 1;
 }
 
 }  // namespace lhip

@@ -27,6 +27,12 @@ lhip_status q8_gemm_split_launch(const int8_t *qs, const __half *ds, const void 
                                  hipStream_t s, bool own_workspace = false, float *ws = nullptr, size_t ws_floats = 0,
                                  const RowsPlan *known = nullptr);
 
+// lhip_q8_0_matmul_plan's answers: for f32 / f16 on the matrix cores within `room` floats of planes; for bf16 (room SIZE_MAX: the plain
+// call; q8_gemm.hip), of which the weight-streaming kernel's.
+void q8_gemm_split_describe(int64_t m, int n, int k, bool f16, size_t room, int32_t plan[3]);
+void q8_gemm_describe(int64_t m, int64_t n, int64_t k, size_t room, int32_t plan[3]);
+void q8_gemm_skinny_describe(int m, int n, int k, size_t room, int32_t plan[3]);
+
 // Blocks of K per slice (whole groups of four).
 int q8_gemm_rows_slice_blocks(int64_t k, int slices);
 // y (m, n) = x (m, k) W^T for f32 or f16 x and y (x 16-byte aligned), any k that is a multiple of 32, any m and n; ldy = row

@@ -221,6 +221,11 @@ double q8_gemm_skinny_us(int m, int n, int k, size_t room) {
     return sk_us(kSkBf16, SkStrip(kSkBf16, index, m), plan.splits, strips * plan.splits, (sk_units(k) + plan.splits - 1) / plan.splits, m, n, 1e30);
 }
 
+void q8_gemm_skinny_describe(int m, int n, int k, size_t room, int32_t plan[3]) {
+    const SkPlan p = sk_plan_within(m, n, k, room);
+    plan[0] = 1, plan[1] = 16 * p.cw, plan[2] = p.splits;
+}
+
 constexpr int kSkMaxRows = 128 * 64;  // passes are the grid's z extent
 
 bool q8_gemm_skinny_supports(int m, int n, int k, int out, const void *y) {
@@ -414,6 +419,21 @@ size_t q8_gemm_split_workspace_floats(int64_t m, int n, int k, RowsPlan *plans) 
         if (splits > 1) most = std::max(most, static_cast<size_t>(splits) * mc * n);
     }
     return most;
+}
+
+void q8_gemm_split_describe(int64_t m, int n, int k, bool f16, size_t room, int32_t plan[3]) {
+    room = std::min(room, kSkScratchFloats);
+    const bool stream = k % kSkUnit == 0 && n % 4 == 0;
+    RowsPlan p = rows_plan(m, n, k, f16, kSkScratchFloats, stream);
+    if (p.floats > room) p = rows_plan(m, n, k, f16, room, stream);
+    if (p.kind == RowsPlan::kStream) {
+        const SkPlan strips = split_plan(static_cast<int>(m < 64 * kSkMaxPasses ? m : 64 * kSkMaxPasses), n, k, room);
+        plan[0] = 1, plan[1] = 16 * strips.cw, plan[2] = strips.splits;
+    } else if (p.kind == RowsPlan::kRows) {
+        plan[0] = 2, plan[1] = p.width, plan[2] = p.n_main ? 0 : p.slices;
+    } else {
+        plan[0] = 3, plan[1] = 0, plan[2] = 1;
+    }
 }
 
 // y (m, N) = x (m, K) W^T for f32 or f16 activations and results, any m; x 16-byte aligned.

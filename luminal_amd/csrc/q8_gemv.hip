@@ -710,6 +710,26 @@ size_t lhip_q8_0_matmul_workspace_nbytes(int64_t m, int64_t n, int64_t k) {
     return q8_gemm_split_workspace_floats(m, static_cast<int>(n), static_cast<int>(k)) * sizeof(float);
 }
 
+lhip_status lhip_q8_0_matmul_plan(int64_t m, int64_t n, int64_t k, int32_t activations, size_t workspace_nbytes, int32_t plan[3]) {
+    if (!plan) return LHIP_ERR_NULL_PTR;
+    if (lhip_status s = check_q8_shape(n, k)) return s;
+    if (m <= 0 || m > kMaxDim || activations < 0 || activations > 2) return LHIP_ERR_INVALID_SHAPE;
+    const bool plain = workspace_nbytes == SIZE_MAX;
+    size_t room = plain ? SIZE_MAX : workspace_nbytes / sizeof(float);
+    if (activations == 2) {
+        if (k % 64 != 0) return LHIP_ERR_UNSUPPORTED;
+        q8_gemm_describe(m, n, k, room, plan);
+        return LHIP_OK;
+    }
+    if (plain && !q8_gemm_split_supports(static_cast<int>(n), static_cast<int>(k), nullptr, nullptr, false)) room = 0;
+    if (on_matrix_cores(m, n, k, nullptr, nullptr, activations == 1, room)) {
+        q8_gemm_split_describe(m, static_cast<int>(n), static_cast<int>(k), activations == 1, room, plan);
+    } else {
+        plan[0] = plan[1] = 0, plan[2] = 1;
+    }
+    return LHIP_OK;
+}
+
 lhip_status lhip_q8_0_matmul_f32_ws(const void *planar_dev, const float *x_dev, float *y_dev, int64_t m, int64_t n,
                                     int64_t k, void *workspace_dev, size_t workspace_nbytes, void *stream) {
     if (lhip_status s = check_args(planar_dev, x_dev, y_dev, m, n, k)) return s;

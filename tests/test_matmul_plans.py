@@ -1,0 +1,59 @@
+"""Whether the sizes of the matmul tests reach the kernels, and the strips, tiles and K slices, that they are listed for.  No GPU."""
+import ctypes as C
+
+import pytest
+
+from luminal_amd import capi
+from matmul_shapes import ROWS, STREAMED_BF16, STREAMED_BF16_ANY_K, STREAMED_F32_F16
+
+TYPES = {"f32": 0, "f16": 1, "bf16": 2}
+PLAIN = (1 << 64) - 1
+MATVEC, STREAM, ROWS_KERNEL, TILES = 0, 1, 2, 3
+
+
+def plan(m, n, k, dtype, workspace=False):
+    """(kernel, weight rows of a workgroup, K slices), of the plain call or with the recommended workspace."""
+    lib, out = capi.load_library(), (C.c_int32 * 3)()
+    room = PLAIN
+    if workspace:
+        room = lib.lhip_q8_0_matmul_bf16_workspace_nbytes(m, n, k, 0) if dtype == "bf16" else lib.lhip_q8_0_matmul_workspace_nbytes(m, n, k)
+    capi.check(lib.lhip_q8_0_matmul_plan(m, n, k, TYPES[dtype], room, out), "lhip_q8_0_matmul_plan")
+    return tuple(out)
+
+
+def cuts(plans):
+    """The (weight rows, whether K is sliced) that occur."""
+    return {(rows, slices > 1) for _, rows, slices in plans}
+
+
+def test_strips_of_the_weight_streaming_kernel():
+    plans = [plan(*s, "bf16") for s in STREAMED_BF16]
+    assert {p[0] for p in plans} == {STREAM}
+    assert cuts(plans) == {(rows, sliced) for rows in (32, 48, 64, 112, 128) for sliced in (False, True)}
+    for dtype in ("f32", "f16"):
+        plans = [plan(*s, dtype) for s in STREAMED_F32_F16]
+        assert {p[0] for p in plans} == {STREAM}, list(zip(STREAMED_F32_F16, plans))
+        assert cuts(plans) == {(rows, sliced) for rows in (32, 48, 64, 128) for sliced in (False, True)}
+
+
+def test_strips_of_the_weight_streaming_kernel_for_any_k():
+    plans = [(plan(*s, "bf16"), plan(*s, "bf16", workspace=True)) for s in STREAMED_BF16_ANY_K]
+    assert all(plain[0] == STREAM for plain, _ in plans) and sum(ws[0] == STREAM for _, ws in plans) >= len(plans) - 1
+    assert all(plain[2] == 1 for plain, _ in plans)  # nothing is kept outside the outputs
+    assert cuts(p for both in plans for p in both if p[0] == STREAM) == {(rows, sliced) for rows in (32, 64, 128) for sliced in (False, True)}
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16"])
+def test_tiles_of_the_kernel_for_several_rows(dtype):
+    plans = [plan(*s, dtype, workspace=True) for s in ROWS[dtype]]
+    assert {p[0] for p in plans} == {ROWS_KERNEL}, list(zip(ROWS[dtype], plans))
+    assert cuts(plans) == {(rows, sliced) for rows in (128, 192, 224, 256) for sliced in (False, True)}, list(zip(ROWS[dtype], plans))
+
+
+def test_plan_errors():
+    lib, out = capi.load_library(), (C.c_int32 * 3)()
+    assert lib.lhip_q8_0_matmul_plan(1, 32, 32, 0, PLAIN, None) == capi.LHIP_ERR_NULL_PTR
+    for bad in ((0, 32, 32, 0), (1, 0, 32, 0), (1, 32, 33, 0), (1, 32, 32, 3), (1, 32, 32, -1)):
+        assert lib.lhip_q8_0_matmul_plan(*bad, PLAIN, out) == capi.LHIP_ERR_INVALID_SHAPE
+    assert lib.lhip_q8_0_matmul_plan(1, 32, 32, 2, PLAIN, out) == capi.LHIP_ERR_UNSUPPORTED  # bf16: K in steps of 64
+    assert plan(1, 4096, 4096, "f32") == (MATVEC, 0, 1) and plan(2048, 14336, 4096, "bf16")[0] == TILES

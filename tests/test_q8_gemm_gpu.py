@@ -15,6 +15,7 @@ torch = pytest.importorskip("torch")
 from conftest import rel_err  # noqa: E402
 from luminal_amd import capi, synth  # noqa: E402
 from luminal_amd.quantized import Q8Weight, QuantizedMatmulBf16  # noqa: E402
+from matmul_shapes import STREAMED_BF16, STREAMED_BF16_ANY_K  # noqa: E402
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -168,16 +169,28 @@ def test_weight_streaming_gemm_vs_oracle(oracle, m, n, k):
         assert np.all(np.abs(y - auto) <= step) and np.mean(y == auto) > 0.98, slices
 
 
-@pytest.mark.parametrize("m,n,k", [
-    (1, 36, 512), (16, 100, 1024), (17, 8188, 1024), (32, 28, 2048),            # strips of 32 rows: ragged, none full
-    (16, 8212, 1024), (33, 12276, 1024),                                        # 48: one row more than 256 strips of 32 hold
-    (65, 8212, 1024), (128, 12300, 1024), (16, 16388, 1024), (64, 14332, 512),  # 64, and one round of them exceeded
-    (16, 4100, 4096), (64, 4092, 4096), (31, 500, 8192), (128, 2044, 8192),     # narrow strips over K slices
-])
+def swiglu_of(lib, st, w, x, m, n, k, *room):
+    """The SwiGLU form of the product, of the plain call or with (workspace address, bytes)."""
+    out = torch.full((m, n // 2), float("nan"), dtype=torch.bfloat16, device=DEV)
+    args = (w.planar.data_ptr(), x.data_ptr(), out.data_ptr(), m, n, k)
+    capi.check(lib.lhip_q8_0_matmul_bf16_ws(*args, capi.LHIP_GEMM_OUT_SWIGLU, *room, st) if room else lib.lhip_q8_0_matmul_bf16_swiglu(*args, st), "swiglu")
+    return out
+
+
+def swiglu_rows(lib, st, y32):
+    """SwiGLU of f32 rows of (gate, up) pairs."""
+    m, n = y32.shape
+    out = torch.empty((m, n // 2), dtype=torch.bfloat16, device=DEV)
+    capi.check(lib.lhip_swiglu_f32_bf16out(y32.data_ptr(), out.data_ptr(), m, n // 2, 1, st), "lhip_swiglu_f32_bf16out")
+    return out
+
+
+@pytest.mark.parametrize("m,n,k", STREAMED_BF16)
 def test_weight_streaming_gemm_by_every_strip_width(oracle, m, n, k):
-    """Sizes on the edges of the strips of 32, 48, 64 and 112 / 128 weight rows, with and without K slices.  The block
-    sums are f32 (32 exact products) and so are their K / 32 additions, so an element is off by less than
-    (32 + K / 32) 2^-24 times the sum of the magnitudes of its terms; the bf16 form is the f32 output rounded once."""
+    """Sizes on the edges of the strips of 32, 48, 64, 112 and 128 weight rows, with and without K slices.  The block
+    sums are f32 (32 exact products) and so are their K / 32 additions (of S slices K / 32 / S + S on a path), so an element is
+    off by less than (32 + K / 32) 2^-24 times the sum of the magnitudes of its terms; the bf16 form is the f32 output
+    rounded once, SwiGLU that of the f32 output."""
     qs, d = synth.q8_0_random(n, k, seed=m + n + k)
     xf, bits = bf16_activations(oracle, m, k, seed=m + 1)
     w = upload(qs, d)
@@ -192,13 +205,10 @@ def test_weight_streaming_gemm_by_every_strip_width(oracle, m, n, k):
     err = (y32.cpu().double() - x64 @ weight.T).abs()
     assert bool((err <= (32 + k // 32) * 2.0 ** -24 * (x64.abs() @ weight.abs().T)).all())
     assert torch.equal(y16, y32.to(torch.bfloat16))
+    assert torch.equal(swiglu_of(lib, st, w, x, m, n, k), swiglu_rows(lib, st, y32))
 
 
-@pytest.mark.parametrize("m,n,k", [
-    (1, 36, 256), (16, 100, 320), (17, 260, 448), (33, 64, 576), (128, 132, 704),  # one to eleven groups of 64
-    (16, 8196, 960), (64, 16388, 1088), (65, 28, 1472), (128, 8252, 1984),         # strips of 32, 64, 128
-    (5, 2880, 2880), (45, 2880, 2880), (100, 2880, 2880), (31, 516, 14272), (128, 1028, 4160),
-])
+@pytest.mark.parametrize("m,n,k", STREAMED_BF16_ANY_K)
 def test_weight_streaming_gemm_of_any_k(oracle, m, n, k):
     """A K that ends inside a step of 512: without K slices (the plain call) and with them (a workspace), to the bound of
     test_weight_streaming_gemm_by_every_strip_width with one more addition per slice; an infinite activation at the end
@@ -222,6 +232,13 @@ def test_weight_streaming_gemm_of_any_k(oracle, m, n, k):
         capi.check(lib.lhip_q8_0_matmul_bf16_f32out(w.planar.data_ptr(), x.data_ptr(), y.data_ptr(), m, n, k, st), "plain")
         capi.check(lib.lhip_q8_0_matmul_bf16_ws(w.planar.data_ptr(), x.data_ptr(), y_ws.data_ptr(), m, n, k, 1,
                                                 space.data_ptr() if nbytes else None, nbytes, st), "ws")
+        if not infinite:  # the bf16 and SwiGLU forms are those of the f32 output
+            room = (space.data_ptr() if nbytes else None, nbytes)
+            for f32, args in ((y, ()), (y_ws, room)):
+                assert torch.equal(swiglu_of(lib, st, w, x, m, n, k, *args), swiglu_rows(lib, st, f32))
+            y16 = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=DEV)
+            capi.check(lib.lhip_q8_0_matmul_bf16(w.planar.data_ptr(), x.data_ptr(), y16.data_ptr(), m, n, k, st), "bf16")
+            assert torch.equal(y16, y.to(torch.bfloat16))
         for got in (y.cpu().double(), y_ws.cpu().double()):
             if infinite:
                 assert bool((got[m // 2] == float("inf")).all())
