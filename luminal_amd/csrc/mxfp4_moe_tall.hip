@@ -4,19 +4,21 @@
 // A workgroup of four waves owns up to 96 routed rows of one expert and 256 weight rows, a wave 64 of these (two tiles of 32;
 // gated: a tile is 16 rows of gate and the same 16 of up).  K goes by in stages of 64.
 //
-// What bounds it: the time goes into the waits of a workgroup's four waves for each other and for LDS and memory at every stage
-// (per CU and stage, three workgroups of 2.25 fragments on average: 1760 cycles of the matrix pipe, 1400 of LDS, 1200 of vector
-// issue, of about 3000 that pass), so as many workgroups as possible share a CU and a stage costs each as little as possible:
+// What bounds it: the matrix pipe is busy for 60 % of the launch at T = 1024 (56 % in the down product), vector instructions are issued for
+// 32 % (27 %), LDS works for 26 % (25 %); the rest are the waits of a workgroup's four waves for each other, for LDS and for memory at
+// every stage, so as many workgroups as possible share a CU and a stage costs each as little as possible (variants' times are of the
+// layer of 32 experts of 2880 x 2880, top 4, while this form took 240 to 246 us at T = 1024 and 147 to 155 at T = 512):
 //   * v_mfma_f32_32x32x16: half the issue slots of 16x16x32, and an activation operand read from LDS feeds two of them (one, with
-//     32 weight rows a wave: LDS holds up the matrix pipe, T = 1024 292 us for the layer and not 246);
+//     32 weight rows a wave: LDS holds up the matrix pipe, T = 1024 292 us);
 //   * everything arrives in LDS by direct loads, and a wave keeps nothing of the next stage in registers: 150 registers, three
 //     workgroups a CU.  Two with a third stage of activations: T = 1024 273 us.  Weights held a stage ahead in registers: the
 //     compiler's waits for them count the direct loads too, and stop at those;
-//   * activation fragments that the tile does not have are not requested (all 96 rows always: 5 % slower at T = 1024).
-// Measured on the benchmark layer (32 experts of 2880 x 2880, top 4), us per layer, before (64-row tiles of mx_moe_gemm_exact_kernel,
-// activations through registers, experts in their own order in the tile list) -> now: T = 192 126 -> 114, T = 512 191 -> 155,
-// T = 1024 284 -> 237 (860 TFLOP/s of useful work), T = 2048 455 -> 393.  Tiles of 128 rows and 64 are level or slower there (T = 1024 289
-// and 259, T = 512 173 and 172), of 160 rows at two workgroups a CU 241 at T = 1024 and 174 at T = 512.
+//   * activation fragments that the tile does not have are not requested (all 96 rows always: 5 % slower at T = 1024);
+//   * tiles of 128 rows, and of 64, are level or slower (T = 1024 289 and 259, T = 512 173 and 172), of 160 rows at two workgroups a CU
+//     241 at T = 1024 and 174 at T = 512.
+// A stage takes longer when the workgroup is alone on its CU (4 experts of 2048 x 2048 at 32 rows, 64 workgroups: 58 us, by 64-row tiles
+// 47), so this is taken only where there are enough (exact_tile_fragments).  Measured, us per layer, 64-row tiles of mx_moe_gemm_exact_kernel -> this: T = 192 117 ->
+// 110, T = 512 186 -> 158, T = 1024 274 -> 236 (860 TFLOP/s of useful work), T = 2048 438 -> 401.
 #include <algorithm>
 
 #include "mxfp4_moe_exact_device.h"
@@ -38,7 +40,8 @@ struct TallShape {
 };
 
 // 64 lanes x 16 (4) bytes from base + the lane's offset to consecutive LDS from `lds` on.  Inline assembly, because the compiler
-// would otherwise wait for the newest of them ahead of every LDS read.
+// would otherwise wait for the newest of them ahead of every LDS read.  (m0 is a reserved register: the compiler keeps nothing in it
+// from one statement to another.)
 template <int BYTES>
 __device__ __forceinline__ void tall_request(const void *base, uint32_t voff, uint32_t lds) {
     if constexpr (BYTES == 16)

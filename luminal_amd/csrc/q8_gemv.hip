@@ -26,23 +26,25 @@
 #include "q8_gemm_rows.h"
 
 namespace lhip {
-// The matrix-core form with f32-accurate (head + tail bf16) operands for several activation rows: q8_gemm_split_launch
-// (q8_gemm_skinny.hip).
-// From this many activation rows on the plain operators take that form where the shape allows it: the weights are
-// then streamed once per 64 rows instead of once per row.  The matrix-core form has a fixed cost (its launch, a
-// reduce launch where K is sliced, staging) that a matvec pass over a small matrix stays under.  Measured, matvec
-// against matrix cores, us: 1024 x 4096 at five rows 6.0 / 10.7; 4096 x 4096 at three rows 12.4 / 12.7, at four
-// 15.8 / 12.4; 14336 x 4096 at two rows 20.6 / 21.5, at three 31.7 / 22.0; 128256 x 4096 at two rows 168 / 130.
+// From this many activation rows on the plain operators take the matrix-core form with f32-accurate operands (q8_gemm_split_launch,
+// q8_gemm_skinny.hip) where the shape allows it: the weights are then streamed once per 64 rows instead of once per row.  That form
+// has a fixed cost (its launch, a reduce launch where K is sliced, staging) that a matvec pass over a small matrix stays under.
+// Measured, matvecs / matrix cores, us, f32 and f16: 1024 x 4096 at five rows 5.9 / 6.9 and 5.2 / 6.5, at six 6.7 / 7.0 and 5.8 / 6.5; 4096 x
+// 4096 at two rows 8.9 / 11.1 and 7.7 / 10.6, at three 12.3 / 11.1 and 10.4 / 10.7, at four 15.9 / 11.2 and 13.0 / 10.7; 14336 x 4096 at
+// two rows 21.1 / 18.8 and 20.1 / 17.9, at three 31.1 / 18.9 and 29.7 / 18.0; 128256 x 4096 at two rows 169 / 128 and 168 / 118.  (The
+// lines were drawn when the matrix cores took 12.7 us at three rows of 4096 x 4096 and 21.5 at two of 14336 x 4096; since its strips
+// follow N the crossing lies up to a row below them there.)
 static int split_min_rows(int64_t n, int64_t k) {
     const int64_t codes = n * k;
     return codes >= (int64_t{256} << 20) ? 2 : codes >= (int64_t{32} << 20) ? 3 : codes >= (int64_t{8} << 20) ? 4 : 6;
 }
 
-// What m matvecs of a K outside the streaming kernel's shapes take, us, and what q8_gemm_rows.hip takes over K slices for few
-// rows, as measured on an MI355X.  A matvec: a launch for all rows, then per row and 1000 weight rows a step of about 1024 of K
-// where K is short, less with more weight rows, and a price per 1000 of K where it is long, less where K is in steps of 512.  The
-// rows kernel: two launches, a slice for each four blocks of K up to 16 of them and longer slices beyond, another half behind 64
-// rows, and the stores of an N that is no multiple of four.
+// What m matvecs of a K outside the streaming kernel's shapes take, us, and an upper bound of what q8_gemm_rows.hip takes over K slices
+// for few rows.  A matvec: a launch for all rows, then per row and 1000 weight rows a step of about 1024 of K where K is short,
+// less with more weight rows, and a price per 1000 of K where it is long, less where K is in steps of 512.  The rows kernel: as
+// measured with tiles of 256 weight rows and a slice for each four blocks of K up to 16 of them, two launches, another half behind
+// 64 rows, and the stores of an N that is no multiple of four; with up to 40 slices and narrower tiles (rows_plan) it takes less
+// where the weight rows are few or K is long: 1000 x 4480 f32 at 12 rows 11.6 and not 19.2, 1001 x 14336 f32 at 8 15.6 and not 36.5.
 static double matvecs_us(int64_t m, int64_t n, int64_t k, bool f16) {
     const double k1000 = static_cast<double>(k) / 1000.0;
     double per_row;
@@ -65,15 +67,17 @@ static double rows_sliced_us(int64_t m, int64_t n, int64_t k, bool f16) {
 
 // Whether a product of m rows is one for the matrix cores.  The streaming kernel's shapes (K in steps of 512, N of 4)
 // from split_min_rows on.  Every other K from 256 on by q8_gemm_rows.hip, from a few rows on and where the costs above say so.
-// Measured, matvecs -> matrix cores, us: 2880 x 2880 f32 at 8 / 45 / 200 rows 18.4 -> 16.3 / 96 -> 18 / 423 -> 28, f16 at 8 / 45
-// rows 9.4 -> 15.8 / 38 -> 15; 1000 x 4480 f32 at 12 / 24 rows 17.0 -> 19.2 / 31.6 -> 19.5; 260 x 544 f32 at 24 / 200 / 512
-// rows 3.3 -> 11.1 / 12.3 -> 15.3 / 29 -> 15; 1001 x 14336 f32 at 8 / 24 rows 20.8 -> 30.6 / 55 -> 30.  (Lines in N K alone
-// sent every product of 12 rows there.)  A K below 256 is a matvec of one or two microseconds per row.
+// Measured, matvecs / matrix cores, us (taken: the first unless marked *): 2880 x 2880 f32 at 4 / 8 / 12* / 45* / 200* rows 11.4 / 11.6, 19.7 / 12.0,
+// 28.1 / 12.4, 97 / 14.3 and 422 / 22.5, f16 at 6 / 12 / 16* / 45* rows 10.2 / 10.5, 16.7 / 11.1, 21.0 / 11.6 and 50 / 12.4; 1000 x 4480 f32 at
+// 6 / 12 / 24* rows 10.6 / 11.0, 19.0 / 11.6 and 34.4 / 12.6; 260 x 544 f32 at 24 / 200 / 512* rows 4.1 / 7.8, 13.2 / 9.5 and 29.5 / 10.2; 1001 x
+// 14336 f32 at 4 / 12 / 24* rows 12.8 / 15.0, 31.5 / 16.1 and 57 / 17.6; 14336 x 4128 f32 at 2 / 3* / 8* rows 31.0 / 34.2, 42.3 / 34.3 and 100 / 34.8.  So
+// the lines, drawn for the kernel with 16 slices, lie some rows above the crossing (6 rows against 12 at 2880 x 2880).  (Lines in
+// N K alone sent every product of 12 rows there.)  A K below 256 is a matvec of one or two microseconds per row.
 // Without room for the slices' planes - the plain operators, which for these K keep nothing outside their outputs, so that
 // calls on several streams may overlap - it is one slice, 1.2 (f32) or 0.66 us (f16) per block of K and round of 256
 // workgroups, against matvecs of 0.17 or 0.085 us per 2^20 codes and row (where they are cheapest, so that nothing gets
-// slower).  Measured, matvecs -> one slice -> sliced, us: 2880 x 2880 f32 at 96 rows 203 -> 86 -> 26, f16 at 128 rows 109 ->
-// 52 -> 21; 14336 x 4128 f32 at 32 rows 367 -> 80 -> 32; 512 x 14304 f32 at 512 rows 1073 -> 424 -> 47.
+// slower).  Measured, matvecs -> one slice -> sliced, us: 2880 x 2880 f32 at 96 rows 202 -> 63 -> 19, f16 at 128 rows 124 ->
+// 46 -> 18; 14336 x 4128 f32 at 32 rows 381 -> 67 -> 36; 512 x 14304 f32 at 512 rows 1069 -> 304 -> 35.
 // `plan` (not for SIZE_MAX): what the answer was worked out with, for the launch; kind kNone where it was not.
 static bool on_matrix_cores(int64_t m, int64_t n, int64_t k, const void *x, const void *y, bool f16, size_t room_floats,
                             RowsPlan *plan = nullptr) {
