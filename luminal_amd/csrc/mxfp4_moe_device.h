@@ -42,18 +42,19 @@ struct MoePlan {
     int *tile_run0, *tile_runlen;
     int *n_tiles;      // [1]
     int max_tiles;     // entries of the tile arrays
+    int by_rows;       // whether experts are listed by their rows (else in their own order)
     int fragment;      // rows of a matrix step: a tile is some number of these, but for the end of an expert
     // 0: tiles are listed in expert order from entry 0.  Otherwise the list is cut into eight ranges of this many
     // entries, one per XCD (range x is read by the workgroups whose dispatch number is x modulo 8), and the
-    // tiles, still in expert order, are dealt to the ranges in eight contiguous, equal shares: the tiles of an
+    // tiles, an expert's behind each other, are dealt to the ranges in eight contiguous, equal shares: the tiles of an
     // expert, and all column blocks of a tile, then run on one XCD and find each other's weights and
     // activation rows in its L2.
     int tiles_per_xcd;
 };
 
 __device__ __forceinline__ void moe_plan_block(const int *__restrict__ sel, int R, int E, int BM, const MoePlan &p) {
-    // The counts of all experts are read by every expert's thread, four at a time.
-    __shared__ __attribute__((aligned(16))) int cnt[1024], tiles[1024];
+    // The counts and places of all experts are read by every expert's thread, four at a time.
+    __shared__ __attribute__((aligned(16))) int cnt[1024], pos[1024], tiles[1024];
     __shared__ int off[1025], cur[1024];
     constexpr int KEEP = 4;  // routed entries a thread keeps in registers between the two passes over them
     int kept[KEEP];
@@ -65,6 +66,7 @@ __device__ __forceinline__ void moe_plan_block(const int *__restrict__ sel, int 
     for (int e = threadIdx.x; e < 1024; e += 1024) {  // (all of them: those from E on are read in fours)
         cnt[e] = 0;
         cur[e] = 0;
+        pos[e] = 1024;
         tiles[e] = 0;
     }
     for (int t = threadIdx.x; t < p.max_tiles; t += 1024) {  // entries no tile is written to stay marked unused
@@ -83,26 +85,45 @@ __device__ __forceinline__ void moe_plan_block(const int *__restrict__ sel, int 
         if (e >= 0 && e < E) atomicAdd(&cnt[e], 1);
     }
     __syncthreads();
-    for (int e = threadIdx.x; e < E; e += 1024) tiles[e] = (cnt[e] + BM - 1) / BM;
-    __syncthreads();
-    const int4 *cnt4 = reinterpret_cast<const int4 *>(cnt), *tiles4 = reinterpret_cast<const int4 *>(tiles);
+    const int4 *cnt4 = reinterpret_cast<const int4 *>(cnt), *pos4 = reinterpret_cast<const int4 *>(pos), *tiles4 = reinterpret_cast<const int4 *>(tiles);
     const int E4 = (E + 3) >> 2;
+    // The list's order of experts: their own, or (by_rows) by rows, the most first, dealt to eight shares back and forth, share
+    // behind share.  Cut into eight ranges of as many tiles, the ranges then have about as many rows each, and tall tiles start
+    // first.  A wave ranks an expert by counting those before it, 64 at a time.
+    for (int e = threadIdx.x; e < E; e += 1024) {
+        tiles[e] = (cnt[e] + BM - 1) / BM;
+        if (!p.by_rows) pos[e] = e;
+    }
+    if (p.by_rows) {
+        const int lane = threadIdx.x & 63;
+        for (int e = threadIdx.x >> 6; e < E; e += 16) {
+            const int mine = cnt[e];
+            int rank = 0;
+            for (int q = lane; q < (E + 63) / 64 * 64; q += 64)  // (counts behind the last expert are zero, and not before any: q > e)
+                rank += __popcll(__ballot(cnt[q] > mine || (cnt[q] == mine && q < e)));
+            const int turn = rank >> 3, whole = E >> 3, more = E & 7;
+            const bool back = turn & 1, last_back = whole & 1;
+            const int share = back ? 7 - (rank & 7) : rank & 7;
+            const int extra = last_back ? max(share - (8 - more), 0) : min(share, more);  // experts of the last turn in the shares before
+            if (lane == 0) pos[e] = share * whole + extra + turn;
+        }
+    }
+    __syncthreads();
     // Thread e lays out expert e: its first slot and first tile are prefix sums over the experts before it, then it writes its
     // own tiles.
     // ceil(cnt / BM) tiles that differ by at most a fragment: 140 rows with BM = 128 become 80 + 60 rather
     // than 128 + 12, and the GEMM skips the row fragments a tile does not have.
     for (int e = threadIdx.x; e < E; e += 1024) {
         int o = 0, nt = 0, total = 0;
+        const int at_e = pos[e];
         for (int q = 0; q < E4; ++q) {
-            const int4 c = cnt4[q], t = tiles4[q];
-            auto add = [&](int n, int tq, int i) {
-                if (4 * q + i < e) {
-                    o += n;
-                    nt += tq;
-                }
+            const int4 c = cnt4[q], at = pos4[q], t = tiles4[q];
+            auto add = [&](int n, int place, int tq, int i) {
+                if (4 * q + i < e) o += n;
+                if (place < at_e) nt += tq;
                 total += tq;
             };
-            add(c.x, t.x, 0), add(c.y, t.y, 1), add(c.z, t.z, 2), add(c.w, t.w, 3);
+            add(c.x, at.x, t.x, 0), add(c.y, at.y, t.y, 1), add(c.z, at.z, t.z, 2), add(c.w, at.w, t.w, 3);
         }
         off[e] = o;
         p.offsets[e] = o;
@@ -130,7 +151,7 @@ __device__ __forceinline__ void moe_plan_block(const int *__restrict__ sel, int 
         if (e == E - 1) {
             off[E] = o + cnt[e];
             p.offsets[E] = o + cnt[e];
-            *p.n_tiles = nt;
+            *p.n_tiles = total;
         }
     }
     __syncthreads();

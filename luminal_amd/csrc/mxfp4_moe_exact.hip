@@ -558,19 +558,19 @@ static lhip_status launch_exact_gemm(const MoeExactArgs &a, int col_blocks, int 
 // read and expanded once), else 64, or 96 (`tall`, mxfp4_moe_tall.hip), cut into equal parts for experts with more.
 // A stage of the 96-row kernel takes longer when its workgroup is alone on a compute unit, and two of its workgroups end no
 // sooner than two of 64 rows; it wins with the third.  So it is taken with two workgroups a compute unit in the first product and one
-// and a half in the second, and there where its tiles are fewer (more than 50 rows an expert: many are two tiles of 64) or
-// hold one fragment of 32 (less than 28).  Measured on 16 layers (4 to 128 experts, H of 1024 to 4096, I of 512 to 14336) at 24 to
-// 384 rows an expert: over 64 rows everywhere 0.98, the better of both 0.97, 96 rows everywhere 1.05.  us, 64 / 96 rows: 32 experts of
-// 2880 x 2880, top 4, T = 192 115 / 108, T = 256 121 / 127, T = 384 142 / 146, T = 512 180 / 153, T = 1024 261 / 233; 8 experts of 4096 x
-// 14336, top 2, T = 128 218 / 314, T = 384 331 / 440; 64 of 2048 x 1408, top 6, T = 512 98 / 106, T = 683 140 / 115; 12 of 2880 x 2880, top 3,
-// T = 192 80 / 85.  16- / 32- / 64-row tiles of the first: T = 32 87 / 94 / 110, T = 64 90 / 95 / 110, T = 128 132 / 99 / 114.
+// and a half in the second, and there where its tiles are fewer (more than 46 rows an expert: some, then many are two tiles of 64) or
+// hold one fragment of 32 (less than 30).  Measured on 16 layers (4 to 128 experts, H of 1024 to 4096, I of 512 to 14336) at 24 to
+// 384 rows an expert: over 64 rows everywhere 0.974, the better of both 0.967, 96 rows everywhere 1.046.  us, 64 / 96 rows: 32 experts of
+// 2880 x 2880, top 4, T = 192 115 / 106, T = 256 120 / 116, T = 384 142 / 142, T = 512 180 / 147, T = 1024 263 / 224; 8 experts of 4096 x
+// 14336, top 2, T = 128 222 / 299, T = 384 329 / 445; 64 of 2048 x 1408, top 6, T = 512 99 / 97, T = 683 135 / 111; 12 of 2880 x 2880, top 3,
+// T = 192 79 / 85.  16- / 32- / 64-row tiles of the first: T = 32 87 / 94 / 110, T = 64 90 / 95 / 110, T = 128 132 / 99 / 114.
 static inline int exact_tile_fragments(int R, int E, int H, int I, bool tall) {
     const int avg = (R + E - 1) / E;
     const int need = avg + 2 * static_cast<int>(sqrtf(static_cast<float>(avg)) + 0.5f);
     if (need <= 32) return need <= 16 ? 1 : 2;
     const int64_t tiles = R / kTallRows + E / 2 > E ? R / kTallRows + E / 2 : E;  // about as many as there will be
     const bool filled = tiles * ((I + 127) / 128) >= 2 * 256 && tiles * ((H + 255) / 256) * 2 >= 3 * 256;
-    return tall && filled && (avg < 28 || avg > 50) ? kTallRows / 16 : 4;
+    return tall && filled && (avg < 30 || avg > 46) ? kTallRows / 16 : 4;
 }
 
 lhip_status moe_exact_forward(const uint8_t *gu, const uint8_t *dn, const __bf16 *x, const int32_t *sel_dev,
@@ -617,6 +617,10 @@ lhip_status moe_exact_forward(const uint8_t *gu, const uint8_t *dn, const __bf16
     const int max_tiles = (R / BM + E + 7) / 8 * 8;
     w.plan.max_tiles = max_tiles;
     w.plan.tiles_per_xcd = max_tiles / 8;
+    // Experts listed by their rows, so that the XCDs have about as many: over own order, where these tiles are taken and an expert has more
+    // than 50 rows on average, 0.986 (32 experts of 2880 x 2880), 0.989 (64 of 2048 x 1024, 48 of 4096 x 1024), 0.996 to 1.003 (16 of 4096 x
+    // 4096, 64 and 60 of 2048 x 1408, 128 of 2048 x 768); at 24 and 28 rows 0.885 to 1.02.
+    w.plan.by_rows = BM == kTallRows;
     w.plan.fragment = BM == kTallRows ? 32 : 16;
     hipLaunchKernelGGL(moe_plan_kernel, dim3(1), dim3(1024), 0, s, sel_dev, R, E, BM, w.plan);
     LHIP_CHECK_LAUNCH();

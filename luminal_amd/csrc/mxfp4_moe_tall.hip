@@ -18,7 +18,7 @@
 //     241 at T = 1024 and 174 at T = 512.
 // A stage takes longer when the workgroup is alone on its CU (4 experts of 2048 x 2048 at 32 rows, 64 workgroups: 58 us, by 64-row tiles
 // 47), so this is taken only where there are enough (exact_tile_fragments).  Measured, us per layer, 64-row tiles of mx_moe_gemm_exact_kernel -> this: T = 192 117 ->
-// 110, T = 512 186 -> 158, T = 1024 274 -> 236 (860 TFLOP/s of useful work), T = 2048 438 -> 401.
+// 110, T = 512 184 -> 147, T = 1024 266 -> 231 (880 TFLOP/s of useful work), T = 2048 449 -> 409.
 #include <algorithm>
 
 #include "mxfp4_moe_exact_device.h"

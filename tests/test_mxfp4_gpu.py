@@ -346,10 +346,11 @@ def test_moe_rows_per_expert_at_the_edges_of_the_96_row_tiles(oracle, e, h, i):
     check_stages_exact(layer, xf, w_gu, w_dn, sel, wts, y, tokens=others)
 
 
-@pytest.mark.parametrize("e,h,i,rows", [(512, 96, 128, 26), (511, 128, 96, 51), (397, 160, 192, 52)])
+@pytest.mark.parametrize("e,h,i,rows", [(516, 96, 128, 29), (511, 128, 96, 47), (397, 160, 192, 52)])
 def test_moe_random_rows_per_expert_in_96_row_tiles(oracle, e, h, i, rows):
     """Routed at random, on both sides of the rows per expert between which tiles of 64 rows are taken instead, and numbers of
-    experts that are no multiple of the eight shares of the tile list (or of the four counts a thread reads at once)."""
+    experts that are no multiple of the eight shares that experts are dealt to by their rows (after an even and an odd number of
+    whole turns), of the four counts a thread reads at once or of the 64 a wave ranks by."""
     layer, w_gu, w_dn = make_layer(oracle, e, h, i, seed=e)
     t = e * rows // 2
     xf, sel, wts, y = run_layer(oracle, layer, t, h, e, 2, seed=rows, scale=0.05)
