@@ -214,6 +214,8 @@ __device__ __forceinline__ float4 merged_attention_piece(const GemvFuse &f, int 
     return make_float4(num.x * inv, num.y * inv, num.z * inv, num.w * inv);
 }
 
+constexpr int kStage = 4;  // pieces of four activations a thread stages from registers (ONE)
+
 struct Located {
     const int8_t *qs;
     const unsigned short *ds;
@@ -233,7 +235,7 @@ __device__ __forceinline__ Located locate(const GemvGroup &p, int gg) {
     return Located{p.qs[w], p.ds[w], p.y[w], p.n[w], (gg - before) * R};
 }
 
-template <int R, int S, int W, int PRO, int EPI>
+template <int R, int S, int W, int PRO, int EPI, bool ONE>
 __global__ __launch_bounds__(W * 64) void q8_gemv_fused_kernel(const int8_t *qs0, const unsigned short *ds0,
                                                                const float *__restrict__ x, const float *aux, int n0,
                                                                int end0, int k, int n_groups, int grid_blocks, float eps,
@@ -262,14 +264,55 @@ __global__ __launch_bounds__(W * 64) void q8_gemv_fused_kernel(const int8_t *qs0
     // EPI_ADD: the residual of a row group is requested together with the group's first weight step, i.e. ahead
     // of loads the pipeline waits for anyway.  Read at the group's end instead, it would be the youngest load in
     // flight and waiting for it would drain the prefetched next step every time (wait counts retire in order).
+    // (Without a branch around it, lanes past the group's rows re-reading its last: a load that some waves skip makes every
+    // later wait count short by one.)
     auto residual_of = [&](const Located &l, bool live) -> float {
-        const int row = l.row0 + static_cast<int>(lane);
-        return (EPI == EPI_ADD && live && lane < static_cast<unsigned>(R) && row < l.n) ? residual[row] : 0.f;
+        if (EPI != EPI_ADD) return 0.f;
+        return residual[live ? min(l.row0 + min(static_cast<int>(lane), R - 1), l.n - 1) : 0];
     };
     float res_cur = 0.f, res_next = 0.f;
 
+    auto located = [&](int gg) { return ONE ? Located{qs0, ds0, p.y[0], n0, gg * R} : locate<R>(p, gg); };
+    auto next = [&](int &gg, int &cc) {
+        if (++cc == chunks) {
+            cc = 0;
+            gg += total_waves;
+        }
+    };
+    auto issue = [&](StepBuf<R, S> &buf, int gg, int cc, bool live) {
+        const Located l = located(live ? gg : 0);
+        if (EPI == EPI_ADD && cc == 0) res_next = residual_of(l, live);
+        load_step(buf, l.qs, l.ds, l.row0, l.n, k, cc * S, lane, live);
+    };
+
+    // One weight, and activations that fit four pieces a thread (ONE): the activations are requested first, then the wave's
+    // first two steps of weights.  Loads retire in order, so the staging waits for its own requests only while both steps are on
+    // their way; with the second step requested behind the staging barrier, the memory system idles from the end of the first
+    // until the barrier and a round trip.  Measured, us a launch in a chain of layers: 6144 x 4096 with the norm 9.2 -> 8.7,
+    // 4096 x 4096 6.5 -> 6.15, 28672 x 4096 with the norm 25.4 -> 23.5, 4096 x 14336 14.4 -> 13.3.
+    const int k4 = k >> 2;
+    const float4 *x4 = reinterpret_cast<const float4 *>(x);
+    const float4 *g4 = reinterpret_cast<const float4 *>(norm_w);
+    auto source = [](int i) { return (i & ~255) | ((i & 63) << 2) | ((i >> 6) & 3); };
     StepBuf<R, S> a, b;
-    {
+    float4 xr[kStage], gr[kStage];
+    int g1 = wave_global, c1 = 0;  // the step behind the one being computed
+    next(g1, c1);
+    if constexpr (ONE) {
+#pragma unroll
+        for (int j = 0; j < kStage; ++j) {
+            const int i = static_cast<int>(threadIdx.x) + j * W * 64;
+            const int src = i < k4 ? source(i) : 0;
+            xr[j] = x4[src];
+            if (NORM) gr[j] = g4[src];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        load_step(a, qs0, ds0, T > 0 ? wave_global * R : 0, n0, k, 0, lane, T > 0);
+        res_cur = residual_of(located(wave_global), T > 0);
+        __builtin_amdgcn_sched_barrier(0);
+        issue(b, g1, c1, T > 1);
+        __builtin_amdgcn_sched_barrier(0);
+    } else {
         const int g0 = wave_global < n_groups ? wave_global : 0;
         if (g0 < end0) {  // wave-uniform
             load_step(a, qs0, ds0, g0 * R, n0, k, 0, lane, T > 0);
@@ -285,27 +328,9 @@ __global__ __launch_bounds__(W * 64) void q8_gemv_fused_kernel(const int8_t *qs0
     // are multiplied by 1/sqrt(mean(x^2) + eps) at the end: the sum of squares rides on the staging loads and
     // is published by the staging barrier.
     {
-        const float4 *x4 = reinterpret_cast<const float4 *>(x);
-        const float4 *g4 = reinterpret_cast<const float4 *>(norm_w);
-        const int k4 = k >> 2;
         float ss = 0.f;
-        int n_active = 0;
-        if (PRO == PRO_MERGE) {  // the key ranges the attention launch cut this position's context into
-            const int n_keys = min(*f.pos + 1, f.max_seq);
-            const int eff = dec_active_splits(n_keys, f.n_splits, true);
-            const int chunk = (n_keys + eff - 1) / eff;
-            n_active = (n_keys + chunk - 1) / chunk;
-        }
-#pragma unroll 4
-        for (int i = threadIdx.x; i < k4; i += W * 64) {
-            const int src = (i & ~255) | ((i & 63) << 2) | ((i >> 6) & 3);
-            float4 v;
-            if (PRO == PRO_MERGE)
-                v = merged_attention_piece(f, src, n_active);
-            else
-                v = x4[src];
+        auto stage = [&](int i, float4 v, const float4 &g) {
             if (NORM) {
-                const float4 g = g4[src];
                 // spelled out, so that every kernel that takes this sum rounds it the same way
                 ss = fmaf(v.x, v.x, ss);
                 ss = fmaf(v.y, v.y, ss);
@@ -314,6 +339,23 @@ __global__ __launch_bounds__(W * 64) void q8_gemv_fused_kernel(const int8_t *qs0
                 v = make_float4(v.x * g.x, v.y * g.y, v.z * g.z, v.w * g.w);
             }
             xs4[i] = v;
+        };
+        if constexpr (ONE) {
+#pragma unroll
+            for (int j = 0; j < kStage; ++j) {
+                const int i = static_cast<int>(threadIdx.x) + j * W * 64;
+                if (i < k4) stage(i, xr[j], gr[j]);
+            }
+        } else if constexpr (PRO == PRO_MERGE) {  // the key ranges the attention launch cut this position's context into
+            const int n_keys = min(*f.pos + 1, f.max_seq);
+            const int eff = dec_active_splits(n_keys, f.n_splits, true);
+            const int chunk = (n_keys + eff - 1) / eff;
+            const int n_active = (n_keys + chunk - 1) / chunk;
+#pragma unroll 4
+            for (int i = threadIdx.x; i < k4; i += W * 64) stage(i, merged_attention_piece(f, source(i), n_active), float4{});
+        } else {
+#pragma unroll 4
+            for (int i = threadIdx.x; i < k4; i += W * 64) stage(i, x4[source(i)], NORM ? g4[source(i)] : float4{});
         }
         if (NORM) {
             ss = wave_sum(ss);
@@ -338,19 +380,8 @@ __global__ __launch_bounds__(W * 64) void q8_gemv_fused_kernel(const int8_t *qs0
     for (int r = 0; r < R; ++r) acc[r] = 0.f;
 
     int t = 0, g = wave_global, c = 0;
-    auto next = [&](int &gg, int &cc) {
-        if (++cc == chunks) {
-            cc = 0;
-            gg += total_waves;
-        }
-    };
-    auto issue = [&](StepBuf<R, S> &buf, int gg, int cc, bool live) {
-        const Located l = locate<R>(p, live ? gg : 0);
-        if (EPI == EPI_ADD && cc == 0) res_next = residual_of(l, live);
-        load_step(buf, l.qs, l.ds, l.row0, l.n, k, cc * S, lane, live);
-    };
     auto finish_group = [&](int gg) {
-        const Located l = locate<R>(p, gg);
+        const Located l = located(gg);
         float sum[R];
 #pragma unroll
         for (int r = 0; r < R; ++r) {
@@ -382,24 +413,28 @@ __global__ __launch_bounds__(W * 64) void q8_gemv_fused_kernel(const int8_t *qs0
         }
     };
 
-    while (true) {
-        int g1 = g, c1 = c;
-        next(g1, c1);
-        issue(b, g1, c1, t + 1 < T);
-        __builtin_amdgcn_sched_barrier(0);
-        compute_step(a, xs4, c * S, lane, acc);
+    if constexpr (!ONE) issue(b, g1, c1, T > 1);
+    __builtin_amdgcn_sched_barrier(0);
+    // Whether a step was the wave's last; otherwise on to the next.
+    auto done = [&]() {
         if (c == chunks - 1) finish_group(g);
-        if (++t >= T) break;
+        if (++t >= T) return true;
         g = g1;
         c = c1;
         next(g1, c1);
+        return false;
+    };
+    compute_step(a, xs4, c * S, lane, acc);
+    if (done()) return;
+    while (true) {
         issue(a, g1, c1, t + 1 < T);
         __builtin_amdgcn_sched_barrier(0);
         compute_step(b, xs4, c * S, lane, acc);
-        if (c == chunks - 1) finish_group(g);
-        if (++t >= T) break;
-        g = g1;
-        c = c1;
+        if (done()) return;
+        issue(b, g1, c1, t + 1 < T);
+        __builtin_amdgcn_sched_barrier(0);
+        compute_step(a, xs4, c * S, lane, acc);
+        if (done()) return;
     }
 }
 
@@ -520,22 +555,31 @@ static void choose(int n, int k, int *rows_per_wave, int *k_unroll, int *blocks_
     }
 }
 
-template <int R, int S, int W, int PRO, int EPI>
-static lhip_status launch_fused(const GemvGroup &p, const GemvFuse &f, const float *x, int k, int n_groups,
-                                int blocks_per_cu, hipStream_t s) {
+template <int R, int S, int W, int PRO, int EPI, bool ONE>
+static lhip_status launch_fused_form(const GemvGroup &p, const GemvFuse &f, const float *x, int k, int n_groups,
+                                     int blocks_per_cu, hipStream_t s) {
     int grid = (n_groups + W - 1) / W;
     const int cap = kNumCUs * blocks_per_cu;
     if (grid > cap) grid = cap;
     const size_t lds_bytes = static_cast<size_t>(k) * sizeof(float);
     static LdsOptIn opt;  // with the static reduction array: beyond the default limit (K = 16384)
-    if (lhip_status st = lds_opt_in(opt, reinterpret_cast<const void *>(q8_gemv_fused_kernel<R, S, W, PRO, EPI>), lds_bytes,
+    if (lhip_status st = lds_opt_in(opt, reinterpret_cast<const void *>(q8_gemv_fused_kernel<R, S, W, PRO, EPI, ONE>), lds_bytes,
                                     lds_bytes + W * sizeof(float) > 64 * 1024))
         return st;
-    hipLaunchKernelGGL((q8_gemv_fused_kernel<R, S, W, PRO, EPI>), dim3(static_cast<unsigned>(grid)), dim3(W * 64),
+    hipLaunchKernelGGL((q8_gemv_fused_kernel<R, S, W, PRO, EPI, ONE>), dim3(static_cast<unsigned>(grid)), dim3(W * 64),
                        lds_bytes, s, p.qs[0], p.ds[0], x, PRO == PRO_NORM ? f.norm_w : f.residual, p.n[0], p.group_end[0], k, n_groups,
                        grid, f.eps, p, f);
     LHIP_CHECK_LAUNCH();
     return LHIP_OK;
+}
+
+template <int R, int S, int W, int PRO, int EPI>
+static lhip_status launch_fused(const GemvGroup &p, const GemvFuse &f, const float *x, int k, int n_groups,
+                                int blocks_per_cu, hipStream_t s) {
+    // (group_end[1] is INT_MAX for one weight only)
+    if (PRO != PRO_MERGE && p.group_end[1] == INT_MAX && k <= kStage * 4 * W * 64)
+        return launch_fused_form<R, S, W, PRO, EPI, PRO != PRO_MERGE>(p, f, x, k, n_groups, blocks_per_cu, s);
+    return launch_fused_form<R, S, W, PRO, EPI, false>(p, f, x, k, n_groups, blocks_per_cu, s);
 }
 
 template <int R, int S, int W>
@@ -562,7 +606,7 @@ static lhip_status dispatch_fused(int r, int sl, int w, int bpc, bool norm, int 
 #define LHIP_CASE(R, S, W) \
     if (r == R && sl == S && w == W) return launch_fused_variant<R, S, W>(norm, epi, p, f, x, k, n_groups, bpc, s);
     LHIP_CASE(2, 4, 4) LHIP_CASE(1, 2, 4) LHIP_CASE(2, 2, 4) LHIP_CASE(1, 1, 4) LHIP_CASE(2, 1, 4)
-    LHIP_CASE(1, 2, 16) LHIP_CASE(2, 2, 8) LHIP_CASE(1, 1, 16) LHIP_CASE(2, 1, 8)
+    LHIP_CASE(1, 2, 16) LHIP_CASE(2, 2, 8) LHIP_CASE(1, 1, 16) LHIP_CASE(2, 1, 8) LHIP_CASE(1, 2, 8)
 #undef LHIP_CASE
     return LHIP_ERR_UNSUPPORTED;
 }
@@ -577,11 +621,21 @@ static void choose_fused(int64_t n_total, int k, int pro, int epi, int *r, int *
     }
     const bool pairs = epi == EPI_SWIGLU;
     *sl = slices >= 2 ? 2 : 1;
-    if (fit >= 3) {
-        // (measured, q|k|v = 6144 rows at K = 4096: four workgroups per CU 7.25 us against 7.55 with three when nothing
-        // precedes the products; with the norm prologue, which every workgroup pays for, three or two: decode 481 tok/s
-        // against 474 with four; the 4096 rows of o: 6.15 with three, 6.25 with four)
-        *r = pairs ? 2 : 1, *w = 4, *bpc = pairs ? 2 : (pro == PRO_NONE && n_total > 4096 ? 4 : 3);
+    // Every workgroup stages (and with the norm sums) the activations, so the fewer workgroups hold the waves the better, as long
+    // as the waves' first two steps keep the memory system busy.  Measured, us a launch, up to 6144 rows two rows a wave in one
+    // workgroup of four waves a CU / one row in one of eight / in two of eight / in three of four (what was taken before):
+    //   norm,  K = 4096: 4096 rows 5.7 / 5.9 / 6.2 / 6.7, 6144 7.3 / 7.5 / 7.7 / 8.4, 12288 11.7 / 11.4 / 11.6 / 12.4
+    //   plain, K = 4096: 4096 rows 5.5 / 5.7 / 5.5 / 5.6, 6144 7.1 / 6.8 / 6.8 / 7.1, 12288 11.6 / 10.9 / 10.8 / 11.1
+    //   K = 8192, norm and plain: 4096 rows 9.4 / 8.9 / 9.4 / 12.1 and 9.0 / 8.1 / 8.5 / 9.6
+    //   K = 2048, norm: 4096 rows 4.7 / 4.8 / 4.8 / 4.6, 6144 5.5 / 5.6 / 5.6 / 5.5 (level)
+    if (*sl == 2 && k > 4096 && k <= 8192) {
+        *r = pairs ? 2 : 1, *w = 8, *bpc = 1;
+    } else if (*sl == 2 && k == 4096 && pro == PRO_NORM && n_total >= 2048) {
+        *r = pairs || n_total <= 6144 ? 2 : 1, *w = n_total <= 6144 ? 4 : 8, *bpc = 1;
+    } else if (*sl == 2 && k == 4096 && !pairs && n_total > 4096) {
+        *r = 1, *w = 8, *bpc = 2;
+    } else if (fit >= 3) {
+        *r = pairs ? 2 : 1, *w = 4, *bpc = pairs ? 2 : 3;
     } else {
         *r = pairs ? 2 : 1, *w = pairs ? 8 : 16, *bpc = 1;
     }

@@ -160,3 +160,27 @@ def test_argument_errors():
     assert lib.lhip_q8_0_matvec_fused_f32_cfg(wp, yp, n, 1, x.data_ptr(), 1024, None, 0.0, None, 2, 1, 1, 4, 1,
                                               s) == capi.LHIP_ERR_UNSUPPORTED  # pairs need two rows per wave
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("k", [1024, 3072, 4096, 8192, 16384])
+@pytest.mark.parametrize("n", [1, 7, 1030, 4100, 6145, 16390])
+def test_one_weight_requests_two_steps_ahead_and_gives_the_grouped_launch_s_bits(n, k):
+    """A launch of one weight requests its first two steps before the activations are staged; a launch of several keeps the
+    staging between them.  Waves with no step, one, two and more; the row arithmetic is the same, so are the bits."""
+    w, _ = make(n, k, n + k)
+    other, _ = make(3, k, 1)
+    x = torch.from_numpy(synth.activations(1, k, seed=n)).to(DEV).reshape(k)
+    g = 1 + 0.1 * torch.sin(torch.arange(k, device=DEV, dtype=torch.float32))
+    res = torch.cos(torch.arange(n, device=DEV, dtype=torch.float32))
+    for cfg in (None, (1, 1, 4, 3), (2, 1, 8, 1), (1, 1, 16, 1)):
+        for norm in (None, g):
+            one, grouped, extra = (torch.full((r,), float("nan"), device=DEV) for r in (n, n, 3))
+            FusedMatvec([w], [one], norm_weight=norm, eps=1e-5, cfg=cfg).run(x)
+            FusedMatvec([w, other], [grouped, extra], norm_weight=norm, eps=1e-5, cfg=cfg or (1, 1, 4, 3)).run(x)
+            if norm is None or cfg is not None:  # (the sum of squares depends on the workgroup's size)
+                assert torch.equal(one, grouped)
+        added = torch.full((n,), float("nan"), device=DEV)
+        FusedMatvec([w], [added], residual=res, epilogue=FusedMatvec.EPI_ADD, cfg=cfg).run(x)
+        plain = torch.empty(n, device=DEV)
+        FusedMatvec([w], [plain], cfg=cfg).run(x)
+        assert torch.equal(added, plain + res)
