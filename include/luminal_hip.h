@@ -110,14 +110,14 @@ lhip_status lhip_q8_0_matmul_f32(const void *planar_dev, const float *x_dev, flo
  * exact.  The f16 form is the f32 form's sum on the widened inputs, rounded once: bit for bit up to 64 rows and for small
  * products, within the order of the f32 additions above.  Any m >= 1.
  * LHIP_ERR_UNSUPPORTED unless K % 512 == 0, N % 4 == 0, x 16-byte and y 16-byte (f16: 8-byte) aligned.
- * lhip_q8_0_matmul_f32 and lhip_q8_0_matmul_f16 take this form by themselves from a few rows on (two for N*K >=
- * 2^28 codes, three from 2^25, four from 2^23, six below: the measured crossovers with the matvec form) where those
- * conditions hold, and may then keep partial sums in the library's scratch array, see the note on overlapping calls at
+ * lhip_q8_0_matmul_f32 and lhip_q8_0_matmul_f16 take this form by themselves from a few rows on (six for N*K < 2^23 codes;
+ * four above, f16 below 2^27 codes five, and fewer where K is so long that their activations do not fit a compute unit's LDS: the
+ * measured crossovers with matvecs, which also stream the weights once for up to five rows) where those conditions hold, and may then keep partial sums in the library's scratch array, see the note on overlapping calls at
  * lhip_q8_0_matmul_bf16: every shape for which lhip_q8_0_matmul_workspace_nbytes is not zero.  Which shapes those are may
  * change from one version of the library to the next (products whose strips fill the chip, e.g. 256 x 14336 x 4096 and 300 x
  * 28672 x 4096, kept nothing there once and do now): a program that overlaps calls asks, or uses the _ws forms.  For every other K >= 256 and every N they keep nothing outside their outputs: the matrix cores
- * without K slices where the rows are many enough for that, else one matvec per row; the _ws forms below with a workspace
- * slice K there and take the matrix cores where they end before the matvecs: from three rows on for the largest matrices, two
+ * without K slices where the rows are many enough for that, else matvecs; the _ws forms below with a workspace
+ * slice K there and take the matrix cores where they end before the matvecs: from five rows on for the largest matrices, two
  * to three hundred for the smallest.  The _cfg entry never does. */
 lhip_status lhip_q8_0_matmul_f32_gemm(const void *planar_dev, const float *x_dev, float *y_dev, int64_t m, int64_t n,
                                       int64_t k, void *stream);
@@ -149,7 +149,8 @@ lhip_status lhip_q8_0_matmul_f32_cfg(const void *planar_dev, const float *x_dev,
  *   grid[1] = m;   // activation rows, 1..65535
  *   hipModuleLaunchKernel(fn, grid[0], grid[1], grid[2], block[0], block[1], block[2],
  *                         lds_bytes, stream, args, NULL);
- * gives the bits of the library call.  It touches no device.  f16 != 0 selects the f16
+ * gives the bits of the library call (which for several rows or a long ragged K may launch a kernel that is not in the
+ * module, with the same arithmetic).  It touches no device.  f16 != 0 selects the f16
  * activation type.  kernel_name receives a NUL-terminated string (64 bytes are enough). */
 lhip_status lhip_q8_0_gemv_kernel_plan(int64_t n, int64_t k, int f16, char *kernel_name, size_t kernel_name_cap,
                                        uint32_t grid[3], uint32_t block[3], uint32_t *lds_bytes);

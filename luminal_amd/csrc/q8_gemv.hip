@@ -24,19 +24,24 @@
 
 #include "common.h"
 #include "q8_gemm_rows.h"
+#include "q8_gemv_rows.h"
 
 namespace lhip {
 // From this many activation rows on the plain operators take the matrix-core form with f32-accurate operands (q8_gemm_split_launch,
-// q8_gemm_skinny.hip) where the shape allows it: the weights are then streamed once per 64 rows instead of once per row.  That form
-// has a fixed cost (its launch, a reduce launch where K is sliced, staging) that a matvec pass over a small matrix stays under.
-// Measured, matvecs / matrix cores, us, f32 and f16: 1024 x 4096 at five rows 5.9 / 6.9 and 5.2 / 6.5, at six 6.7 / 7.0 and 5.8 / 6.5; 4096 x
-// 4096 at two rows 8.9 / 11.1 and 7.7 / 10.6, at three 12.3 / 11.1 and 10.4 / 10.7, at four 15.9 / 11.2 and 13.0 / 10.7; 14336 x 4096 at
-// two rows 21.1 / 18.8 and 20.1 / 17.9, at three 31.1 / 18.9 and 29.7 / 18.0; 128256 x 4096 at two rows 169 / 128 and 168 / 118.  (The
-// lines were drawn when the matrix cores took 12.7 us at three rows of 4096 x 4096 and 21.5 at two of 14336 x 4096; since its strips
-// follow N the crossing lies up to a row below them there.)
-static int split_min_rows(int64_t n, int64_t k) {
+// q8_gemm_skinny.hip) where the shape allows it: the weights are then streamed once per 64 rows and multiplied on the matrix cores.
+// That form has a fixed cost (its launch, a reduce launch where K is sliced, staging) that matvecs of a few rows, which also stream
+// the weights once (q8_gemv_rows.hip) and pay 16 vector instructions per row and 16 codes, stay under.  Measured, matvecs / matrix
+// cores, us, f32 and f16: 4096 x 4096 at three rows 7.1 / 11.1 and 6.9 / 10.7, at four (f16 only) 7.5 / 11.0; 14336 x 4096 at three
+// rows 16.6 / 19.4 and 16.0 / 18.2, at four 18.1 / 20.0 and 18.3 / 18.6; 97184 x 4096 at three 82 / 115 and 88 / 99; 600 x 1024 at
+// five rows 3.9 / 5.8 either way.  Where the rows' activations do not fit the LDS of one pass, the line is two rows lower at most:
+// 4096 x 14336 f32 at three rows 27.8 / 22.3.
+static int split_min_rows(int64_t n, int64_t k, bool f16) {
     const int64_t codes = n * k;
-    return codes >= (int64_t{256} << 20) ? 2 : codes >= (int64_t{32} << 20) ? 3 : codes >= (int64_t{8} << 20) ? 4 : 6;
+    if (codes < int64_t{8} << 20) return 6;
+    const int rows = f16 && codes < int64_t{128} << 20 ? 4 : 3, fit = q8_gemv_rows_per_pass(k, f16);
+    if (rows <= fit) return rows + 1;
+    if (fit >= 2) return fit + 1;
+    return codes >= (int64_t{256} << 20) ? 2 : codes >= (int64_t{32} << 20) ? 3 : 4;
 }
 
 // What m matvecs of a K outside the streaming kernel's shapes take, us, and an upper bound of what q8_gemm_rows.hip takes over K slices
@@ -81,11 +86,14 @@ static double rows_sliced_us(int64_t m, int64_t n, int64_t k, bool f16) {
 // `plan` (not for SIZE_MAX): what the answer was worked out with, for the launch; kind kNone where it was not.
 static bool on_matrix_cores(int64_t m, int64_t n, int64_t k, const void *x, const void *y, bool f16, size_t room_floats,
                             RowsPlan *plan = nullptr) {
-    if (q8_gemm_split_supports(static_cast<int>(n), static_cast<int>(k), x, y, f16)) return m >= split_min_rows(n, k);
+    if (q8_gemm_split_supports(static_cast<int>(n), static_cast<int>(k), x, y, f16)) return m >= split_min_rows(n, k, f16);
     if (k < 256 || !aligned(x, 16)) return false;
     const int64_t codes = n * k;
     const int64_t min_rows = codes >= (int64_t{32} << 20) ? 3 : codes >= (int64_t{16} << 20) ? 6 : codes >= (int64_t{8} << 20) ? 8 : 12;
     if (m < (f16 ? min_rows * 5 / 4 : min_rows)) return false;
+    // up to four rows of one pass over the weights: 10944 x 3552 f32 at four rows 24.7 on the matrix cores, 16.4 as matvecs, f16 21.4 and
+    // 16.8; at five and more of such sizes within a tenth of each other
+    if (m <= 4 && m <= q8_gemv_rows_per_pass(k, f16)) return false;
     bool room = room_floats == SIZE_MAX;
     if (!room) {
         RowsPlan plans[2];
@@ -663,6 +671,20 @@ static lhip_status matrix_cores(const void *planar, const void *x, void *y, int6
                                 plan && plan->kind != RowsPlan::kNone ? plan : nullptr);
 }
 
+// Matvecs of several rows a pass over the weights (q8_gemv_rows.hip); the passes are the grid's y dimension.
+static lhip_status rows_matvecs(const void *planar, const void *x, void *y, int64_t m, int64_t n, int64_t k, bool f16, void *stream) {
+    auto *base = static_cast<const uint8_t *>(planar);
+    const int64_t size = f16 ? 2 : 4;
+    for (int64_t m0 = 0; m0 < m; m0 += kMaxGridRows) {
+        const int mc = static_cast<int>(m - m0 < kMaxGridRows ? m - m0 : kMaxGridRows);
+        if (lhip_status st = q8_gemv_rows_launch(reinterpret_cast<const int8_t *>(base), reinterpret_cast<const __half *>(base + q8_scale_offset(n, k)),
+                                                 static_cast<const uint8_t *>(x) + m0 * k * size, static_cast<uint8_t *>(y) + m0 * n * size, mc,
+                                                 static_cast<int>(n), static_cast<int>(k), f16, as_stream(stream)))
+            return st;
+    }
+    return LHIP_OK;
+}
+
 extern "C" {
 
 lhip_status lhip_q8_0_matmul_f32_cfg(const void *planar_dev, const float *x_dev, float *y_dev, int64_t m, int64_t n,
@@ -689,6 +711,7 @@ lhip_status lhip_q8_0_matmul_f32(const void *planar_dev, const float *x_dev, flo
     if (on_matrix_cores(m, n, k, x_dev, y_dev, false, 0, &plan))
         return matrix_cores(planar_dev, x_dev, y_dev, m, n, k, false, stream,
                             !q8_gemm_split_supports(static_cast<int>(n), static_cast<int>(k), x_dev, y_dev, false), nullptr, 0, &plan);
+    if (q8_gemv_rows_pays(m, n, k, false)) return rows_matvecs(planar_dev, x_dev, y_dev, m, n, k, false, stream);
     int r, u, b, w;
     choose(static_cast<int>(n), static_cast<int>(k), &r, &u, &b, &w);
     return lhip_q8_0_matmul_f32_cfg(planar_dev, x_dev, y_dev, m, n, k, r, u, b, w, stream);
@@ -728,6 +751,7 @@ lhip_status lhip_q8_0_matmul_f16(const void *planar_dev, const void *x_f16_dev, 
     if (on_matrix_cores(m, n, k, x_f16_dev, y_f16_dev, true, 0, &plan))
         return matrix_cores(planar_dev, x_f16_dev, y_f16_dev, m, n, k, true, stream,
                             !q8_gemm_split_supports(static_cast<int>(n), static_cast<int>(k), x_f16_dev, y_f16_dev, true), nullptr, 0, &plan);
+    if (q8_gemv_rows_pays(m, n, k, true)) return rows_matvecs(planar_dev, x_f16_dev, y_f16_dev, m, n, k, true, stream);
     auto *base = static_cast<const uint8_t *>(planar_dev);
     int r, u, b, w;
     choose(static_cast<int>(n), static_cast<int>(k), &r, &u, &b, &w);

@@ -1,0 +1,104 @@
+// Q8_0 matvecs of a few activation rows and of any K (the kernel: q8_gemv_rows_device.h): launch shapes and launches.
+#include "q8_gemv_rows.h"
+#include "q8_gemv_rows_device.h"
+
+namespace lhip {
+
+constexpr int kRowsWaves = 8, kRowsMax = 5;           // waves of a workgroup; activation rows of a pass
+constexpr size_t kRowsLds = size_t{160} * 1024;       // of a CU
+
+// The launch shape: weight rows and slices of 1024 of K a step, activation rows of a pass, workgroups a CU.
+struct GemvRowsShape {
+    int r, s, mr, bpc;
+    size_t lds;
+};
+
+static int rows_slices(int64_t k) { return static_cast<int>((k + 1023) / 1024); }
+static size_t lds_of(int64_t k, int s, int mr, bool f16) {
+    return static_cast<size_t>(mr) * ((rows_slices(k) + s - 1) / s * s) * 1024 * (f16 ? 2 : 4);
+}
+
+// Slices a step: two where K is an even number of them from four on, so that no wave reads past K for half a step.
+static int rows_step(int64_t k) { return rows_slices(k) % 2 == 0 && rows_slices(k) >= 4 ? 2 : 1; }
+
+int q8_gemv_rows_per_pass(int64_t k, bool f16) {
+    if (k > (int64_t{1} << 16)) return 0;
+    const size_t rows = kRowsLds / lds_of(k, rows_step(k), 1, f16);
+    return rows < kRowsMax ? static_cast<int>(rows) : kRowsMax;
+}
+
+// Two weight rows a wave for a ragged K of up to three slices (a step is short there and reads past K cost most: 2880 x 2880 f32 at three
+// rows 6.3 -> 5.9 us), else one.  Two workgroups a CU where their activations fit and a wave has several row groups even so; with f32 and
+// 4096 weight rows one is better, which stages half as much (4096 x 4096 at three rows 7.7 -> 7.1 us).
+static GemvRowsShape rows_shape(int64_t m, int64_t n, int64_t k, bool f16) {
+    GemvRowsShape p;
+    p.r = k % 1024 != 0 && rows_slices(k) <= 3 ? 2 : 1;
+    p.s = rows_step(k);
+    const int most = q8_gemv_rows_per_pass(k, f16);
+    int64_t passes = (m + most - 1) / most;
+    // further passes while all of them together have a wave for each row group: 300 x 8000 at five rows, one row a pass, 5.3 us, all
+    // five in one 7.1
+    const int64_t groups = (n + p.r - 1) / p.r;
+    while (passes < m && (passes + 1) * groups <= 256 * kRowsWaves) ++passes;
+    p.mr = static_cast<int>((m + passes - 1) / passes);
+    p.lds = lds_of(k, p.s, p.mr, f16);
+    p.bpc = (n > 4096 || f16) && 2 * p.lds <= kRowsLds ? 2 : 1;
+    return p;
+}
+
+// Over 700 random sizes of up to 24 rows: 1.20 (f32) and 1.15 (f16) times as fast as a matvec a row where taken, few more than 4 %
+// slower.  The staging of the activations costs half a microsecond over the kernel without (512 x 544 2.2 -> 2.9 us, 5190 x 1024
+// at two rows 4.3 -> 5.3), which further rows earn back from some 8 M codes on (2452 x 2048 at two rows 5.2 -> 4.8; 2880 x 2880 f32 7.2 ->
+// 5.5, at five 13.9 -> 6.4), later where a short ragged K leaves lanes idle and where halves, which the other kernel reads in half the
+// time (6524 x 960 f16 at three rows 4.8 -> 5.9, 2260 x 3872 f16 at one 4.8 -> 5.6, 5113 x 1696 f16 at two 5.2 -> 6.5, 2880 x 2880 f16 4.8 -> 5.4, at three 6.9 -> 5.7).  A long
+// ragged K has no other kernel that streams: 14336 x 4128 at one row 19.7 -> 15.0, 644 x 13696 9.7 -> 6.7.
+bool q8_gemv_rows_pays(int64_t m, int64_t n, int64_t k, bool f16) {
+    if (q8_gemv_rows_per_pass(k, f16) == 0) return false;
+    if (k % 1024 != 0 && k > (f16 ? 4096 : 3072)) return true;
+    if (f16 && k < 1024) return false;
+    const double millions = (f16 ? k % 1024 == 0 && k > 1024 : k >= 1024) ? 8.0 : 12.0;
+    return static_cast<double>(m - 1) * static_cast<double>(n) * static_cast<double>(k) >= millions * 1e6;
+}
+
+template <int R, int S, int MR, bool RAG, typename XT>
+static lhip_status rows_launch(const GemvRowsShape &p, const int8_t *qs, const __half *ds, const XT *x, XT *y, int m, int n, int k,
+                               hipStream_t s) {
+    constexpr int W = kRowsWaves;
+    int grid = ((n + R - 1) / R + W - 1) / W;
+    if (grid > 256 * p.bpc) grid = 256 * p.bpc;
+    const unsigned row_groups = static_cast<unsigned>((rows_slices(k) + S - 1) / S * S * RowsX<XT>::kPer);
+    static LdsOptIn opt;
+    if (lhip_status st = lds_opt_in(opt, reinterpret_cast<const void *>(q8_gemv_rows_kernel<R, S, W, MR, RAG, XT>), p.lds)) return st;
+    hipLaunchKernelGGL((q8_gemv_rows_kernel<R, S, W, MR, RAG, XT>), dim3(static_cast<unsigned>(grid), static_cast<unsigned>((m + MR - 1) / MR)),
+                       dim3(W * 64), p.lds, s, qs, reinterpret_cast<const unsigned short *>(ds), x, y, m, n, k, grid, 65536u / row_groups + 1);
+    LHIP_CHECK_LAUNCH();
+    return LHIP_OK;
+}
+
+template <int R, int S, bool RAG, typename XT>
+static lhip_status rows_launch_mr(const GemvRowsShape &p, const int8_t *qs, const __half *ds, const XT *x, XT *y, int m, int n, int k,
+                                  hipStream_t s) {
+    switch (p.mr) {
+        case 1: return rows_launch<R, S, 1, RAG>(p, qs, ds, x, y, m, n, k, s);
+        case 2: return rows_launch<R, S, 2, RAG>(p, qs, ds, x, y, m, n, k, s);
+        case 3: return rows_launch<R, S, 3, RAG>(p, qs, ds, x, y, m, n, k, s);
+        case 4: return rows_launch<R, S, 4, RAG>(p, qs, ds, x, y, m, n, k, s);
+        default: return rows_launch<R, S, 5, RAG>(p, qs, ds, x, y, m, n, k, s);
+    }
+}
+
+template <typename XT>
+static lhip_status rows_launch_any(const int8_t *qs, const __half *ds, const XT *x, XT *y, int m, int n, int k, hipStream_t s) {
+    const GemvRowsShape p = rows_shape(m, n, k, sizeof(XT) == 2);
+    if (p.r == 2) return rows_launch_mr<2, 1, true>(p, qs, ds, x, y, m, n, k, s);
+    if (p.s == 2)
+        return k % 2048 != 0 ? rows_launch_mr<1, 2, true>(p, qs, ds, x, y, m, n, k, s) : rows_launch_mr<1, 2, false>(p, qs, ds, x, y, m, n, k, s);
+    return k % 1024 != 0 ? rows_launch_mr<1, 1, true>(p, qs, ds, x, y, m, n, k, s) : rows_launch_mr<1, 1, false>(p, qs, ds, x, y, m, n, k, s);
+}
+
+lhip_status q8_gemv_rows_launch(const int8_t *qs, const __half *ds, const void *x, void *y, int m, int n, int k, bool f16, hipStream_t s) {
+    if (f16) return rows_launch_any(qs, ds, static_cast<const __half *>(x), static_cast<__half *>(y), m, n, k, s);
+    return rows_launch_any(qs, ds, static_cast<const float *>(x), static_cast<float *>(y), m, n, k, s);
+}
+
+}  // namespace lhip
