@@ -24,20 +24,6 @@
 
 namespace lhip {
 
-// The 32 codes of one block (four dwords, even k in the low nibble) times 2^(code - 127), as the four weight
-// operands of the block's matrix steps.
-__device__ __forceinline__ void mx_expand_block(const mu32x4 &q, uint32_t scale_code, v8bf (&w)[4]) {
-    const float s = __uint_as_float(scale_code << 23);
-#pragma unroll
-    for (int d = 0; d < 4; ++d) {
-        const v2bf p0 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(q[d], s, 0);
-        const v2bf p1 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(q[d], s, 1);
-        const v2bf p2 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(q[d], s, 2);
-        const v2bf p3 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(q[d], s, 3);
-        w[d] = v8bf{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
-    }
-}
-
 // LDS byte offset, inside a row's two planes of `plane_bytes` each, of 16-byte piece j (k = 8j .. 8j+7) of a chunk.
 __device__ __forceinline__ int exact_piece_offset(int j, int plane_bytes) {
     const int g = j >> 2, d = j & 3;
@@ -278,247 +264,6 @@ __global__ __launch_bounds__(256 * WR) void mx_moe_gemm_exact_kernel(MoeExactArg
         }
 }
 
-// ---------------------------------------------------------------------------
-// Direct form for a handful of routed rows (at most 4: one token's top-4, batch-1 decode), two launches.
-//
-// Gate|up: row tile t is routed entry t (expert sel[t], no plan); the token's row of x is staged whole in LDS once,
-// the K loop is nothing but the weight stream, D chunks of weights in flight per wave.
-// ---------------------------------------------------------------------------
-struct MoeDirectExactArgs {
-    const __bf16 *x;      // [T][K]
-    const int *sel;       // [R]
-    int a_div;            // routed entry / a_div = token
-    const uint8_t *w_nib, *w_sc;
-    int rows_per_expert, K, Kp, N;
-    int n_experts, direct_rows;
-    int *slot_of;         // gets the identity (or -1 for an entry that names no expert)
-    __bf16 *act;          // [R][N]
-};
-
-// Stage `rows` bf16 rows of K elements (row stride `stride` elements) into the two-plane layout, zeros past K.
-__device__ __forceinline__ void exact_stage_rows(unsigned char *lds, const __bf16 *src, size_t stride, int rows, int K,
-                                                 int Kp, int a_row, int a_plane, int tid) {
-    const int per_row = Kp / 8;  // 16-byte pieces per row
-    for (int q = tid; q < rows * per_row; q += 256) {
-        const int row = q / per_row, piece = q - row * per_row;
-        const int chunk = piece >> 4, j = piece & 15;
-        mu32x4 v = {0, 0, 0, 0};
-        if (piece * 8 < K) v = *reinterpret_cast<const mu32x4 *>(src + row * stride + piece * 8);
-        *reinterpret_cast<mu32x4 *>(lds + row * a_row + chunk * kChunk + exact_piece_offset(j, a_plane)) = v;
-    }
-}
-
-// The leading arguments are what stands between the launch and the first weight load (sel[tile] -> expert -> address):
-// as scalars they reach the wave in registers, where a by-value struct is read from the argument buffer first.
-template <int D>
-__global__ __launch_bounds__(256) void mx_moe_gateup_direct_exact_kernel(const int *sel, const uint8_t *w_nib, const uint8_t *w_sc,
-                                                                         const __bf16 *x, int rows_per_expert, int k_in,
-                                                                         int k_padded, int n_out, int n_experts,
-                                                                         int direct_rows, MoeDirectExactArgs rest) {
-    MoeDirectExactArgs g = rest;
-    g.sel = sel; g.w_nib = w_nib; g.w_sc = w_sc; g.x = x;
-    g.rows_per_expert = rows_per_expert; g.K = k_in; g.Kp = k_padded; g.N = n_out; g.n_experts = n_experts; g.direct_rows = direct_rows;
-    constexpr int NT = 2;  // a gate fragment and its up fragment
-    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-    const int tile = blockIdx.y;
-    if (tile >= g.direct_rows) return;
-    const int expert = g.sel[tile];
-    const bool known = expert >= 0 && expert < g.n_experts;
-    if (blockIdx.x == 0 && threadIdx.x == 0) g.slot_of[tile] = known ? tile : -1;
-    if (!known) return;
-
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int r = lane & 15, grp = lane >> 4;
-    const int Kp = g.Kp;
-    const int chunks = Kp / kChunk;
-    const int steps = (chunks + D - 1) / D * D;
-    const int a_row = moe_small_pitch(Kp);
-    const int a_plane = 16 * a_row;
-
-    const int n0 = (blockIdx.x * 4 + wave) * 16;
-    const int col = n0 + r;
-    const uint8_t *w_tile[NT];
-    const uint8_t *s_tile[NT];
-#pragma unroll
-    for (int f = 0; f < NT; ++f) {
-        const int wrow0 = (f ? g.N : 0) + min(n0, g.N - 16);
-        const size_t panel = (static_cast<size_t>(expert) * g.rows_per_expert + wrow0) >> 4;
-        w_tile[f] = g.w_nib + (panel * chunks * 64 + lane) * 16;
-        s_tile[f] = g.w_sc + panel * chunks * 64 + (lane & ~3);  // the dword that holds this lane's scale byte
-    }
-    const int s_shift = 8 * (lane & 3);
-    BSet<1, NT> bs[D];
-    auto load_b = [&](int set, int c) {
-        bs[set].valid = c < chunks;
-        const int cc = min(c, chunks - 1);
-#pragma unroll
-        for (int f = 0; f < NT; ++f) {
-            bs[set].q[f] = __builtin_nontemporal_load(reinterpret_cast<const mu32x4 *>(w_tile[f] + static_cast<size_t>(cc) * 1024));
-            bs[set].s[f] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t *>(s_tile[f] + cc * 64));
-        }
-    };
-    // Weights first: their trip to memory overlaps the staging of the activations.
-#pragma unroll
-    for (int j = 0; j < D; ++j) load_b(j, j);
-    exact_stage_rows(lds, g.x + static_cast<size_t>(tile / g.a_div) * g.K, 0, 1, g.K, Kp, a_row, a_plane, tid);
-    __syncthreads();
-
-    v4f acc[NT];
-#pragma unroll
-    for (int f = 0; f < NT; ++f) acc[f] = v4f{0.f, 0.f, 0.f, 0.f};
-    // Rows 1..15 of the tile hold whatever LDS held before; a row's products stay in that row's results, which are
-    // never stored.
-    const unsigned char *ap = lds + r * a_row + grp * 16;
-    auto compute = [&](int set, int c) {
-        const int cc = min(c, chunks - 1);
-        const unsigned char *p = ap + cc * kChunk;
-        v8bf a[4];
-        a[0] = *reinterpret_cast<const v8bf *>(p);
-        a[1] = *reinterpret_cast<const v8bf *>(p + 64);
-        a[2] = *reinterpret_cast<const v8bf *>(p + a_plane);
-        a[3] = *reinterpret_cast<const v8bf *>(p + a_plane + 64);
-#pragma unroll
-        for (int f = 0; f < NT; ++f) {
-            asm volatile("" : "+v"(bs[set].q[f]), "+v"(bs[set].s[f]));
-            const mu32x4 zero = {0, 0, 0, 0};
-            const mu32x4 q = bs[set].valid ? bs[set].q[f] : zero;  // a dead chunk adds zeros
-            v8bf wb[4];
-            mx_expand_block(q, (bs[set].s[f] >> s_shift) & 0xffu, wb);
-#pragma unroll
-            for (int d = 0; d < 4; ++d) acc[f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[d], wb[d], acc[f], 0, 0, 0);
-            asm volatile("" : "+a"(acc[f]));
-        }
-    };
-    for (int c0 = 0; c0 < steps; c0 += D) {
-#pragma unroll
-        for (int j = 0; j < D; ++j) {
-            compute(j, c0 + j);
-            __builtin_amdgcn_sched_barrier(0);
-            load_b(j, c0 + j + D);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    }
-    // row 0 of the fragment is the routed row: element 0 of the lanes of group 0
-    if (grp == 0 && col < g.N) g.act[static_cast<size_t>(tile) * g.N + col] = static_cast<__bf16>(exact_swiglu(acc[0][0], acc[1][0]));
-}
-
-// Down projection of the routed rows with the weighted sum over a token's experts folded in (see
-// mx_moe_down_direct_kernel: a workgroup owns 16 output columns for all routed rows, the four waves split K and meet
-// in LDS, every wave requests its whole share of the weights before anything else).
-struct MoeDownDirectExactArgs {
-    const __bf16 *act;    // [R][K]
-    const uint8_t *w_nib, *w_sc;
-    int rows_per_expert, K, Kp, N;
-    const int *sel;
-    const float *wts;
-    int R, topk, n_experts;
-    float *out;           // [R][N]
-    __bf16 *y;            // [R / topk][N]
-};
-
-__global__ __launch_bounds__(256) void mx_moe_down_direct_exact_kernel(const int *sel, const uint8_t *w_nib, const uint8_t *w_sc,
-                                                                       const __bf16 *act, int rows_per_expert, int k_in,
-                                                                       int k_padded, int n_out, int n_experts, int n_rows,
-                                                                       MoeDownDirectExactArgs rest) {
-    MoeDownDirectExactArgs g = rest;  // (leading scalars as in the gate/up kernel)
-    g.sel = sel; g.w_nib = w_nib; g.w_sc = w_sc; g.act = act;
-    g.rows_per_expert = rows_per_expert; g.K = k_in; g.Kp = k_padded; g.N = n_out; g.n_experts = n_experts; g.R = n_rows;
-    constexpr int D = 8;  // chunks of a routed row per wave: K up to 4 * D * kChunk
-    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int r = lane & 15, grp = lane >> 4;
-    const int Kp = g.Kp, chunks = Kp / kChunk, R = g.R;
-    const int a_row = moe_small_pitch(Kp), a_plane = 16 * a_row;
-    const int n0 = blockIdx.x * 16;  // N is a multiple of 16
-    const int col = n0 + r;
-
-    unsigned off_lo, off_hi, known;
-    {
-        const int t = lane & (kDirectRows - 1);
-        const int e = t < R ? g.sel[t] : -1;
-        const bool ok = e >= 0 && e < g.n_experts;
-        const size_t off = ((static_cast<size_t>(ok ? e : 0) * g.rows_per_expert + n0) >> 4) * chunks * 64;
-        off_lo = static_cast<unsigned>(off);
-        off_hi = static_cast<unsigned>(off >> 32);
-        known = static_cast<unsigned>(__ballot(ok)) & ((1u << kDirectRows) - 1u);
-    }
-    const uint8_t *w_lane = g.w_nib + lane * 16;
-    const uint8_t *s_lane = g.w_sc + (lane & ~3);
-    const int s_shift = 8 * (lane & 3);
-    static_assert(D * 4 * kChunk >= 4096, "K up to 4096");
-    BSet<1, 1> bs[kDirectRows][D];
-#pragma unroll
-    for (int t = 0; t < kDirectRows; ++t) {
-        const int tc = min(t, R - 1);
-        const size_t off = static_cast<size_t>(__builtin_amdgcn_readlane(off_hi, tc)) << 32 | __builtin_amdgcn_readlane(off_lo, tc);
-        const uint8_t *wb = w_lane + off * 16;
-        const uint8_t *sb = s_lane + off;
-#pragma unroll
-        for (int j = 0; j < D; ++j) {
-            const int cc = min(wave + 4 * j, chunks - 1);
-            bs[t][j].q[0] = __builtin_nontemporal_load(reinterpret_cast<const mu32x4 *>(wb + static_cast<size_t>(cc) * 1024));
-            bs[t][j].s[0] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t *>(sb + cc * 64));
-        }
-    }
-    exact_stage_rows(lds, g.act, static_cast<size_t>(g.K), R, g.K, Kp, a_row, a_plane, tid);
-    __syncthreads();
-
-    const unsigned char *ap = lds + r * a_row + grp * 16;
-    float vals[kDirectRows];
-#pragma unroll
-    for (int t = 0; t < kDirectRows; ++t) {
-        v4f acc = v4f{0.f, 0.f, 0.f, 0.f};
-        const bool live = (t < R) & ((known >> t) & 1u);
-#pragma unroll
-        for (int j = 0; j < D; ++j) {
-            const int c = wave + 4 * j;
-            asm volatile("" : "+v"(bs[t][j].q[0]), "+v"(bs[t][j].s[0]));
-            if (live & (c < chunks)) {  // wave-uniform
-                const unsigned char *p = ap + c * kChunk;
-                v8bf a[4], wb[4];
-                a[0] = *reinterpret_cast<const v8bf *>(p);
-                a[1] = *reinterpret_cast<const v8bf *>(p + 64);
-                a[2] = *reinterpret_cast<const v8bf *>(p + a_plane);
-                a[3] = *reinterpret_cast<const v8bf *>(p + a_plane + 64);
-                mx_expand_block(bs[t][j].q[0], (bs[t][j].s[0] >> s_shift) & 0xffu, wb);
-#pragma unroll
-                for (int d = 0; d < 4; ++d) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[d], wb[d], acc, 0, 0, 0);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        vals[t] = acc[t];  // routed row t is row t of the fragment: element t of the lanes of group 0
-    }
-
-    __syncthreads();
-    float *part = reinterpret_cast<float *>(lds);  // [4 waves][kDirectRows][16 columns]
-    if (grp == 0) {
-#pragma unroll
-        for (int t = 0; t < kDirectRows; ++t) part[(wave * kDirectRows + t) * 16 + r] = vals[t];
-    }
-    __syncthreads();
-    if (wave != 0 || grp != 0 || col >= g.N) return;
-    float down[kDirectRows];
-#pragma unroll
-    for (int t = 0; t < kDirectRows; ++t) {
-        down[t] = ((part[t * 16 + r] + part[(kDirectRows + t) * 16 + r]) + part[(2 * kDirectRows + t) * 16 + r]) +
-                  part[(3 * kDirectRows + t) * 16 + r];
-        if (t < R) g.out[static_cast<size_t>(t) * g.N + col] = ((known >> t) & 1u) ? down[t] : 0.f;
-    }
-    for (int token = 0; token * g.topk < R; ++token) {
-        float a = 0.f;
-        for (int sidx = 0; sidx < g.topk; ++sidx) {
-            const int t = token * g.topk + sidx;
-            const float d = t == 0 ? down[0] : t == 1 ? down[1] : t == 2 ? down[2] : down[3];
-            if ((known >> t) & 1u) a = fmaf(g.wts[t], d, a);
-        }
-        g.y[static_cast<size_t>(token) * g.N + col] = static_cast<__bf16>(a);
-    }
-}
-
 __global__ __launch_bounds__(1024) void moe_plan_kernel(const int *__restrict__ sel, int R, int E, int BM, MoePlan p) {
     moe_plan_block(sel, R, E, BM, p);
 }
@@ -581,36 +326,10 @@ lhip_status moe_exact_forward(const uint8_t *gu, const uint8_t *dn, const __bf16
     const uint8_t *gu_sc = gu + mx_scale_offset(static_cast<int64_t>(E) * 2 * I, H);
     const uint8_t *dn_sc = dn + mx_scale_offset(static_cast<int64_t>(E) * H, I);
 
-    if (R <= kDirectRows && moe_small_lds_bytes(Hp) <= 150 * 1024 && moe_small_lds_bytes(Ip) <= 150 * 1024 && Ip <= 4096) {
-        MoeDirectExactArgs a1{};
-        a1.x = x; a1.sel = sel_dev; a1.a_div = topk;
-        a1.w_nib = gu; a1.w_sc = gu_sc;
-        a1.rows_per_expert = 2 * I; a1.K = H; a1.Kp = Hp; a1.N = I;
-        a1.n_experts = E; a1.direct_rows = R; a1.slot_of = w.plan.slot_of; a1.act = w.act;
-        {
-            const size_t lds_bytes = moe_small_lds_bytes(Hp);
-            auto kern = mx_moe_gateup_direct_exact_kernel<8>;
-            static LdsOptIn opt;
-            if (lhip_status st = lds_opt_in(opt, reinterpret_cast<const void *>(kern), lds_bytes)) return st;
-            hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>((I + 63) / 64), static_cast<unsigned>(R)), dim3(256), lds_bytes, s,
-                               a1.sel, a1.w_nib, a1.w_sc, a1.x, a1.rows_per_expert, a1.K, a1.Kp, a1.N, a1.n_experts, a1.direct_rows, a1);
-            LHIP_CHECK_LAUNCH();
-        }
-        MoeDownDirectExactArgs a2{};
-        a2.act = w.act; a2.w_nib = dn; a2.w_sc = dn_sc;
-        a2.rows_per_expert = H; a2.K = I; a2.Kp = Ip; a2.N = H;
-        a2.sel = sel_dev; a2.wts = wts_dev; a2.R = R; a2.topk = topk; a2.n_experts = E;
-        a2.out = w.out; a2.y = y;
-        {
-            const size_t lds_bytes = moe_small_lds_bytes(Ip);
-            static LdsOptIn opt;
-            if (lhip_status st = lds_opt_in(opt, reinterpret_cast<const void *>(mx_moe_down_direct_exact_kernel), lds_bytes)) return st;
-            hipLaunchKernelGGL(mx_moe_down_direct_exact_kernel, dim3(static_cast<unsigned>(H / 16)), dim3(256), lds_bytes, s,
-                               a2.sel, a2.w_nib, a2.w_sc, a2.act, a2.rows_per_expert, a2.K, a2.Kp, a2.N, a2.n_experts, a2.R, a2);
-            LHIP_CHECK_LAUNCH();
-        }
-        return LHIP_OK;
-    }
+    // (A K of several segments pays while the tiles are few: 8 experts of 4096 x 14336, top 2, T = 1 118 -> 43 us, T = 16 145 -> 141, T = 32
+    // 150 -> 163; 32 of 5120 x 5120, top 2, T = 6 103 -> 97, T = 8 110 -> 116.)
+    if (R <= kFewRows && ((H <= 4096 && I <= 4096) || R <= (E <= 16 ? 32 : 12)))
+        return moe_few_forward(MoeFewLayer{gu, gu_sc, dn, dn_sc, x, sel_dev, wts_dev, y, w.act, w.out, w.plan.slot_of, T, H, I, E, topk}, s);
 
     const int mt = exact_tile_fragments(R, E, H, I, moe_tall_supports(T, H, I));
     const int BM = 16 * mt;

@@ -14,6 +14,20 @@ __device__ __forceinline__ float exact_swiglu(float gate, float up) {
     return up * (gate * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504f * gate)));
 }
 
+// The 32 codes of one block (four dwords, even k in the low nibble) times 2^(code - 127), as the four weight
+// operands of the block's matrix steps.
+__device__ __forceinline__ void mx_expand_block(const mu32x4 &q, uint32_t scale_code, v8bf (&w)[4]) {
+    const float s = __uint_as_float(scale_code << 23);
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+        const v2bf p0 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(q[d], s, 0);
+        const v2bf p1 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(q[d], s, 1);
+        const v2bf p2 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(q[d], s, 2);
+        const v2bf p3 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(q[d], s, 3);
+        w[d] = v8bf{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
+    }
+}
+
 struct MoeExactArgs {
     const __bf16 *a;      // activation rows, K elements each
     const int *a_index;   // slot -> routed entry (GEMM 1) or nullptr (rows are slots)
@@ -61,6 +75,20 @@ __device__ __forceinline__ void exact_tile(const MoeExactArgs &g, int &tile, int
         rows = g.tile_rows[tile];
     }
 }
+
+// mxfp4_moe_few.hip: the layer for up to kFewRows routed rows, without a plan; `act`, `out` and `slot_of` as the workspace holds them.
+constexpr int kFewRows = 64;
+struct MoeFewLayer {
+    const uint8_t *gu, *gu_sc, *dn, *dn_sc;
+    const __bf16 *x;
+    const int *sel;
+    const float *wts;
+    __bf16 *y, *act;
+    float *out;
+    int *slot_of;
+    int T, H, I, E, topk;
+};
+lhip_status moe_few_forward(const MoeFewLayer &l, hipStream_t s);
 
 // mxfp4_moe_tall.hip.  Whether its 32-bit offsets reach everywhere for t tokens of width h and experts of width i.
 constexpr int kTallRows = 96;
