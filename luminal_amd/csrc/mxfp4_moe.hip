@@ -187,12 +187,6 @@ struct MoeGemmArgs {
     // (planes of row stride q_kp, scales of row stride q_kp / 32) instead of writing `out`.
     uint8_t *q_hi, *q_lo, *q_sc;
     int q_kp;
-    // Direct form (a handful of routed rows, no plan launch in front): row tile t is routed entry t, its expert
-    // sel[t]; the activations are the bf16 rows of x, quantised by the workgroup itself; slot_of gets the identity.
-    const int *sel;
-    const __bf16 *x;
-    int *slot_of;
-    int n_experts, direct_rows;
 };
 
 
@@ -528,368 +522,6 @@ void mx_moe_gemm_kernel(MoeGemmArgs g) {
         }
 }
 
-// ---------------------------------------------------------------------------
-// Decode-sized variant: row tiles of at most 16 routed rows (one row fragment).
-// The tile's whole quantised activation rows (all of K) are staged in LDS once,
-// so the K loop is nothing but the weight stream — no activation loads, no
-// barriers — with D = 8 chunks of weights in flight per wave.  Needs
-// 2 * 16 * pitch + 16 * Kp/32 bytes of LDS (K up to ~4.6k).
-// ---------------------------------------------------------------------------
-template <int NT, bool GATED, bool DIRECT = false, int D = 8>
-__global__ __launch_bounds__(256) void mx_moe_gemm_small_kernel(MoeGemmArgs g) {
-    static_assert(!GATED || NT % 2 == 0, "gated tiles pair each gate fragment with its up fragment");
-    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-
-    const int tile = blockIdx.y;
-    int expert, row0, rows;
-    if (DIRECT) {
-        if (tile >= g.direct_rows) return;
-        expert = g.sel[tile];
-        const bool known = expert >= 0 && expert < g.n_experts;
-        if (blockIdx.x == 0 && threadIdx.x == 0) g.slot_of[tile] = known ? tile : -1;
-        if (!known) return;
-        row0 = tile;
-        rows = 1;
-    } else {
-        if (tile >= *g.n_tiles) return;
-        expert = g.tile_expert[tile];
-        row0 = g.tile_row0[tile];
-        rows = g.tile_rows[tile];  // 1..16
-    }
-
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int r = lane & 15, grp = lane >> 4;
-    const int Kp = g.Kp;
-    const int chunks = Kp / kChunk;
-    const int steps = (chunks + D - 1) / D * D;
-    const int a_row = moe_small_pitch(Kp);  // LDS bytes per activation row
-    const int a_plane = 16 * a_row;
-    const int sc_row = Kp / 32;            // scale bytes per row
-    unsigned char *lds_sc = lds + 2 * a_plane;
-
-    const uint8_t *w_tile[NT];
-    const uint8_t *s_tile[NT];
-    int col[NT];
-#pragma unroll
-    for (int f = 0; f < NT; ++f) {
-        int n0, wrow0;
-        if (GATED) {
-            n0 = ((blockIdx.x * 4 + wave) * (NT / 2) + (f >> 1)) * 16;
-            wrow0 = ((f & 1) ? g.N : 0) + min(n0, g.N - 16);
-        } else {
-            n0 = ((blockIdx.x * 4 + wave) * NT + f) * 16;
-            wrow0 = min(n0, g.N - 16);
-        }
-        col[f] = n0 + r;
-        const size_t panel = (static_cast<size_t>(expert) * g.rows_per_expert + wrow0) >> 4;
-        w_tile[f] = g.w_nib + (panel * chunks * 64 + lane) * 16;
-        s_tile[f] = g.w_sc + panel * chunks * 64 + (lane & ~3);  // the dword that holds this lane's scale byte
-    }
-    // A lane's scale is requested as the aligned dword around it and shifted down at its use: a byte load is
-    // widened after the loop's phi, i.e. at the top of every trip for all D sets, and that widening waits for the
-    // set requested last.
-    const int s_shift = 8 * (lane & 3);
-    BSet<1, NT> bs[D];
-    auto load_b = [&](int set, int c) {
-        bs[set].valid = c < chunks;
-        const int cc = min(c, chunks - 1);
-#pragma unroll
-        for (int f = 0; f < NT; ++f) {
-            bs[set].q[f] = __builtin_nontemporal_load(reinterpret_cast<const mu32x4 *>(w_tile[f] + static_cast<size_t>(cc) * 1024));
-            bs[set].s[f] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t *>(s_tile[f] + cc * 64));
-        }
-    };
-    // Weights first: their HBM round trip overlaps the staging of the activations.
-#pragma unroll
-    for (int j = 0; j < D; ++j) load_b(j, j);
-
-    if (DIRECT) {
-        // the routed entry's row of x, quantised here as the plan launch would have (groups of four threads share
-        // a 32-block: Kp / 8 is a multiple of four, so a group is whole or absent)
-        const __bf16 *x_row = g.x + static_cast<size_t>(tile / g.a_div) * g.K;
-        for (int q = tid; q < Kp / 8; q += 256) mx_quantize_act_item(q, x_row, lds, lds + a_plane, lds_sc, 1, g.K, Kp);
-    } else {
-        const int per_row = Kp / 16;  // 16-byte pieces per row and plane
-        const int pieces = rows * per_row * 2;
-        for (int q = tid; q < pieces; q += 256) {
-            const int plane = q / (rows * per_row), rem = q - plane * (rows * per_row);
-            const int row = rem / per_row, c16 = rem - row * per_row;
-            const int slot = row0 + row;
-            const int arow = g.a_index ? g.a_index[slot] / g.a_div : slot;
-            const mu32x4 v = *reinterpret_cast<const mu32x4 *>((plane ? g.a_lo : g.a_hi) +
-                                                                static_cast<size_t>(arow) * Kp + c16 * 16);
-            *reinterpret_cast<mu32x4 *>(lds + plane * a_plane + row * a_row + c16 * 16) = v;
-        }
-        const int sc_words = rows * (sc_row / 4);
-        for (int q = tid; q < sc_words; q += 256) {
-            const int row = q / (sc_row / 4), w4 = q - row * (sc_row / 4);
-            const int slot = row0 + row;
-            const int arow = g.a_index ? g.a_index[slot] / g.a_div : slot;
-            reinterpret_cast<uint32_t *>(lds_sc + row * sc_row)[w4] =
-                reinterpret_cast<const uint32_t *>(g.a_sc + static_cast<size_t>(arow) * sc_row)[w4];
-        }
-    }
-    __syncthreads();
-
-    v4f acc[NT];
-#pragma unroll
-    for (int f = 0; f < NT; ++f) acc[f] = v4f{0.f, 0.f, 0.f, 0.f};
-
-    // Rows past the tile hold stale LDS bytes; their results are never stored.
-    const unsigned char *ap = lds + r * a_row + grp * 16;
-    const unsigned char *sp = lds_sc + r * sc_row + grp;
-    auto compute = [&](int set, int c) {
-        const int cc = min(c, chunks - 1);
-        const unsigned char *p = ap + cc * kChunk;
-        const mu32x4 h0 = *reinterpret_cast<const mu32x4 *>(p);
-        const mu32x4 h1 = *reinterpret_cast<const mu32x4 *>(p + 64);
-        const mu32x4 l0 = *reinterpret_cast<const mu32x4 *>(p + a_plane);
-        const mu32x4 l1 = *reinterpret_cast<const mu32x4 *>(p + a_plane + 64);
-        const int sa = sp[cc * 4];
-        const v8i ah = {(int)h0.x, (int)h0.y, (int)h0.z, (int)h0.w, (int)h1.x, (int)h1.y, (int)h1.z, (int)h1.w};
-        const v8i al = {(int)l0.x, (int)l0.y, (int)l0.z, (int)l0.w, (int)l1.x, (int)l1.y, (int)l1.z, (int)l1.w};
-#pragma unroll
-        for (int f = 0; f < NT; ++f) {
-            asm volatile("" : "+v"(bs[set].q[f]), "+v"(bs[set].s[f]));
-            const mu32x4 zero = {0, 0, 0, 0};
-            const mu32x4 q = bs[set].valid ? bs[set].q[f] : zero;
-            const int sb = bs[set].valid ? static_cast<int>(bs[set].s[f] >> s_shift) : 127;  // the matrix core reads byte 0
-            const v8i b = {(int)q.x, (int)q.y, (int)q.z, (int)q.w, 0, 0, 0, 0};
-            acc[f] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ah, b, acc[f], 0, 4, 0, sa, 0, sb);
-            acc[f] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(al, b, acc[f], 0, 4, 0, sa - kLoShift, 0, sb);
-            asm volatile("" : "+a"(acc[f]));
-        }
-    };
-    for (int c0 = 0; c0 < steps; c0 += D) {
-#pragma unroll
-        for (int j = 0; j < D; ++j) {
-            compute(j, c0 + j);
-            __builtin_amdgcn_sched_barrier(0);
-            load_b(j, c0 + j + D);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    }
-
-    if constexpr (GATED && NT == 2) {
-        if (g.q_hi) {
-            // Quantise the result for the next GEMM here (same arithmetic as mx_quantize_act_item on the
-            // bf16-rounded values).  A wave holds 16 of a block's 32 columns; the two waves of a block exchange
-            // their row maxima through LDS, which the K loop no longer needs.
-            __syncthreads();  // every wave is done reading the staged activations
-            float *pmax = reinterpret_cast<float *>(lds);  // [4 waves][16 rows]
-            float a[4];
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const float gate = acc[0][v], up = acc[1][v];
-                const float act = up * (gate * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504f * gate)));
-                a[v] = col[0] < g.N ? static_cast<float>(static_cast<__bf16>(act)) : 0.f;
-                const float mx = row16_max(fabsf(a[v]));
-                if (r == 0) pmax[wave * 16 + 4 * grp + v] = mx;
-            }
-            __syncthreads();
-            const int b = blockIdx.x * 2 + (wave >> 1);  // quantisation block of this wave's columns
-            const int half = (wave & 1) * 16;
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int m = 4 * grp + v;
-                if (m >= rows) continue;
-                const float amax = fmaxf(pmax[wave * 16 + m], pmax[(wave ^ 1) * 16 + m]);
-                int e = 127;
-                float inv = 1.0f;
-                if (amax > 0.f && amax < __uint_as_float(0x7f800000u)) {
-                    const int ex = static_cast<int>((__float_as_uint(amax) >> 23) & 0xff);
-                    e = max(ex - 7, kLoShift + 1);
-                    inv = __uint_as_float(static_cast<uint32_t>(254 - e) << 23);
-                }
-                const float s0 = a[v] * inv;
-                const int h = __builtin_amdgcn_cvt_pk_fp8_f32(s0, 0.f, 0, false);
-                const int l = __builtin_amdgcn_cvt_pk_fp8_f32((s0 - __builtin_amdgcn_cvt_f32_fp8(h, 0)) * kLoGain, 0.f, 0, false);
-                const size_t at = static_cast<size_t>(row0 + m) * g.q_kp + b * 32 + half + r;
-                g.q_hi[at] = static_cast<uint8_t>(h);
-                g.q_lo[at] = static_cast<uint8_t>(l);
-                const size_t sc_at = static_cast<size_t>(row0 + m) * (g.q_kp / 32);
-                if (r == 0 && half == 0) g.q_sc[sc_at + b] = static_cast<uint8_t>(e);
-                // The last column block also fills the padding past N up to the padded row length: zeros, scale 2^0.
-                if (blockIdx.x == gridDim.x - 1 && wave == 0) {
-                    const int k0 = (g.N + 63) / 64 * 64;  // the column blocks end here
-                    for (int k = k0 + r; k < g.q_kp; k += 16) {
-                        g.q_hi[static_cast<size_t>(row0 + m) * g.q_kp + k] = 0;
-                        g.q_lo[static_cast<size_t>(row0 + m) * g.q_kp + k] = 0;
-                    }
-                    if (r == 0)
-                        for (int kb = k0 / 32; kb < g.q_kp / 32; ++kb) g.q_sc[sc_at + kb] = 127;
-                }
-            }
-            return;
-        }
-    }
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        const int m = 4 * grp + v;
-        if (m >= rows) continue;
-        const size_t orow = static_cast<size_t>(row0 + m) * g.N;
-        if (GATED) {
-#pragma unroll
-            for (int p = 0; p < NT / 2; ++p)
-                if (col[2 * p] < g.N) {
-                    const float gate = acc[2 * p][v], up = acc[2 * p + 1][v];
-                    const float act = up * (gate * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504f * gate)));
-                    static_cast<__bf16 *>(g.out)[orow + col[2 * p]] = static_cast<__bf16>(act);
-                }
-        } else {
-#pragma unroll
-            for (int f = 0; f < NT; ++f)
-                if (col[f] < g.N) static_cast<float *>(g.out)[orow + col[f]] = acc[f][v];
-        }
-    }
-}
-
-// ---------------------------------------------------------------------------
-// Down projection of a handful of routed rows (at most 4: one token's top-4) with the weighted sum over a token's
-// experts folded in, for the direct form: no plan, no combine launch.  A workgroup owns 16 output columns for
-// ALL routed rows: routed row t multiplies the 16 weight rows of expert sel[t]; the four waves split K (chunk c
-// belongs to wave c % 4) and meet in LDS, then y[token][col] = bf16(sum_s wts * down) in the combine kernel's
-// order.  The rows' quantised activations (all of K) are staged in LDS once; a wave requests its whole share of
-// the weights (all routed rows, K up to 4096) before anything else and holds it in registers.
-// ---------------------------------------------------------------------------
-
-struct MoeDownDirectArgs {
-    const uint8_t *a_hi, *a_lo, *a_sc;  // quantised activations: R rows of Kp / Kp/32 bytes, row = routed entry
-    const uint8_t *w_nib, *w_sc;        // planar down weights of all experts, rows_per_expert rows each
-    int rows_per_expert, Kp, N;
-    const int *sel;
-    const float *wts;
-    int R, topk, n_experts;
-    float *out;                         // [R][N] f32 rows (read back by lhip_mxfp4_moe_read_intermediates)
-    __bf16 *y;                          // [R / topk][N]
-};
-
-__global__ __launch_bounds__(256) void mx_moe_down_direct_kernel(MoeDownDirectArgs g) {
-    constexpr int D = 8;  // chunks of a routed row per wave: K up to 4 * D * kChunk
-    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int r = lane & 15, grp = lane >> 4;
-    const int Kp = g.Kp, chunks = Kp / kChunk, R = g.R;
-    const int a_row = moe_small_pitch(Kp), a_plane = 16 * a_row, sc_row = Kp / 32;
-    unsigned char *lds_sc = lds + 2 * a_plane;
-    const int n0 = blockIdx.x * 16;  // N is a multiple of 16
-    const int col = n0 + r;
-
-    // Per routed row: where its expert's weights start (lane t of a register pair holds routed row t's, read with
-    // v_readlane) and whether it names a real expert (a bit mask).  The loads below stay free of branches and of
-    // selects between 64-bit scalars (which compile to branches): a branch between loads makes the compiler's
-    // wait counts for the sets in flight fall back to "wait for everything".
-    unsigned off_lo, off_hi, known;
-    {
-        const int t = lane & (kDirectRows - 1);
-        const int e = t < R ? g.sel[t] : -1;
-        const bool ok = e >= 0 && e < g.n_experts;
-        const size_t off = ((static_cast<size_t>(ok ? e : 0) * g.rows_per_expert + n0) >> 4) * chunks * 64;
-        off_lo = static_cast<unsigned>(off);
-        off_hi = static_cast<unsigned>(off >> 32);
-        known = static_cast<unsigned>(__ballot(ok)) & ((1u << kDirectRows) - 1u);  // lanes 0..3 are rows 0..3
-    }
-    const uint8_t *w_lane = g.w_nib + lane * 16;
-    const uint8_t *s_lane = g.w_sc + (lane & ~3);
-    const int s_shift = 8 * (lane & 3);
-    // Chunk wave + 4 * j of routed row t is weight set (t, j), j < D: all of a wave's share - at most
-    // kDirectRows * D kilobytes - is requested up front and held in registers (a workgroup has the SIMDs to
-    // itself: 512 registers per lane), so the whole launch costs one trip to memory instead of one per D chunks.
-    static_assert(D * 4 * kChunk >= 4096, "K up to 4096");
-    BSet<1, 1> bs[kDirectRows][D];
-#pragma unroll
-    for (int t = 0; t < kDirectRows; ++t) {
-        const int tc = min(t, R - 1);  // rows past R re-read the last row's lines: never used
-        const size_t off = static_cast<size_t>(__builtin_amdgcn_readlane(off_hi, tc)) << 32 | __builtin_amdgcn_readlane(off_lo, tc);
-        const uint8_t *wb = w_lane + off * 16;
-        const uint8_t *sb = s_lane + off;
-#pragma unroll
-        for (int j = 0; j < D; ++j) {
-            const int cc = min(wave + 4 * j, chunks - 1);  // chunks past the end re-read the last one: never used
-            bs[t][j].q[0] = __builtin_nontemporal_load(reinterpret_cast<const mu32x4 *>(wb + static_cast<size_t>(cc) * 1024));
-            bs[t][j].s[0] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t *>(sb + cc * 64));
-        }
-    }
-    {
-        const int per_row = Kp / 16;
-        const int pieces = R * per_row * 2;
-        for (int q = tid; q < pieces; q += 256) {
-            const int plane = q / (R * per_row), rem = q - plane * (R * per_row);
-            const int row = rem / per_row, c16 = rem - row * per_row;
-            const mu32x4 v = *reinterpret_cast<const mu32x4 *>((plane ? g.a_lo : g.a_hi) + static_cast<size_t>(row) * Kp + c16 * 16);
-            *reinterpret_cast<mu32x4 *>(lds + plane * a_plane + row * a_row + c16 * 16) = v;
-        }
-        const int sc_words = R * (sc_row / 4);
-        for (int q = tid; q < sc_words; q += 256) {
-            const int row = q / (sc_row / 4), w4 = q - row * (sc_row / 4);
-            reinterpret_cast<uint32_t *>(lds_sc + row * sc_row)[w4] =
-                reinterpret_cast<const uint32_t *>(g.a_sc + static_cast<size_t>(row) * sc_row)[w4];
-        }
-    }
-    __syncthreads();
-
-    // Rows past R hold stale LDS bytes; their results are never used.
-    const unsigned char *ap = lds + r * a_row + grp * 16;
-    const unsigned char *sp = lds_sc + r * sc_row + grp;
-    float vals[kDirectRows];  // this wave's share of routed row t's 16 outputs (lanes 0..15)
-#pragma unroll
-    for (int t = 0; t < kDirectRows; ++t) {
-        v4f acc = v4f{0.f, 0.f, 0.f, 0.f};
-        const bool live = (t < R) & ((known >> t) & 1u);
-#pragma unroll
-        for (int j = 0; j < D; ++j) {
-            const int c = wave + 4 * j;
-            asm volatile("" : "+v"(bs[t][j].q[0]), "+v"(bs[t][j].s[0]));
-            if (live & (c < chunks)) {  // wave-uniform
-                const unsigned char *p = ap + c * kChunk;
-                const mu32x4 h0 = *reinterpret_cast<const mu32x4 *>(p);
-                const mu32x4 h1 = *reinterpret_cast<const mu32x4 *>(p + 64);
-                const mu32x4 l0 = *reinterpret_cast<const mu32x4 *>(p + a_plane);
-                const mu32x4 l1 = *reinterpret_cast<const mu32x4 *>(p + a_plane + 64);
-                const int sa = sp[c * 4];
-                const v8i ah = {(int)h0.x, (int)h0.y, (int)h0.z, (int)h0.w, (int)h1.x, (int)h1.y, (int)h1.z, (int)h1.w};
-                const v8i al = {(int)l0.x, (int)l0.y, (int)l0.z, (int)l0.w, (int)l1.x, (int)l1.y, (int)l1.z, (int)l1.w};
-                const mu32x4 q = bs[t][j].q[0];
-                const int sb = static_cast<int>(bs[t][j].s[0] >> s_shift);
-                const v8i b = {(int)q.x, (int)q.y, (int)q.z, (int)q.w, 0, 0, 0, 0};
-                acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ah, b, acc, 0, 4, 0, sa, 0, sb);
-                acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(al, b, acc, 0, 4, 0, sa - kLoShift, 0, sb);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        vals[t] = acc[t];  // routed row t is row t of the fragment
-    }
-
-    __syncthreads();  // every wave is done reading the staged activations
-    float *part = reinterpret_cast<float *>(lds);  // [4 waves][kDirectRows][16 columns]
-    if (grp == 0) {
-#pragma unroll
-        for (int t = 0; t < kDirectRows; ++t) part[(wave * kDirectRows + t) * 16 + r] = vals[t];
-    }
-    __syncthreads();
-    if (wave != 0 || grp != 0 || col >= g.N) return;
-    float down[kDirectRows];
-#pragma unroll
-    for (int t = 0; t < kDirectRows; ++t) {
-        down[t] = ((part[t * 16 + r] + part[(kDirectRows + t) * 16 + r]) + part[(2 * kDirectRows + t) * 16 + r]) +
-                  part[(3 * kDirectRows + t) * 16 + r];
-        if (t < R) g.out[static_cast<size_t>(t) * g.N + col] = ((known >> t) & 1u) ? down[t] : 0.f;
-    }
-    for (int token = 0; token * g.topk < R; ++token) {
-        float a = 0.f;
-        for (int sidx = 0; sidx < g.topk; ++sidx) {
-            const int t = token * g.topk + sidx;
-            const float d = t == 0 ? down[0] : t == 1 ? down[1] : t == 2 ? down[2] : down[3];
-            if ((known >> t) & 1u) a = fmaf(g.wts[t], d, a);
-        }
-        g.y[static_cast<size_t>(token) * g.N + col] = static_cast<__bf16>(a);
-    }
-}
-
 // y[t][h] = bf16( sum_s wts[t][s] * out[slot_of[t*topk+s]][h] ), 4 columns per thread
 __global__ __launch_bounds__(256) void moe_combine_kernel(const float *__restrict__ out, const int *__restrict__ slot_of,
                                                           const float *__restrict__ wts, __bf16 *__restrict__ y, int T,
@@ -958,18 +590,6 @@ static lhip_status launch_moe_gemm(const MoeGemmArgs &a, int col_blocks, int max
     return LHIP_OK;
 }
 
-
-template <int NT, bool GATED>
-static lhip_status launch_moe_gemm_small(const MoeGemmArgs &a, int col_blocks, int max_tiles, hipStream_t s) {
-    const size_t lds_bytes = moe_small_lds_bytes(a.Kp);
-    auto kern = mx_moe_gemm_small_kernel<NT, GATED>;
-    static LdsOptIn opt;
-    if (lhip_status st = lds_opt_in(opt, reinterpret_cast<const void *>(kern), lds_bytes)) return st;
-    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(col_blocks), static_cast<unsigned>(max_tiles)), dim3(256),
-                       lds_bytes, s, a);
-    LHIP_CHECK_LAUNCH();
-    return LHIP_OK;
-}
 
 // Scratch memory of lhip_mxfp4_moe_bf16_static: the layer's workspace for callers that cannot allocate one.  One copy
 // per device, held until the process ends; every call of that entry point on a device shares it.
@@ -1064,7 +684,7 @@ lhip_status lhip_mxfp4_moe_bf16_mode(const void *w_gate_up_planar, const void *w
     const int T = static_cast<int>(t), H = static_cast<int>(h), I = static_cast<int>(i), E = static_cast<int>(e);
     const int topk_i = static_cast<int>(topk), R = T * topk_i;
     MoeWorkspace w = carve(workspace_dev, t, h, i, e, topk);
-    if (mode == LHIP_MOE_EXACT)
+    if (mode == LHIP_MOE_EXACT || moe_few_takes(T, H, I, E, topk_i))
         return moe_exact_forward(static_cast<const uint8_t *>(w_gate_up_planar), static_cast<const uint8_t *>(w_down_planar),
                                  static_cast<const __bf16 *>(x_dev), sel_dev, wts_dev, static_cast<__bf16 *>(y_dev), T, H, I,
                                  E, topk_i, w, s);
@@ -1084,51 +704,10 @@ lhip_status lhip_mxfp4_moe_bf16_mode(const void *w_gate_up_planar, const void *w
     const int mt = need <= 16 ? 1 : need <= 32 ? 2 : need <= 64 ? 4 : need <= 80 ? 5 : need <= 128 ? 8 : 5;
     const int BM = 16 * mt;
     const int max_tiles = (R / BM + E + 7) / 8 * 8;  // upper bound of the tile count, whole eighths for the per-XCD list
-    // One token's worth of routed rows (batch-1 decode): stage each tile's activation rows whole and run the
-    // barrier-free weight stream.  From two tokens on the chunked kernel below is faster (measured, us per layer,
-    // whole-row kernel / chunked: T = 1 31.6 / 39.5, T = 2 45.9 / 42.8, T = 8 80 / 64, T = 32 126 / 92).
-    const bool decode_sized = R <= 4;
-
     auto *gu = static_cast<const uint8_t *>(w_gate_up_planar);
     auto *dn = static_cast<const uint8_t *>(w_down_planar);
-    if (decode_sized && R <= kDirectRows && moe_small_lds_bytes(Hp) <= 150 * 1024 && Ip <= 4096) {
-        // Direct form: two launches.  The gate/up GEMM takes routed entry t as its row tile t and quantises the
-        // token's row of x itself; the down GEMM sums over the token's experts as it finishes.
-        MoeGemmArgs a1{};
-        a1.a_div = topk_i;
-        a1.w_nib = gu; a1.w_sc = gu + mx_scale_offset(e * 2 * i, h);
-        a1.rows_per_expert = 2 * I; a1.K = H; a1.Kp = Hp; a1.N = I;
-        a1.out = w.act;
-        a1.q_hi = w.a_hi; a1.q_lo = w.a_lo; a1.q_sc = w.a_sc; a1.q_kp = Ip;
-        a1.sel = sel_dev; a1.x = static_cast<const __bf16 *>(x_dev); a1.slot_of = w.plan.slot_of;
-        a1.n_experts = E; a1.direct_rows = R;
-        {
-            const size_t lds_bytes = moe_small_lds_bytes(Hp);
-            auto kern = mx_moe_gemm_small_kernel<2, true, true>;
-            static LdsOptIn opt;
-            if (lhip_status st = lds_opt_in(opt, reinterpret_cast<const void *>(kern), lds_bytes)) return st;
-            hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>((I + 63) / 64), static_cast<unsigned>(R)), dim3(256), lds_bytes, s, a1);
-            LHIP_CHECK_LAUNCH();
-        }
-        MoeDownDirectArgs a2{};
-        a2.a_hi = w.a_hi; a2.a_lo = w.a_lo; a2.a_sc = w.a_sc;
-        a2.w_nib = dn; a2.w_sc = dn + mx_scale_offset(e * h, i);
-        a2.rows_per_expert = H; a2.Kp = Ip; a2.N = H;
-        a2.sel = sel_dev; a2.wts = wts_dev; a2.R = R; a2.topk = topk_i; a2.n_experts = E;
-        a2.out = w.out; a2.y = static_cast<__bf16 *>(y_dev);
-        {
-            const size_t lds_bytes = moe_small_lds_bytes(Ip);
-            static LdsOptIn opt;
-            if (lhip_status st = lds_opt_in(opt, reinterpret_cast<const void *>(mx_moe_down_direct_kernel), lds_bytes)) return st;
-            hipLaunchKernelGGL(mx_moe_down_direct_kernel, dim3(static_cast<unsigned>(H / 16)), dim3(256), lds_bytes, s, a2);
-            LHIP_CHECK_LAUNCH();
-        }
-        return LHIP_OK;
-    }
-
-    // The decode-sized kernels walk the plain tile list; the chunked kernels take the one laid out per XCD.
     w.plan.max_tiles = max_tiles;
-    w.plan.tiles_per_xcd = decode_sized ? 0 : max_tiles / 8;
+    w.plan.tiles_per_xcd = max_tiles / 8;
     {
         const size_t items = static_cast<size_t>(T) * (Hp / 8);
         hipLaunchKernelGGL(moe_prepare_kernel, dim3(static_cast<unsigned>(1 + (items + 1023) / 1024)), dim3(1024), 0, s,
@@ -1143,18 +722,14 @@ lhip_status lhip_mxfp4_moe_bf16_mode(const void *w_gate_up_planar, const void *w
     a1.tile_expert = w.plan.tile_expert; a1.tile_row0 = w.plan.tile_row0; a1.tile_rows = w.plan.tile_rows;
     a1.tile_run0 = w.plan.tile_run0; a1.tile_runlen = w.plan.tile_runlen;
     a1.n_tiles = w.plan.n_tiles; a1.tiles_per_xcd = w.plan.tiles_per_xcd; a1.out = w.act;
-    const bool whole_rows = mt == 1 && decode_sized && moe_small_lds_bytes(Hp) <= 150 * 1024;
     // Every gated kernel launched below quantises its result for the down GEMM in its epilogue.
     a1.q_hi = w.a_hi; a1.q_lo = w.a_lo; a1.q_sc = w.a_sc; a1.q_kp = Ip;
     // Column blocks: 4 waves x (NT/2) gate/up pairs of 16.  Tall row tiles take 4 weight
     // fragments per wave, so each activation fragment read from LDS feeds twice the MFMAs.
-    const int cb1 = (I + 63) / 64, cb1w = (I + 127) / 128;
+    const int cb1w = (I + 127) / 128;
     lhip_status st;
     switch (mt) {
-        case 1:
-            st = whole_rows ? launch_moe_gemm_small<2, true>(a1, cb1, max_tiles, s)
-                                                       : launch_moe_gemm<1, 4, true>(a1, cb1w, max_tiles, s);
-            break;
+        case 1: st = launch_moe_gemm<1, 4, true>(a1, cb1w, max_tiles, s); break;
         case 2: st = launch_moe_gemm<2, 4, true>(a1, cb1w, max_tiles, s); break;
         case 4: st = launch_moe_gemm<4, 4, true, 1, 2>(a1, cb1w, max_tiles, s); break;
         case 5: st = launch_moe_gemm<5, 4, true, 1, 2>(a1, cb1w, max_tiles, s); break;
@@ -1170,9 +745,7 @@ lhip_status lhip_mxfp4_moe_bf16_mode(const void *w_gate_up_planar, const void *w
     a2.tile_run0 = w.plan.tile_run0; a2.tile_runlen = w.plan.tile_runlen;
     a2.n_tiles = w.plan.n_tiles; a2.tiles_per_xcd = w.plan.tiles_per_xcd; a2.out = w.out;
     if (mt == 1) {
-        st = decode_sized && moe_small_lds_bytes(Ip) <= 150 * 1024
-                 ? launch_moe_gemm_small<1, false>(a2, (H + 63) / 64, max_tiles, s)
-                                                   : launch_moe_gemm<1, 2, false>(a2, (H + 127) / 128, max_tiles, s);
+        st = launch_moe_gemm<1, 2, false>(a2, (H + 127) / 128, max_tiles, s);
     } else {
         const int cb2 = (H + 127) / 128, cb2w = (H + 255) / 256;  // 4 waves x NT fragments of 16
         switch (mt) {
@@ -1212,7 +785,7 @@ lhip_status lhip_mxfp4_moe_read_intermediates_mode(const void *workspace_dev, fl
     if (!act_dev && !down_dev) return LHIP_OK;
     MoeWorkspace w = carve(const_cast<void *>(workspace_dev), t, h, i, e, topk);
     const int R = static_cast<int>(t * topk);
-    if (mode == LHIP_MOE_EXACT)
+    if (mode == LHIP_MOE_EXACT || moe_few_takes(static_cast<int>(t), static_cast<int>(h), static_cast<int>(i), static_cast<int>(e), static_cast<int>(topk)))
         return moe_exact_read_intermediates(w, act_dev, down_dev, R, static_cast<int>(i), static_cast<int>(h), as_stream(stream));
     hipLaunchKernelGGL(moe_read_intermediates_kernel, dim3(static_cast<unsigned>(R)), dim3(256), 0, as_stream(stream),
                        w.plan.slot_of, w.a_hi, w.a_lo, w.a_sc, w.out, act_dev, down_dev, R, static_cast<int>(i),

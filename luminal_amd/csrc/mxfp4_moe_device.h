@@ -21,9 +21,6 @@ constexpr int kARow = 160;       // LDS bytes per activation row of a chunk: 128
                                  // lane (r, g) at r * pitch + 16 g, take twice as long: measured 8.0 against 4.3 cycles per read)
 
 static inline int64_t pad128(int64_t k) { return (k + 127) / 128 * 128; }
-// Row pitch of a whole quantised activation row in LDS (Kp a multiple of 128): the row plus padding that makes the
-// pitch 160 mod 256, the residue measured free of bank conflicts for the fragment reads.
-__host__ __device__ static inline int moe_small_pitch(int Kp) { return Kp + ((Kp & 255) ? 32 : 160); }
 
 // ---------------------------------------------------------------------------
 // Plan: group the R = T*topk routed entries by expert and cut each expert's rows
@@ -254,14 +251,16 @@ static inline MoeWorkspace carve(void *base, int64_t T, int64_t H, int64_t I, in
     return w;
 }
 
-static inline size_t moe_small_lds_bytes(int Kp) { return 2 * 16 * static_cast<size_t>(moe_small_pitch(Kp)) + 16 * (Kp / 32); }
-
-// Routed rows the direct (two-launch) forms take: one token's top-4.
+// Routed rows whose down product adds the experts up itself: one token's top-4.
 constexpr int kDirectRows = 4;
 
 // mxfp4_moe.hip: y[t][h] = bf16( sum_s wts[t][s] * out[slot_of[t*topk+s]][h] )
 lhip_status moe_launch_combine(const float *out, const int *slot_of, const float *wts, __bf16 *y, int T, int H, int topk,
                                hipStream_t s);
+// mxfp4_moe_few.hip: whether a layer of so few routed rows goes to its kernels, which expand the weights exactly, in either mode: the
+// block-scaled form, whose price is its quantised activations' launch and tiles, was slower there (us, block-scaled / exact, 32
+// experts of 2880 x 2880, top 4: T = 1 24.5 / 21.3, T = 4 52 / 41, T = 8 73 / 58, T = 16 82 / 74).
+bool moe_few_takes(int T, int H, int I, int E, int topk);
 // mxfp4_moe_exact.hip: the layer on the bf16 matrix instruction (weights expanded exactly), and its intermediates.
 lhip_status moe_exact_forward(const uint8_t *gu, const uint8_t *dn, const __bf16 *x, const int32_t *sel_dev,
                               const float *wts_dev, __bf16 *y, int T, int H, int I, int E, int topk, MoeWorkspace &w,

@@ -326,9 +326,7 @@ lhip_status moe_exact_forward(const uint8_t *gu, const uint8_t *dn, const __bf16
     const uint8_t *gu_sc = gu + mx_scale_offset(static_cast<int64_t>(E) * 2 * I, H);
     const uint8_t *dn_sc = dn + mx_scale_offset(static_cast<int64_t>(E) * H, I);
 
-    // (A K of several segments pays while the tiles are few: 8 experts of 4096 x 14336, top 2, T = 1 118 -> 43 us, T = 16 145 -> 141, T = 32
-    // 150 -> 163; 32 of 5120 x 5120, top 2, T = 6 103 -> 97, T = 8 110 -> 116.)
-    if (R <= kFewRows && ((H <= 4096 && I <= 4096) || R <= (E <= 16 ? 32 : 12)))
+    if (moe_few_takes(T, H, I, E, topk))
         return moe_few_forward(MoeFewLayer{gu, gu_sc, dn, dn_sc, x, sel_dev, wts_dev, y, w.act, w.out, w.plan.slot_of, T, H, I, E, topk}, s);
 
     const int mt = exact_tile_fragments(R, E, H, I, moe_tall_supports(T, H, I));

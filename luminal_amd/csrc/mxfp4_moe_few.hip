@@ -303,6 +303,13 @@ static lhip_status launch_few(const uint8_t *nib, const uint8_t *sc, const __bf1
     return LHIP_OK;
 }
 
+// (A K of several segments pays while the tiles are few: 8 experts of 4096 x 14336, top 2, T = 1 118 -> 43 us, T = 16 145 -> 141, T = 32
+// 150 -> 163; 32 of 5120 x 5120, top 2, T = 6 103 -> 97, T = 8 110 -> 116.)
+bool moe_few_takes(int T, int H, int I, int E, int topk) {
+    const int64_t R = static_cast<int64_t>(T) * topk;
+    return R <= kFewRows && ((H <= 512 * kFewD && I <= 512 * kFewD) || R <= (E <= 16 ? 32 : 12));
+}
+
 lhip_status moe_few_forward(const MoeFewLayer &l, hipStream_t s) {
     const int R = l.T * l.topk;
     if (lhip_status st = launch_few<true>(l.gu, l.gu_sc, l.x, l, 2 * l.I, l.H, l.I, l.act, s)) return st;
