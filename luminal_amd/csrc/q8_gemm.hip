@@ -9,8 +9,9 @@
 // (crates/luminal_metal/src/quantized.rs:54-61,63-199).  That kernel rounds
 // q * d to the activation type first; these keep the weights exact: the int8
 // codes go to the matrix cores as they are (exact in bf16) and the block's scale
-// multiplies the f32 sum of the block's products.  Three kernels share the shapes:
+// multiplies the f32 sum of the block's products.  Four kernels share the shapes:
 //   * at most 128 rows: q8_gemm_skinny.hip, bound by streaming the weights;
+//   * more rows, or an odd N, and so few tiles that K would have to be sliced: q8_gemm_deep.hip;
 //   * more rows: q8_gemm_wide.hip, tiles of 256x256 and 128x256, over slices of K
 //     where those are few;
 //   * more rows but too few such tiles and a K too short to slice: the kernel in
@@ -34,6 +35,7 @@
 #include <utility>
 
 #include "common.h"
+#include "q8_gemm_deep.h"
 #include "q8_gemm_rows.h"
 #include "q8_gemm_wide.h"
 #include "q8_mma_device.h"
@@ -347,6 +349,7 @@ constexpr int kTileSkinny = 5;        // K slices chosen by the library
 constexpr int kTileSkinnySplit = 50;  // + number of K slices
 constexpr int kTileSliced = 120;      // + number of K slices: the large tile over slices of K, then a reduction
 constexpr int kTileTail = 200;        // more than one round of large tiles, whatever ends its last round first
+constexpr int kTileDeep = 1000;       // + 10 mt + nt: q8_gemm_deep.hip; not by name from outside
 
 // A product of more than 256 tiles of 128x256 runs in rounds of 256 workgroups (one per CU), and a last round that
 // is partly filled takes as long as a full one.  The plan below gives whole rounds to one launch and the remaining
@@ -437,6 +440,8 @@ static lhip_status gemm_dispatch(const void *planar_dev, const void *x_dev, void
         return q8_gemm_skinny_launch(qs, ds, x_dev, y_dev, mi, ni, ki, out, tile == kTileSkinny ? 0 : tile - kTileSkinnySplit, s,
                                      scratch.own || k % 512 != 0, scratch.ws, scratch.floats);
     }
+    if (tile > kTileDeep)
+        return q8_gemm_deep_launch(qs, ds, x_dev, kWdBf16, y_dev, mi, ni, ki, out, DeepPlan{(tile - kTileDeep) / 10, tile % 10}, s);
     if (tile > kTileSliced && tile <= kTileSliced + 16) {
         // Few output tiles (the down projection of a 512-token prompt: 64 tiles of 128x256): slices of K fill the chip,
         // f32 partial planes go to the scratch array and are added in slice order.
@@ -555,8 +560,9 @@ static int gemm_tiles(int64_t m, int64_t n, int64_t k, int out, const void *y, s
     return tile;
 }
 
-static int gemm_auto_tile(int64_t m, int64_t n, int64_t k, int out, const void *y, size_t room) {
-    double us;
+// The weight-streaming kernel, or slices or tiles; *us: what the latter take.
+static int gemm_slices_or_tiles(int64_t m, int64_t n, int64_t k, int out, const void *y, size_t room, double *us) {
+    *us = 0.0;
     // Few activation rows: the product is bound by the weight stream.  A K that is no multiple of 512 is one for that kernel
     // unless the tiles end within a tenth of it, which they do for a K of one step and for many weight rows.  Measured, us,
     // tiles -> streamed, without and with a workspace: 16 x 2880 x 2880 33 -> 9.9 and 33 -> 8.6, 45 x 2880 x 2880 33 -> 17 and 15.9 ->
@@ -565,16 +571,35 @@ static int gemm_auto_tile(int64_t m, int64_t n, int64_t k, int out, const void *
     if (m <= 128 && n <= kMaxDim && k <= kMaxDim &&
         q8_gemm_skinny_supports(static_cast<int>(m), static_cast<int>(n), static_cast<int>(k), out, y)) {
         if (k % 512 == 0) return kTileSkinny;
-        const int tile = gemm_tiles(m, n, k, out, y, room, &us);
-        return 1.1 * q8_gemm_skinny_us(static_cast<int>(m), static_cast<int>(n), static_cast<int>(k), room) < us ? kTileSkinny : tile;
+        const int tile = gemm_tiles(m, n, k, out, y, room, us);
+        return 1.1 * q8_gemm_skinny_us(static_cast<int>(m), static_cast<int>(n), static_cast<int>(k), room) < *us ? kTileSkinny : tile;
     }
-    return gemm_tiles(m, n, k, out, y, room, &us);
+    return gemm_tiles(m, n, k, out, y, room, us);
+}
+
+// Those, or the kernel whose workgroups walk all of K, where it ends a twentieth sooner, the spread of the estimates.  Measured, us,
+// tiles and slices -> that kernel: 192 x 6000 x 1536 23.3 -> 11.7, 256 x 4096 x 4096 27.0 -> 20.5, 1024 x 1024 x 4096 28.6 -> 22.6, 352 x
+// 3067 x 12288 (no slices for an odd N) 191 -> 69; the other way 256 x 14336 x 4096 54 <- 66, 592 x 9820 x 768 23 <- 38.  Up to 128 rows the
+// streaming kernel and its lines stand, and so do the slices that the header promises a long K: at 8192 and more they are ahead for
+// most sizes (350 x 6364 x 10688 82 <- 119, 207 x 2276 x 12992 40 <- 43), though not for few weight rows (171 x 544 x 8192 26.3 -> 19.8).
+static int gemm_auto_tile(int64_t m, int64_t n, int64_t k, int out, const void *y, size_t room) {
+    double us, deep_us;
+    const int tile = gemm_slices_or_tiles(m, n, k, out, y, room, &us);
+    const bool streams = m <= 128 && q8_gemm_skinny_supports(static_cast<int>(m), static_cast<int>(n), static_cast<int>(k), out, y);
+    const bool long_slices = tile > kTileSliced && tile < kTileTail && k >= 8192;
+    if (streams || long_slices || k < 256 || !q8_gemm_deep_supports(k, nullptr)) return tile;
+    const DeepPlan deep = q8_gemm_deep_plan(m, n, k, &deep_us);
+    return 1.05 * deep_us < us ? kTileDeep + 10 * deep.mt + deep.nt : tile;
 }
 
 void q8_gemm_describe(int64_t m, int64_t n, int64_t k, size_t room, int32_t plan[3]) {
     room = room == SIZE_MAX ? gemm_plain_room(k) : room < kGemmScratchFloats ? room : kGemmScratchFloats;
     const int tile = gemm_auto_tile(m, n, k, kOutBf16, nullptr, room);
     if (tile == kTileSkinny) return q8_gemm_skinny_describe(static_cast<int>(m), static_cast<int>(n), static_cast<int>(k), room, plan);
+    if (tile > kTileDeep) {
+        plan[0] = 4, plan[1] = 32 * (tile % 10), plan[2] = 1;
+        return;
+    }
     plan[0] = 3, plan[1] = 0;
     plan[2] = tile == kTileTail ? 0 : tile > kTileSliced ? tile - kTileSliced : 1;
 }
@@ -587,6 +612,7 @@ extern "C" {
 
 lhip_status lhip_q8_0_matmul_bf16_cfg(const void *planar_dev, const void *x_dev, void *y_dev, int64_t m, int64_t n,
                                       int64_t k, int tile, void *stream) {
+    if (tile > kTileTail) return LHIP_ERR_UNSUPPORTED;
     if (tile > kTileSliced && tile <= kTileSliced + 16 && k % (kBK * 4 * (tile - kTileSliced)) != 0) return LHIP_ERR_UNSUPPORTED;
     if ((tile == kTileSkinny || (tile > kTileSkinnySplit && tile <= kTileSkinnySplit + 64)) && k % 512 != 0) return LHIP_ERR_UNSUPPORTED;
     return gemm_dispatch(planar_dev, x_dev, y_dev, m, n, k, tile, kOutBf16, stream);
@@ -610,8 +636,10 @@ lhip_status lhip_q8_0_matmul_bf16_swiglu(const void *planar_dev, const void *x_d
 size_t lhip_q8_0_matmul_bf16_workspace_nbytes(int64_t m, int64_t n, int64_t k, int32_t out_form) {
     if (check_q8_shape(n, k) != LHIP_OK || m <= 0 || m > kMaxDim || k % kBK != 0) return 0;
     if (out_form < kOutBf16 || out_form > kOutSwiglu) return 0;
-    // the plan with all its slices (an aligned output is assumed: K is sliced for aligned outputs only)
-    const int tile = gemm_auto_tile(m, n, k, out_form, nullptr, kGemmScratchFloats);
+    // the plan with all its slices (an aligned output is assumed: K is sliced for aligned outputs only), also where the kernel that
+    // needs no planes is ahead of it: callers' sizes stay what they were
+    double us;
+    const int tile = gemm_slices_or_tiles(m, n, k, out_form, nullptr, kGemmScratchFloats, &us);
     size_t floats = 0;
     if (tile > kTileSliced && tile <= kTileSliced + 16)
         floats = static_cast<size_t>(tile - kTileSliced) * m * n;

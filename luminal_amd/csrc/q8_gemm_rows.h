@@ -6,16 +6,18 @@
 #include <stdint.h>
 
 #include "common.h"
+#include "q8_gemm_deep.h"
 
 namespace lhip {
 
 // How a product is run: by passes of 64 rows of q8_gemm_skinny_device.h (kStream), by q8_gemm_rows.hip (kRows: `n_main` leading
-// weight rows in whole rounds of workgroups, the others over `slices` K slices; n_main = 0: all of them), or by the
-// tiles of q8_gemm_wide.hip (kWide).
+// weight rows in whole rounds of workgroups, the others over `slices` K slices; n_main = 0: all of them), by the
+// tiles of q8_gemm_wide.hip (kWide), or by q8_gemm_deep.hip (kDeep, f16 only).
 struct RowsPlan {
-    enum Kind { kStream, kRows, kWide, kNone } kind = kStream;
+    enum Kind { kStream, kRows, kWide, kDeep, kNone } kind = kStream;
     int n_main = 0, slices = 1, width = 256;  // width = weight rows of a tile (of the n_main: 256)
     size_t floats = 0;  // of partial planes
+    DeepPlan deep;
 };
 // Floats of partial planes the plan of (m, n, k) uses when it has the library's own scratch array to itself: what a caller's workspace
 // must hold for the same plan (and the same bits) with either activation type.  plans[0], plans[1]: those of f32 and f16.

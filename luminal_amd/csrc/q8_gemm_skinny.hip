@@ -397,7 +397,21 @@ static RowsPlan rows_plan(int64_t m, int n, int k, bool f16, size_t room, bool s
     // A product of which the plain call kept nothing in the library's array, so that its calls may overlap, when these plans had tiles
     // of 256 in up to 16 slices, none of them behind a number that leaves one empty, at 1.2 (f32) or 0.66 us per block (`early`), keeps
     // nothing there now.
-    return stream && early.floats == 0 && !(early.kind == RowsPlan::kStream && planes) ? bare : best;
+    if (stream && early.floats == 0 && !(early.kind == RowsPlan::kStream && planes)) best = bare, best_us = bare_us;
+    // The kernel whose workgroups walk all of K, for f16 (three limbs an f32 value are staged for too few weight rows there): from one
+    // round of its quads of blocks on, and above 128 rows where the streaming kernel takes the K, whose strips serve both types up to
+    // there.  A tenth ahead, the spread of the estimates.  Measured, us, what the rules above choose -> that kernel: 45 x 2880 x 2880
+    // 11.8 -> 8.3, 128 x 2880 x 2880 17.8 -> 10.9, 256 x 6000 x 1536 22.6 -> 14.1, 256 x 4096 x 4096 24.7 -> 20.7; the other way 256 x
+    // 4096 x 14336 58 <- 75, 512 x 14336 x 4096 84 <- 130, 186 x 9184 x 3072 30.5 <- 32.4.
+    if (f16 && k >= 512 && (!stream || m > 128) && q8_gemm_deep_supports(k, nullptr)) {
+        double us;
+        const DeepPlan deep = q8_gemm_deep_plan(m, n, k, &us);
+        if (1.1 * us < best_us) {
+            best = RowsPlan{RowsPlan::kDeep, 0, 1, 0, best.floats};  // (it needs no planes; callers' sizes stay what they were)
+            best.deep = deep;
+        }
+    }
+    return best;
 }
 
 size_t q8_gemm_split_workspace_floats(int64_t m, int n, int k, RowsPlan *plans) {
@@ -431,6 +445,8 @@ void q8_gemm_split_describe(int64_t m, int n, int k, bool f16, size_t room, int3
         plan[0] = 1, plan[1] = 16 * strips.cw, plan[2] = strips.splits;
     } else if (p.kind == RowsPlan::kRows) {
         plan[0] = 2, plan[1] = p.width, plan[2] = p.n_main ? 0 : p.slices;
+    } else if (p.kind == RowsPlan::kDeep) {
+        plan[0] = 4, plan[1] = 32 * p.deep.nt, plan[2] = 1;
     } else {
         plan[0] = 3, plan[1] = 0, plan[2] = 1;
     }
@@ -448,6 +464,8 @@ lhip_status q8_gemm_split_launch(const int8_t *qs, const __half *ds, const void 
     if (plan.floats > room) plan = rows_plan(m, n, k, f16, room, stream);
     float *scratch = own_workspace ? ws : (plan.kind == RowsPlan::kRows && plan.slices > 1 ? sk_scratch_ptr() : nullptr);
     if (plan.kind == RowsPlan::kWide) return q8_gemm_wide_launch(qs, ds, x, kWdF16, y, static_cast<int>(m), n, k, kWdOutF16, s);
+    if (plan.kind == RowsPlan::kDeep)
+        return q8_gemm_deep_launch(qs, ds, x, kWdF16, y, static_cast<int>(m), n, k, kWdOutF16, plan.deep, s);
     if (plan.kind == RowsPlan::kRows) {
         if (plan.slices > 1 && !scratch) return LHIP_ERR_HIP;
         const int mi = static_cast<int>(m), tail = n - plan.n_main;
