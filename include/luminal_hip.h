@@ -411,7 +411,8 @@ lhip_status lhip_attention_f32(const float *qkv_dev, const float *k_cache_dev, c
  * [(q_heads + 2*kv_heads)*head_dim] and is not modified; out_dev [q_heads*head_dim].  The keys of every KV head
  * are split over several workgroups whose partial softmax states meet in workspace_dev
  * (lhip_attention_decode_workspace_nbytes bytes, 256-byte aligned, contents irrelevant on entry; calls sharing a
- * workspace must be ordered on one stream) and are merged by a second small kernel.  Built for head_dim 64 or 128 and
+ * workspace must be ordered on one stream) and are merged by a second small kernel; a cache of at most 512 positions
+ * (of 16 per range: 256 / kv_heads ranges, at most 32) takes one kernel for both, with the same bits.  Built for head_dim 64 or 128 and
  * q_heads / kv_heads in {1, 2, 4, 8}: LHIP_ERR_UNSUPPORTED otherwise (the workspace size is then 0). */
 size_t lhip_attention_decode_workspace_nbytes(int64_t q_heads, int64_t kv_heads, int64_t head_dim);
 lhip_status lhip_attention_decode_f32(const float *qkv_dev, float *k_cache_dev, float *v_cache_dev, float *out_dev,
