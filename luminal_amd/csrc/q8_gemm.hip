@@ -10,8 +10,8 @@
 // q * d to the activation type first; these keep the weights exact: the int8
 // codes go to the matrix cores as they are (exact in bf16) and the block's scale
 // multiplies the f32 sum of the block's products.  Four kernels share the shapes:
-//   * at most 128 rows: q8_gemm_skinny.hip, bound by streaming the weights;
-//   * more rows, or an odd N, and so few tiles that K would have to be sliced: q8_gemm_deep.hip;
+//   * few rows, 128 at most: q8_gemm_skinny.hip, bound by streaming the weights;
+//   * some dozens to hundreds of rows, or an odd N, and so few tiles that K would have to be sliced: q8_gemm_deep.hip;
 //   * more rows: q8_gemm_wide.hip, tiles of 256x256 and 128x256, over slices of K
 //     where those are few;
 //   * more rows but too few such tiles and a K too short to slice: the kernel in
@@ -579,17 +579,28 @@ static int gemm_slices_or_tiles(int64_t m, int64_t n, int64_t k, int out, const 
 
 // Those, or the kernel whose workgroups walk all of K, where it ends a twentieth sooner, the spread of the estimates.  Measured, us,
 // tiles and slices -> that kernel: 192 x 6000 x 1536 23.3 -> 11.7, 256 x 4096 x 4096 27.0 -> 20.5, 1024 x 1024 x 4096 28.6 -> 22.6, 352 x
-// 3067 x 12288 (no slices for an odd N) 191 -> 69; the other way 256 x 14336 x 4096 54 <- 66, 592 x 9820 x 768 23 <- 38.  Up to 128 rows the
-// streaming kernel and its lines stand, and so do the slices that the header promises a long K: at 8192 and more they are ahead for
-// most sizes (350 x 6364 x 10688 82 <- 119, 207 x 2276 x 12992 40 <- 43), though not for few weight rows (171 x 544 x 8192 26.3 -> 19.8).
+// 3067 x 12288 (no slices for an odd N) 191 -> 69; the other way 256 x 14336 x 4096 54 <- 66, 592 x 9820 x 768 23 <- 38.  The slices that the
+// header promises a long K stay: at 8192 and more they are ahead for most sizes (350 x 6364 x 10688 82 <- 119, 207 x 2276 x 12992 40
+// <- 43), though not for few weight rows (171 x 544 x 8192 26.3 -> 19.8).
+// Up to 128 rows the streaming kernel stays for K below three of its steps of 512 and for every other K.  From three steps on the
+// other kernel takes what it ends a tenth sooner above 64 rows, for which the strips are bound by their reads of the activations and no
+// longer by the weights, and a quarter sooner from 33 on.  Measured, us, strips -> that kernel: 80 x 4096 x 4096 16.8 -> 12.7, 96 x 14336 x
+// 4096 33.7 -> 29.8, 128 x 6000 x 1536 13.8 -> 9.9, 96 x 8148 x 2048 15.8 -> 11.4, 45 x 6144 x 4096 17.8 -> 12.8, 45 x 14336 x 4096 27.6 -> 22.6;
+// the other way 45 x 4096 x 4096 12.7, 64 x 6144 x 4096 15.4 <- 15.7 and 64 x 6000 x 1536 9.2 <- 9.3 as they are.
 static int gemm_auto_tile(int64_t m, int64_t n, int64_t k, int out, const void *y, size_t room) {
     double us, deep_us;
     const int tile = gemm_slices_or_tiles(m, n, k, out, y, room, &us);
     const bool streams = m <= 128 && q8_gemm_skinny_supports(static_cast<int>(m), static_cast<int>(n), static_cast<int>(k), out, y);
     const bool long_slices = tile > kTileSliced && tile < kTileTail && k >= 8192;
-    if (streams || long_slices || k < 256 || !q8_gemm_deep_supports(k, nullptr)) return tile;
+    double margin = 1.05;
+    if (streams) {
+        if (m <= 32 || k % 512 != 0 || k < 1536) return tile;
+        us = q8_gemm_skinny_us(static_cast<int>(m), static_cast<int>(n), static_cast<int>(k), room);
+        margin = m > 64 ? 1.1 : 1.25;
+    }
+    if (long_slices || k < 256 || !q8_gemm_deep_supports(k, nullptr)) return tile;
     const DeepPlan deep = q8_gemm_deep_plan(m, n, k, &deep_us);
-    return 1.05 * deep_us < us ? kTileDeep + 10 * deep.mt + deep.nt : tile;
+    return margin * deep_us < us ? kTileDeep + 10 * deep.mt + deep.nt : tile;
 }
 
 void q8_gemm_describe(int64_t m, int64_t n, int64_t k, size_t room, int32_t plan[3]) {

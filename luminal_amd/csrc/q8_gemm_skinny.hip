@@ -399,11 +399,13 @@ static RowsPlan rows_plan(int64_t m, int n, int k, bool f16, size_t room, bool s
     // nothing there now.
     if (stream && early.floats == 0 && !(early.kind == RowsPlan::kStream && planes)) best = bare, best_us = bare_us;
     // The kernel whose workgroups walk all of K, for f16 (three limbs an f32 value are staged for too few weight rows there): from one
-    // round of its quads of blocks on, and above 128 rows where the streaming kernel takes the K, whose strips serve both types up to
-    // there.  A tenth ahead, the spread of the estimates.  Measured, us, what the rules above choose -> that kernel: 45 x 2880 x 2880
-    // 11.8 -> 8.3, 128 x 2880 x 2880 17.8 -> 10.9, 256 x 6000 x 1536 22.6 -> 14.1, 256 x 4096 x 4096 24.7 -> 20.7; the other way 256 x
-    // 4096 x 14336 58 <- 75, 512 x 14336 x 4096 84 <- 130, 186 x 9184 x 3072 30.5 <- 32.4.
-    if (f16 && k >= 512 && (!stream || m > 128) && q8_gemm_deep_supports(k, nullptr)) {
+    // round of its quads of blocks on, and where the streaming kernel takes the K, from three of that kernel's steps on or above 128
+    // rows (up to 64, where its f16 results are those of f32 rounded, this rule is not reached).  A tenth ahead, the spread of the
+    // estimates.  Measured, us, what the rules above choose -> that kernel: 45 x 2880 x 2880 11.8 -> 8.3, 128 x 2880 x 2880 17.8 -> 10.9,
+    // 256 x 6000 x 1536 22.6 -> 14.1, 256 x 4096 x 4096 24.7 -> 20.7, 80 x 4096 x 4096 17.6 -> 12.6, 96 x 8148 x 2048
+    // 18.8 -> 11.3; the other way 256 x 4096 x 14336 58 <- 75, 512 x 14336 x 4096
+    // 84 <- 130, 186 x 9184 x 3072 30.5 <- 32.4.
+    if (f16 && k >= 512 && (!stream || k >= 1536 || m > 128) && q8_gemm_deep_supports(k, nullptr)) {
         double us;
         const DeepPlan deep = q8_gemm_deep_plan(m, n, k, &us);
         if (1.1 * us < best_us) {
