@@ -588,7 +588,7 @@ static int gemm_slices_or_tiles(int64_t m, int64_t n, int64_t k, int out, const 
 // 4096 33.7 -> 29.8, 128 x 6000 x 1536 13.8 -> 9.9, 96 x 8148 x 2048 15.8 -> 11.4, 45 x 6144 x 4096 17.8 -> 12.8, 45 x 14336 x 4096 27.6 -> 22.6;
 // the other way 45 x 4096 x 4096 12.7, 64 x 6144 x 4096 15.4 <- 15.7 and 64 x 6000 x 1536 9.2 <- 9.3 as they are.
 static int gemm_auto_tile(int64_t m, int64_t n, int64_t k, int out, const void *y, size_t room) {
-    double us, deep_us;
+    double us;
     const int tile = gemm_slices_or_tiles(m, n, k, out, y, room, &us);
     const bool streams = m <= 128 && q8_gemm_skinny_supports(static_cast<int>(m), static_cast<int>(n), static_cast<int>(k), out, y);
     const bool long_slices = tile > kTileSliced && tile < kTileTail && k >= 8192;
@@ -599,8 +599,8 @@ static int gemm_auto_tile(int64_t m, int64_t n, int64_t k, int out, const void *
         margin = m > 64 ? 1.1 : 1.25;
     }
     if (long_slices || k < 256 || !q8_gemm_deep_supports(k, nullptr)) return tile;
-    const DeepPlan deep = q8_gemm_deep_plan(m, n, k, &deep_us);
-    return margin * deep_us < us ? kTileDeep + 10 * deep.mt + deep.nt : tile;
+    const DeepPlan deep = q8_gemm_deep_plan(m, n, k, us / margin);
+    return deep.mt ? kTileDeep + 10 * deep.mt + deep.nt : tile;
 }
 
 void q8_gemm_describe(int64_t m, int64_t n, int64_t k, size_t room, int32_t plan[3]) {

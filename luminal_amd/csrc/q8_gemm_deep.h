@@ -15,8 +15,8 @@ struct DeepPlan {
     int mt = 0, nt = 0;  // 0: not by this kernel
 };
 bool q8_gemm_deep_supports(int64_t k, const void *x);
-// The form that ends first for a product of K >= 128, and its time, us.
-DeepPlan q8_gemm_deep_plan(int64_t m, int64_t n, int64_t k, double *us);
+// The form that ends first for a product of K >= 128 if it takes less than `limit` us (else mt = 0).
+DeepPlan q8_gemm_deep_plan(int64_t m, int64_t n, int64_t k, double limit);
 lhip_status q8_gemm_deep_launch(const int8_t *qs, const __half *ds, const void *x, WdType type, void *y, int m, int n, int k,
                                 int out, DeepPlan plan, hipStream_t s);
 

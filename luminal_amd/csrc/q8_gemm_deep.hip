@@ -359,16 +359,19 @@ static constexpr DeepTimes kDpTimes[] = {
     {{8, 1}, 3.85, 1.50, 1.86, 0.40}, {{2, 2}, 4.31, 0.49, 1.41, 0.03}, {{3, 2}, 4.41, 0.61, 1.58, 0.09}, {{4, 2}, 4.10, 1.94, 1.87, 0.25},
     {{6, 2}, 3.98, 2.24, 2.39, 0.31}, {{8, 2}, 4.06, 2.57, 3.01, 0.33}};
 
-DeepPlan q8_gemm_deep_plan(int64_t m, int64_t n, int64_t k, double *us) {
+DeepPlan q8_gemm_deep_plan(int64_t m, int64_t n, int64_t k, double limit) {
     const double walks = static_cast<double>((k + 511) / 512);
     DeepPlan best;
-    *us = 1e30;
+    if (3.85 + 0.76 * walks >= limit || m > (1 << 30) || n > (1 << 30)) return best;  // (no form takes less)
+    const uint32_t mu = static_cast<uint32_t>(m), nu = static_cast<uint32_t>(n);
+#pragma unroll
     for (const DeepTimes &t : kDpTimes) {
-        const int64_t groups = ((m + 16 * t.plan.mt - 1) / (16 * t.plan.mt)) * ((n + 32 * t.plan.nt - 1) / (32 * t.plan.nt));
+        const uint32_t mr = 16 * t.plan.mt, nr = 32 * t.plan.nt;
+        const int64_t groups = static_cast<int64_t>((mu + mr - 1) / mr) * ((nu + nr - 1) / nr);
         if (groups > 0x7ffffff0) continue;  // the grid's x extent
-        const double rounds = static_cast<double>((groups + 255) / 256), chips = static_cast<double>(groups) / 256.0;
-        const double t_us = t.launch + (rounds - 1.0) * t.round + walks * (rounds * t.walk + chips * t.fill);
-        if (t_us < *us) *us = t_us, best = t.plan;
+        const double rounds = static_cast<double>((groups + 255) >> 8), chips = static_cast<double>(groups) * (1.0 / 256.0);
+        const double us = t.launch + (rounds - 1.0) * t.round + walks * (rounds * t.walk + chips * t.fill);
+        if (us < limit) limit = us, best = t.plan;
     }
     return best;
 }

@@ -406,9 +406,8 @@ static RowsPlan rows_plan(int64_t m, int n, int k, bool f16, size_t room, bool s
     // 18.8 -> 11.3; the other way 256 x 4096 x 14336 58 <- 75, 512 x 14336 x 4096
     // 84 <- 130, 186 x 9184 x 3072 30.5 <- 32.4.
     if (f16 && k >= 512 && (!stream || k >= 1536 || m > 128) && q8_gemm_deep_supports(k, nullptr)) {
-        double us;
-        const DeepPlan deep = q8_gemm_deep_plan(m, n, k, &us);
-        if (1.1 * us < best_us) {
+        const DeepPlan deep = q8_gemm_deep_plan(m, n, k, best_us / 1.1);
+        if (deep.mt) {
             best = RowsPlan{RowsPlan::kDeep, 0, 1, 0, best.floats};  // (it needs no planes; callers' sizes stay what they were)
             best.deep = deep;
         }

@@ -88,6 +88,17 @@ static bool on_matrix_cores(int64_t m, int64_t n, int64_t k, const void *x, cons
                             RowsPlan *plan = nullptr) {
     if (q8_gemm_split_supports(static_cast<int>(n), static_cast<int>(k), x, y, f16)) return m >= split_min_rows(n, k, f16);
     if (k < 256 || !aligned(x, 16)) return false;
+    // f16 by the kernel that walks all of K, which keeps no planes (more rows than these are for the matrix cores by the lines below too):
+    // 2880 x 2880 at 10 / 12 / 14 rows 9.8 / 11.3 / 12.7 as matvecs, 7.9 there; 6000 x 1600 at 8 9.2 and 5.9, 23 x 4830 x 1024 13.9 and 6.1.
+    if (f16 && k >= 512 && m <= 32 && m > q8_gemv_rows_per_pass(k, f16) && q8_gemm_deep_supports(k, x) &&
+        q8_gemm_deep_plan(m, n, k, matvecs_us(m, n, k, f16) / 1.1).mt) {
+        RowsPlan plans[2];
+        q8_gemm_split_workspace_floats(m, static_cast<int>(n), static_cast<int>(k), plans);
+        if (plans[1].kind == RowsPlan::kDeep) {
+            if (plan) *plan = plans[1];
+            return true;
+        }
+    }
     const int64_t codes = n * k;
     const int64_t min_rows = codes >= (int64_t{32} << 20) ? 3 : codes >= (int64_t{16} << 20) ? 6 : codes >= (int64_t{8} << 20) ? 8 : 12;
     if (m < (f16 ? min_rows * 5 / 4 : min_rows)) return false;

@@ -70,3 +70,17 @@ def test_an_infinity_and_a_nan_stay_in_their_rows():
     rest = [r for r in range(m) if r not in (3, 70)]
     assert bool(((y - want).abs() <= bound + want.abs() * 2.0 ** -8)[rest].all())
     assert bool(y[70].isnan().all()) and not bool(y[3].isfinite().any())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(10, 2880, 2880), (8, 6000, 1600), (23, 4831, 1024)])
+def test_f16_of_a_few_rows(m, n, k):
+    """Fewer rows than a tile, that would be matvecs otherwise; the plain C call, which has no workspace, gives the operator's bits."""
+    assert kernel_of(m, n, k, 1) == (4, 1)
+    w, x, want, bound = operands(m, n, k, torch.float16)
+    y = QuantizedMatmul().process(x, w)
+    assert bool(((y.double() - want).abs() <= bound + want.abs() * 2.0 ** -11 + 2.0 ** -25).all())
+    plain = torch.full_like(y, float("nan"))
+    capi.check(capi.load_library().lhip_q8_0_matmul_f16(w.planar.data_ptr(), x.data_ptr(), plain.data_ptr(), m, n, k,
+                                                        torch.cuda.current_stream().cuda_stream), "f16")
+    assert torch.equal(plain.view(torch.int16), y.view(torch.int16))
