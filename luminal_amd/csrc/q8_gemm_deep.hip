@@ -83,8 +83,7 @@ __global__ __launch_bounds__(512) void q8_gemm_deep_kernel(const int8_t *qs, con
     const int m0 = mt * (16 * MT), n0 = nt * S::BN + nh * (16 * NT);
     const int rounds = (quads + kDpQuads - 1) / kDpQuads;
 
-    // ---- activations: this wave's half of its quad column's, eight rows of a pair a load, three steps ahead of their use: two in
-    // registers, one in LDS
+    // ---- activations: this wave's half of its quad column's, eight rows of a pair a request, ST - 1 steps ahead of their use
     auto a_swizzle = [](int row) { return (row >> 1) & 7; };
     const unsigned char *xb = reinterpret_cast<const unsigned char *>(x) + static_cast<size_t>(m0) * K * 2;
     const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char *)dp_lds));
