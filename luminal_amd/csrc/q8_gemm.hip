@@ -384,12 +384,13 @@ static GemmTail gemm_tail_plan(int64_t m, int64_t n, int64_t k, int out, const v
 
 // Whether the sliced remainder ends before one launch of mixed tiles: half units of a 128x256 tile over all of K (0.64
 // us per 64 of K), the remainder's share of a round, and 25 us for its launch, its planes and their sum.  Measured,
-// sliced remainder against mixed tiles: 2048 x 14336 x 4096 313 against 273 us.
+// sliced remainder against mixed tiles: 2048 x 14336 x 4096 313 against 273 us.  A remainder of two column tiles or less is compared with
+// tiles of 256 and 128 rows only and stays as it was: 1024 x 8692 x 4096 120.7 in slices and 118.7 in one launch with 192 rows.
 static bool gemm_tail_pays(const GemmTail &t, int64_t m, int64_t n, int64_t k) {
     if (t.slices < 2) return false;
     const double unit = 0.64 * static_cast<double>(k / kBK);
-    return static_cast<double>(q8_gemm_wide_ends(m, t.n_main)) * unit + 2.0 * unit / t.slices + 25.0 <
-           static_cast<double>(q8_gemm_wide_ends(m, n)) * unit;
+    return q8_gemm_wide_ends(m, t.n_main) * unit + 2.0 * unit / t.slices + 25.0 <
+           q8_gemm_wide_ends(m, n, n - t.n_main > 512) * unit;
 }
 
 // M tiles per group of the raster: the activation tiles of a group of rows stay in an XCD's L2 while its N tiles pass.
@@ -515,7 +516,7 @@ static double gemm_unsliced_us(int64_t m, int64_t n, int64_t k, int *tile) {
     double us = small < 64 ? 3.0 + 0.6 * ahead * kt : small <= 256 ? 4.3 + 1.0 * ahead * kt : 5.9 + 1.22 * ahead * kt;
     *tile = small < 64 ? 3 : 2;
     if (large >= 32 && q8_gemm_wide_supports(k)) {
-        const double wide = (n % 2 != 0 ? 7.7 : 5.4) + static_cast<double>(q8_gemm_wide_ends(m, n)) * 0.535 * kt;
+        const double wide = (n % 2 != 0 ? 7.7 : 5.4) + q8_gemm_wide_ends(m, n) * 0.535 * kt;
         if (small > 512 || wide <= us) us = wide, *tile = 0;
     }
     return us;

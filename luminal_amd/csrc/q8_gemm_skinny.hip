@@ -347,7 +347,7 @@ static RowsPlan rows_plan(int64_t m, int n, int k, bool f16, size_t room, bool s
         if (mc == m) best_us *= split_plan(mc, n, k, room).of_base;
     }
     if (f16 && q8_gemm_wide_supports(k)) {
-        const double us = 8.0 + static_cast<double>(q8_gemm_wide_ends(m, n)) * 0.32 * nblk;
+        const double us = 8.0 + q8_gemm_wide_ends(m, n) * 0.32 * nblk;
         if (us < best_us) best_us = us, best.kind = RowsPlan::kWide;
     }
     early = bare = best, early_us = bare_us = best_us;

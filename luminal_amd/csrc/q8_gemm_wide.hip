@@ -44,7 +44,7 @@ constexpr int kWdBN = 256;  // weight rows per workgroup: eight waves of 32
 template <int BM>
 struct WdShape {
     static constexpr int A_ROW = 128, B_ROW = 64;            // bytes of an activation row and of a row of codes
-    static constexpr int A_BYTES = BM * A_ROW;
+    static constexpr int A_BYTES = (BM + 63) / 64 * 64 * A_ROW;  // in whole requests of eight waves
     static constexpr int B_WAVE = 32 * B_ROW;                // the codes of a wave's weight rows
     static constexpr int B_BYTES = 8 * B_WAVE;
     static constexpr int S_BYTES = 8 * 256;                  // one dword (two blocks' scales) per lane
@@ -295,7 +295,7 @@ __device__ __forceinline__ void wd_tile_body(unsigned char *lds, const int8_t *_
 #pragma unroll
                 for (int e = 0; e < C; ++e) v[e] = swiglu_value(v[2 * e], v[2 * e + 1]);
             }
-            if (row >= M) continue;
+            if (row >= M || (NI % 4 != 0 && i0 * 16 + er >= BM)) continue;
             OT *p = yo + static_cast<size_t>(row) * pitch + col / PER;
             if (C > 1 && col + W <= n_end) {
                 typedef OT otxc __attribute__((ext_vector_type(C)));
@@ -315,7 +315,7 @@ __device__ __forceinline__ void wd_tile_body(unsigned char *lds, const int8_t *_
 #pragma unroll
     for (int i0 = 0; i0 < NI; i0 += 4) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < (NI - i0 < 4 ? NI - i0 : 4); ++i)
 #pragma unroll
             for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -326,13 +326,13 @@ __device__ __forceinline__ void wd_tile_body(unsigned char *lds, const int8_t *_
     }
 }
 
-// Weight rows below n_big in tiles of 256x256 (the first big_blocks workgroups), the others in tiles of 128x256
-// (wd_big_rows chooses the cut).  With `slices` > 1 every slice of kt_slice K tiles goes into an f32 plane of (M, N) of its
-// own.
+// Weight rows below n_big in tiles of 256x256 (the first big_blocks workgroups), the others in tiles of 128, 192 or 224 rows (`small`) x 256
+// (wd_cut chooses both).  With `slices` > 1 every slice of kt_slice K tiles goes into an f32 plane of (M, N) of its
+// own (tiles of 128x256).
 template <typename XT, int OUT>
 __global__ __launch_bounds__(512) void q8_gemm_wide_kernel(const int8_t *__restrict__ qs, const __half *__restrict__ ds,
                                                            const XT *__restrict__ x, void *__restrict__ y, int M, int N, int K,
-                                                           int n_big, int big_blocks, int slices, int kt_slice, int ldy) {
+                                                           int n_big, int big_blocks, int small, int slices, int kt_slice, int ldy) {
     extern __shared__ __attribute__((aligned(16))) unsigned char wd_lds[];
     const int kt_all = K / 64;
     int mt, nt, slice;
@@ -342,62 +342,99 @@ __global__ __launch_bounds__(512) void q8_gemm_wide_kernel(const int8_t *__restr
         wd_tile_body<256, XT, OUT>(wd_lds, qs, ds, x, y, M, K, mt * 256, nt * kWdBN, n_big, 0, kt_all, ldy);
         return;
     }
-    const int m_tiles = (M + 127) / 128;
-    if (!wd_tile(static_cast<int>(blockIdx.x) - big_blocks, m_tiles, (N - n_big + kWdBN - 1) / kWdBN, slices, min(m_tiles, 16), mt, nt, slice))
+    const int m_tiles = (M + small - 1) / small;
+    if (!wd_tile(static_cast<int>(blockIdx.x) - big_blocks, m_tiles, (N - n_big + kWdBN - 1) / kWdBN, slices, min(m_tiles, 2048 / small), mt, nt, slice))
         return;
-    const int kt0 = slice * kt_slice;
-    if (slices > 1) y = static_cast<float *>(y) + static_cast<size_t>(slice) * M * N;
-    wd_tile_body<128, XT, OUT>(wd_lds, qs, ds, x, y, M, K, mt * 128, n_big + nt * kWdBN, N, kt0, min(kt_slice, kt_all - kt0), ldy);
+    const int n0 = n_big + nt * kWdBN;
+    if (small == 192) {
+        wd_tile_body<192, XT, OUT>(wd_lds, qs, ds, x, y, M, K, mt * 192, n0, N, 0, kt_all, ldy);
+    } else if (small == 224) {
+        wd_tile_body<224, XT, OUT>(wd_lds, qs, ds, x, y, M, K, mt * 224, n0, N, 0, kt_all, ldy);
+    } else {
+        const int kt0 = slice * kt_slice;
+        if (slices > 1) y = static_cast<float *>(y) + static_cast<size_t>(slice) * M * N;
+        wd_tile_body<128, XT, OUT>(wd_lds, qs, ds, x, y, M, K, mt * 128, n0, N, kt0, min(kt_slice, kt_all - kt0), ldy);
+    }
 }
 
-// How many weight rows go to 256x256 tiles.  A tile of either height takes the same time whatever its neighbours do, a
-// 256-row one about 1.5 times a 128-row one (2.0 against 1.2-1.3 us per 64 of K), and the launch ends with its slowest CU, so
-// the cut is taken where the list of big tiles followed by small ones, dealt to 256 CUs in order, ends first: after the
-// last or last but one whole round of big tiles, or with tiles of one height only.
-static int wd_big_rows(int64_t m, int64_t n, int64_t *end = nullptr) {
-    const int64_t mt256 = (m + 255) / 256, mt128 = (m + 127) / 128;
-    const int64_t n_tiles = n / kWdBN, n_all = (n + kWdBN - 1) / kWdBN;  // whole tiles, all of them
-    auto ends = [&](int64_t c) {  // in half units of a small tile's time: a big tile is 3, a small one 2
-        const int64_t big = mt256 * c, small = mt128 * (n_all - c);
-        const int64_t t0 = big / 256 * 3, busy = big % 256;  // 256 - busy CUs are free from t0 on, busy of them from t0 + 3
-        int64_t q = busy ? 3 : 0;
-        if ((2 * small + 3 * busy) / 256 - 2 > q) q = (2 * small + 3 * busy) / 256 - 2;
-        while ((256 - busy) * (q / 2) + (q > 3 ? busy * ((q - 3) / 2) : 0) < small) ++q;
-        return t0 + q;
-    };
+// How many weight rows go to 256x256 tiles, and the height of the tiles for the others.  A tile takes the same time whatever its
+// neighbours do, one of 256 / 224 / 192 rows 1.5 / 1.37 / 1.18 times one of 128 (one round of each at K = 4096: 125, 116, 100 and 86
+// us), and the launch ends with its slowest CU, so what is taken is the list of big tiles followed by smaller ones that ends first when
+// dealt to 256 CUs in order: big tiles up to the last or last but one whole round of them, all of them, or none.  Tiles of 192 and 224
+// rows are for a last (or only) round that 128-row tiles overfill and 256-row tiles leave CUs out of; they have to be 5 % ahead (at 3 % a
+// second round of 224 rows at 2048 x 14336 x 4096 gave nothing).
+// Measured, us, 256 and 128 rows -> with them: 1500 x 6144 x 4096 (144 tiles of 256 or 288 of 128) 126 -> 102 by 192 of 192 rows, 2000 x 6144
+// x 4096 127 -> 120 by 216 of 224 rows, 700 x 14336 x 4096 126 -> 107, 800 x 10000 x 2880 90 -> 74, 1700 x 14336 x 4096 262 -> 224.
+struct WdCut {
+    int n_big = 0, small = 128;
+    double end = 0.0;  // in half units of a 128x256 tile's time
+};
+static WdCut wd_cut(int64_t m, int64_t n, bool all_heights = true) {
+    const int64_t mt256 = (m + 255) / 256, n_tiles = n / kWdBN, n_all = (n + kWdBN - 1) / kWdBN;  // whole tiles, all of them
     const int64_t rounds = mt256 * n_tiles / 256;
-    const int64_t cuts[3] = {n_tiles, rounds * 256 / mt256, (rounds - 1) * 256 / mt256};
-    int64_t best = 0, best_t = ends(0);
-    for (int64_t c : cuts)
-        if (c > 0 && ends(c) < best_t) best = c, best_t = ends(c);
-    if (end) *end = best_t;
-    return static_cast<int>(best) * kWdBN;
+    const int64_t cuts[4] = {0, n_tiles, rounds * 256 / mt256, (rounds - 1) * 256 / mt256};
+    constexpr double kBig = 3.0;
+    constexpr struct {
+        int rows;
+        double time, margin;
+    } heights[3] = {{128, 2.0, 1.0}, {192, 2.35, 1.05}, {224, 2.74, 1.05}};
+    WdCut best;
+    best.end = 1e300;
+#pragma unroll
+    for (const auto &h : heights) {
+        if (h.rows != 128 && !all_heights) break;
+        const int64_t mt = (m + h.rows - 1) / h.rows;
+        for (int i = 0; i < 4; ++i) {
+            const int64_t c = cuts[i];
+            if ((i > 0 && c <= 0) || (h.rows != 128 && c == n_all)) continue;
+            const int64_t big = mt256 * c, small = mt * (n_all - c);
+            const int64_t busy = big % 256, free = 256 - busy;  // CUs free from t0 on, and from t0 + kBig on
+            const double t0 = static_cast<double>(big / 256) * kBig;
+            double end = busy ? kBig : 0.0;
+            if (small > 0) {
+                // by whole tiles on the CUs that are free first, or on the others; from about their share of rounds on
+                auto done = [&](double t) {
+                    const int64_t f = static_cast<int64_t>(t / h.time + 1e-6), g = t > kBig ? static_cast<int64_t>((t - kBig) / h.time + 1e-6) : 0;
+                    return free * f + busy * g;
+                };
+                int64_t f = small / 256 > 0 ? small / 256 : 1;
+                while (done(static_cast<double>(f) * h.time) < small) ++f;
+                double t = static_cast<double>(f) * h.time;
+                if (busy)
+                    for (int64_t g = f; g >= 1; --g) {
+                        const double u = kBig + static_cast<double>(g) * h.time;
+                        if (u < t && done(u) >= small) t = u;
+                        if (u < t - 2.0 * h.time - kBig) break;
+                    }
+                if (t > end) end = t;
+            }
+            end += t0;
+            if (end * h.margin < best.end) best.n_big = static_cast<int>(c) * kWdBN, best.small = h.rows, best.end = end;
+        }
+    }
+    return best;
 }
 
-int64_t q8_gemm_wide_ends(int64_t m, int64_t n) {
-    int64_t end = 0;
-    wd_big_rows(m, n, &end);
-    return end;
-}
+double q8_gemm_wide_ends(int64_t m, int64_t n, bool all_heights) { return wd_cut(m, n, all_heights).end; }
 
 template <typename XT, int OUT>
 static lhip_status wd_launch_t(const int8_t *qs, const __half *ds, const void *x, void *y, int m, int n, int k, int slices,
                                int ldy, hipStream_t s) {
-    const int n_big = slices == 1 ? wd_big_rows(m, n) : 0;
+    const WdCut cut = slices == 1 ? wd_cut(m, n) : WdCut{};
     auto blocks = [](int64_t m_tiles, int64_t n_tiles) { return (m_tiles * n_tiles + 7) / 8 * 8; };  // whole eights, see wd_tile
-    const int64_t big = blocks((m + 255) / 256, n_big / kWdBN);
-    const int64_t small = blocks((m + 127) / 128, static_cast<int64_t>((n - n_big + kWdBN - 1) / kWdBN) * slices);
+    const int64_t big = blocks((m + 255) / 256, cut.n_big / kWdBN);
+    const int64_t small = blocks((m + cut.small - 1) / cut.small, static_cast<int64_t>((n - cut.n_big + kWdBN - 1) / kWdBN) * slices);
     if (big + small > 0x7fffffff) return LHIP_ERR_INVALID_SHAPE;  // the grid's x extent
     auto kern = q8_gemm_wide_kernel<XT, OUT>;
     constexpr int lds_small = WdShape<128>::LDS, lds_most = WdShape<256>::LDS;
-    static_assert(lds_most >= lds_small, "the opt-in covers both heights");
+    static_assert(lds_most >= lds_small && lds_most >= WdShape<192>::LDS && lds_most >= WdShape<224>::LDS, "the opt-in covers all heights");
     static LdsOptIn opt;
     if (lhip_status st = lds_opt_in(opt, reinterpret_cast<const void *>(kern), lds_most)) return st;
     const int kt = k / 64, kt_slice = (kt + slices - 1) / slices;
     if (slices < 1 || (slices - 1) * kt_slice >= kt) return LHIP_ERR_UNSUPPORTED;  // an empty slice
     hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(big + small)), dim3(512),
-                       static_cast<unsigned>(n_big > 0 ? lds_most : lds_small), s, qs, ds, static_cast<const XT *>(x), y, m, n, k,
-                       n_big, static_cast<int>(big), slices, kt_slice, ldy > 0 ? ldy : n);
+                       static_cast<unsigned>(cut.n_big > 0 || cut.small != 128 ? lds_most : lds_small), s, qs, ds, static_cast<const XT *>(x), y, m, n, k,
+                       cut.n_big, static_cast<int>(big), cut.small, slices, kt_slice, ldy > 0 ? ldy : n);
     LHIP_CHECK_LAUNCH();
     return LHIP_OK;
 }
