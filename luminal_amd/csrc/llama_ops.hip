@@ -117,10 +117,42 @@ __global__ __launch_bounds__(1024) void rms_norm_kernel(const float *x, const fl
 
 // Rotary embedding on adjacent pairs (the ggml layout of model.rs:52-72) for the q and k
 // parts of a fused qkv row, then k and v are appended to the cache at position pos0 + s.
-// qkv: [S][(hq + 2*hkv) * hd]; caches: [hkv][max_seq][hd].  A block takes a token and a share of its heads: a
-// thread keeps its pair and works out the angle once for all its heads (a power, a sine and a cosine, which one block per (token, head)
-// of 64 threads was bound by): 2000 tokens of 32 + 2 x 8 heads of 128 30.0 -> 18.3 us, 5.4 TB/s, 700 of 64 + 2 x 8 of 64 17.8 -> 7.1.
-constexpr int kRopeThreads = 256, kRopeAhead = 6;  // heads of a thread in flight
+// qkv: [S][(hq + 2*hkv) * hd]; caches: [hkv][max_seq][hd].
+// A few tokens (kRopeFew): one block per (token, head).
+__global__ __launch_bounds__(64) void rope_kv_few_kernel(float *__restrict__ qkv, float *__restrict__ k_cache,
+                                                         float *__restrict__ v_cache, const int *__restrict__ pos_dev,
+                                                         int hq, int hkv, int hd, int max_seq, float theta) {
+    const int s = blockIdx.x, head = blockIdx.y;  // head in [0, hq + 2*hkv)
+    const int pos = *pos_dev + s;
+    float *row = qkv + (static_cast<size_t>(s) * (hq + 2 * hkv) + head) * hd;
+    const int half = hd / 2;
+    if (head < hq + hkv) {  // q or k: rotate
+        for (int j = threadIdx.x; j < half; j += 64) {
+            const float inv_freq = 1.0f / powf(theta, static_cast<float>(2 * j) / static_cast<float>(hd));
+            const float ang = static_cast<float>(pos) * inv_freq;
+            float sn, cs;
+            sincosf(ang, &sn, &cs);
+            const float x0 = row[2 * j], x1 = row[2 * j + 1];
+            const float y0 = fmaf(x0, cs, -(x1 * sn)), y1 = fmaf(x1, cs, x0 * sn);
+            row[2 * j] = y0;
+            row[2 * j + 1] = y1;
+            if (head >= hq && pos < max_seq) {
+                float *kc = k_cache + (static_cast<size_t>(head - hq) * max_seq + pos) * hd;
+                kc[2 * j] = y0;
+                kc[2 * j + 1] = y1;
+            }
+        }
+    } else if (pos < max_seq) {  // v: copy
+        float *vc = v_cache + (static_cast<size_t>(head - hq - hkv) * max_seq + pos) * hd;
+        for (int j = threadIdx.x; j < hd; j += 64) vc[j] = row[j];
+    }
+}
+
+// More of them: a block takes a token and a share of its heads, a thread keeps its pair and works out the angle - a power, a sine and a
+// cosine, which bound the kernel above - once for all its heads, under their first loads.  The same products and sums, so the same
+// bits.  32 + 2 x 8 heads of 128, above / here, us a layer from a graph: 20 tokens 2.7 / 2.95, 64 3.35 / 3.3, 300 6.7 / 5.1, 1000 16.0 / 8.9,
+// 2000 28.8 / 17.3 (5.7 TB/s).
+constexpr int kRopeFew = 64, kRopeThreads = 256, kRopeAhead = 4;  // heads of a thread in flight
 __global__ __launch_bounds__(kRopeThreads) void rope_kv_kernel(float *__restrict__ qkv, float *__restrict__ k_cache,
                                                                float *__restrict__ v_cache, const int *__restrict__ pos_dev,
                                                                int hq, int hkv, int hd, int max_seq, float theta, int pairs) {
@@ -130,32 +162,38 @@ __global__ __launch_bounds__(kRopeThreads) void rope_kv_kernel(float *__restrict
     if (threadIdx.x >= pairs * lanes) return;
     const int pos = *pos_dev + s;
     float *token = qkv + static_cast<size_t>(s) * heads * hd;
+    const int q_and_k = hq + hkv;
     for (int j = threadIdx.x % pairs; j < half; j += pairs) {
+        float x0[kRopeAhead], x1[kRopeAhead];
+        auto load = [&](int h0) __attribute__((always_inline)) {
+#pragma unroll
+            for (int u = 0; u < kRopeAhead; ++u) {
+                if (h0 + u * step >= heads) break;
+                const float *row = token + static_cast<size_t>(h0 + u * step) * hd;
+                x0[u] = row[2 * j], x1[u] = row[2 * j + 1];
+            }
+        };
+        load(first);  // (under the arithmetic of the angle)
         const float inv_freq = 1.0f / powf(theta, static_cast<float>(2 * j) / static_cast<float>(hd));
         const float ang = static_cast<float>(pos) * inv_freq;
         float sn, cs;
         sincosf(ang, &sn, &cs);
         for (int h0 = first; h0 < heads; h0 += step * kRopeAhead) {
-            float x0[kRopeAhead], x1[kRopeAhead];
-#pragma unroll
-            for (int u = 0; u < kRopeAhead; ++u) {
-                const float *row = token + static_cast<size_t>(min(h0 + u * step, heads - 1)) * hd;
-                x0[u] = row[2 * j], x1[u] = row[2 * j + 1];
-            }
+            if (h0 != first) load(h0);
 #pragma unroll
             for (int u = 0; u < kRopeAhead; ++u) {
                 const int head = h0 + u * step;
                 if (head >= heads) break;
                 float y0 = x0[u], y1 = x1[u];
-                if (head < hq + hkv) {  // q or k: rotate
+                if (head < q_and_k) {  // q or k: rotate
                     y0 = fmaf(x0[u], cs, -(x1[u] * sn)), y1 = fmaf(x1[u], cs, x0[u] * sn);
                     float *row = token + static_cast<size_t>(head) * hd;
                     row[2 * j] = y0;
                     row[2 * j + 1] = y1;
                 }
                 if (head >= hq && pos < max_seq) {
-                    float *cache = head < hq + hkv ? k_cache + static_cast<size_t>(head - hq) * max_seq * hd
-                                                   : v_cache + static_cast<size_t>(head - hq - hkv) * max_seq * hd;
+                    float *cache = head < q_and_k ? k_cache + static_cast<size_t>(head - hq) * max_seq * hd
+                                                  : v_cache + static_cast<size_t>(head - q_and_k) * max_seq * hd;
                     cache += static_cast<size_t>(pos) * hd;
                     cache[2 * j] = y0;
                     cache[2 * j + 1] = y1;
@@ -525,9 +563,17 @@ lhip_status lhip_rope_kv_append_f32(float *qkv_dev, float *k_cache_dev, float *v
     if (tokens <= 0 || q_heads <= 0 || kv_heads <= 0 || head_dim <= 0 || head_dim % 2 != 0 || max_seq <= 0 ||
         q_heads % kv_heads != 0 || tokens > kMaxDim || q_heads + 2 * kv_heads > 65535 || max_seq > kMaxDim)
         return LHIP_ERR_INVALID_SHAPE;
+    if (tokens < kRopeFew) {
+        hipLaunchKernelGGL(rope_kv_few_kernel, dim3(static_cast<unsigned>(tokens), static_cast<unsigned>(q_heads + 2 * kv_heads)),
+                           dim3(64), 0, as_stream(stream), qkv_dev, k_cache_dev, v_cache_dev, pos_dev,
+                           static_cast<int>(q_heads), static_cast<int>(kv_heads), static_cast<int>(head_dim),
+                           static_cast<int>(max_seq), theta);
+        LHIP_CHECK_LAUNCH();
+        return LHIP_OK;
+    }
+    // fewer tokens: fewer heads a thread, so that there are two blocks a compute unit
     const int heads = static_cast<int>(q_heads + 2 * kv_heads);
     const int pairs = static_cast<int>(head_dim / 2 < kRopeThreads ? head_dim / 2 : kRopeThreads), lanes = kRopeThreads / pairs;
-    // few tokens: fewer heads a thread, so that there are two blocks a compute unit
     int64_t parts = (512 + tokens - 1) / tokens;
     if (parts > (heads + lanes - 1) / lanes) parts = (heads + lanes - 1) / lanes;
     hipLaunchKernelGGL(rope_kv_kernel, dim3(static_cast<unsigned>(tokens), static_cast<unsigned>(parts)), dim3(kRopeThreads), 0,

@@ -584,10 +584,11 @@ static int gemm_slices_or_tiles(int64_t m, int64_t n, int64_t k, int out, const 
 // header promises a long K stay: at 8192 and more they are ahead for most sizes (350 x 6364 x 10688 82 <- 119, 207 x 2276 x 12992 40
 // <- 43), though not for few weight rows (171 x 544 x 8192 26.3 -> 19.8).
 // Up to 128 rows the streaming kernel stays for K below three of its steps of 512 and for every other K.  From three steps on the
-// other kernel takes what it ends a tenth sooner above 64 rows, for which the strips are bound by their reads of the activations and no
-// longer by the weights, and a quarter sooner from 33 on.  Measured, us, strips -> that kernel: 80 x 4096 x 4096 16.8 -> 12.7, 96 x 14336 x
-// 4096 33.7 -> 29.8, 128 x 6000 x 1536 13.8 -> 9.9, 96 x 8148 x 2048 15.8 -> 11.4, 45 x 6144 x 4096 17.8 -> 12.8, 45 x 14336 x 4096 27.6 -> 22.6;
-// the other way 45 x 4096 x 4096 12.7, 64 x 6144 x 4096 15.4 <- 15.7 and 64 x 6000 x 1536 9.2 <- 9.3 as they are.
+// other kernel takes what it ends a fifth sooner above 64 rows, for which the strips are bound by their reads of the activations and no
+// longer by the weights, and a quarter sooner from 33 on: the estimates are of weights that the memory-side cache holds, and from memory
+// that kernel loses 1.5 to 2 us more.  Measured, us, strips -> that kernel, weights from memory: 80 x 4096 x 4096 16.8 -> 14.8, 80 x 6144 x
+// 4096 21.9 -> 20.4, 48 x 6144 x 4096 18.8 -> 15.2, the other way 100 x 4096 x 4096 17.7 <- 19.1; from the cache: 80 x 4096 x 4096 16.8 ->
+// 12.7, 96 x 14336 x 4096 33.7 -> 29.8, 128 x 6000 x 1536 13.8 -> 9.9, 96 x 8148 x 2048 15.8 -> 11.4, 45 x 14336 x 4096 27.6 -> 22.6.
 static int gemm_auto_tile(int64_t m, int64_t n, int64_t k, int out, const void *y, size_t room) {
     double us;
     const int tile = gemm_slices_or_tiles(m, n, k, out, y, room, &us);
@@ -597,7 +598,7 @@ static int gemm_auto_tile(int64_t m, int64_t n, int64_t k, int out, const void *
     if (streams) {
         if (m <= 32 || k % 512 != 0 || k < 1536) return tile;
         us = q8_gemm_skinny_us(static_cast<int>(m), static_cast<int>(n), static_cast<int>(k), room);
-        margin = m > 64 ? 1.1 : 1.25;
+        margin = m > 64 ? 1.2 : 1.25;
     }
     if (long_slices || k < 256 || !q8_gemm_deep_supports(k, nullptr)) return tile;
     const DeepPlan deep = q8_gemm_deep_plan(m, n, k, us / margin);

@@ -13,8 +13,8 @@ pytestmark = pytest.mark.gpu
 DEV, THETA = "cuda:0", 500000.0
 
 
-@pytest.mark.parametrize("tokens,hq,hkv,hd,pos", [(1, 32, 8, 128, 5), (700, 4, 2, 64, 0), (33, 4, 2, 6, 9), (9, 3, 1, 600, 3),
-                                                  (5, 2, 2, 512, 40), (17, 7, 7, 192, 0), (600, 1, 1, 2, 1)])
+@pytest.mark.parametrize("tokens,hq,hkv,hd,pos", [(63, 32, 8, 128, 5), (64, 32, 8, 128, 5), (700, 4, 2, 64, 0), (65, 4, 2, 6, 9), (70, 3, 1, 600, 3),
+                                                  (64, 2, 2, 512, 40), (130, 7, 7, 192, 0), (600, 1, 1, 2, 1)])
 def test_rope_and_append(tokens, hq, hkv, hd, pos):
     lib = capi.load_library()
     rng = np.random.default_rng(tokens + hd)
