@@ -583,7 +583,10 @@ static int gemm_slices_or_tiles(int64_t m, int64_t n, int64_t k, int out, const 
 // 3067 x 12288 (no slices for an odd N) 191 -> 69; the other way 256 x 14336 x 4096 54 <- 66, 592 x 9820 x 768 23 <- 38.  The slices that the
 // header promises a long K stay: at 8192 and more they are ahead for most sizes (350 x 6364 x 10688 82 <- 119, 207 x 2276 x 12992 40
 // <- 43), though not for few weight rows (171 x 544 x 8192 26.3 -> 19.8).
-// Up to 128 rows the streaming kernel stays for K below three of its steps of 512 and for every other K.  From three steps on the
+// Up to 128 rows the streaming kernel stays for K below three of its steps of 512 and, where it is ahead of tiles and slices, for every
+// K outside those steps.  Where they are ahead of it, the other kernel takes what it ends a seventh sooner; us, weights from memory (from the
+// cache), tiles or slices -> it: 128 x 2880 x 2880 22.0 -> 13.9 (20.6 -> 10.9), 101 x 468 x 576 10.5 -> 4.4, 57 x 6512 x 5760 27.3 -> 25.4 (26.3 ->
+// 20.0); mean of 62 sizes 1.55 (1.72) times as fast, none slower; at a twentieth 124 x 14128 x 4480 39.3 <- 41.3.  From three steps on the
 // other kernel takes what it ends a fifth sooner above 64 rows, for which the strips are bound by their reads of the activations and no
 // longer by the weights, and a quarter sooner from 33 on: the estimates are of weights that the memory-side cache holds, and from memory
 // that kernel loses 1.5 to 2 us more.  Measured, us, strips -> that kernel, weights from memory: 80 x 4096 x 4096 16.8 -> 14.8, 80 x 6144 x
@@ -594,8 +597,8 @@ static int gemm_auto_tile(int64_t m, int64_t n, int64_t k, int out, const void *
     const int tile = gemm_slices_or_tiles(m, n, k, out, y, room, &us);
     const bool streams = m <= 128 && q8_gemm_skinny_supports(static_cast<int>(m), static_cast<int>(n), static_cast<int>(k), out, y);
     const bool long_slices = tile > kTileSliced && tile < kTileTail && k >= 8192;
-    double margin = 1.05;
-    if (streams) {
+    double margin = streams ? 1.15 : 1.05;
+    if (streams && tile == kTileSkinny) {
         if (m <= 32 || k % 512 != 0 || k < 1536) return tile;
         us = q8_gemm_skinny_us(static_cast<int>(m), static_cast<int>(n), static_cast<int>(k), room);
         margin = m > 64 ? 1.2 : 1.25;

@@ -13,7 +13,8 @@ DEV = "cuda:0"
 # By tile (activation rows x weight rows): 32, 48, 64, 96 and 128 x 32, then x 64
 BOTH = [(49, 3725, 512), (130, 2068, 512), (255, 1696, 576), (161, 2750, 576), (193, 2568, 512),
         (129, 2480, 512), (130, 3660, 576), (257, 2728, 512), (130, 5452, 512), (97, 8339, 576)]
-BF16_ONLY = [(300, 36, 448), (17, 1001, 576), (130, 257, 320), (200, 1030, 1152), (132, 2880, 2880)]
+BF16_ONLY = [(300, 36, 448), (17, 1001, 576), (130, 257, 320), (200, 1030, 1152), (132, 2880, 2880),
+             (76, 3224, 768), (101, 468, 576), (112, 1196, 704)]
 
 
 def kernel_of(m, n, k, activations):
