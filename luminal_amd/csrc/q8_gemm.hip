@@ -585,7 +585,7 @@ static int gemm_slices_or_tiles(int64_t m, int64_t n, int64_t k, int out, const 
 // <- 43), though not for few weight rows (171 x 544 x 8192 26.3 -> 19.8).
 // Up to 128 rows the streaming kernel stays for K below three of its steps of 512 and, where it is ahead of tiles and slices, for every
 // K outside those steps.  Where they are ahead of it, the other kernel takes what it ends a seventh sooner; us, weights from memory (from the
-// cache), tiles or slices -> it: 128 x 2880 x 2880 22.0 -> 13.9 (20.6 -> 10.9), 101 x 468 x 576 10.5 -> 4.4, 57 x 6512 x 5760 27.3 -> 25.4 (26.3 ->
+// cache), tiles or slices -> it: 128 x 2880 x 2880 22.0 -> 13.9 (20.6 -> 10.9), 101 x 468 x 576 9.1 -> 4.2, 57 x 6512 x 5760 27.3 -> 25.4 (26.3 ->
 // 20.0); mean of 62 sizes 1.55 (1.72) times as fast, none slower; at a twentieth 124 x 14128 x 4480 39.3 <- 41.3.  From three steps on the
 // other kernel takes what it ends a fifth sooner above 64 rows, for which the strips are bound by their reads of the activations and no
 // longer by the weights, and a quarter sooner from 33 on: the estimates are of weights that the memory-side cache holds, and from memory
