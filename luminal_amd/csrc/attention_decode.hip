@@ -191,8 +191,11 @@ __global__ __launch_bounds__(kShortThreads) void attention_decode_short_kernel(
             float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
             for (int u = 0; u < KPG; ++u) {
-                const float w = p_s[range][kg + KG * u];  // 0 for keys past the range
-                const float4 v = k0 + kg + KG * u == pos ? vnew[c0 + c] : vreg[t][u];
+                const int key = k0 + kg + KG * u;
+                const float w = p_s[range][kg + KG * u];
+                // behind the new position, the last key, nothing is multiplied, not even by zero (as in attention_decode_body): the row
+                // read there may be the new position's, which the workgroup that appends it has written by now or not
+                const float4 v = key < pos ? vreg[t][u] : key == pos && key < min(n_keys, k0 + chunk) ? vnew[c0 + c] : make_float4(0.f, 0.f, 0.f, 0.f);
                 a.x = fmaf(w, v.x, a.x); a.y = fmaf(w, v.y, a.y);
                 a.z = fmaf(w, v.z, a.z); a.w = fmaf(w, v.w, a.w);
             }

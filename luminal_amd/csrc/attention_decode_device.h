@@ -378,7 +378,8 @@ __device__ __forceinline__ void attention_decode_body(IO io, AttnShared<G, HD> &
                 }
 #pragma unroll
             for (int u = 0; u < KPG; ++u)
-                if (t0 + kgp + KG * u == pos) vreg[u] = sh.vnew[c4];
+                if (t0 + kgp + KG * u >= pos)  // behind it lies no key: zero weight times a row that was never written need not be zero
+                    vreg[u] = t0 + kgp + KG * u == pos && pos < k1 ? sh.vnew[c4] : make_float4(0.f, 0.f, 0.f, 0.f);
             // ---- scores, key by key: the second key's rows may still be on their way
 #pragma unroll
             for (int i = 0; i < 2; ++i) {

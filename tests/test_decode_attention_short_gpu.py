@@ -36,3 +36,28 @@ def test_one_launch_gives_the_bits_of_two(hq, hkv, hd, short):
         one, two = decode(lib, qkv, ks, vs, pos, hq, hkv, hd, short), decode(lib, qkv, kl, vl, pos, hq, hkv, hd, long)
         assert torch.equal(one.view(torch.int32), two.view(torch.int32)), pos
         assert torch.equal(ks, kl[:, :short]) and torch.equal(vs, vl[:, :short]) and not torch.equal(kl, k_long), pos
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("hq,hkv,hd,short", SHAPES)
+def test_rows_not_written_yet_and_an_infinite_value_stay_where_they_belong(hq, hkv, hd, short):
+    """From the new position on the caches hold NaN and the new value has infinities, at positions that a range begins with (all below
+    the number of ranges, multiples of a range's keys) and others: neither reaches a slot behind the range's end, by either form."""
+    lib = capi.load_library()
+    gen = torch.Generator(device=DEV).manual_seed(hq + hd + 1)
+    long = 1024
+    keys, values = (torch.randn((hkv, long, hd), device=DEV, generator=gen) for _ in range(2))
+    for pos in (0, 1, 2, 15, 30, 31, 32, 33, 40, 96, 97, 200, 252, 300, short - 1):
+        if pos >= short:
+            continue
+        qkv = torch.randn(((hq + 2 * hkv) * hd,), device=DEV, generator=gen)
+        kc, vc = keys.clone(), values.clone()
+        clean = decode(lib, qkv, kc, vc, pos, hq, hkv, hd, long).view(hq, hd)
+        qkv.view(-1, hd)[hq + hkv:, 3::8] = float("inf")
+        for max_seq in (short, long):
+            kc, vc = (t[:, :max_seq].clone() for t in (keys, values))
+            kc[:, pos:] = vc[:, pos:] = float("nan")
+            out = decode(lib, qkv, kc, vc, pos, hq, hkv, hd, max_seq).view(hq, hd)
+            assert bool((out[:, 3::8] == float("inf")).all()), (pos, max_seq)
+            rest = [c for c in range(hd) if c % 8 != 3]
+            assert torch.equal(out[:, rest].view(torch.int32), clean[:, rest].view(torch.int32)), (pos, max_seq)
