@@ -234,6 +234,7 @@ __device__ __forceinline__ float4 merged_attention_piece(const GemvFuse &f, int 
 }
 
 constexpr int kStage = 4;  // pieces of four activations a thread stages from registers (ONE)
+constexpr int kNormWaves = 4;  // waves that take the norm's sum of squares
 
 struct Located {
     const int8_t *qs;
@@ -345,16 +346,22 @@ __global__ __launch_bounds__(W * 64) void q8_gemv_fused_kernel(const int8_t *qs0
 
     // The norm's scalar factor commutes with the matrix product, so x * g is staged at once and the row sums
     // are multiplied by 1/sqrt(mean(x^2) + eps) at the end: the sum of squares rides on the staging loads and
-    // is published by the staging barrier.
+    // is published by the staging barrier.  It is that of 256 threads over every 256th piece whatever the workgroup, the order of
+    // the decode program too: in a larger one the pieces also go to LDS as they are, where the first four waves add them up (eight waves
+    // 0.1 to 0.3 us, 8192 x 8192 14.9 -> 15.2; sixteen 0.9).
+    float ss = 0.f;
+    // spelled out, so that every kernel that takes this sum rounds it the same way
+    auto add_squares = [&](const float4 &v) {
+        ss = fmaf(v.x, v.x, ss);
+        ss = fmaf(v.y, v.y, ss);
+        ss = fmaf(v.z, v.z, ss);
+        ss = fmaf(v.w, v.w, ss);
+    };
     {
-        float ss = 0.f;
         auto stage = [&](int i, float4 v, const float4 &g) {
             if (NORM) {
-                // spelled out, so that every kernel that takes this sum rounds it the same way
-                ss = fmaf(v.x, v.x, ss);
-                ss = fmaf(v.y, v.y, ss);
-                ss = fmaf(v.z, v.z, ss);
-                ss = fmaf(v.w, v.w, ss);
+                if (W == kNormWaves) add_squares(v);
+                else xs4[k4 + i] = v;
                 v = make_float4(v.x * g.x, v.y * g.y, v.z * g.z, v.w * g.w);
             }
             xs4[i] = v;
@@ -376,7 +383,7 @@ __global__ __launch_bounds__(W * 64) void q8_gemv_fused_kernel(const int8_t *qs0
 #pragma unroll 4
             for (int i = threadIdx.x; i < k4; i += W * 64) stage(i, x4[source(i)], NORM ? g4[source(i)] : float4{});
         }
-        if (NORM) {
+        if (NORM && W == kNormWaves) {
             ss = wave_sum(ss);
             if (lane == 0) red[wave] = ss;
         }
@@ -385,12 +392,21 @@ __global__ __launch_bounds__(W * 64) void q8_gemv_fused_kernel(const int8_t *qs0
     // the pipeline loop, the read would stall the second step of every wave.
     asm volatile("" ::"s"(p.group_end[1]), "s"(p.group_end[2]), "s"(p.n[1]));
     __syncthreads();
+    if (NORM && W != kNormWaves) {
+        if (wave < kNormWaves) {
+#pragma unroll 4
+            for (int i = threadIdx.x; i < k4; i += kNormWaves * 64) add_squares(xs4[k4 + i]);
+            ss = wave_sum(ss);
+            if (lane == 0) red[wave] = ss;
+        }
+        __syncthreads();  // (behind the first step instead: the same within 0.1 us)
+    }
     if (T == 0) return;
     float scale = 1.f;
     if (NORM) {
         float total = 0.f;
 #pragma unroll
-        for (int w = 0; w < W; ++w) total += red[w];
+        for (int w = 0; w < kNormWaves; ++w) total += red[w];
         scale = 1.0f / sqrtf(total / static_cast<float>(k) + eps);
     }
 
@@ -580,7 +596,7 @@ static lhip_status launch_fused_form(const GemvGroup &p, const GemvFuse &f, cons
     int grid = (n_groups + W - 1) / W;
     const int cap = kNumCUs * blocks_per_cu;
     if (grid > cap) grid = cap;
-    const size_t lds_bytes = static_cast<size_t>(k) * sizeof(float);
+    const size_t lds_bytes = static_cast<size_t>(k) * sizeof(float) * (PRO == PRO_NORM && W != kNormWaves ? 2 : 1);
     static LdsOptIn opt;  // with the static reduction array: beyond the default limit (K = 16384)
     if (lhip_status st = lds_opt_in(opt, reinterpret_cast<const void *>(q8_gemv_fused_kernel<R, S, W, PRO, EPI, ONE>), lds_bytes,
                                     lds_bytes + W * sizeof(float) > 64 * 1024))

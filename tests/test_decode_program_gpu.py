@@ -50,6 +50,23 @@ def test_single_matvec_phase_equals_the_fused_matvec(n, k, norm):
     assert torch.equal(bits(y), bits(y_ref))
 
 
+# widths and row counts for which the fused matvec takes workgroups of eight and sixteen waves, whose sum of squares has the order of four
+@pytest.mark.parametrize("n,k", [(5000, 8192), (300, 6144), (12288, 4096), (37, 14336)])
+def test_norm_of_a_single_phase_whatever_the_fused_launch_s_workgroup(n, k):
+    w = weight(n, k, n + k)
+    pos = torch.zeros(1, dtype=torch.int32, device=DEV)
+    for seed in range(6):
+        torch.manual_seed(seed)
+        x, g = torch.randn(k, device=DEV), 1 + 0.1 * torch.randn(k, device=DEV)
+        y_ref, y = torch.empty(n, device=DEV), torch.full((n,), float("nan"), device=DEV)
+        FusedMatvec([w], [y_ref], norm_weight=g, eps=1e-5).run(x)
+        prog = DecodeProgram(pos=pos).matvec(w, x, y, norm_weight=g, eps=1e-5).build()
+        prog.run()
+        torch.cuda.synchronize()
+        assert not prog.timed_out()
+        assert torch.equal(bits(y), bits(y_ref)), seed
+
+
 def test_chain_of_phases_with_every_epilogue_equals_the_fused_matvecs():
     """h -> (norm) gate|up + SwiGLU -> down + residual -> (norm) head, twice over, as 6 phases of one launch."""
     d, f, v = 2048, 3072, 1500

@@ -184,3 +184,20 @@ def test_one_weight_requests_two_steps_ahead_and_gives_the_grouped_launch_s_bits
         plain = torch.empty(n, device=DEV)
         FusedMatvec([w], [plain], cfg=cfg).run(x)
         assert torch.equal(added, plain + res)
+
+
+@pytest.mark.parametrize("n,k", [(7, 1024), (1030, 3072), (300, 13312), (4100, 16384)])
+def test_norm_does_not_depend_on_the_workgroup_s_size(n, k):
+    """The sum of squares is that of four waves in workgroups of four, eight and sixteen, for one weight and for several."""
+    w, _ = make(n, k, n + k)
+    other, _ = make(3, k, 1)
+    for seed in range(4):
+        x = torch.from_numpy(synth.activations(1, k, seed=seed)).to(DEV).reshape(k)
+        g = 1 + 0.1 * torch.sin(torch.arange(k, device=DEV, dtype=torch.float32))
+        outs = []
+        for cfg in (None, (1, 1, 4, 2), (2, 1, 4, 1), (2, 1, 8, 1), (1, 1, 16, 1)):
+            for ws in ([w], [w, other]):
+                ys = [torch.full((v.n,), float("nan"), device=DEV) for v in ws]
+                FusedMatvec(ws, ys, norm_weight=g, eps=1e-5, cfg=cfg).run(x)
+                outs.append(ys[0])
+        assert all(torch.equal(o, outs[0]) for o in outs), seed
