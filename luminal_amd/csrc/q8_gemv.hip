@@ -647,7 +647,7 @@ static lhip_status dispatch_fused(int r, int sl, int w, int bpc, bool norm, int 
 }
 
 // Default launch shape of the fused kernel for n_total rows (all weights together).
-static void choose_fused(int64_t n_total, int k, int pro, int epi, int *r, int *sl, int *w, int *bpc) {
+static void choose_fused(int64_t n_total, bool grouped, int k, int pro, int epi, int *r, int *sl, int *w, int *bpc) {
     const int slices = k % 4096 == 0 ? 4 : (k % 2048 == 0 ? 2 : 1);
     const int fit = (160 * 1024) / (k * 4);
     if (n_total >= 16384 && slices == 4 && fit >= 1) {
@@ -663,14 +663,24 @@ static void choose_fused(int64_t n_total, int k, int pro, int epi, int *r, int *
     //   plain, K = 4096: 4096 rows 5.5 / 5.7 / 5.5 / 5.6, 6144 7.1 / 6.8 / 6.8 / 7.1, 12288 11.6 / 10.9 / 10.8 / 11.1
     //   K = 8192, norm and plain: 4096 rows 9.4 / 8.9 / 9.4 / 12.1 and 9.0 / 8.1 / 8.5 / 9.6
     //   K = 2048, norm: 4096 rows 4.7 / 4.8 / 4.8 / 4.6, 6144 5.5 / 5.6 / 5.6 / 5.5 (level)
-    if (*sl == 2 && k > 4096 && k <= 8192) {
+    // A launch of several weights (grouped) has no early second step: with more than 4096 rows workgroups of four waves where those are not behind, eight waves
+    // against three of four, 8192 + 1024 + 1024 rows of 6144 15.4 / 14.6 plain and 16.0 / 15.2 with the norm, of 8192 with the norm 19.4 / 21.1.
+    // A fourth workgroup pays without the norm where a step is one slice (12288 rows of 5120 17.4 -> 15.8 us, of 7168 22.9 -> 20.9, of 9216 28.3 ->
+    // 26.2, of 3072 10.1 -> 9.7) and for groups of 6144 (12288 rows 17.0 -> 16.3); of 10240 and more 3 % behind, of 8192 3.5 %.
+    // Sixteen waves behind the norm add up the squares in 0.9 us: 1024 rows of 14336 12.0 us, two workgroups of four waves 8.8, from 4096 rows
+    // on 15.3 and 17.1.
+    const bool eight = *sl == 2 && k > 4096 && k <= 8192;
+    if (eight && (!grouped || n_total <= 4096 || (pro == PRO_NORM && (k == 8192 || n_total <= 6144)))) {
         *r = pairs ? 2 : 1, *w = 8, *bpc = 1;
     } else if (*sl == 2 && k == 4096 && pro == PRO_NORM && n_total >= 2048) {
         *r = pairs || n_total <= 6144 ? 2 : 1, *w = n_total <= 6144 ? 4 : 8, *bpc = 1;
-    } else if (*sl == 2 && k == 4096 && !pairs && n_total > 4096) {
+    } else if (*sl == 2 && k == 4096 && !pairs && !grouped && n_total > 4096) {
         *r = 1, *w = 8, *bpc = 2;
     } else if (fit >= 3) {
-        *r = pairs ? 2 : 1, *w = 4, *bpc = pairs ? 2 : 3;
+        const bool four = pro == PRO_NONE && n_total > 4096 && fit >= 4 && (*sl == 1 || (k > 4096 && k < 8192));
+        *r = pairs ? 2 : 1, *w = 4, *bpc = pairs ? 2 : four ? 4 : 3;
+    } else if (pro == PRO_NORM && n_total <= 2048) {
+        *r = pairs ? 2 : 1, *w = 4, *bpc = 2;
     } else {
         *r = pairs ? 2 : 1, *w = pairs ? 8 : 16, *bpc = 1;
     }
@@ -955,7 +965,7 @@ lhip_status lhip_q8_0_matvec_fused_f32(const void *const *planar_dev, float *con
     int64_t total = 0;
     for (int i = 0; i < count; ++i) total += n[i] > 0 ? n[i] : 0;
     int r, sl, w, bpc;
-    choose_fused(total, static_cast<int>(k), norm_weight_dev ? PRO_NORM : PRO_NONE, epilogue, &r, &sl, &w, &bpc);
+    choose_fused(total, count > 1, static_cast<int>(k), norm_weight_dev ? PRO_NORM : PRO_NONE, epilogue, &r, &sl, &w, &bpc);
     return lhip_q8_0_matvec_fused_f32_cfg(planar_dev, y_dev, n, count, x_dev, k, norm_weight_dev, eps, residual_dev,
                                           epilogue, r, sl, w, bpc, stream);
 }
