@@ -722,6 +722,48 @@ static lhip_status rows_matvecs(const void *planar, const void *x, void *y, int6
     return LHIP_OK;
 }
 
+// `named`: the caller names the launch shape, one of the header's list; (1, 2, 8) is the library's own.
+static lhip_status fused_matvec(const void *const *planar_dev, float *const *y_dev, const int64_t *n, int count, const float *x_dev,
+                                int64_t k, const float *norm_weight_dev, float eps, const float *residual_dev, int epilogue,
+                                int rows_per_wave, int k_unroll, int waves_per_block, int blocks_per_cu, bool named, void *stream) {
+    if (!planar_dev || !y_dev || !n || !x_dev) return LHIP_ERR_NULL_PTR;
+    if (count < 1 || count > kMaxGroup) return LHIP_ERR_INVALID_SHAPE;
+    if (epilogue != EPI_NONE && epilogue != EPI_ADD && epilogue != EPI_SWIGLU) return LHIP_ERR_UNSUPPORTED;
+    if (epilogue == EPI_ADD && (!residual_dev || count != 1)) return residual_dev ? LHIP_ERR_UNSUPPORTED : LHIP_ERR_NULL_PTR;
+    if (!aligned(x_dev, 16) || (norm_weight_dev && !aligned(norm_weight_dev, 16))) return LHIP_ERR_MISALIGNED;
+    if (k <= 0 || k % 1024 != 0 || k > kMaxLdsK) return k > 0 && k % 32 == 0 ? LHIP_ERR_UNSUPPORTED : LHIP_ERR_INVALID_SHAPE;
+    if (rows_per_wave < 1 || k_unroll < 1 || blocks_per_cu < 1 || blocks_per_cu > 16 || k % (k_unroll * 1024) != 0)
+        return LHIP_ERR_UNSUPPORTED;
+    GemvGroup p;
+    int64_t groups = 0;
+    for (int i = 0; i < kMaxGroup; ++i) {
+        if (i < count) {
+            if (!planar_dev[i] || !y_dev[i]) return LHIP_ERR_NULL_PTR;
+            if (lhip_status st = check_q8_shape(n[i], k)) return st;
+            if (epilogue == EPI_SWIGLU && n[i] % 2 != 0) return LHIP_ERR_INVALID_SHAPE;
+            if (!aligned(planar_dev[i], 256) || !aligned(y_dev[i], 4)) return LHIP_ERR_MISALIGNED;
+            auto *base = static_cast<const uint8_t *>(planar_dev[i]);
+            p.qs[i] = reinterpret_cast<const int8_t *>(base);
+            p.ds[i] = reinterpret_cast<const unsigned short *>(base + q8_scale_offset(n[i], k));
+            p.y[i] = y_dev[i];
+            p.n[i] = static_cast<int>(n[i]);
+            groups += (n[i] + rows_per_wave - 1) / rows_per_wave;
+            if (groups > kMaxDim) return LHIP_ERR_INVALID_SHAPE;
+            p.group_end[i] = static_cast<int>(groups);
+        } else {
+            p.qs[i] = p.qs[0], p.ds[i] = p.ds[0], p.y[i] = p.y[0], p.n[i] = p.n[0];
+            p.group_end[i] = INT_MAX;
+        }
+    }
+    if (named && rows_per_wave == 1 && k_unroll == 2 && waves_per_block == 8) return LHIP_ERR_UNSUPPORTED;
+    GemvFuse f{};
+    f.norm_w = norm_weight_dev;
+    f.eps = eps;
+    f.residual = residual_dev;
+    return dispatch_fused(rows_per_wave, k_unroll, waves_per_block, blocks_per_cu, norm_weight_dev != nullptr, epilogue,
+                          p, f, x_dev, static_cast<int>(k), static_cast<int>(groups), as_stream(stream));
+}
+
 extern "C" {
 
 lhip_status lhip_q8_0_matmul_f32_cfg(const void *planar_dev, const float *x_dev, float *y_dev, int64_t m, int64_t n,
@@ -876,41 +918,8 @@ lhip_status lhip_q8_0_matvec_fused_f32_cfg(const void *const *planar_dev, float 
                                            int count, const float *x_dev, int64_t k, const float *norm_weight_dev,
                                            float eps, const float *residual_dev, int epilogue, int rows_per_wave,
                                            int k_unroll, int waves_per_block, int blocks_per_cu, void *stream) {
-    if (!planar_dev || !y_dev || !n || !x_dev) return LHIP_ERR_NULL_PTR;
-    if (count < 1 || count > kMaxGroup) return LHIP_ERR_INVALID_SHAPE;
-    if (epilogue != EPI_NONE && epilogue != EPI_ADD && epilogue != EPI_SWIGLU) return LHIP_ERR_UNSUPPORTED;
-    if (epilogue == EPI_ADD && (!residual_dev || count != 1)) return residual_dev ? LHIP_ERR_UNSUPPORTED : LHIP_ERR_NULL_PTR;
-    if (!aligned(x_dev, 16) || (norm_weight_dev && !aligned(norm_weight_dev, 16))) return LHIP_ERR_MISALIGNED;
-    if (k <= 0 || k % 1024 != 0 || k > kMaxLdsK) return k > 0 && k % 32 == 0 ? LHIP_ERR_UNSUPPORTED : LHIP_ERR_INVALID_SHAPE;
-    if (rows_per_wave < 1 || k_unroll < 1 || blocks_per_cu < 1 || blocks_per_cu > 16 || k % (k_unroll * 1024) != 0)
-        return LHIP_ERR_UNSUPPORTED;
-    GemvGroup p;
-    int64_t groups = 0;
-    for (int i = 0; i < kMaxGroup; ++i) {
-        if (i < count) {
-            if (!planar_dev[i] || !y_dev[i]) return LHIP_ERR_NULL_PTR;
-            if (lhip_status st = check_q8_shape(n[i], k)) return st;
-            if (epilogue == EPI_SWIGLU && n[i] % 2 != 0) return LHIP_ERR_INVALID_SHAPE;
-            if (!aligned(planar_dev[i], 256) || !aligned(y_dev[i], 4)) return LHIP_ERR_MISALIGNED;
-            auto *base = static_cast<const uint8_t *>(planar_dev[i]);
-            p.qs[i] = reinterpret_cast<const int8_t *>(base);
-            p.ds[i] = reinterpret_cast<const unsigned short *>(base + q8_scale_offset(n[i], k));
-            p.y[i] = y_dev[i];
-            p.n[i] = static_cast<int>(n[i]);
-            groups += (n[i] + rows_per_wave - 1) / rows_per_wave;
-            if (groups > kMaxDim) return LHIP_ERR_INVALID_SHAPE;
-            p.group_end[i] = static_cast<int>(groups);
-        } else {
-            p.qs[i] = p.qs[0], p.ds[i] = p.ds[0], p.y[i] = p.y[0], p.n[i] = p.n[0];
-            p.group_end[i] = INT_MAX;
-        }
-    }
-    GemvFuse f{};
-    f.norm_w = norm_weight_dev;
-    f.eps = eps;
-    f.residual = residual_dev;
-    return dispatch_fused(rows_per_wave, k_unroll, waves_per_block, blocks_per_cu, norm_weight_dev != nullptr, epilogue,
-                          p, f, x_dev, static_cast<int>(k), static_cast<int>(groups), as_stream(stream));
+    return fused_matvec(planar_dev, y_dev, n, count, x_dev, k, norm_weight_dev, eps, residual_dev, epilogue, rows_per_wave, k_unroll,
+                        waves_per_block, blocks_per_cu, true, stream);
 }
 
 lhip_status lhip_q8_0_matvec_attn_merge_f32(const void *planar_dev, float *y_dev, int64_t n, int64_t k,
@@ -966,8 +975,8 @@ lhip_status lhip_q8_0_matvec_fused_f32(const void *const *planar_dev, float *con
     for (int i = 0; i < count; ++i) total += n[i] > 0 ? n[i] : 0;
     int r, sl, w, bpc;
     choose_fused(total, count > 1, static_cast<int>(k), norm_weight_dev ? PRO_NORM : PRO_NONE, epilogue, &r, &sl, &w, &bpc);
-    return lhip_q8_0_matvec_fused_f32_cfg(planar_dev, y_dev, n, count, x_dev, k, norm_weight_dev, eps, residual_dev,
-                                          epilogue, r, sl, w, bpc, stream);
+    return fused_matvec(planar_dev, y_dev, n, count, x_dev, k, norm_weight_dev, eps, residual_dev, epilogue, r, sl, w, bpc, false,
+                        stream);
 }
 
 }  // extern "C"

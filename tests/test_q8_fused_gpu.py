@@ -201,3 +201,13 @@ def test_norm_does_not_depend_on_the_workgroup_s_size(n, k):
                 FusedMatvec(ws, ys, norm_weight=g, eps=1e-5, cfg=cfg).run(x)
                 outs.append(ys[0])
         assert all(torch.equal(o, outs[0]) for o in outs), seed
+
+
+def test_launch_shapes_that_are_not_in_the_header_s_list_are_refused():
+    w, _ = make(64, 4096, 1)
+    x, y = torch.ones(4096, device=DEV), torch.empty(64, device=DEV)
+    for shape in ((1, 2, 8), (1, 4, 4), (2, 2, 16), (1, 1, 8), (4, 1, 4)):
+        for norm in (None, x):
+            with pytest.raises(capi.LhipError) as e:
+                FusedMatvec([w], [y], norm_weight=norm, eps=1e-5, cfg=(*shape, 1)).run(x)
+            assert e.value.status == capi.LHIP_ERR_UNSUPPORTED, shape
