@@ -866,9 +866,12 @@ lhip_status lhip_q8_0_matmul_f16_gemm(const void *planar_dev, const void *x_f16_
 
 size_t lhip_q8_0_matmul_workspace_nbytes(int64_t m, int64_t n, int64_t k) {
     if (check_q8_shape(n, k) != LHIP_OK || m <= 0 || m > kMaxDim) return 0;
-    // (the matvec kernels keep nothing outside their outputs)
-    if (!on_matrix_cores(m, n, k, nullptr, nullptr, false, SIZE_MAX) && !on_matrix_cores(m, n, k, nullptr, nullptr, true, SIZE_MAX)) return 0;
-    return q8_gemm_split_workspace_floats(m, static_cast<int>(n), static_cast<int>(k)) * sizeof(float);
+    // (the matvec kernels and the f16 kernel that walks all of K keep nothing outside their outputs)
+    const bool f32 = on_matrix_cores(m, n, k, nullptr, nullptr, false, SIZE_MAX), f16 = on_matrix_cores(m, n, k, nullptr, nullptr, true, SIZE_MAX);
+    if (!f32 && !f16) return 0;
+    RowsPlan plans[2];
+    const size_t floats = q8_gemm_split_workspace_floats(m, static_cast<int>(n), static_cast<int>(k), plans);
+    return !f32 && plans[1].kind == RowsPlan::kDeep ? 0 : floats * sizeof(float);
 }
 
 lhip_status lhip_q8_0_matmul_plan(int64_t m, int64_t n, int64_t k, int32_t activations, size_t workspace_nbytes, int32_t plan[3]) {

@@ -50,6 +50,18 @@ def test_tiles_of_the_kernel_for_several_rows(dtype):
     assert cuts(plans) == {(rows, sliced) for rows in (128, 192, 224, 256) for sliced in (False, True)}, list(zip(ROWS[dtype], plans))
 
 
+def test_no_room_is_asked_for_where_neither_type_keeps_anything_in_it():
+    """A K outside the weight-streaming kernel's shapes: the recommended workspace is used by the f32 or the f16 call, or it is 0."""
+    lib, asked = capi.load_library(), 0
+    for m in (2, 5, 6, 8, 10, 12, 24, 45, 128):
+        for n in (256, 1000, 2880, 6001, 10944, 14336):
+            for k in (544, 576, 960, 1600, 2880, 4160, 8000):
+                if lib.lhip_q8_0_matmul_workspace_nbytes(m, n, k):
+                    asked += 1
+                    assert any(plan(m, n, k, t, workspace=True)[2] != 1 for t in ("f32", "f16")), (m, n, k)
+    assert asked > 50
+
+
 def test_plan_errors():
     lib, out = capi.load_library(), (C.c_int32 * 3)()
     assert lib.lhip_q8_0_matmul_plan(1, 32, 32, 0, PLAIN, None) == capi.LHIP_ERR_NULL_PTR
