@@ -242,7 +242,8 @@ lhip_status lhip_q8_0_matmul_bf16_cfg(const void *planar_dev, const void *x_dev,
  * aligned arguments and may answer differently from version to version.  workspace_nbytes: the room a `_ws` form is given,
  * (size_t)-1 for the plain call.  plan[0] = 0: matvecs, 1: the weight-streaming kernel, 2: the f32 / f16 kernel for several
  * rows, 3: the bf16 / f16 tiles, 4: the bf16 / f16 kernel whose workgroups walk all of K; plan[1] = weight rows of a workgroup of
- * kernels 1, 2 and 4 (else 0); plan[2] = slices of K (0: of the columns that whole rounds of tiles leave over only). */
+ * kernels 1, 2 and 4, activation rows of a pass where matvecs take several (else 0), of the last or only round's tiles where those are
+ * of 192 or 224 (else 0); plan[2] = slices of K (0: of the columns that whole rounds of tiles leave over only). */
 lhip_status lhip_q8_0_matmul_plan(int64_t m, int64_t n, int64_t k, int32_t activations, size_t workspace_nbytes, int32_t plan[3]);
 
 /* Row gather: out[t][j] = dequant(W[(int)idx[t]][j]), idx carried as f32 like

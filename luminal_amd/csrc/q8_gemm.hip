@@ -616,7 +616,7 @@ void q8_gemm_describe(int64_t m, int64_t n, int64_t k, size_t room, int32_t plan
         plan[0] = 4, plan[1] = 32 * (tile % 10), plan[2] = 1;
         return;
     }
-    plan[0] = 3, plan[1] = 0;
+    plan[0] = 3, plan[1] = tile == 0 && q8_gemm_wide_supports(k) ? q8_gemm_wide_special_height(m, n) : 0;
     plan[2] = tile == kTileTail ? 0 : tile > kTileSliced ? tile - kTileSliced : 1;
 }
 

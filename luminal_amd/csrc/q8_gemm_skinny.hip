@@ -449,7 +449,7 @@ void q8_gemm_split_describe(int64_t m, int n, int k, bool f16, size_t room, int3
     } else if (p.kind == RowsPlan::kDeep) {
         plan[0] = 4, plan[1] = 32 * p.deep.nt, plan[2] = 1;
     } else {
-        plan[0] = 3, plan[1] = 0, plan[2] = 1;
+        plan[0] = 3, plan[1] = q8_gemm_wide_special_height(m, n), plan[2] = 1;
     }
 }
 

@@ -417,6 +417,11 @@ static WdCut wd_cut(int64_t m, int64_t n, bool all_heights = true) {
 
 double q8_gemm_wide_ends(int64_t m, int64_t n, bool all_heights) { return wd_cut(m, n, all_heights).end; }
 
+int q8_gemm_wide_special_height(int64_t m, int64_t n) {
+    const WdCut cut = wd_cut(m, n);
+    return cut.small != 128 ? cut.small : 0;
+}
+
 template <typename XT, int OUT>
 static lhip_status wd_launch_t(const int8_t *qs, const __half *ds, const void *x, void *y, int m, int n, int k, int slices,
                                int ldy, hipStream_t s) {

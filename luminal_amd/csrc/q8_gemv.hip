@@ -889,7 +889,8 @@ lhip_status lhip_q8_0_matmul_plan(int64_t m, int64_t n, int64_t k, int32_t activ
     if (on_matrix_cores(m, n, k, nullptr, nullptr, activations == 1, room)) {
         q8_gemm_split_describe(m, static_cast<int>(n), static_cast<int>(k), activations == 1, room, plan);
     } else {
-        plan[0] = plan[1] = 0, plan[2] = 1;
+        plan[0] = 0, plan[2] = 1;
+        plan[1] = q8_gemv_rows_pays(m, n, k, activations == 1) ? q8_gemv_rows_of_pass(m, n, k, activations == 1) : 0;
     }
     return LHIP_OK;
 }

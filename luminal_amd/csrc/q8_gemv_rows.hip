@@ -60,6 +60,8 @@ bool q8_gemv_rows_pays(int64_t m, int64_t n, int64_t k, bool f16) {
     return static_cast<double>(m - 1) * static_cast<double>(n) * static_cast<double>(k) >= millions * 1e6;
 }
 
+int q8_gemv_rows_of_pass(int64_t m, int64_t n, int64_t k, bool f16) { return rows_shape(m, n, k, f16).mr; }
+
 template <int R, int S, int MR, bool RAG, typename XT>
 static lhip_status rows_launch(const GemvRowsShape &p, const int8_t *qs, const __half *ds, const XT *x, XT *y, int m, int n, int k,
                                hipStream_t s) {
