@@ -46,27 +46,21 @@ static GemvRowsShape rows_shape(int64_t m, int64_t n, int64_t k, bool f16) {
     return p;
 }
 
-// By the weight rows that matvecs read beyond the first activation row's, (m - 1) n: the staging of the activations costs half a
-// microsecond over the kernel without, which further rows earn back the later the fewer waves they would fill, the more lanes the last
-// slice of a short K leaves idle, and for halves, which the other kernel reads in half the time.  The lines are those of the least loss
-// over 5200 random sizes, weights from memory: 0.55 % behind the faster kernel on average (lines by (m - 1) n k and for every long ragged
-// K: 1.4 %, and up to 30 % for few weight rows, which matvecs a row take in, us, 24 x 256 x 2880 f16 4.4 <- 5.6, 5 x 256 x 4160 4.2 <- 4.8, 2 x 2240 x
-// 4096 4.6 <- 5.5).  Mean times of this kernel within a factor of four below and above a line, in those of the other: f32
-// K of 3072 and 4096 1.03 / 0.82, f32 ragged K up to 1024 1.13 / 0.85, f16 ragged K of 2048 to 3072 1.11 / 0.83, f16 K from 5120 on in whole
-// slices 1.03 / 0.72.  A long ragged K has no other kernel that streams: 14336 x 4128 f32 at one row 19.7 -> 15.0, 644 x 13696 9.7 -> 6.7 (2380
-// x 5088 6.6 <- 7.2); one f16 row only where the weight rows fill the chip or K is longest (4644 x 4352 6.5 <- 8.0, 7464 x 4608 8.6 <- 10.3,
-// 14168 x 8640 30.7 -> 26.0).
+// The staging of the activations costs half a microsecond over a matvec a row, which further activation rows earn back by what is read
+// beyond the first one's weight rows or by the results there are, later for halves of a short ragged K, which the other kernel reads in
+// half the time; a ragged K from 3072 on it walks without a load ahead and is behind for any size.  Drawn over 10000 random sizes of up to
+// 512 rows: 0.3 (f32) and 0.5 % (f16) behind the faster kernel on average, weights from memory, 0.4 and 0.7 % with those from the cache
+// among them.  (Lines by (m - 1) n k and for every long ragged K: 1.2 to 1.4 %, and up to 30 % for small products, which matvecs a row take in, us,
+// 24 x 256 x 2880 f16 4.4 <- 5.6, 12 x 213 x 4096 4.5 <- 5.2, 2 x 2240 x 4096 4.6 <- 5.5.)  One row: where K is long or its weight rows fill the
+// chip twice: 14336 x 4128 f32 19.7 -> 15.0, 644 x 13696 9.7 -> 6.7, 14168 x 8640 f16 30.7 -> 26.0; the other way 2380 x 5088 f32 6.6 <- 7.2.
 bool q8_gemv_rows_pays(int64_t m, int64_t n, int64_t k, bool f16) {
     if (q8_gemv_rows_per_pass(k, f16) == 0) return false;
     const bool ragged = k % 1024 != 0;
-    if (m == 1) return ragged && (f16 ? k > 4096 && (n > 8192 || (k > 8192 && n <= 4096)) : k > 5120 || (k > 4096 && n > 4096));
-    constexpr int lines[2][2][6] = {{{8500, 4200, 3000, 2500, 3000, 1500}, {10000, 3000, 3000, 0, 1500, 0}},
-                                    {{7500, 3500, 3000, 3000, 2500, 2000}, {27000, 5000, 6000, 0, 3000, 0}}};  // by slices
-    const int slices = rows_slices(k);
-    double line = lines[f16][ragged][slices < 6 ? slices - 1 : 5];
-    if (slices == 1 && k <= 600) line *= f16 ? 2.6 : 1.6;
-    if (ragged && slices == 2) line *= (f16 ? 2048.0 / k : 1.0) * 2048.0 / k;
-    return static_cast<double>((m - 1) * n) > line;
+    if (m == 1) return ragged && k > 1024 && (k > 5120 || n > (k <= 3072 ? 8200 : 4100));
+    const int64_t further = (m - 1) * n;
+    if (f16 && ragged && k <= 3072) return static_cast<double>(further) * static_cast<double>(k < 640 ? 640 : k) > (k <= 1024 ? 18e6 : 11e6);
+    if (k <= 1024) return further > (f16 ? 7000 : 10000);
+    return (ragged && k > 3072) || m * n > (ragged ? 3100 : 2400);
 }
 
 int q8_gemv_rows_of_pass(int64_t m, int64_t n, int64_t k, bool f16) { return rows_shape(m, n, k, f16).mr; }
