@@ -44,77 +44,62 @@ static int split_min_rows(int64_t n, int64_t k, bool f16) {
     return codes >= (int64_t{256} << 20) ? 2 : codes >= (int64_t{32} << 20) ? 3 : 4;
 }
 
-// What m matvecs of a K outside the streaming kernel's shapes take, us, and an upper bound of what q8_gemm_rows.hip takes over K slices
-// for few rows.  A matvec: a launch for all rows, then per row and 1000 weight rows a step of about 1024 of K where K is short,
-// less with more weight rows, and a price per 1000 of K where it is long, less where K is in steps of 512.  The rows kernel: as
-// measured with tiles of 256 weight rows and a slice for each four blocks of K up to 16 of them, two launches, another half behind
-// 64 rows, and the stores of an N that is no multiple of four; with up to 40 slices and narrower tiles (rows_plan) it takes less
-// where the weight rows are few or K is long: 1000 x 4480 f32 at 12 rows 11.6 and not 19.2, 1001 x 14336 f32 at 8 15.6 and not 36.5.
+// What matvecs of a K outside the streaming kernel's shapes take, us, by the kernel that runs them (q8_gemv_rows_pays): one launch, then
+// for a matvec a row its share per 1000 results and per million codes and row; for several rows a pass the products over whole slices of K
+// and, where the passes do not run side by side, the weights once a pass.  Fitted to 3100 launches, weights from memory, standard deviation
+// 9 to 16 %.
 static double matvecs_us(int64_t m, int64_t n, int64_t k, bool f16) {
-    const double k1000 = static_cast<double>(k) / 1000.0;
-    double per_row;
-    if (k % 512 == 0) {
-        per_row = (n < 4096 ? (f16 ? 0.13 : 0.15) : (f16 ? 0.09 : 0.10)) * k1000;
-    } else {
-        const double step = n < 4096 ? (f16 ? 0.11 : 0.20) : n < 12288 ? (f16 ? 0.09 : 0.115) : (f16 ? 0.083 : 0.085);
-        const double slope = n < 4096 ? (f16 ? 0.11 : 0.26) : (f16 ? 0.085 : 0.18);
-        const double steps = static_cast<double>((k + 1023) / 1024);
-        per_row = step * steps > slope * k1000 ? step * steps : slope * k1000;
-    }
-    return 1.5 + static_cast<double>(m) * static_cast<double>(n) / 1000.0 * per_row;
+    const double k1000 = static_cast<double>(k) / 1000.0, rows = static_cast<double>(m), codes = static_cast<double>(n) * k1000 / 1000.0;
+    const double results = rows * static_cast<double>(n) / 1000.0;
+    if (!q8_gemv_rows_pays(m, n, k, f16)) return f16 ? 2.5 + 0.283 * k1000 + 0.08 * results + 0.11 * rows * codes : 2.4 + 0.365 * k1000 + 0.143 * results + 0.103 * rows * codes;
+    const double products = results * static_cast<double>((k + 1023) / 1024) * 1.024;
+    if (q8_gemv_rows_one_round(m, n, k, f16)) return f16 ? 3.1 + 0.30 * k1000 + 0.048 * products + 0.085 * results : 3.4 + 0.25 * k1000 + 0.083 * products + 0.0007 * results;
+    const int most = q8_gemv_rows_per_pass(k, f16);
+    const double read = codes * static_cast<double>((m + most - 1) / most);
+    return f16 ? 3.9 + 0.38 * k1000 + 0.037 * read + 0.053 * products + 0.02 * results : 4.0 + 0.465 * k1000 + 0.10 * read + 0.054 * products + 0.0037 * results;
 }
+// And what q8_gemm_rows.hip takes over K slices, launch of their sum included: the blocks of K, which lie in slices beyond 33 of them, the weight
+// stream, the stores of an N that is no multiple of four, the products; up to 64 rows and above.  Fitted to as many launches, 8 to 10 %.
 static double rows_sliced_us(int64_t m, int64_t n, int64_t k, bool f16) {
-    const double nblk = static_cast<double>(k / 32), few = nblk < 33 ? nblk : 33, more = nblk - few;
-    const double odd = n % 4 != 0 ? 0.045 * static_cast<double>(m < 128 ? m : 128) : 0.0;
-    if (f16) return 7.3 + 0.115 * few + 0.035 * more + (m > 64 ? 1.8 : 0.0) + odd;
-    return 8.0 + 0.16 * few + 0.055 * more + (m > 64 ? 2.0 + 0.09 * few : 0.0) + odd;
+    static constexpr double times[2][2][6] = {{{6.9, 0.034, 0.011, 0.33, 0.015, 0.0048}, {9.4, 0.072, 0.009, 0.16, 0.0036, 0.0068}},
+                                              {{5.6, 0.063, 0.009, 0.27, 0.012, 0.0044}, {7.1, 0.096, 0.011, 0.25, 0.0165, 0.0031}}};
+    const double *t = times[f16][m > 64];
+    const double nblk = static_cast<double>(k / 32), few = nblk < 33 ? nblk : 33, codes = static_cast<double>(n) * static_cast<double>(k) * 1e-6;
+    return t[0] + t[1] * few + t[2] * (nblk - few) + t[3] * codes + (n % 4 != 0 ? t[4] * static_cast<double>(m) * static_cast<double>(n) * 1e-3 : 0.0) +
+           t[5] * static_cast<double>(m) * codes;
 }
 
-// Whether a product of m rows is one for the matrix cores.  The streaming kernel's shapes (K in steps of 512, N of 4)
-// from split_min_rows on.  Every other K from 256 on by q8_gemm_rows.hip, from a few rows on and where the costs above say so.
-// Measured, matvecs / matrix cores, us (taken: the first unless marked *): 2880 x 2880 f32 at 4 / 8 / 12* / 45* / 200* rows 11.4 / 11.6, 19.7 / 12.0,
-// 28.1 / 12.4, 97 / 14.3 and 422 / 22.5, f16 at 6 / 12 / 16* / 45* rows 10.2 / 10.5, 16.7 / 11.1, 21.0 / 11.6 and 50 / 12.4; 1000 x 4480 f32 at
-// 6 / 12 / 24* rows 10.6 / 11.0, 19.0 / 11.6 and 34.4 / 12.6; 260 x 544 f32 at 24 / 200 / 512* rows 4.1 / 7.8, 13.2 / 9.5 and 29.5 / 10.2; 1001 x
-// 14336 f32 at 4 / 12 / 24* rows 12.8 / 15.0, 31.5 / 16.1 and 57 / 17.6; 14336 x 4128 f32 at 2 / 3* / 8* rows 31.0 / 34.2, 42.3 / 34.3 and 100 / 34.8.  So
-// the lines, drawn for the kernel with 16 slices, lie some rows above the crossing (6 rows against 12 at 2880 x 2880).  (Lines in
-// N K alone sent every product of 12 rows there.)  A K below 256 is a matvec of one or two microseconds per row.
+// Whether a product of m rows is one for the matrix cores.  The streaming kernel's shapes (K in steps of 512, N of 4) from split_min_rows
+// on.  Every other K from 256 on where the costs above say so: of 3086 random sizes of up to 512 rows the choice is 0.4 % (f32) and 0.3 %
+// (f16) behind the faster form on average, 1.3 and 1.6 % by the prices of a matvec a row and least rows by N K (5 x 14336 x 2880 f32 25.1 -> 16.9 us,
+// 6 x 6000 x 2880 14.7 -> 11.8, 12 x 10944 x 544 f16 19.1 -> 9.7); up to 1100 weight rows, whose estimates
+// spread most, the matrix cores have to be a fourteenth ahead, a quarter for up to 8 rows of x (8 x 1001 x 14336 f32: 19 us as matvecs, 16), beyond
+// them and 32 rows of x the matvecs a seventh.  A K below 256 is a matvec of one or two microseconds per row.
+// f16 goes by the kernel that walks all of K, which keeps no planes, where that ends a tenth before the matvecs and is the matrix cores'
+// own choice: 2880 x 2880 at 12 rows 11.0 as matvecs, 7.9 there; 6000 x 1600 at 8 9.2 and 5.9, 23 x 4830 x 1024 13.9 and 6.1, 12 x 14336 x 544
+// 22.9 and 8.2.
 // Without room for the slices' planes - the plain operators, which for these K keep nothing outside their outputs, so that
 // calls on several streams may overlap - it is one slice, 1.2 (f32) or 0.66 us (f16) per block of K and round of 256
-// workgroups, against matvecs of 0.17 or 0.085 us per 2^20 codes and row (where they are cheapest, so that nothing gets
-// slower).  Measured, matvecs -> one slice -> sliced, us: 2880 x 2880 f32 at 96 rows 202 -> 63 -> 19, f16 at 128 rows 124 ->
-// 46 -> 18; 14336 x 4128 f32 at 32 rows 381 -> 67 -> 36; 512 x 14304 f32 at 512 rows 1069 -> 304 -> 35.
+// workgroups.  Measured, one slice -> sliced, us: 2880 x 2880 f32 at 96 rows 63 -> 19, f16 at 128 rows 46 -> 18; 14336 x 4128 f32 at 32
+// rows 67 -> 36; 512 x 14304 f32 at 512 rows 304 -> 35.
 // `plan` (not for SIZE_MAX): what the answer was worked out with, for the launch; kind kNone where it was not.
 static bool on_matrix_cores(int64_t m, int64_t n, int64_t k, const void *x, const void *y, bool f16, size_t room_floats,
                             RowsPlan *plan = nullptr) {
     if (q8_gemm_split_supports(static_cast<int>(n), static_cast<int>(k), x, y, f16)) return m >= split_min_rows(n, k, f16);
     if (k < 256 || !aligned(x, 16)) return false;
-    // f16 by the kernel that walks all of K, which keeps no planes (more rows than these are for the matrix cores by the lines below too):
-    // 2880 x 2880 at 10 / 12 / 14 rows 9.8 / 11.3 / 12.7 as matvecs, 7.9 there; 6000 x 1600 at 8 9.2 and 5.9, 23 x 4830 x 1024 13.9 and 6.1.
-    if (f16 && k >= 512 && m <= 32 && m > q8_gemv_rows_per_pass(k, f16) && q8_gemm_deep_supports(k, x) &&
-        q8_gemm_deep_plan(m, n, k, matvecs_us(m, n, k, f16) / 1.1).mt) {
-        RowsPlan plans[2];
-        q8_gemm_split_workspace_floats(m, static_cast<int>(n), static_cast<int>(k), plans);
-        if (plans[1].kind == RowsPlan::kDeep) {
-            if (plan) *plan = plans[1];
-            return true;
-        }
-    }
-    const int64_t codes = n * k;
-    const int64_t min_rows = codes >= (int64_t{32} << 20) ? 3 : codes >= (int64_t{16} << 20) ? 6 : codes >= (int64_t{8} << 20) ? 8 : 12;
-    if (m < (f16 ? min_rows * 5 / 4 : min_rows)) return false;
-    // up to four rows of one pass over the weights: 10944 x 3552 f32 at four rows 24.7 on the matrix cores, 16.4 as matvecs, f16 21.4 and
-    // 16.8; at five and more of such sizes within a tenth of each other
-    if (m <= 4 && m <= q8_gemv_rows_per_pass(k, f16)) return false;
-    bool room = room_floats == SIZE_MAX;
-    if (!room) {
-        RowsPlan plans[2];
-        room = room_floats >= q8_gemm_split_workspace_floats(m, static_cast<int>(n), static_cast<int>(k), plans);
-        if (plan && (k % 512 != 0 || n % 4 != 0)) *plan = plans[f16];
-    }
-    if (room) return rows_sliced_us(m, n, k, f16) < matvecs_us(m, n, k, f16);
+    const double matvecs = matvecs_us(m, n, k, f16);
+    const bool sliced = rows_sliced_us(m, n, k, f16) < matvecs * (n <= 1100 ? (m <= 8 ? 0.75 : 0.93) : m > 32 ? 1.15 : 1.0);
+    if (room_floats == SIZE_MAX) return sliced;
+    const bool deep = f16 && k >= 512 && q8_gemm_deep_supports(k, x) && q8_gemm_deep_plan(m, n, k, matvecs / 1.1).mt;
     const int64_t rounds = ((m + 127) / 128 * ((n + 255) / 256) + 255) / 256;
-    return static_cast<double>(m) * static_cast<double>(codes) * (f16 ? 0.085 : 0.17) / (1 << 20) >
-           8.0 + static_cast<double>(rounds * (k / 32)) * (f16 ? 0.66 : 1.2);
+    const bool whole = 8.0 + static_cast<double>(rounds * (k / 32)) * (f16 ? 0.66 : 1.2) < matvecs;
+    if (!deep && !sliced && !whole) return false;
+    RowsPlan plans[2];
+    q8_gemm_split_workspace_floats(m, static_cast<int>(n), static_cast<int>(k), plans);
+    const bool room = room_floats >= plans[f16].floats;
+    if (plan && (k % 512 != 0 || n % 4 != 0)) *plan = plans[f16];
+    if (deep && plans[1].kind == RowsPlan::kDeep) return true;
+    return room ? sliced : whole;
 }
 
 }  // namespace lhip
@@ -871,7 +856,9 @@ size_t lhip_q8_0_matmul_workspace_nbytes(int64_t m, int64_t n, int64_t k) {
     if (!f32 && !f16) return 0;
     RowsPlan plans[2];
     const size_t floats = q8_gemm_split_workspace_floats(m, static_cast<int>(n), static_cast<int>(k), plans);
-    return !f32 && plans[1].kind == RowsPlan::kDeep ? 0 : floats * sizeof(float);
+    if (k % 512 == 0 && n % 4 == 0) return floats * sizeof(float);
+    const size_t f32_floats = f32 ? plans[0].floats : 0, f16_floats = f16 && plans[1].kind != RowsPlan::kDeep ? plans[1].floats : 0;
+    return (f32_floats > f16_floats ? f32_floats : f16_floats) * sizeof(float);
 }
 
 lhip_status lhip_q8_0_matmul_plan(int64_t m, int64_t n, int64_t k, int32_t activations, size_t workspace_nbytes, int32_t plan[3]) {

@@ -63,6 +63,11 @@ bool q8_gemv_rows_pays(int64_t m, int64_t n, int64_t k, bool f16) {
     return (ragged && k > 3072) || m * n > (ragged ? 3100 : 2400);
 }
 
+bool q8_gemv_rows_one_round(int64_t m, int64_t n, int64_t k, bool f16) {
+    const GemvRowsShape p = rows_shape(m, n, k, f16);
+    return (m + p.mr - 1) / p.mr * ((n + p.r - 1) / p.r) <= 256 * kRowsWaves;
+}
+
 int q8_gemv_rows_of_pass(int64_t m, int64_t n, int64_t k, bool f16) { return rows_shape(m, n, k, f16).mr; }
 
 template <int R, int S, int MR, bool RAG, typename XT>
