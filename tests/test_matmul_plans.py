@@ -50,6 +50,14 @@ def test_tiles_of_the_kernel_for_several_rows(dtype):
     assert cuts(plans) == {(rows, sliced) for rows in (128, 192, 224, 256) for sliced in (False, True)}, list(zip(ROWS[dtype], plans))
 
 
+def test_f16_products_of_a_large_ragged_matrix_stay_with_k_slices():
+    """Weights that no cache holds: the kernel that walks all of K was up to a fifth behind there, ahead for smaller ones."""
+    for s in ((6, 8369, 6144), (11, 5048, 11904), (32, 5204, 13888), (10, 12398, 10880)):
+        assert plan(*s, "f16", workspace=True)[0] == ROWS_KERNEL, s
+    for s in ((45, 2880, 2880), (23, 4830, 1024), (251, 848, 5184), (9, 3208, 2304)):
+        assert plan(*s, "f16", workspace=True)[0] == 4, s
+
+
 def test_no_room_is_asked_for_where_neither_type_keeps_anything_in_it():
     """A K outside the weight-streaming kernel's shapes: the recommended workspace is used by the f32 or the f16 call, or it is 0."""
     lib, asked = capi.load_library(), 0
