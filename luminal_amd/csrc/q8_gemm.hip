@@ -582,7 +582,8 @@ static int gemm_slices_or_tiles(int64_t m, int64_t n, int64_t k, int out, const 
 // tiles and slices -> that kernel: 192 x 6000 x 1536 23.3 -> 11.7, 256 x 4096 x 4096 27.0 -> 20.5, 1024 x 1024 x 4096 28.6 -> 22.6, 352 x
 // 3067 x 12288 (no slices for an odd N) 191 -> 69; the other way 256 x 14336 x 4096 54 <- 66, 592 x 9820 x 768 23 <- 38.  The slices that the
 // header promises a long K stay: at 8192 and more they are ahead for most sizes (350 x 6364 x 10688 82 <- 119, 207 x 2276 x 12992 40
-// <- 43), though not for few weight rows (171 x 544 x 8192 26.3 -> 19.8).
+// <- 43), though not for few weight rows (171 x 544 x 8192 26.3 -> 19.8).  From 6144 on a seventh, for weights from memory: 141 x 3540 x 6144 28.0 <-
+// 30.0, 167 x 3528 x 7552 31.2 <- 34.0, 312 x 1928 x 7424 31.3 <- 33.6.
 // Up to 128 rows the streaming kernel stays for K below three of its steps of 512 and, where it is ahead of tiles and slices, for every
 // K outside those steps.  Where they are ahead of it, the other kernel takes what it ends a seventh sooner; us, weights from memory (from the
 // cache), tiles or slices -> it: 128 x 2880 x 2880 22.0 -> 13.9 (20.6 -> 10.9), 101 x 468 x 576 9.1 -> 4.2, 57 x 6512 x 5760 27.3 -> 25.4 (26.3 ->
@@ -596,14 +597,14 @@ static int gemm_auto_tile(int64_t m, int64_t n, int64_t k, int out, const void *
     double us;
     const int tile = gemm_slices_or_tiles(m, n, k, out, y, room, &us);
     const bool streams = m <= 128 && q8_gemm_skinny_supports(static_cast<int>(m), static_cast<int>(n), static_cast<int>(k), out, y);
-    const bool long_slices = tile > kTileSliced && tile < kTileTail && k >= 8192;
-    double margin = streams ? 1.15 : 1.05;
+    const bool sliced = tile > kTileSliced && tile < kTileTail;
+    double margin = streams || (sliced && k >= 6144) ? 1.15 : 1.05;
     if (streams && tile == kTileSkinny) {
         if (m <= 32 || k % 512 != 0 || k < 1536) return tile;
         us = q8_gemm_skinny_us(static_cast<int>(m), static_cast<int>(n), static_cast<int>(k), room);
         margin = m > 64 ? 1.2 : 1.25;
     }
-    if (long_slices || k < 256 || !q8_gemm_deep_supports(k, nullptr)) return tile;
+    if ((sliced && k >= 8192) || k < 256 || !q8_gemm_deep_supports(k, nullptr)) return tile;
     const DeepPlan deep = q8_gemm_deep_plan(m, n, k, us / margin);
     return deep.mt ? kTileDeep + 10 * deep.mt + deep.nt : tile;
 }
