@@ -265,17 +265,34 @@ __global__ __launch_bounds__(64 * 4 * kDirectRows) void mx_moe_few_down_kernel(c
     }
 }
 
-// Column blocks a workgroup walks.  Two workgroups are resident a CU; with as many as one round of them takes, requests never stop;
-// three blocks at least once that leaves a workgroup for every CU, five (32 columns: six) at most, beyond which workgroups of few tiles
-// leave the CUs at different times.
-// Measured, us a layer by (gate|up, down) blocks: T = 2 (3, 3) 29.2, (5, 3) 32.4, (2, 1) 33.6; T = 4 (5, 3) 41.6, (3, 3) 43.9, (12, 6)
-// 42.5; T = 8 (5, 5) 59.2, (3, 1) 69.5; T = 16 (5, 6) 73.1, (3, 3) 79.9, (8, 4) 83.8.
-static int few_blocks(const MoeFewLayer &l, int all, int most) {
+// Experts that T tokens' choices are expected to touch (T small).
+static double few_tiles(int T, int E, int topk) {
     double none = 1.0;  // an expert's chance of no row
-    for (int i = 0; i < l.T; ++i) none *= 1.0 - static_cast<double>(l.topk) / l.E;
-    const double units = l.E * (1.0 - none) * all;
-    const int blocks = static_cast<int>(units / 480.0) + 1, least = units > 512.0 ? 3 : units > 256.0 ? 2 : 1;
-    return blocks < least ? least : blocks > most ? most : blocks;
+    for (int i = 0; i < T; ++i) none *= 1.0 - static_cast<double>(topk) / E;
+    return E * (1.0 - none);
+}
+
+// Column blocks a workgroup walks.  Two workgroups are resident a CU; with as many as one round of them takes, requests never stop, and
+// five (32 columns: six) are the most, beyond which workgroups of few tiles leave the CUs at different times.  Where the blocks of all
+// expected tiles are about one to four a CU, the number with which the fullest CU walks the fewest: between, some CUs have twice the
+// work of others.
+// Measured, us a layer by (gate|up, down) blocks, 32 experts of 2880 x 2880, top 4: T = 2 (3, 3) 29.2, (5, 3) 32.4, (2, 1) 33.6; T = 4 (5, 3) 41.6,
+// (3, 3) 43.9, (12, 6) 42.5; T = 8 (5, 5) 59.2, (3, 1) 69.5; T = 16 (5, 6) 73.1, (3, 3) 79.9, (8, 4) 83.8.  By the fullest CU: four tiles of
+// 4096 x 4096, gate|up in 2 / 3 / 4 blocks 27.7 / 30.0 / 27.8, of 3584 27.5 / 30.0 / 27.2, of 2880 22.9 / 21.9 / 22.6; eight of 4096, down 44.4 / 46.6 /
+// 44.4 (three blocks at least were taken before).
+static int few_blocks(const MoeFewLayer &l, int all, int most) {
+    const double tiles = few_tiles(l.T, l.E, l.topk), units = tiles * all;
+    if (units <= 1100.0) {
+        int blocks = 1;
+        double least = 1e30;
+        for (int b = 1; b <= 4; ++b) {
+            const double turns = b * ceil(tiles * ((all + b - 1) / b) / 256.0 - 0.05);
+            if (turns <= least) least = turns, blocks = b;
+        }
+        return blocks;
+    }
+    const int blocks = static_cast<int>(units / 480.0) + 1;
+    return blocks > most ? most : blocks;
 }
 
 template <bool GATED>
