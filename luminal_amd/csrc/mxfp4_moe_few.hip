@@ -320,11 +320,16 @@ static lhip_status launch_few(const uint8_t *nib, const uint8_t *sc, const __bf1
     return LHIP_OK;
 }
 
-// (A K of several segments pays while the tiles are few: 8 experts of 4096 x 14336, top 2, T = 1 118 -> 43 us, T = 16 145 -> 141, T = 32
-// 150 -> 163; 32 of 5120 x 5120, top 2, T = 6 103 -> 97, T = 8 110 -> 116.)
+// A K of several segments pays while the tiles are few: 8 experts of 4096 x 14336, top 2, T = 1 118 -> 43 us, T = 16 147 -> 125 (T = 20 of them
+// 150 and 131); 32 of 5120 x 5120, top 2, T = 6 103 -> 97, T = 8 110 <- 116.  A hidden size of several segments re-reads the activations
+// besides: from seven experts and 420 MB of weights on the plan's tiles are ahead (16 of 5120 x 8192, top 1, T = 8 104 <- 116, T = 24 160 <- 182;
+// 8 of 6144 x 6144, top 2, T = 12 98 <- 109; the other way T = 6 96 -> 85, 4 of 8192 x 8192, T = 8 112 -> 93).
 bool moe_few_takes(int T, int H, int I, int E, int topk) {
     const int64_t R = static_cast<int64_t>(T) * topk;
-    return R <= kFewRows && ((H <= 512 * kFewD && I <= 512 * kFewD) || R <= (E <= 16 ? 32 : 12));
+    if (R > kFewRows || (H <= 512 * kFewD && I <= 512 * kFewD)) return R <= kFewRows;
+    const double experts = few_tiles(T, E, topk);
+    if (H > 512 * kFewD && experts > 6.0 && experts * 1.6 * H * I > 420e6) return false;
+    return R <= (E <= 16 ? 32 : 12);
 }
 
 lhip_status moe_few_forward(const MoeFewLayer &l, hipStream_t s) {
