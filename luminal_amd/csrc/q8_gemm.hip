@@ -383,14 +383,17 @@ static GemmTail gemm_tail_plan(int64_t m, int64_t n, int64_t k, int out, const v
 }
 
 // Whether the sliced remainder ends before one launch of mixed tiles: half units of a 128x256 tile over all of K (0.64
-// us per 64 of K), the remainder's share of a round, and 25 us for its launch, its planes and their sum.  Measured,
-// sliced remainder against mixed tiles: 2048 x 14336 x 4096 313 against 273 us.  A remainder of two column tiles or less is compared with
-// tiles of 256 and 128 rows only and stays as it was: 1024 x 8692 x 4096 120.7 in slices and 118.7 in one launch with 192 rows.
+// us per 64 of K), the remainder's share of a round, and its launch, its planes and their sum: 25 us behind several rounds, where the two
+// are level at 1.06 of the one launch's time; behind a single one, whose planes are few, 2 us, unless 25 are a fifth of it.  Measured, us,
+// sliced and one launch: 2023 x 17016 x 4096 321 and 335, 916 x 25056 x 4096 245 and 225; behind a single round 439 x 16896 x 5120 136 and 126,
+// 794 x 8352 x 14336 320 and 282, 952 x 9028 x 2048 73 and 62, 479 x 16540 x 8192 194 and 212, 1906 x 4456 x 8192 194 and 197, 960 x 8196 x 4096 106
+// and 106, 1024 x 8692 x 4096 111 and 108, 1962 x 4356 x 4096 113 and 107 (these three are sliced).
 static bool gemm_tail_pays(const GemmTail &t, int64_t m, int64_t n, int64_t k) {
     if (t.slices < 2) return false;
     const double unit = 0.64 * static_cast<double>(k / kBK);
-    return q8_gemm_wide_ends(m, t.n_main) * unit + 2.0 * unit / t.slices + 25.0 <
-           q8_gemm_wide_ends(m, n, n - t.n_main > 512) * unit;
+    const bool one_round = (m + 255) / 256 * (t.n_main / 128) <= 256;
+    const double one = q8_gemm_wide_ends(m, n) * unit, sliced = q8_gemm_wide_ends(m, t.n_main) * unit + 2.0 * unit / t.slices;
+    return one_round ? sliced + 2.0 < one && sliced + 25.0 < 1.22 * one : sliced + 25.0 < 1.06 * one;
 }
 
 // M tiles per group of the raster: the activation tiles of a group of rows stay in an XCD's L2 while its N tiles pass.

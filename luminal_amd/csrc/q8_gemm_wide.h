@@ -21,8 +21,7 @@ bool q8_gemm_wide_supports(int64_t k);
 lhip_status q8_gemm_wide_launch(const int8_t *qs, const __half *ds, const void *x, WdType type, void *y, int m, int n, int k,
                                 int out, hipStream_t s, int slices = 1, int ldy = 0);
 // When a launch of that product ends, in half units of a 128x256 tile's time over all of K (1.3 us per 64 of K).
-// (all_heights: its tiles of 192 and 224 rows too.)
-double q8_gemm_wide_ends(int64_t m, int64_t n, bool all_heights = true);
+double q8_gemm_wide_ends(int64_t m, int64_t n);
 // 192 or 224 where a launch over all of K takes tiles of so many rows for its last or only round, else 0.
 int q8_gemm_wide_special_height(int64_t m, int64_t n);
 

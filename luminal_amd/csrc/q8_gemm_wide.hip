@@ -369,7 +369,7 @@ struct WdCut {
     int n_big = 0, small = 128;
     double end = 0.0;  // in half units of a 128x256 tile's time
 };
-static WdCut wd_cut(int64_t m, int64_t n, bool all_heights = true) {
+static WdCut wd_cut(int64_t m, int64_t n) {
     const int64_t mt256 = (m + 255) / 256, n_tiles = n / kWdBN, n_all = (n + kWdBN - 1) / kWdBN;  // whole tiles, all of them
     const int64_t rounds = mt256 * n_tiles / 256;
     const int64_t cuts[4] = {0, n_tiles, rounds * 256 / mt256, (rounds - 1) * 256 / mt256};
@@ -382,7 +382,6 @@ static WdCut wd_cut(int64_t m, int64_t n, bool all_heights = true) {
     best.end = 1e300;
 #pragma unroll
     for (const auto &h : heights) {
-        if (h.rows != 128 && !all_heights) break;
         const int64_t mt = (m + h.rows - 1) / h.rows;
         for (int i = 0; i < 4; ++i) {
             const int64_t c = cuts[i];
@@ -415,7 +414,7 @@ static WdCut wd_cut(int64_t m, int64_t n, bool all_heights = true) {
     return best;
 }
 
-double q8_gemm_wide_ends(int64_t m, int64_t n, bool all_heights) { return wd_cut(m, n, all_heights).end; }
+double q8_gemm_wide_ends(int64_t m, int64_t n) { return wd_cut(m, n).end; }
 
 int q8_gemm_wide_special_height(int64_t m, int64_t n) {
     const WdCut cut = wd_cut(m, n);
