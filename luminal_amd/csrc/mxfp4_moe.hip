@@ -182,9 +182,8 @@ struct MoeGemmArgs {
     const int *tile_expert, *tile_row0, *tile_rows, *n_tiles;
     const int *tile_run0, *tile_runlen; // runs of tiles of one expert (MoePlan)
     int tiles_per_xcd;                  // layout of the tile list (MoePlan::tiles_per_xcd)
-    void *out;                          // bf16 [R][N] (gated) or f32 [R][N]
-    // Gated GEMM with NT == 4 only: when q_hi is set, the epilogue quantises its bf16 result for the next GEMM
-    // (planes of row stride q_kp, scales of row stride q_kp / 32) instead of writing `out`.
+    float *out;                         // [R][N], down GEMM
+    // Gated GEMM: its epilogue quantises the bf16 result for the next GEMM (planes of row stride q_kp, scales of row stride q_kp / 32).
     uint8_t *q_hi, *q_lo, *q_sc;
     int q_kp;
 };
@@ -197,7 +196,7 @@ struct MoeGemmArgs {
 template <int MT, int NT, bool GATED, int WR, int D>
 __global__ __launch_bounds__(256 * WR) __attribute__((amdgpu_waves_per_eu(1, (MT >= 8 && WR == 1) ? 1 : 8)))
 void mx_moe_gemm_kernel(MoeGemmArgs g) {
-    static_assert(!GATED || NT % 2 == 0, "gated tiles pair each gate fragment with its up fragment");
+    static_assert(!GATED || NT == 4, "a wave's two pairs of gate and up fragments are one block of the next GEMM's activations");
     static_assert(MT % WR == 0 && D % 2 == 0, "tile shape");
     constexpr int BM = 16 * MT;
     constexpr int MTW = MT / WR;      // row fragments per wave
@@ -210,36 +209,26 @@ void mx_moe_gemm_kernel(MoeGemmArgs g) {
 
     // Which tile and which column block.  Workgroups are dispatched in the order of their linear number
     // (x fastest) and dealt to the eight XCDs in turn, so the workgroups with the same number modulo 8 share an L2.
-    // With a tile list laid out per XCD, those take the entries of their XCD's range in order, all column blocks
+    // They take the entries of their XCD's range of the tile list in order, all column blocks
     // of one tile after another: the tile's activation rows, which every column block reads, come out of that L2
     // after their first use.  Where an expert was cut into a run of several tiles, the run is walked column block
     // by column block instead (all tiles of the run for one block, then the next block): the workgroups that read
     // the same weights are dispatched next to each other and share one fetch of them.  Entries without a tile have
     // no rows.
-    int tile = blockIdx.y, cb = blockIdx.x;
-    int expert, row0, rows;
-    if (g.tiles_per_xcd) {
-        const int linear = blockIdx.y * gridDim.x + blockIdx.x;
-        const int turn = linear >> 3, cols = static_cast<int>(gridDim.x);
-        const int base = (linear & 7) * g.tiles_per_xcd;
-        const int entry = turn / cols;  // < gridDim.y / 8 = tiles_per_xcd
-        cb = turn - entry * cols;
-        tile = base + entry;
-        // (the entry's own tile is read in the same trip to memory; only a workgroup inside a run pays a second one,
-        // and not for the expert, which the run shares)
-        expert = g.tile_expert[tile];
-        row0 = g.tile_row0[tile];
-        rows = g.tile_rows[tile];
-        const int run0 = g.tile_run0[tile], runlen = g.tile_runlen[tile];
-        if (runlen > 1) {
-            const int local = turn - (run0 - base) * cols;  // position among the run's runlen * cols workgroups
-            cb = local / runlen;
-            tile = run0 + (local - cb * runlen);
-            row0 = g.tile_row0[tile];
-            rows = g.tile_rows[tile];
-        }
-    } else {
-        expert = g.tile_expert[tile];
+    const int linear = blockIdx.y * gridDim.x + blockIdx.x;
+    const int turn = linear >> 3, cols = static_cast<int>(gridDim.x);
+    const int base = (linear & 7) * g.tiles_per_xcd;
+    const int entry = turn / cols;  // < gridDim.y / 8 = tiles_per_xcd
+    int cb = turn - entry * cols, tile = base + entry;
+    // (the entry's own tile is read in the same trip to memory; only a workgroup inside a run pays a second one,
+    // and not for the expert, which the run shares)
+    const int expert = g.tile_expert[tile];
+    int row0 = g.tile_row0[tile], rows = g.tile_rows[tile];
+    const int run0 = g.tile_run0[tile], runlen = g.tile_runlen[tile];
+    if (runlen > 1) {
+        const int local = turn - (run0 - base) * cols;  // position among the run's runlen * cols workgroups
+        cb = local / runlen;
+        tile = run0 + (local - cb * runlen);
         row0 = g.tile_row0[tile];
         rows = g.tile_rows[tile];
     }
@@ -454,72 +443,58 @@ void mx_moe_gemm_kernel(MoeGemmArgs g) {
     }
 
     // ---- epilogue: acc[i][f][v] is row i*16 + 4*grp + v, column fragment f, column r
-    if constexpr (GATED && NT == 4) {
-        if (g.q_hi) {
-            // The wave's two (gate, up) pairs are the 32 intermediate columns [32 b, 32 b + 32), b = 4 cb +
-            // wave: one quantisation block of the next GEMM's activations.  Same arithmetic as
-            // mx_quantize_act_item on the bf16-rounded result (block maximum over the 16 lanes of a row group),
-            // so the intermediate activations never go through memory as bf16.
-            const int b = cb * 4 + wave;
+    if constexpr (GATED) {
+        // The wave's two (gate, up) pairs are the 32 intermediate columns [32 b, 32 b + 32), b = 4 cb +
+        // wave: one quantisation block of the next GEMM's activations.  Same arithmetic as
+        // mx_quantize_act_item on the bf16-rounded result (block maximum over the 16 lanes of a row group),
+        // so the intermediate activations never go through memory as bf16.
+        const int b = cb * 4 + wave;
 #pragma unroll
-            for (int i = 0; i < MTW; ++i)
+        for (int i = 0; i < MTW; ++i)
 #pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const int m = (i * WR + wrow) * 16 + 4 * grp + v;
-                    if (m >= rows) continue;  // uniform over the 16 lanes that exchange values below
-                    float a[2];
+            for (int v = 0; v < 4; ++v) {
+                const int m = (i * WR + wrow) * 16 + 4 * grp + v;
+                if (m >= rows) continue;  // uniform over the 16 lanes that exchange values below
+                float a[2];
 #pragma unroll
-                    for (int p = 0; p < 2; ++p) {
-                        const float gate = acc[i][2 * p][v], up = acc[i][2 * p + 1][v];
-                        const float act = up * (gate * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504f * gate)));
-                        a[p] = col[2 * p] < g.N ? static_cast<float>(static_cast<__bf16>(act)) : 0.f;
-                    }
-                    const float amax = row16_max(fmaxf(fabsf(a[0]), fabsf(a[1])));
-                    int e = 127;
-                    float inv = 1.0f;
-                    if (amax > 0.f && amax < __uint_as_float(0x7f800000u)) {
-                        const int ex = static_cast<int>((__float_as_uint(amax) >> 23) & 0xff);
-                        e = max(ex - 7, kLoShift + 1);
-                        inv = __uint_as_float(static_cast<uint32_t>(254 - e) << 23);
-                    }
-                    const float s0 = a[0] * inv, s1 = a[1] * inv;
-                    const int h = __builtin_amdgcn_cvt_pk_fp8_f32(s0, s1, 0, false);
-                    const float r0 = s0 - __builtin_amdgcn_cvt_f32_fp8(h, 0), r1 = s1 - __builtin_amdgcn_cvt_f32_fp8(h, 1);
-                    const int l = __builtin_amdgcn_cvt_pk_fp8_f32(r0 * kLoGain, r1 * kLoGain, 0, false);
-                    const size_t at = static_cast<size_t>(row0 + m) * g.q_kp + b * 32 + r;
-                    g.q_hi[at] = static_cast<uint8_t>(h);
-                    g.q_hi[at + 16] = static_cast<uint8_t>(h >> 8);
-                    g.q_lo[at] = static_cast<uint8_t>(l);
-                    g.q_lo[at + 16] = static_cast<uint8_t>(l >> 8);
-                    if (r == 0)
-                        g.q_sc[static_cast<size_t>(row0 + m) * (g.q_kp / 32) + b] = static_cast<uint8_t>(b * 32 < g.N ? e : 127);
+                for (int p = 0; p < 2; ++p) {
+                    const float gate = acc[i][2 * p][v], up = acc[i][2 * p + 1][v];
+                    const float act = up * (gate * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504f * gate)));
+                    a[p] = col[2 * p] < g.N ? static_cast<float>(static_cast<__bf16>(act)) : 0.f;
                 }
-            return;
-        }
-    }
+                const float amax = row16_max(fmaxf(fabsf(a[0]), fabsf(a[1])));
+                int e = 127;
+                float inv = 1.0f;
+                if (amax > 0.f && amax < __uint_as_float(0x7f800000u)) {
+                    const int ex = static_cast<int>((__float_as_uint(amax) >> 23) & 0xff);
+                    e = max(ex - 7, kLoShift + 1);
+                    inv = __uint_as_float(static_cast<uint32_t>(254 - e) << 23);
+                }
+                const float s0 = a[0] * inv, s1 = a[1] * inv;
+                const int h = __builtin_amdgcn_cvt_pk_fp8_f32(s0, s1, 0, false);
+                const float r0 = s0 - __builtin_amdgcn_cvt_f32_fp8(h, 0), r1 = s1 - __builtin_amdgcn_cvt_f32_fp8(h, 1);
+                const int l = __builtin_amdgcn_cvt_pk_fp8_f32(r0 * kLoGain, r1 * kLoGain, 0, false);
+                const size_t at = static_cast<size_t>(row0 + m) * g.q_kp + b * 32 + r;
+                g.q_hi[at] = static_cast<uint8_t>(h);
+                g.q_hi[at + 16] = static_cast<uint8_t>(h >> 8);
+                g.q_lo[at] = static_cast<uint8_t>(l);
+                g.q_lo[at + 16] = static_cast<uint8_t>(l >> 8);
+                if (r == 0)
+                    g.q_sc[static_cast<size_t>(row0 + m) * (g.q_kp / 32) + b] = static_cast<uint8_t>(b * 32 < g.N ? e : 127);
+            }
+    } else {
 #pragma unroll
-    for (int i = 0; i < MTW; ++i)
+        for (int i = 0; i < MTW; ++i)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int m = (i * WR + wrow) * 16 + 4 * grp + v;
-            if (m >= rows) continue;
-            const size_t orow = static_cast<size_t>(row0 + m) * g.N;
-            if (GATED) {
-#pragma unroll
-                for (int p = 0; p < NT / 2; ++p)
-                    if (col[2 * p] < g.N) {
-                        const float gate = acc[i][2 * p][v], up = acc[i][2 * p + 1][v];
-                        // Hardware exp2 and reciprocal (1 ulp each): the result is rounded to bf16 right away,
-                        // and the library forms cost more than the tile's matrix work is worth.
-                        const float act = up * (gate * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504f * gate)));
-                        static_cast<__bf16 *>(g.out)[orow + col[2 * p]] = static_cast<__bf16>(act);
-                    }
-            } else {
+            for (int v = 0; v < 4; ++v) {
+                const int m = (i * WR + wrow) * 16 + 4 * grp + v;
+                if (m >= rows) continue;
+                const size_t orow = static_cast<size_t>(row0 + m) * g.N;
 #pragma unroll
                 for (int f = 0; f < NT; ++f)
-                    if (col[f] < g.N) static_cast<float *>(g.out)[orow + col[f]] = acc[i][f][v];
+                    if (col[f] < g.N) g.out[orow + col[f]] = acc[i][f][v];
             }
-        }
+    }
 }
 
 // y[t][h] = bf16( sum_s wts[t][s] * out[slot_of[t*topk+s]][h] ), 4 columns per thread
@@ -721,8 +696,7 @@ lhip_status lhip_mxfp4_moe_bf16_mode(const void *w_gate_up_planar, const void *w
     a1.rows_per_expert = 2 * I; a1.K = H; a1.Kp = Hp; a1.N = I;
     a1.tile_expert = w.plan.tile_expert; a1.tile_row0 = w.plan.tile_row0; a1.tile_rows = w.plan.tile_rows;
     a1.tile_run0 = w.plan.tile_run0; a1.tile_runlen = w.plan.tile_runlen;
-    a1.n_tiles = w.plan.n_tiles; a1.tiles_per_xcd = w.plan.tiles_per_xcd; a1.out = w.act;
-    // Every gated kernel launched below quantises its result for the down GEMM in its epilogue.
+    a1.n_tiles = w.plan.n_tiles; a1.tiles_per_xcd = w.plan.tiles_per_xcd;
     a1.q_hi = w.a_hi; a1.q_lo = w.a_lo; a1.q_sc = w.a_sc; a1.q_kp = Ip;
     // Column blocks: 4 waves x (NT/2) gate/up pairs of 16.  Tall row tiles take 4 weight
     // fragments per wave, so each activation fragment read from LDS feeds twice the MFMAs.

@@ -33,16 +33,16 @@ struct MoePlan {
     int *tile_expert;  // [max_tiles]
     int *tile_row0;    // [max_tiles] first slot of the tile
     int *tile_rows;    // [max_tiles] valid rows in the tile (0 = unused entry)
-    // [max_tiles] the run of a tile: the consecutive list entries that hold tiles of the same expert (on the same XCD,
-    // when the list is cut per XCD) start at entry tile_run0 and number tile_runlen (0 = unused entry).  The exact
+    // [max_tiles] the run of a tile: the consecutive list entries that hold tiles of the same expert (on the same XCD)
+    // start at entry tile_run0 and number tile_runlen (0 = unused entry).  The exact
     // GEMMs walk a run column block by column block, so that the workgroups that read the same weights run together.
     int *tile_run0, *tile_runlen;
     int *n_tiles;      // [1]
     int max_tiles;     // entries of the tile arrays
     int by_rows;       // whether experts are listed by their rows (else in their own order)
     int fragment;      // rows of a matrix step: a tile is some number of these, but for the end of an expert
-    // 0: tiles are listed in expert order from entry 0.  Otherwise the list is cut into eight ranges of this many
-    // entries, one per XCD (range x is read by the workgroups whose dispatch number is x modulo 8), and the
+    // The list is cut into eight ranges of this many entries, one per XCD (range x is read by the workgroups whose
+    // dispatch number is x modulo 8), and the
     // tiles, an expert's behind each other, are dealt to the ranges in eight contiguous, equal shares: the tiles of an
     // expert, and all column blocks of a tile, then run on one XCD and find each other's weights and
     // activation rows in its L2.
@@ -129,14 +129,11 @@ __device__ __forceinline__ void moe_plan_block(const int *__restrict__ sel, int 
         const int nt_first = nt, nt_end = nt + tiles_e;
         for (int m0 = 0, i = 0; m0 < cnt[e]; ++i) {
             const int per = (frags_e / tiles_e + (i < frags_e % tiles_e ? 1 : 0)) * p.fragment;
-            int at = nt, run_first = nt_first, run_end = nt_end;
-            if (p.tiles_per_xcd) {  // tile nt of `total` goes to range x = floor(8 nt / total), behind that range's earlier tiles
-                const int x = nt * 8 / total;
-                const int x_first = (x * total + 7) / 8, x_end = ((x + 1) * total + 7) / 8;  // the tiles of range x
-                at = x * p.tiles_per_xcd + nt - x_first;
-                run_first = max(nt_first, x_first);
-                run_end = min(nt_end, x_end);
-            }
+            // tile nt of `total` goes to range x = floor(8 nt / total), behind that range's earlier tiles
+            const int x = nt * 8 / total;
+            const int x_first = (x * total + 7) / 8, x_end = ((x + 1) * total + 7) / 8;  // the tiles of range x
+            const int at = x * p.tiles_per_xcd + nt - x_first;
+            const int run_first = max(nt_first, x_first), run_end = min(nt_end, x_end);
             p.tile_expert[at] = e;
             p.tile_row0[at] = o + m0;
             p.tile_rows[at] = min(per, cnt[e] - m0);

@@ -42,35 +42,28 @@ struct MoeExactArgs {
     void *out;            // bf16 [R][N] (gated) or f32 [R][N]
 };
 
-// Tile and column block of this workgroup (see MoePlan::tiles_per_xcd for the per-XCD list).
+// Tile and column block of this workgroup (by MoePlan::tiles_per_xcd).
 // Within a run of tiles of one expert the workgroups are ordered column block by column block: the tiles that
 // read the same weights are dispatched next to each other and share one fetch of them out of the XCD's L2.
 __device__ __forceinline__ void exact_tile(const MoeExactArgs &g, int &tile, int &cb, int &expert, int &row0, int &rows) {
-    tile = blockIdx.y, cb = blockIdx.x;
-    if (g.tiles_per_xcd) {
-        const int linear = blockIdx.y * gridDim.x + blockIdx.x;
-        const int turn = linear >> 3, cols = static_cast<int>(gridDim.x);
-        const int base = (linear & 7) * g.tiles_per_xcd;
-        const int entry = turn / cols;
-        cb = turn - entry * cols;
-        tile = base + entry;
-        // (the entry's own tile is read in the same trip to memory; only a workgroup inside a run pays a second one,
-        // and not for the expert, which the run shares)
-        expert = g.tile_expert[tile];
-        row0 = g.tile_row0[tile];
-        rows = g.tile_rows[tile];
-        const int run0 = g.tile_run0[tile], runlen = g.tile_runlen[tile];
-        if (runlen > 1) {
-            const int local = turn - (run0 - base) * cols;  // position among the run's runlen * cols workgroups
-            cb = local / runlen;
-            // (Tall tiles first in a run: dealt to 32 compute units in turn, a run of two would give every other one tall tiles only.
-            // So the tiles trade places from one 32 to the next: T = 1024 241 -> 235 us.)
-            tile = run0 + (local - cb * runlen + ((turn - local + cb * runlen) >> 5)) % runlen;
-            row0 = g.tile_row0[tile];
-            rows = g.tile_rows[tile];
-        }
-    } else {
-        expert = g.tile_expert[tile];
+    const int linear = blockIdx.y * gridDim.x + blockIdx.x;
+    const int turn = linear >> 3, cols = static_cast<int>(gridDim.x);
+    const int base = (linear & 7) * g.tiles_per_xcd;
+    const int entry = turn / cols;
+    cb = turn - entry * cols;
+    tile = base + entry;
+    // (the entry's own tile is read in the same trip to memory; only a workgroup inside a run pays a second one,
+    // and not for the expert, which the run shares)
+    expert = g.tile_expert[tile];
+    row0 = g.tile_row0[tile];
+    rows = g.tile_rows[tile];
+    const int run0 = g.tile_run0[tile], runlen = g.tile_runlen[tile];
+    if (runlen > 1) {
+        const int local = turn - (run0 - base) * cols;  // position among the run's runlen * cols workgroups
+        cb = local / runlen;
+        // (Tall tiles first in a run: dealt to 32 compute units in turn, a run of two would give every other one tall tiles only.
+        // So the tiles trade places from one 32 to the next: T = 1024 241 -> 235 us.)
+        tile = run0 + (local - cb * runlen + ((turn - local + cb * runlen) >> 5)) % runlen;
         row0 = g.tile_row0[tile];
         rows = g.tile_rows[tile];
     }
