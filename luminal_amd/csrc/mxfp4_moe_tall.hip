@@ -21,6 +21,7 @@
 // 110, T = 512 184 -> 147, T = 1024 266 -> 231 (880 TFLOP/s of useful work), T = 2048 449 -> 409.
 #include <algorithm>
 
+#include "lds_request.h"
 #include "mxfp4_moe_exact_device.h"
 
 namespace lhip {
@@ -39,16 +40,6 @@ struct TallShape {
     static_assert(3 * LDS <= 160 * 1024, "three workgroups a CU");
 };
 
-// 64 lanes x 16 (4) bytes from base + the lane's offset to consecutive LDS from `lds` on.  Inline assembly, because the compiler
-// would otherwise wait for the newest of them ahead of every LDS read.  (m0 is a reserved register: the compiler keeps nothing in it
-// from one statement to another.)
-template <int BYTES>
-__device__ __forceinline__ void tall_request(const void *base, uint32_t voff, uint32_t lds) {
-    if constexpr (BYTES == 16)
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base) : "memory");
-    else
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(voff), "s"(base) : "memory");
-}
 // Until at most N of this wave's requests are under way and its LDS accesses are done.
 template <int N>
 __device__ __forceinline__ void tall_wait() {
@@ -95,8 +86,8 @@ __global__ __launch_bounds__(64 * TallShape::NW, 3) void mx_moe_gemm_tall_kernel
         const int tt = min(t, stages - 1);  // past the end: the last stage again, never used
         const uint32_t dst = lds0 + w_lds + buf * S::W_WAVE;
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) tall_request<16>(w_base + static_cast<size_t>(tt) * 512, w_off[j], dst + j * 1024);
-        tall_request<4>(s_base + static_cast<size_t>(tt) * 32, s_off, dst + NJ * 1024);
+        for (int j = 0; j < NJ; ++j) lds_request<16>(w_base + static_cast<size_t>(tt) * 512, w_off[j], dst + j * 1024);
+        lds_request<4>(s_base + static_cast<size_t>(tt) * 32, s_off, dst + NJ * 1024);
     };
 
     // ---- requests of activations: number q of a wave brings eight rows of fragment q; piece p of a row lies at slot
@@ -120,8 +111,8 @@ __global__ __launch_bounds__(64 * TallShape::NW, 3) void mx_moe_gemm_tall_kernel
         for (int q = 0; q < MF; ++q) {
             if (q >= frags) continue;
             const int at = buf * S::A_STAGE + (q * NW + wave) * 1024;
-            if (whole) tall_request<16>(base, a_off[q], lds0 + at);
-            else if (in) tall_request<16>(base, a_off[q], lds0 + at);
+            if (whole) lds_request<16>(base, a_off[q], lds0 + at);
+            else if (in) lds_request<16>(base, a_off[q], lds0 + at);
             else *reinterpret_cast<mu32x4 *>(lds + at + lane * 16) = mu32x4{0, 0, 0, 0};
         }
     };

@@ -25,6 +25,7 @@
 #include <utility>
 
 #include "common.h"
+#include "lds_request.h"
 #include "q8_gemm_deep.h"
 #include "q8_mma_device.h"
 
@@ -46,21 +47,7 @@ struct DpShape {
     static_assert(LDS <= 160 * 1024, "LDS");
 };
 
-// 64 lanes x 16 bytes from base + the lane's offset to consecutive LDS from `lds` on (as in q8_gemm_wide.hip).
-__device__ __forceinline__ void dp_request(const void *base, uint32_t voff, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base) : "memory");
-}
-template <int N>
-__device__ __forceinline__ void dp_wait() {  // until at most N of this wave's loads are under way
-    asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory");
-}
-__device__ __forceinline__ void dp_barrier() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
-
-// (qs and ds without __restrict__: the loads through them keep their place among the requests, which dp_wait counts.)
+// (qs and ds without __restrict__: the loads through them keep their place among the requests, which wait_loads counts.)
 template <int MT, int NT, typename XT, int OUT>
 __global__ __launch_bounds__(512) void q8_gemm_deep_kernel(const int8_t *qs, const unsigned short *ds, const XT *x, void *y, int M, int N, int K,
                                                            int m_tiles, int n_tiles) {
@@ -98,7 +85,7 @@ __global__ __launch_bounds__(512) void q8_gemm_deep_kernel(const int8_t *qs, con
         const int pair = min(((t >> 1) * kDpQuads + kq) * 2 + (t & 1), pairs - 1);
         const uint32_t st = lds0 + stage * S::STAGE + kq * S::PAIR + nh * (MT * 1024);
 #pragma unroll
-        for (int u = 0; u < MT; ++u) dp_request(xb + static_cast<size_t>(pair) * 128, a_off[u], st + u * 1024);
+        for (int u = 0; u < MT; ++u) lds_request<16>(xb + static_cast<size_t>(pair) * 128, a_off[u], st + u * 1024);
     };
 
     // ---- codes and scales of a quad: lane (r, g) loads 16 codes of each pair of row r
@@ -221,8 +208,8 @@ __global__ __launch_bounds__(512) void q8_gemm_deep_kernel(const int8_t *qs, con
     auto last_stage = [&]() { return stage == 0 ? ST - 1 : stage - 1; };  // the one that the step before this has read
     auto quad = [&](int qi) __attribute__((always_inline)) {
         const int left = pairs - (qi * kDpQuads + kq) * 2;  // pairs of the quad that are there
-        dp_wait<(ST - 2) * MT>();
-        dp_barrier();
+        wait_loads<(ST - 2) * MT>();
+        bare_barrier();
         take(qi);
         __builtin_amdgcn_sched_barrier(0);
         load_scales(qi + 1);
@@ -238,8 +225,8 @@ __global__ __launch_bounds__(512) void q8_gemm_deep_kernel(const int8_t *qs, con
         }
         stage = next_stage();
         __builtin_amdgcn_sched_barrier(0);
-        dp_wait<(ST - 2) * MT + CODES>();
-        dp_barrier();
+        wait_loads<(ST - 2) * MT + CODES>();
+        bare_barrier();
         request(2 * qi + ST, last_stage());
         __builtin_amdgcn_sched_barrier(0);
         if (left > 1) blocks(dp_lds + stage * S::STAGE, std::integral_constant<int, 2>{});
@@ -257,8 +244,8 @@ __global__ __launch_bounds__(512) void q8_gemm_deep_kernel(const int8_t *qs, con
     __builtin_amdgcn_sched_barrier(0);
     int qi = 0;
     do quad(qi); while (++qi < rounds);  // (at least once: behind a test the first loads would be moved past it)
-    dp_wait<0>();  // no request outlives its buffer, which the epilogue now takes over
-    dp_barrier();
+    wait_loads<0>();  // no request outlives its buffer, which the epilogue now takes over
+    bare_barrier();
 
     // ---- epilogue: the quad columns' sums through LDS, added in their order.  Element v of lane (r, g) is row 4 g + v,
     // column r of its 16 x 16 tile.

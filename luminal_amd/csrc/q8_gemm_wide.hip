@@ -31,6 +31,7 @@
 #include <utility>
 
 #include "common.h"
+#include "lds_request.h"
 #include "q8_gemm_wide.h"
 #include "q8_mma_device.h"
 
@@ -56,25 +57,6 @@ struct WdShape {
     static constexpr int REQ = A_REQ + B_REQ + 1;            // scales
     static_assert(LDS <= 160 * 1024 && A_REQ * 8 * 1024 == A_BYTES && B_REQ * 1024 == B_WAVE, "staging split");
 };
-
-// The tile's requests: 64 lanes x 16 (4) bytes from base + the lane's offset to consecutive LDS from `lds` on.
-// Inline assembly, because the compiler would otherwise wait for the newest of them ahead of every LDS read.
-template <int BYTES>
-__device__ __forceinline__ void wd_request(const void *base, uint32_t voff, uint32_t lds) {
-    if constexpr (BYTES == 16)
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base) : "memory");
-    else
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(voff), "s"(base) : "memory");
-}
-template <int N>
-__device__ __forceinline__ void wd_wait_requests() {  // until at most N of this wave's requests are under way
-    asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory");
-}
-__device__ __forceinline__ void wd_barrier() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
 
 // Order of the tiles.  An XCD runs its workgroups in order, 32 at a time.  The (M tile, N tile, K slice) triples are numbered with the M tiles of a group of m_group (2048 rows)
 // innermost, then the slices of an N tile, then the N tiles, then the groups, and each XCD takes an equal share of
@@ -140,12 +122,12 @@ __device__ __forceinline__ void wd_tile_body(unsigned char *lds, const int8_t *_
         const int tt = min(t, KT - 1);  // past the end: the last tile again, never used
         const uint32_t st = lds0 + stage * S::STAGE;
         if constexpr (p < S::A_REQ) {
-            wd_request<16>(xb + static_cast<size_t>(tt) * 128, a_off[p], st + (wave * S::A_REQ + p) * 1024);
+            lds_request<16>(xb + static_cast<size_t>(tt) * 128, a_off[p], st + (wave * S::A_REQ + p) * 1024);
         } else if constexpr (p < S::A_REQ + S::B_REQ) {
             constexpr int q = p - S::A_REQ;
-            wd_request<16>(qb + static_cast<size_t>(tt) * 64, b_off[q], st + S::A_BYTES + wave * S::B_WAVE + q * 1024);
+            lds_request<16>(qb + static_cast<size_t>(tt) * 64, b_off[q], st + S::A_BYTES + wave * S::B_WAVE + q * 1024);
         } else {  // a row's two scales are one aligned dword (K / 32 is even)
-            wd_request<4>(db + static_cast<size_t>(tt) * 2, s_off, st + S::A_BYTES + S::B_BYTES + wave * 256);
+            lds_request<4>(db + static_cast<size_t>(tt) * 2, s_off, st + S::A_BYTES + S::B_BYTES + wave * 256);
         }
     };
     auto request = [&](int t, int stage) __attribute__((always_inline)) {
@@ -191,8 +173,8 @@ __device__ __forceinline__ void wd_tile_body(unsigned char *lds, const int8_t *_
 
 #pragma unroll
     for (int i = 0; i < S::STAGES - 1; ++i) request(i, i);
-    wd_wait_requests<(S::STAGES - 2) * S::REQ>();
-    wd_barrier();
+    wait_loads<(S::STAGES - 2) * S::REQ>();
+    bare_barrier();
 #pragma unroll
     for (int f = 0; f < AHEAD; ++f) ar[f] = *reinterpret_cast<const mma_u32x4 *>(lds + a_lane + f * 16 * S::A_ROW);
     read_raw(lds + b_lane);
@@ -215,8 +197,8 @@ __device__ __forceinline__ void wd_tile_body(unsigned char *lds, const int8_t *_
             if constexpr (f == NI) {
                 // This wave's requests for the next tile have landed, and behind the barrier everybody's; the buffer of
                 // the tile before this one is free.
-                wd_wait_requests<(S::STAGES - 3) * S::REQ>();
-                wd_barrier();
+                wait_loads<(S::STAGES - 3) * S::REQ>();
+                bare_barrier();
                 read_raw(st_next + b_lane);
                 read_scales(st_next);
             }
@@ -256,8 +238,8 @@ __device__ __forceinline__ void wd_tile_body(unsigned char *lds, const int8_t *_
         set_scales();
         stage = next;
     }
-    wd_wait_requests<0>();  // no request outlives its buffer, which the epilogue now takes over
-    wd_barrier();
+    wait_loads<0>();  // no request outlives its buffer, which the epilogue now takes over
+    bare_barrier();
 
     // ---- epilogue.  Accumulator element v of lane (r, g) is row 4 g + v, column r of its 16 x 16 tile: two-byte stores
     // of 32-byte runs.  The wave turns 64 rows at a time round in its own part of LDS, so that the lanes of a store are
