@@ -58,6 +58,14 @@ def test_f16_products_of_a_large_ragged_matrix_stay_with_k_slices():
         assert plan(*s, "f16", workspace=True)[0] == 4, s
 
 
+def test_matvecs_of_a_long_k_take_several_rows_a_pass():
+    """Whole slices of a K beyond 12288: a matvec a row was up to twice as slow there, by how few results there are (weights of any size)."""
+    for s, t in (((2, 360, 40960), "f16"), ((3, 512, 40960), "f32"), ((2, 848, 16384), "f32"), ((4, 280, 14336), "f16"), ((2, 804, 12288), "f16")):
+        assert plan(*s, t)[0] == MATVEC and plan(*s, t)[1] > 0, (s, t)
+    for s in ((3, 167, 12288), (2, 240, 4096)):
+        assert plan(*s, "f32") == (MATVEC, 0, 1), s
+
+
 def test_no_room_is_asked_for_where_neither_type_keeps_anything_in_it():
     """A K outside the weight-streaming kernel's shapes: the recommended workspace is used by the f32 or the f16 call, or it is 0."""
     lib, asked = capi.load_library(), 0
