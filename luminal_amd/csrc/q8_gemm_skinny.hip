@@ -405,12 +405,10 @@ static RowsPlan rows_plan(int64_t m, int n, int k, bool f16, size_t room, bool s
     // 256 x 6000 x 1536 22.6 -> 14.1, 256 x 4096 x 4096 24.7 -> 20.7, 80 x 4096 x 4096 17.6 -> 12.6, 96 x 8148 x 2048
     // 18.8 -> 11.3; the other way 256 x 4096 x 14336 58 <- 75, 512 x 14336 x 4096
     // 84 <- 130, 186 x 9184 x 3072 30.5 <- 32.4.
-    // Against K slices: the estimates are of weights in the memory-side cache, and from memory that kernel loses some 0.1 us more per MB of them,
-    // which shows for a large or long matrix.
+    // Against K slices it is further what it loses from memory.
     // Measured, us, weights from memory, slices and that kernel: 6 x 8369 x 6144 24.4 and 29.1, 11 x 5048 x 11904 25.9 and 35.6, 32 x 5204 x 13888 35.2
     // and 42.2; the other way 251 x 848 x 5184 16.4 and 12.9.
-    const double large = static_cast<double>(n) * static_cast<double>(k) * 1e-6 - (k < 8192 ? 16.0 : 0.0);
-    const double from_memory = best.kind == RowsPlan::kRows && best.slices > 1 && large > 0.0 ? 0.12 * large : 0.0;
+    const double from_memory = best.kind == RowsPlan::kRows && best.slices > 1 ? q8_gemm_deep_from_memory_us(n, k) : 0.0;
     if (f16 && k >= 512 && (!stream || k >= 1536 || m > 128) && q8_gemm_deep_supports(k, nullptr)) {
         const DeepPlan deep = q8_gemm_deep_plan(m, n, k, (best_us - from_memory) / 1.1);
         if (deep.mt) {

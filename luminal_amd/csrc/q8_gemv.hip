@@ -46,17 +46,21 @@ static int split_min_rows(int64_t n, int64_t k, bool f16) {
 
 // What matvecs of a K outside the streaming kernel's shapes take, us, by the kernel that runs them (q8_gemv_rows_pays): one launch, then
 // for a matvec a row its share per 1000 results and per million codes and row; for several rows a pass the products over whole slices of K
-// and, where the passes do not run side by side, the weights once a pass.  Fitted to 3100 launches, weights from memory, standard deviation
-// 9 to 16 %.
+// and, where the passes do not run side by side, the weights once a pass.  Fitted to 3100 launches with a K of up to 14336, weights from
+// memory, standard deviation 9 to 16 %; beyond it f16 and several passes are a quarter to a half above that (11448 x 33696 f16 at three rows,
+// two passes, 196 us, as K slices 141; 18824 x 14976 f32 149 and 108).  A K of which the LDS holds no row of activations: by what a matvec a row
+// measures there (5796 x 56672 f32 at three rows 354, as K slices 134; 1688 x 52544 f16 57.6 and 39.5).
 static double matvecs_us(int64_t m, int64_t n, int64_t k, bool f16) {
     const double k1000 = static_cast<double>(k) / 1000.0, rows = static_cast<double>(m), codes = static_cast<double>(n) * k1000 / 1000.0;
     const double results = rows * static_cast<double>(n) / 1000.0;
+    const int most = q8_gemv_rows_per_pass(k, f16);
+    if (most == 0) return 2.5 + 0.37 * k1000 + (f16 ? 0.25 : 0.36) * rows * codes;
     if (!q8_gemv_rows_pays(m, n, k, f16)) return f16 ? 2.5 + 0.283 * k1000 + 0.08 * results + 0.11 * rows * codes : 2.4 + 0.365 * k1000 + 0.143 * results + 0.103 * rows * codes;
     const double products = results * static_cast<double>((k + 1023) / 1024) * 1.024;
     if (q8_gemv_rows_one_round(m, n, k, f16)) return f16 ? 3.1 + 0.30 * k1000 + 0.048 * products + 0.085 * results : 3.4 + 0.25 * k1000 + 0.083 * products + 0.0007 * results;
-    const int most = q8_gemv_rows_per_pass(k, f16);
     const double read = codes * static_cast<double>((m + most - 1) / most);
-    return f16 ? 3.9 + 0.38 * k1000 + 0.037 * read + 0.053 * products + 0.02 * results : 4.0 + 0.465 * k1000 + 0.10 * read + 0.054 * products + 0.0037 * results;
+    const double beyond = k <= 14336 ? 1.0 : m <= most ? (f16 ? 1.35 : 1.0) : f16 ? 1.6 : 1.25;
+    return beyond * (f16 ? 3.9 + 0.38 * k1000 + 0.037 * read + 0.053 * products + 0.02 * results : 4.0 + 0.465 * k1000 + 0.10 * read + 0.054 * products + 0.0037 * results);
 }
 // And what q8_gemm_rows.hip takes over K slices, launch of their sum included: the blocks of K, which lie in slices beyond 33 of them, the weight
 // stream, the stores of an N that is no multiple of four, the products; up to 64 rows and above.  Fitted to as many launches, 8 to 10 %.
@@ -74,7 +78,8 @@ static double rows_sliced_us(int64_t m, int64_t n, int64_t k, bool f16) {
 // (f16) behind the faster form on average, 1.3 and 1.6 % by the prices of a matvec a row and least rows by N K (5 x 14336 x 2880 f32 25.1 -> 16.9 us,
 // 6 x 6000 x 2880 14.7 -> 11.8, 12 x 10944 x 544 f16 19.1 -> 9.7); up to 1100 weight rows, whose estimates
 // spread most, the matrix cores have to be a fourteenth ahead, a quarter for up to 8 rows of x (8 x 1001 x 14336 f32: 19 us as matvecs, 16), beyond
-// them and 32 rows of x the matvecs a seventh.  A K below 256 is a matvec of one or two microseconds per row.
+// them the matvecs a seventh for more than 32 rows of x, and for up to four the matrix cores (3 x 95540 x 544 f32 25.1 us as matvecs, 27.8).  A single row
+// is a matvec for any size.  A K below 256 is a matvec of one or two microseconds per row.
 // f16 goes by the kernel that walks all of K, which keeps no planes, where that ends a tenth before the matvecs and is the matrix cores'
 // own choice: 2880 x 2880 at 12 rows 11.0 as matvecs, 7.9 there; 6000 x 1600 at 8 9.2 and 5.9, 23 x 4830 x 1024 13.9 and 6.1, 12 x 14336 x 544
 // 22.9 and 8.2.
@@ -86,11 +91,11 @@ static double rows_sliced_us(int64_t m, int64_t n, int64_t k, bool f16) {
 static bool on_matrix_cores(int64_t m, int64_t n, int64_t k, const void *x, const void *y, bool f16, size_t room_floats,
                             RowsPlan *plan = nullptr) {
     if (q8_gemm_split_supports(static_cast<int>(n), static_cast<int>(k), x, y, f16)) return m >= split_min_rows(n, k, f16);
-    if (k < 256 || !aligned(x, 16)) return false;
+    if (m == 1 || k < 256 || !aligned(x, 16)) return false;
     const double matvecs = matvecs_us(m, n, k, f16);
-    const bool sliced = rows_sliced_us(m, n, k, f16) < matvecs * (n <= 1100 ? (m <= 8 ? 0.75 : 0.93) : m > 32 ? 1.15 : 1.0);
+    const bool sliced = rows_sliced_us(m, n, k, f16) < matvecs * (n <= 1100 ? (m <= 8 ? 0.75 : 0.93) : m > 32 ? 1.15 : m <= 4 ? 0.85 : 1.0);
     if (room_floats == SIZE_MAX) return sliced;
-    const bool deep = f16 && k >= 512 && q8_gemm_deep_supports(k, x) && q8_gemm_deep_plan(m, n, k, matvecs / 1.1).mt;
+    const bool deep = f16 && k >= 512 && q8_gemm_deep_supports(k, x) && q8_gemm_deep_plan(m, n, k, (matvecs - q8_gemm_deep_from_memory_us(n, k)) / 1.1).mt;
     const int64_t rounds = ((m + 127) / 128 * ((n + 255) / 256) + 255) / 256;
     const bool whole = 8.0 + static_cast<double>(rounds * (k / 32)) * (f16 ? 0.66 : 1.2) < matvecs;
     if (!deep && !sliced && !whole) return false;

@@ -61,7 +61,7 @@ bool q8_gemv_rows_pays(int64_t m, int64_t n, int64_t k, bool f16) {
     const int64_t further = (m - 1) * n;
     if (f16 && ragged && k <= 3072) return static_cast<double>(further) * static_cast<double>(k < 640 ? 640 : k) > (k <= 1024 ? 18e6 : 11e6);
     if (k <= 1024) return further > (f16 ? 7000 : 10000);
-    return (ragged && k > 3072) || k > 12288 || m * n > (ragged ? 3100 : k >= 12288 ? 800 : 2400);
+    return (ragged && k > 3072) || k > 12288 || m * n > (ragged ? 3100 : k >= 12288 ? 1200 : 2400);
 }
 
 bool q8_gemv_rows_one_round(int64_t m, int64_t n, int64_t k, bool f16) {

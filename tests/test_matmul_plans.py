@@ -66,6 +66,26 @@ def test_matvecs_of_a_long_k_take_several_rows_a_pass():
         assert plan(*s, "f32") == (MATVEC, 0, 1), s
 
 
+def test_a_single_row_is_a_matvec_for_any_size():
+    """Also where K is short and the weight rows are very many (128256 x 288 went to the matrix cores)."""
+    lib = capi.load_library()
+    for n in (1, 1000, 14336, 65536, 128256, 262144):
+        for k in (256, 288, 512, 1056, 2880, 8000, 14368, 40992, 70016):
+            assert lib.lhip_q8_0_matmul_workspace_nbytes(1, n, k) == 0, (n, k)
+            for dtype in ("f32", "f16"):
+                assert plan(1, n, k, dtype)[0] == plan(1, n, k, dtype, workspace=True)[0] == MATVEC, (n, k, dtype)
+
+
+def test_ragged_products_of_a_very_long_k():
+    """Where matvecs take several passes over the weights, or LDS holds no row of their activations, K slices end up to 2.6 times sooner."""
+    for s, t in (((3, 5796, 56672), "f32"), ((3, 1688, 52544), "f16"), ((3, 11448, 33696), "f16"), ((3, 18824, 14976), "f32")):
+        assert plan(*s, t, workspace=True)[0] == ROWS_KERNEL, (s, t)
+    for s, t in (((3, 6808, 22592), "f16"), ((2, 16514, 34464), "f32"), ((3, 95540, 544), "f32"), ((3, 29325, 7680), "f16")):
+        assert plan(*s, t, workspace=True)[0] == MATVEC, (s, t)
+    for s in ((8, 27324, 10368), (6, 16272, 30336)):  # (weights beyond any cache: what they cost from memory is in the estimates of both)
+        assert plan(*s, "f16", workspace=True)[0] == 4, s
+
+
 def test_no_room_is_asked_for_where_neither_type_keeps_anything_in_it():
     """A K outside the weight-streaming kernel's shapes: the recommended workspace is used by the f32 or the f16 call, or it is 0."""
     lib, asked = capi.load_library(), 0

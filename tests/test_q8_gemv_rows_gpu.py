@@ -18,7 +18,7 @@ ONE_SHOT = QuantizedMatmul(1, 1, 0, 4)
 # workgroups; the activations of one row filling a pass; K of one slice
 SIZES = [(2, 3073, 4096), (3, 4096, 4096), (4, 2051, 4096), (5, 1501, 2048), (5, 2880, 2880), (1, 7, 10272), (5, 259, 5152), (1, 1001, 14304),
          (24, 260, 3136), (13, 300, 8000), (2, 4096, 14336), (3, 1601, 13312), (1, 33, 20512), (2, 1065, 40928), (12, 1100, 2016),
-         (11, 1601, 1024), (3, 4097, 3072), (2, 12001, 1504), (7, 2050, 5120)]
+         (11, 1601, 1024), (3, 4097, 3072), (2, 12001, 1504), (7, 2050, 5120), (2, 848, 16384), (2, 360, 40960)]
 F32_ONLY = [(11, 2001, 992), (11, 1100, 1056), (2, 8193, 1056)]
 
 
