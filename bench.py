@@ -390,7 +390,7 @@ def bench_prefill_gemm(args, cpu_seconds=None):
                      "achieved": round(ach, 1), "peak": MFMA_BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(ach / MFMA_BF16_PEAK_TFLOPS, 4), "traffic": TRAFFIC["gemm"][0],
                      "traffic_source": TRAFFIC["gemm"][1], "avg_launch_us": round(us, 1)},
-        "roofline_m128": {"bound": "hbm", "kernel": "lhip::q8_gemm_skinny_kernel<8, *, 8, __bf16> (gate/up, M=128)",
+        "roofline_m128": {"bound": "hbm", "kernel": "lhip::q8_gemm_deep_kernel<*, *, __bf16, *> (gate/up, M=128)",
                           "achieved": g128["gbs"], "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": g128["frac_hbm"],
                           "traffic": None}}
     if cpu_seconds:

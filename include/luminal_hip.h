@@ -117,8 +117,9 @@ lhip_status lhip_q8_0_matmul_f32(const void *planar_dev, const float *x_dev, flo
  * change from one version of the library to the next (products whose strips fill the chip, e.g. 256 x 14336 x 4096 and 300 x
  * 28672 x 4096, kept nothing there once and do now): a program that overlaps calls asks, or uses the _ws forms.  For every other K >= 256 and every N they keep nothing outside their outputs: the matrix cores
  * without K slices where the rows are many enough for that, else matvecs; the _ws forms below with a workspace
- * slice K there and take the matrix cores where they end before the matvecs: from five rows on for the largest matrices, two
- * to three hundred for the smallest.  The _cfg entry never does. */
+ * slice K there and take the matrix cores where they end before the matvecs: from two to five rows on for large matrices, some tens for
+ * small ones, never for the smallest; a single row is a matvec.  There an f16 result is within the order of the f32 additions of the
+ * f32 form's, rounded, and of that of a call with its row alone: another kernel may have added.  The _cfg entry never does. */
 lhip_status lhip_q8_0_matmul_f32_gemm(const void *planar_dev, const float *x_dev, float *y_dev, int64_t m, int64_t n,
                                       int64_t k, void *stream);
 lhip_status lhip_q8_0_matmul_f16_gemm(const void *planar_dev, const void *x_f16_dev, void *y_f16_dev, int64_t m,

@@ -126,7 +126,7 @@ __global__ __launch_bounds__(kShortThreads) void attention_decode_short_kernel(
             }
         }
     }
-    // ---- rotary (adjacent pairs, as the rope operator: products rounded one by one)
+    // ---- rotary (adjacent pairs, the products rounded one by one; the operator of prompts, lhip_rope_kv_append_f32, fuses one of the two)
     if (tid < 2 * HD && (tid & 1) == 0) {
         const float2 sc = rope_sin_cos(theta, 2 * pj, HD, pos);
         const float sn = sc.x, cs = sc.y;

@@ -321,7 +321,7 @@ __device__ __forceinline__ void attention_decode_body(IO io, AttnShared<G, HD> &
     };
     if (on && k0 < k1) load_tile(k0);
 
-    // ---- rotary on the G query rows and the new key (adjacent pairs, as the rope operator), copy of the new value
+    // ---- rotary on the G query rows and the new key (adjacent pairs), copy of the new value
     if (on) {
         constexpr int NPAIR = (G + 1) * (HD / 2);
         constexpr int ITER = (NPAIR + kDecThreads - 1) / kDecThreads;
@@ -346,7 +346,7 @@ __device__ __forceinline__ void attention_decode_body(IO io, AttnShared<G, HD> &
                 const float2 sc = rope_sin_cos(theta, 2 * j, HD, pos);
                 const float sn = sc.x, cs = sc.y;
                 float *dst = r < G ? reinterpret_cast<float *>(sh.q_s[r]) : reinterpret_cast<float *>(sh.knew);
-                // products rounded one by one, as the rope operator of the graph does
+                // products rounded one by one (the operator of prompts, lhip_rope_kv_append_f32, fuses one of the two)
                 dst[2 * j] = __fsub_rn(__fmul_rn(xr[it].x, cs), __fmul_rn(xr[it].y, sn));
                 dst[2 * j + 1] = __fadd_rn(__fmul_rn(xr[it].x, sn), __fmul_rn(xr[it].y, cs));
             }

@@ -142,8 +142,8 @@ class Q8Weight:
 class QuantizedMatmul:
     """(.., M, K) x Q8_0 (N, K) -> (.., M, N) in the activation type T = f32 or f16, f32 accumulation either way
     (QuantizedMatmul<T>::process, crates/luminal_cuda/src/quantized.rs:116-168).  The library runs one matvec per
-    row or group of up to five rows, as the reference does per row, or, where that ends earlier (from three to six rows on for a K in steps
-    of 512, by cost for every other K), the matrix-core form with exact products (x as three bf16 limbs, an f16 x as two or as it
+    row or group of up to five rows, as the reference does per row, or, where that ends earlier (from four to six rows on for a K in steps
+    of 512, from two where K is so long that LDS holds few rows of it, by cost for every other K), the matrix-core form with exact products (x as three bf16 limbs, an f16 x as two or as it
     is), which streams the weights once per 64 or 128 rows.  A launch shape can be chosen for f32 only and always means the matvec form."""
 
     def __init__(self, rows_per_wave: int | None = None, k_unroll: int | None = None, blocks_per_cu: int = 0,

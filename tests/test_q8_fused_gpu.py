@@ -177,8 +177,7 @@ def test_one_weight_requests_two_steps_ahead_and_gives_the_grouped_launch_s_bits
             one, grouped, extra = (torch.full((r,), float("nan"), device=DEV) for r in (n, n, 3))
             FusedMatvec([w], [one], norm_weight=norm, eps=1e-5, cfg=cfg).run(x)
             FusedMatvec([w, other], [grouped, extra], norm_weight=norm, eps=1e-5, cfg=cfg or (1, 1, 4, 3)).run(x)
-            if norm is None or cfg is not None:  # (the sum of squares depends on the workgroup's size)
-                assert torch.equal(one, grouped)
+            assert torch.equal(one, grouped)
         added = torch.full((n,), float("nan"), device=DEV)
         FusedMatvec([w], [added], residual=res, epilogue=FusedMatvec.EPI_ADD, cfg=cfg).run(x)
         plain = torch.empty(n, device=DEV)
