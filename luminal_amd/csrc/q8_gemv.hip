@@ -653,6 +653,7 @@ static void choose_fused(int64_t n_total, bool grouped, int k, int pro, int epi,
     //   plain, K = 4096: 4096 rows 5.5 / 5.7 / 5.5 / 5.6, 6144 7.1 / 6.8 / 6.8 / 7.1, 12288 11.6 / 10.9 / 10.8 / 11.1
     //   K = 8192, norm and plain: 4096 rows 9.4 / 8.9 / 9.4 / 12.1 and 9.0 / 8.1 / 8.5 / 9.6
     //   K = 2048, norm: 4096 rows 4.7 / 4.8 / 4.8 / 4.6, 6144 5.5 / 5.6 / 5.6 / 5.5 (level)
+    // (the norm by eight waves 0.1 to 0.3 more since the squares are added up in the order of four)
     // A launch of several weights (grouped) has no early second step: with more than 4096 rows workgroups of four waves where those are not behind, eight waves
     // against three of four, 8192 + 1024 + 1024 rows of 6144 15.4 / 14.6 plain and 16.0 / 15.2 with the norm, of 8192 with the norm 19.4 / 21.1.
     // A fourth workgroup pays without the norm where a step is one slice (12288 rows of 5120 17.4 -> 15.8 us, of 7168 22.9 -> 20.9, of 9216 28.3 ->
