@@ -54,11 +54,12 @@ static GemvRowsShape rows_shape(int64_t m, int64_t n, int64_t k, bool f16) {
 // among them.  (Lines by (m - 1) n k and for every long ragged K: 1.2 to 1.4 %, and up to 30 % for small products, which matvecs a row take in, us,
 // 24 x 256 x 2880 f16 4.4 <- 5.6, 12 x 213 x 4096 4.5 <- 5.2, 2 x 2240 x 4096 4.6 <- 5.5.)  One row: where K is long, or its weight rows fill the
 // chip twice or do not once: 14336 x 4128 f32 19.7 -> 15.0, 644 x 13696 9.7 -> 6.7, 14168 x 8640 f16 30.7 -> 26.0, 1920 x 3936 f32 4.9 -> 4.5; the
-// other way 2380 x 5088 f32 6.6 <- 7.2, 3576 x 4704 f16 6.2 <- 6.7.  (4000 x 4608 f32 8.2 -> 7.5.)
+// other way 2380 x 5088 f32 6.6 <- 7.2, 3576 x 4704 f16 6.2 <- 6.7.  (4000 x 4608 f32 8.2 -> 7.5; 7084 x 3840 f16 7.6 <- 8.5,
+// 8316 x 3904 14.5 -> 9.1.)
 bool q8_gemv_rows_pays(int64_t m, int64_t n, int64_t k, bool f16) {
     if (q8_gemv_rows_per_pass(k, f16) == 0) return false;
     const bool ragged = k % 1024 != 0;
-    if (m == 1) return ragged && k > 1024 && (k > 5120 || n > (k <= 3072 ? 8200 : f16 ? 4100 : 3000) || (n <= 256 * kRowsWaves && k > (f16 ? 4096 : 3072)));
+    if (m == 1) return ragged && k > 1024 && (k > 5120 || n > (k <= (f16 ? 4096 : 3072) ? 8192 : f16 ? 4100 : 3000) || (n <= 256 * kRowsWaves && k > (f16 ? 4096 : 3072)));
     const int64_t further = (m - 1) * n;
     if (f16 && ragged && k <= 3072) return static_cast<double>(further) * static_cast<double>(k < 640 ? 640 : k) > (k <= 1024 ? 18e6 : 11e6);
     if (k <= 1024) return further > (f16 ? 7000 : 10000);

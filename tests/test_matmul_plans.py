@@ -68,7 +68,7 @@ def test_matvecs_of_a_long_k_take_several_rows_a_pass():
 
 def test_the_matvec_of_one_row_of_a_ragged_k():
     """The kernel of several rows also takes one where its waves have at most one weight row each (up to a seventh sooner), not for twice as many."""
-    for n, k, t, rows in ((160, 3552, "f32", 1), (1920, 3936, "f32", 1), (1141, 4608, "f16", 1), (2380, 5088, "f32", 0), (3576, 4704, "f16", 0), (4000, 4608, "f32", 1),
+    for n, k, t, rows in ((160, 3552, "f32", 1), (1920, 3936, "f32", 1), (1141, 4608, "f16", 1), (2380, 5088, "f32", 0), (3576, 4704, "f16", 0), (4000, 4608, "f32", 1), (7084, 3840, "f16", 0), (8316, 3904, "f16", 1),
                           (1920, 3040, "f32", 0), (1141, 4064, "f16", 0)):
         assert plan(1, n, k, t) == (MATVEC, rows, 1), (n, k, t)
 
