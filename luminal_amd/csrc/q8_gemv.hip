@@ -77,9 +77,9 @@ static double rows_sliced_us(int64_t m, int64_t n, int64_t k, bool f16) {
 // on.  Every other K from 256 on where the costs above say so: of 3086 random sizes of up to 512 rows the choice is 0.4 % (f32) and 0.3 %
 // (f16) behind the faster form on average, 1.3 and 1.6 % by the prices of a matvec a row and least rows by N K (5 x 14336 x 2880 f32 25.1 -> 16.9 us,
 // 6 x 6000 x 2880 14.7 -> 11.8, 12 x 10944 x 544 f16 19.1 -> 9.7); up to 1100 weight rows, whose estimates
-// spread most, the matrix cores have to be a fourteenth ahead, a quarter for up to 8 rows of x (8 x 1001 x 14336 f32: 19 us as matvecs, 16), beyond
-// them the matvecs a seventh for more than 32 rows of x, and for up to four the matrix cores (3 x 95540 x 544 f32 25.1 us as matvecs, 27.8).  A single row
-// is a matvec for any size.  A K below 256 is a matvec of one or two microseconds per row.
+// spread most, the matrix cores have to be a fourteenth ahead, a quarter for up to 8 rows of x (8 x 1001 x 14336 f32: 19 us as matvecs, 16). Beyond
+// them a ninth from 9 to 32 rows (mean loss of 9 to 12 f32 rows 1.4 -> 0.8 %: 11 x 1928 x 3648 10.5 as matvecs, 12.6), a sixth for up to four (3 x
+// 95540 x 544 f32 25.1, 27.8), and above 32 rows the matvecs a seventh.  A single row is a matvec for any size.  A K below 256 is a matvec of one or two microseconds per row.
 // f16 goes by the kernel that walks all of K, which keeps no planes, where that ends a tenth before the matvecs and is the matrix cores'
 // own choice: 2880 x 2880 at 12 rows 11.0 as matvecs, 7.9 there; 6000 x 1600 at 8 9.2 and 5.9, 23 x 4830 x 1024 13.9 and 6.1, 12 x 14336 x 544
 // 22.9 and 8.2.
@@ -93,7 +93,7 @@ static bool on_matrix_cores(int64_t m, int64_t n, int64_t k, const void *x, cons
     if (q8_gemm_split_supports(static_cast<int>(n), static_cast<int>(k), x, y, f16)) return m >= split_min_rows(n, k, f16);
     if (m == 1 || k < 256 || !aligned(x, 16)) return false;
     const double matvecs = matvecs_us(m, n, k, f16);
-    const bool sliced = rows_sliced_us(m, n, k, f16) < matvecs * (n <= 1100 ? (m <= 8 ? 0.75 : 0.93) : m > 32 ? 1.15 : m <= 4 ? 0.85 : 1.0);
+    const bool sliced = rows_sliced_us(m, n, k, f16) < matvecs * (n <= 1100 ? (m <= 8 ? 0.75 : 0.93) : m > 32 ? 1.15 : m > 8 ? 0.9 : m > 4 ? 1.0 : 0.85);
     if (room_floats == SIZE_MAX) return sliced;
     const bool deep = f16 && k >= 512 && q8_gemm_deep_supports(k, x) && q8_gemm_deep_plan(m, n, k, (matvecs - q8_gemm_deep_from_memory_us(n, k)) / 1.1).mt;
     const int64_t rounds = ((m + 127) / 128 * ((n + 255) / 256) + 255) / 256;

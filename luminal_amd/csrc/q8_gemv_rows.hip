@@ -49,20 +49,25 @@ static GemvRowsShape rows_shape(int64_t m, int64_t n, int64_t k, bool f16) {
 // The staging of the activations costs half a microsecond over a matvec a row, which further activation rows earn back by what is read
 // beyond the first one's weight rows or by the results there are, later for halves of a short ragged K, which the other kernel reads in
 // half the time; a ragged K from 3072 on it walks without a load ahead and is behind for any size, as it is for any K beyond 12288
-// (848 x 16384 f32 at two rows 11.2 -> 8.7 us, 280 x 14336 f16 at four 10.1 -> 7.2, 360 x 40960 at two 25 -> 14; at 12288 804 rows of f16 at two 6.9 ->
-// 6.5, 167 of f32 at three 6.1 <- 6.5).  Drawn over 10000 random sizes of K up to 14336 and of up to 512 rows: 0.3 (f32) and 0.5 % (f16) behind the faster kernel on average, weights from memory, 0.4 and 0.7 % with those from the cache
-// among them.  (Lines by (m - 1) n k and for every long ragged K: 1.2 to 1.4 %, and up to 30 % for small products, which matvecs a row take in, us,
-// 24 x 256 x 2880 f16 4.4 <- 5.6, 12 x 213 x 4096 4.5 <- 5.2, 2 x 2240 x 4096 4.6 <- 5.5.)  One row: where K is long, or its weight rows fill the
-// chip twice or do not once: 14336 x 4128 f32 19.7 -> 15.0, 644 x 13696 9.7 -> 6.7, 14168 x 8640 f16 30.7 -> 26.0, 1920 x 3936 f32 4.9 -> 4.5; the
-// other way 2380 x 5088 f32 6.6 <- 7.2, 3576 x 4704 f16 6.2 <- 6.7.  (4000 x 4608 f32 8.2 -> 7.5; 7084 x 3840 f16 7.6 <- 8.5,
-// 8316 x 3904 14.5 -> 9.1.)
+// (848 x 16384 f32 at two rows 11.2 -> 8.7 us, 280 x 14336 f16 at four 10.1 -> 7.2, 360 x 40960 at two 25 -> 14; at 12288 804 rows of f16 at
+// two 6.9 -> 6.5, 167 of f32 at three 6.1 <- 6.5).  Drawn over 10000 random sizes of K up to 14336 and of up to 512 rows: 0.3 (f32) and 0.5 % (f16)
+// behind the faster kernel on average, weights from memory, 0.4 and 0.7 % with those from the cache among them.  (Lines by (m - 1) n k and for
+// every long ragged K: 1.2 to 1.4 %, and up to 30 % for small products, which matvecs a row take in, us, 24 x 256 x 2880 f16 4.4 <- 5.6, 12 x 213 x
+// 4096 4.5 <- 5.2, 2 x 2240 x 4096 4.6 <- 5.5.)  A short f32 K whose weight rows fill the waves by themselves needs more further rows: 3 x 5195 x
+// 416 5.1 <- 6.1, 4 x 8020 x 512 7.9 -> 6.5; 4 x 2862 x 1024 5.5 -> 4.6.
+// One row: where K is long, or its weight rows fill the chip twice or do not once: 14336 x 4128 f32 19.7 -> 15.0, 644 x 13696 9.7 -> 6.7, 14168 x
+// 8640 f16 30.7 -> 26.0, 1920 x 3936 f32 4.9 -> 4.5, 4000 x 4608 f32 8.2 -> 7.5, 8316 x 3904 f16 14.5 -> 9.1; the other way 2380 x 5088 f32 6.6 <- 7.2,
+// 3576 x 4704 f16 6.2 <- 6.7, 7084 x 3840 f16 7.6 <- 8.5.
 bool q8_gemv_rows_pays(int64_t m, int64_t n, int64_t k, bool f16) {
     if (q8_gemv_rows_per_pass(k, f16) == 0) return false;
     const bool ragged = k % 1024 != 0;
-    if (m == 1) return ragged && k > 1024 && (k > 5120 || n > (k <= (f16 ? 4096 : 3072) ? 8192 : f16 ? 4100 : 3000) || (n <= 256 * kRowsWaves && k > (f16 ? 4096 : 3072)));
+    if (m == 1) {
+        const int long_k = f16 ? 4096 : 3072;
+        return ragged && k > 1024 && (k > 5120 || n > (k <= long_k ? 8192 : f16 ? 4100 : 3000) || (k > long_k && n <= 256 * kRowsWaves));
+    }
     const int64_t further = (m - 1) * n;
     if (f16 && ragged && k <= 3072) return static_cast<double>(further) * static_cast<double>(k < 640 ? 640 : k) > (k <= 1024 ? 18e6 : 11e6);
-    if (k <= 1024) return further > (f16 ? 7000 : 10000);
+    if (k <= 1024) return further > (f16 ? 7000 : k >= 640 ? 8000 : n > 4096 ? 20000 : 10000);
     return (ragged && k > 3072) || k > 12288 || m * n > (ragged ? 3100 : k >= 12288 ? 1200 : 2400);
 }
 

@@ -58,11 +58,12 @@ def test_f16_products_of_a_large_ragged_matrix_stay_with_k_slices():
         assert plan(*s, "f16", workspace=True)[0] == 4, s
 
 
-def test_matvecs_of_a_long_k_take_several_rows_a_pass():
-    """Whole slices of a K beyond 12288: a matvec a row was up to twice as slow there, by how few results there are (weights of any size)."""
-    for s, t in (((2, 360, 40960), "f16"), ((3, 512, 40960), "f32"), ((2, 848, 16384), "f32"), ((4, 280, 14336), "f16"), ((2, 804, 12288), "f16")):
+def test_matvecs_of_several_rows_a_pass_where_they_pay():
+    """Whole slices of a K beyond 12288, where a matvec a row was up to twice as slow; a short K by the further rows."""
+    for s, t in (((2, 360, 40960), "f16"), ((3, 512, 40960), "f32"), ((2, 848, 16384), "f32"), ((4, 280, 14336), "f16"), ((2, 804, 12288), "f16"),
+                 ((4, 2862, 1024), "f32"), ((4, 8020, 512), "f32")):
         assert plan(*s, t)[0] == MATVEC and plan(*s, t)[1] > 0, (s, t)
-    for s in ((3, 167, 12288), (2, 240, 4096)):
+    for s in ((3, 167, 12288), (2, 240, 4096), (3, 5195, 416)):
         assert plan(*s, "f32") == (MATVEC, 0, 1), s
 
 
@@ -87,7 +88,8 @@ def test_ragged_products_of_a_very_long_k():
     """Where matvecs take several passes over the weights, or LDS holds no row of their activations, K slices end up to 2.6 times sooner."""
     for s, t in (((3, 5796, 56672), "f32"), ((3, 1688, 52544), "f16"), ((3, 11448, 33696), "f16"), ((3, 18824, 14976), "f32")):
         assert plan(*s, t, workspace=True)[0] == ROWS_KERNEL, (s, t)
-    for s, t in (((3, 6808, 22592), "f16"), ((2, 16514, 34464), "f32"), ((3, 95540, 544), "f32"), ((3, 29325, 7680), "f16")):
+    for s, t in (((11, 1928, 3648), "f32"), ((3, 6808, 22592), "f16"), ((2, 16514, 34464), "f32"), ((3, 95540, 544), "f32"),
+                 ((3, 29325, 7680), "f16")):
         assert plan(*s, t, workspace=True)[0] == MATVEC, (s, t)
     for s in ((8, 27324, 10368), (6, 16272, 30336)):  # (weights beyond any cache: what they cost from memory is in the estimates of both)
         assert plan(*s, "f16", workspace=True)[0] == 4, s
