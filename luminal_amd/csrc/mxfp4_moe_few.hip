@@ -274,20 +274,24 @@ static double few_tiles(int T, int E, int topk) {
 
 // Column blocks a workgroup walks.  Two workgroups are resident a CU; with as many as one round of them takes, requests never stop, and
 // five (32 columns: six) are the most, beyond which workgroups of few tiles leave the CUs at different times.  Where the blocks of all
-// expected tiles are about one to four a CU, the number with which the fullest CU walks the fewest: between, some CUs have twice the
-// work of others.
+// expected tiles are up to six a CU, the number of at most three with which the fullest CU walks the fewest, half a block counted for each
+// of its workgroups: of 1080 launches (760 layers of 4 to 64 experts, up to 6144 wide, T = 1 to 8) 1.0 % behind the best number on average.
 // Measured, us a layer by (gate|up, down) blocks, 32 experts of 2880 x 2880, top 4: T = 2 (3, 3) 29.2, (5, 3) 32.4, (2, 1) 33.6; T = 4 (5, 3) 41.6,
-// (3, 3) 43.9, (12, 6) 42.5; T = 8 (5, 5) 59.2, (3, 1) 69.5; T = 16 (5, 6) 73.1, (3, 3) 79.9, (8, 4) 83.8.  By the fullest CU: four tiles of
-// 4096 x 4096, gate|up in 2 / 3 / 4 blocks 27.7 / 30.0 / 27.8, of 3584 27.5 / 30.0 / 27.2, of 2880 22.9 / 21.9 / 22.6; eight of 4096, down 44.4 / 46.6 /
-// 44.4 (three blocks at least were taken before).
+// (3, 3) 43.9, (12, 6) 42.5; T = 8 (5, 5) 59.2, (3, 1) 69.5; T = 16 (5, 6) 73.1, (3, 3) 79.9, (8, 4) 83.8.  By the fullest CU, gate|up in 1 / 2 / 3 /
+// 4 blocks: four tiles of 4096 x 4096 - / 27.7 / 30.0 / 27.8, of 3840 x 2240 (three) 18.5 / 17.7 / 19.2 / 20.3, of 2880 - / 22.9 / 21.9 / 22.6, of 3392 x 896
+// 12.8 / 14.1 / 15.0 / 16.4.
 static int few_blocks(const MoeFewLayer &l, int all, int most) {
     const double tiles = few_tiles(l.T, l.E, l.topk), units = tiles * all;
-    if (units <= 1100.0) {
+    if (units <= 1500.0) {
         int blocks = 1;
         double least = 1e30;
-        for (int b = 1; b <= 4; ++b) {
-            const double turns = b * ceil(tiles * ((all + b - 1) / b) / 256.0 - 0.05);
-            if (turns <= least) least = turns, blocks = b;
+        const int whole = static_cast<int>(tiles);
+        const double more = tiles - whole;
+        for (int b = 1; b <= 3; ++b) {
+            const int columns = (all + b - 1) / b;
+            auto turns = [&](int n) { return (b + 0.5) * ((n * columns + 255) / 256); };  // of n tiles
+            const double expected = (1.0 - more) * turns(whole) + more * turns(whole + 1);
+            if (expected < least) least = expected, blocks = b;
         }
         return blocks;
     }
