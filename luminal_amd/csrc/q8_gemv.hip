@@ -660,20 +660,36 @@ static void choose_fused(int64_t n_total, bool grouped, int k, int pro, int epi,
     // against three of four, 8192 + 1024 + 1024 rows of 6144 15.4 / 14.6 plain and 16.0 / 15.2 with the norm, of 8192 with the norm 19.4 / 21.1.
     // A fourth workgroup pays without the norm where a step is one slice (12288 rows of 5120 17.4 -> 15.8 us, of 7168 22.9 -> 20.9, of 9216 28.3 ->
     // 26.2, of 3072 10.1 -> 9.7) and for groups of 6144 (12288 rows 17.0 -> 16.3); of 10240 and more 3 % behind, of 8192 3.5 %.
-    // Sixteen waves behind the norm add up the squares in 0.9 us: 1024 rows of 14336 12.0 us, two workgroups of four waves 8.8, from 4096 rows
-    // on 15.3 and 17.1.
-    const bool eight = *sl == 2 && k > 4096 && k <= 8192;
-    if (eight && (!grouped || n_total <= 4096 || (pro == PRO_NORM && (k == 8192 || n_total <= 6144)))) {
+    // Sixteen waves behind the norm add up the squares in 0.9 us, so that fewer are ahead there, us, two workgroups of four with one and with two
+    // rows a wave / one of eight with two / one of sixteen with one: K = 14336 1000 rows 8.8 / 9.2 / 10.7 / 11.9, 2000 11.9 / 10.4 / 11.8 / 12.7, 3100 16.6 / 14.5 /
+    // 13.4 / 14.2, 12000 36.4 / 35.6 / 33.7 / 34.2; K = 16384 the same up to 4096 rows, 5000 22.5 / 23.4 / 24.9 / 24.7, 9000 33.6 / 34.1 / 36.9 / 36.9; K = 15360
+    // one weight of 2000 rows 15.2 / 14.3 / 14.8 / 13.6, 2048 rows of three weights 15.3 / 14.2 / 14.8 / 16.0.
+    // SwiGLU of up to 2048 rows behind the norm, one of eight waves / two of four: K = 6144 700 rows 6.4 / 5.7, 2000 6.65 / 6.2, 3000 7.0 / 7.4, K = 8192 700
+    // rows 7.2 / 6.4; of more than 4096 of K = 16384 5000 rows 25.1 / 22.8, 14000 49.9 / 46.7.
+    // Several weights of 6144, three of four / one of eight: 700 rows together 5.1 / 5.2 plain and 5.3 / 5.9 with the norm, 2048 5.8 / 5.6, 2346 6.2 / 6.9, 3072
+    // 6.8 / 7.3, 4096 8.2 / 7.9; of 8192 700 rows 5.3 / 5.6, 2048 6.8 / 6.4, 2346 7.9 / 8.6, 4096 9.8 / 9.5.  Plain SwiGLU of 8192 300 rows 6.0 by eight waves, 5.6.
+    // One weight of 6144, plain, three of four / one of eight: 19300 rows 23.6 / 24.1, 14000 17.9 / 18.4, 12000 16.2 either way.
+    const bool norm = pro == PRO_NORM;
+    bool eight = *sl == 2 && k > 4096 && k <= 8192;
+    if (pairs)
+        eight = eight && n_total > (norm ? 2048 : 1024);
+    else if (grouped)
+        eight = eight && n_total > 1024 && (norm ? k == 8192 || n_total <= 6144 : n_total <= 2048 || (n_total > 3072 && n_total <= 4096));
+    else if (k == 6144 && !norm)
+        eight = eight && n_total <= 12288;
+    if (eight) {
         *r = pairs ? 2 : 1, *w = 8, *bpc = 1;
-    } else if (*sl == 2 && k == 4096 && pro == PRO_NORM && n_total >= 2048) {
+    } else if (*sl == 2 && k == 4096 && norm && n_total >= 2048) {
         *r = pairs || n_total <= 6144 ? 2 : 1, *w = n_total <= 6144 ? 4 : 8, *bpc = 1;
     } else if (*sl == 2 && k == 4096 && !pairs && !grouped && n_total > 4096) {
         *r = 1, *w = 8, *bpc = 2;
     } else if (fit >= 3) {
         const bool four = pro == PRO_NONE && n_total > 4096 && fit >= 4 && (*sl == 1 || (k > 4096 && k < 8192));
         *r = pairs ? 2 : 1, *w = 4, *bpc = pairs ? 2 : four ? 4 : 3;
-    } else if (pro == PRO_NORM && n_total <= 2048) {
-        *r = pairs ? 2 : 1, *w = 4, *bpc = 2;
+    } else if (norm && (n_total <= (*sl == 2 || grouped || pairs ? 2048 : 1024) || (k == 16384 && !grouped && epi != EPI_ADD && n_total > 4096))) {
+        *r = pairs || (n_total > 1024 && n_total <= 2048) ? 2 : 1, *w = 4, *bpc = 2;
+    } else if (norm && *sl == 2 && epi != EPI_ADD) {
+        *r = 2, *w = 8, *bpc = 1;
     } else {
         *r = pairs ? 2 : 1, *w = pairs ? 8 : 16, *bpc = 1;
     }

@@ -185,7 +185,7 @@ def test_one_weight_requests_two_steps_ahead_and_gives_the_grouped_launch_s_bits
         assert torch.equal(added, plain + res)
 
 
-@pytest.mark.parametrize("n,k", [(7, 1024), (1030, 3072), (300, 13312), (4100, 16384)])
+@pytest.mark.parametrize("n,k", [(7, 1024), (1030, 3072), (300, 13312), (4100, 16384), (1501, 14336), (3001, 14336), (1030, 15360)])
 def test_norm_does_not_depend_on_the_workgroup_s_size(n, k):
     """The sum of squares is that of four waves in workgroups of four, eight and sixteen, for one weight and for several."""
     w, _ = make(n, k, n + k)
